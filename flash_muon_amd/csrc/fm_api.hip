@@ -159,6 +159,8 @@ size_t fm_syrk_workspace_bytes(int M, int K) {
   return p.total > plain ? p.total : plain;
 }
 
+size_t fm_syrk_f32_workspace_bytes(int M, int K) { return M <= 0 || K <= 0 ? 0 : syrk_f32_workspace_bytes(M, K); }
+
 static int syrk_impl(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64_t ldy_col, int M, int K,
                      void* ws, size_t ws_bytes, fm_stream_t stream, int elem, bool may_pad = true) {
   if (M < 0 || K < 0) return FM_ERR_SHAPE;
@@ -185,13 +187,16 @@ static int syrk_impl(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64
     if (K > 0 && overlaps(mat_range(X, M, K, ldx, es), y)) return FM_ERR_ALIAS;
   }
   hipStream_t hs = static_cast<hipStream_t>(stream);
+  if (elem == kElemF32)
+    return hip_status(launch_syrk_f32(static_cast<const float*>(X), ldx, static_cast<float*>(Y), ldy_row, ldy_col, M, K,
+                                      usable_ws(ws), ws_bytes, hs));
   GemmArgs a = {};
   a.E = nullptr; a.lde = 0;
   a.alpha = 0.0f; a.beta = 1.0f; a.symmetric = 1; a.elem = elem;
   SyrkPad p;
   // Y is symmetric, so a unit stride in either direction makes its lines rows for the copy out
   const int64_t ldy = ldy_col == 1 ? ldy_row : ldy_row == 1 ? ldy_col : 0;
-  if (may_pad && elem != kElemF32 && ldy >= M && usable_ws(ws) && syrk_pad_layout(M, K, &p) && ws_bytes >= p.total &&
+  if (may_pad && ldy >= M && usable_ws(ws) && syrk_pad_layout(M, K, &p) && ws_bytes >= p.total &&
       !overlaps(mat_range(X, M, K, ldx, es), Range{reinterpret_cast<uintptr_t>(ws), reinterpret_cast<uintptr_t>(ws) + p.total}) &&
       !overlaps(mat_range(Y, M, M, ldy, es), Range{reinterpret_cast<uintptr_t>(ws), reinterpret_cast<uintptr_t>(ws) + p.total})) {
     unsigned char* w = static_cast<unsigned char*>(ws);

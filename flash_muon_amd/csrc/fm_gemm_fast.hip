@@ -1945,7 +1945,7 @@ static void fast_schedule(int num_tiles, int nk, long long max_slots, FastArgs& 
 // what both tile shapes ask of a problem: whole tiles of edge `tile`, whole k stages, 16-byte
 // accesses everywhere
 static bool tiled_dma_eligible(const GemmArgs& a, int tile) {
-  if (a.elem == kElemF32 || (a.elem == kElemF16 && a.E)) return false;
+  if (a.elem == kElemF16 && a.E) return false;
   if (a.Kc < BKF || a.Kc % BKF != 0) return false;
   if (a.lda % 8 != 0 || a.ldb % 8 != 0) return false;
   if ((reinterpret_cast<uintptr_t>(a.A) & 15) || (reinterpret_cast<uintptr_t>(a.B) & 15)) return false;

@@ -71,8 +71,7 @@ template <bool F16> __device__ __forceinline__ float elem_to_f32(unsigned short 
 //     if diag_out and i == j:  diag_out[i] = v (fp32) and v = 0
 //     C [i*c_rs  + j*c_cs ] = round(v)               (if C  != nullptr)
 //     C2[j*c2_rs + i*c2_cs] = round(v)               (if C2 != nullptr; the mirrored copy)
-// A, B, E, C and C2 hold bf16; without E they may hold fp16 or fp32 instead (`elem`; pointers stay
-// typed bf16_t, leading dimensions and strides stay in elements).
+// A, B, E, C and C2 hold bf16; without E they may hold fp16 instead (`elem`; pointers stay typed bf16_t).
 // With `symmetric` set, A == B, only tiles on or above the diagonal are computed and C2 == C.
 struct GemmArgs {
   const bf16_t* A;  int64_t lda;
@@ -86,7 +85,7 @@ struct GemmArgs {
   const float* row_alpha;   // optional per-row addition to alpha
   float* diag_out;          // optional fp32 copy of the diagonal, which is then stored as zero
   int symmetric;
-  int elem;                 // element type of A, B, C, C2: kElemBf16, kElemF16, or kElemF32 (general path only)
+  int elem;                 // element type of A, B, C, C2: kElemBf16 or kElemF16
   // `batch` independent problems of the same shape in one launch: matrix b of an operand starts
   // b * stride elements after matrix 0 (strides of absent operands are ignored)
   int batch;
@@ -120,6 +119,11 @@ __host__ __device__ inline GemmArgs batch_view(const GemmArgs& g, int b) {
 // Returns a hipError_t value.
 int launch_gemm_nt(GemmArgs args, void* ws, size_t ws_bytes, hipStream_t stream);
 int launch_gemm_general(GemmArgs args, hipStream_t stream);
+// Y = X X^T in fp32 (fm_gemm_f32.hip), any shape, strides and alignment; without a workspace of
+// syrk_f32_workspace_bytes the tiles stay whole
+size_t syrk_f32_workspace_bytes(int M, int K);
+int launch_syrk_f32(const float* X, int64_t ldx, float* Y, int64_t rs, int64_t cs, int M, int K, void* ws,
+                    size_t ws_bytes, hipStream_t stream);
 bool gemm_fast_eligible(const GemmArgs& a);
 // bytes of fp32 partial tiles the 256x256 path can need for `batch` Ma x Nb outputs, whatever k is
 // (0 when no schedule of this shape cuts a tile)

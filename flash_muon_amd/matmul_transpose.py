@@ -47,7 +47,7 @@ def matmul_transpose_assign(d_in, d_out):
         dst = torch.empty((M, M), device=d_in.device, dtype=d_in.dtype)
     with _lib.on_device(d_in.device):
         stream = _lib.stream_ptr(d_in.device)
-        need = 0 if d_in.dtype == torch.float32 else lib.fm_syrk_workspace_bytes(M, K)
+        need = (lib.fm_syrk_f32_workspace_bytes if d_in.dtype == torch.float32 else lib.fm_syrk_workspace_bytes)(M, K)
         ws, ws_bytes = _lib.gemm_workspace(need, d_in.device, stream)
         st = getattr(lib, entry)(d_in.data_ptr(), ldx, dst.data_ptr(),
                                  dst.stride(0) if M > 1 else M, dst.stride(1) if M > 1 else 1,

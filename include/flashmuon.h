@@ -84,7 +84,7 @@ FM_API int fm_set_knob(int knob, long long value);
 
 /* ---------------------------------------------------------------------------------------------
  * Scratch for the three GEMM-shaped entry points below, by the shape of their OUTPUT: (M, M) for
- * fm_syrk_bf16, fm_syrk_f16, fm_syrk_f32 and fm_syrk_poly_bf16, (M, K) for fm_gemm_axpby_bf16.  It holds the
+ * fm_syrk_bf16, fm_syrk_f16 and fm_syrk_poly_bf16, (M, K) for fm_gemm_axpby_bf16.  It holds the
  * fp32 partial tiles of output tiles whose k range is split over several workgroups: 256 KiB per
  * part, at most 256 parts (64 MiB) when the output has more 256x256 tiles than the GPU has CUs,
  * at most 768 (192 MiB) below that; 16 MiB (256 parts of 64 KiB) for outputs of at most 128 tiles
@@ -148,8 +148,12 @@ FM_API int fm_syrk_f16(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int
                 int M, int K, void* ws, size_t ws_bytes, fm_stream_t stream);
 
 /* The same product for fp32 X and Y, on fp32 MFMA (32x32x2): fp32 products and accumulation, no
- * rounding of the result.  Runs on the general tiled schedule for every shape; ws is not used.
+ * rounding of the result.  Every shape, stride and alignment runs on 64x64 tiles; with a workspace of
+ * fm_syrk_f32_workspace_bytes (0 or 16 MiB) the tiles left after the last full round are shared out
+ * evenly over the GPU, as fp32 parts that a second kernel adds up in k order; without one they stay
+ * whole, which is slower.
  */
+FM_API size_t fm_syrk_f32_workspace_bytes(int M, int K);
 FM_API int fm_syrk_f32(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64_t ldy_col,
                 int M, int K, void* ws, size_t ws_bytes, fm_stream_t stream);
 
