@@ -29,11 +29,15 @@ inline void* usable_ws(void* ws) { return (reinterpret_cast<uintptr_t>(ws) % 256
 // workspace of fm_newtonschulz_batched_bf16, carved in this order; per-matrix arrays are
 // batch-major with the strides below
 struct NsLayout {
-  size_t sumsq, partials, pdiag, x[2], xt[2], a, p, gemm, total;
+  size_t partials, pdiag, x[2], xt[2], a, p, gemm, total;
   size_t pdiag_stride;   // floats between the fp32 diagonals of consecutive matrices
   int M, K;              // the sizes the iteration runs on: those of the matrix, or padded (below)
   bool padded;
+  int edge_s, edge_x;    // tiles of the one-launch iteration
+  bool flow;             // one launch for all products: x[0], a and p hold kFlowSteps (+ 1) iterates and squares
+  size_t counters;
 };
+constexpr int kFlowSteps = 5;   // steps per launch of the one-launch iteration
 // A matrix whose sides are not whole 128-tiles would take the general GEMM path in every stage
 // (0.5-0.8 times the vendor GEMMs).  Its iterates live in the workspace anyway, so they are kept
 // zero-padded to whole tiles instead: zero rows and columns stay zero through every step, and the
@@ -51,10 +55,52 @@ static int ns_pad(int n) {
   if (p >= kPad256From && p % 256 != 0) p += 128;
   return p;
 }
+// Which matrices iterate in one launch (fm_flow.hip), and on which tiles: M x K with M <= K, `batch` of them.
+// Five steps in us, one launch / launches per product: 256^2 91 / 109, 512 x 2048 133 / 154, 768^2 121 / 146,
+// 1024^2 137 / 158, 24 of 768^2 360 / 393, 8 of 1024 x 2816 593 / 705, 16 of 768 x 3072 649 / 967.  The launches per
+// product win where the 256x256 tiles fill the GPU by themselves (24 of 2048^2 4600 / 4200, 1536^2 288 / 254), and for
+// few matrices with a long side, whose first product they cut along k (1024 x 4096 267 / 228, 4 of 1024 x 2048
+// 313 / 297, 1280 x 5120 385 / 304).
+bool ns_flow_chosen(int batch, int m, int k) {
+  const double r = (double)k / m;
+  if (k >= (1 << 21)) return false;   // in-tile byte offsets stay below 2^31
+  if (m <= 512) return true;
+  if (m <= 1024) return r <= 1.5 || batch >= 8 || (r <= 2.25 && batch <= 2);
+  if (m <= 1280) return batch >= 12 || (batch == 1 && r <= 2.25) || (batch == 2 && r <= 1.5);
+  return false;
+}
+// 64x64 tiles for X' as long as every CU gets at most one, and for the symmetric products as long as they are
+// about one round (a longer K makes the 64-tiles of A = X X^T pay a little further): 512^2 104 us on 64x64
+// tiles, 115 with X' on 128x128, 144 all on 128x128; 8 of 384 x 768 152, 111 and 133; 24 of 768^2 520, 423 and 360.
+void ns_flow_edges(int batch, int m, int k, int* es, int* ex) {
+  const int64_t t = (m + 63) / 64, sym = t * (t + 1) / 2 * batch, rect = t * ((k + 63) / 64) * batch;
+  *ex = rect <= 256 ? 64 : 128;
+  *es = rect <= 256 || sym <= 256 || (sym <= 440 && k >= 2 * m) ? 64 : 128;
+}
 NsLayout ns_layout(int batch, int rows, int cols) {
   const int m = rows < cols ? rows : cols, k = rows < cols ? cols : rows;
   const size_t B = (size_t)batch;
-  NsLayout l;
+  NsLayout l = {};
+  if (ns_flow_chosen(batch, m, k)) {
+    l.flow = true;
+    ns_flow_edges(batch, m, k, &l.edge_s, &l.edge_x);
+    l.M = (m + l.edge_x - 1) / l.edge_x * l.edge_x;
+    l.K = (k + l.edge_x - 1) / l.edge_x * l.edge_x;
+    l.padded = l.M != m || l.K != k;
+    size_t off = 0;
+    auto take = [&](size_t bytes) { size_t o = off; off += align_up(bytes, 256); return o; };
+    const size_t M = (size_t)l.M, K = (size_t)l.K;
+    l.partials = take(B * kSumsqBlocks * sizeof(float));
+    l.pdiag_stride = M;
+    l.pdiag = take(B * M * kFlowSteps * sizeof(float));
+    l.x[0] = take(B * M * K * 2 * (kFlowSteps + 1));
+    l.a = take(B * M * M * 2 * kFlowSteps);
+    l.p = take(B * M * M * 2 * kFlowSteps);
+    l.counters = take((size_t)flow_counter_words(batch, kFlowSteps) * sizeof(unsigned));
+    l.gemm = off;
+    l.total = off;
+    return l;
+  }
   l.M = (m + 127) / 128 * 128;
   l.K = (k + 127) / 128 * 128;
   {
@@ -67,7 +113,6 @@ NsLayout ns_layout(int batch, int rows, int cols) {
   const size_t M = (size_t)l.M, K = (size_t)l.K;
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off += align_up(bytes, 256); return o; };
-  l.sumsq = take(B * 64 * sizeof(float));                 // one float per matrix, 256 bytes apart
   l.partials = take(B * kSumsqBlocks * sizeof(float));
   l.pdiag_stride = align_up(M, 64);
   l.pdiag = take(B * l.pdiag_stride * sizeof(float));
@@ -372,13 +417,48 @@ int fm_newtonschulz_batched_bf16(const void* const* G, int dtype, int batch, int
   }
 
   unsigned char* w = static_cast<unsigned char*>(ws);
+  if (l.flow && steps > 0) {
+    hipStream_t hs = static_cast<hipStream_t>(stream);
+    const bool tall = rows > cols;
+    float* sumsq = reinterpret_cast<float*>(w + l.partials);
+    const int parts = sumsq_parts((int64_t)rows * cols);
+    unsigned* counters = reinterpret_cast<unsigned*>(w + l.counters);
+    const int n_counters = flow_counter_words(batch, steps < kFlowSteps ? steps : kFlowSteps);
+    const int64_t mk = (int64_t)l.M * l.K;
+    bf16_t* X = reinterpret_cast<bf16_t*>(w + l.x[0]);
+    if (launch_sumsq_parts_batched(G, batch, dtype, rows, cols, ldg, sumsq, hs, counters, n_counters)) return FM_ERR_LAUNCH;
+    bf16_t* x[kMaxBatch];
+    for (int i = 0; i < batch; ++i) x[i] = X + i * mk;
+    if (launch_scale_cast_batched(G, batch, dtype, rows, cols, ldg, sumsq, parts, eps, tall ? nullptr : x, l.K, tall ? x : nullptr, l.K,
+                                  hs, tall ? l.K : l.M, tall ? l.M : l.K))
+      return FM_ERR_LAUNCH;
+    FlowProblem f = {};
+    f.X = X; f.x_step = batch * mk;
+    f.A = reinterpret_cast<bf16_t*>(w + l.a); f.P = reinterpret_cast<bf16_t*>(w + l.p); f.a_step = (int64_t)batch * l.M * l.M;
+    f.pdiag = reinterpret_cast<float*>(w + l.pdiag); f.d_step = (int64_t)batch * l.pdiag_stride; f.d_mat = (int64_t)l.pdiag_stride;
+    f.M = l.M; f.K = l.K; f.batch = batch; f.edge_s = l.edge_s; f.edge_x = l.edge_x;
+    f.a = a; f.b = b; f.c = c;
+    f.counters = counters;
+    for (int s = 0; s < steps; s += kFlowSteps) {
+      f.steps = steps - s < kFlowSteps ? steps - s : kFlowSteps;
+      const bool last = s + f.steps == steps;
+      // what is not the last launch leaves its result in the slot behind its own, from where the next one
+      // goes the other way
+      void* o[kMaxBatch];
+      for (int i = 0; i < batch; ++i) o[i] = last ? out[i] : (void*)(f.X + f.steps * f.x_step + i * mk);
+      f.out = o;
+      f.ldout = last ? ldout : l.K;
+      f.rows = last ? rows : l.M; f.cols = last ? cols : l.K; f.tall = last && tall;
+      if (s > 0 && launch_zero_words(counters, n_counters, hs)) return FM_ERR_LAUNCH;
+      if (launch_ns_flow(f, hs)) return FM_ERR_LAUNCH;
+      f.X += f.steps * f.x_step;
+      f.x_step = -f.x_step;
+    }
+    return FM_OK;
+  }
   void* gws = w + l.gemm;
   const size_t gws_bytes = l.total - l.gemm;
   hipStream_t hs = static_cast<hipStream_t>(stream);
-  // the last 256 bytes of the GEMM scratch hold the ticket word of the sub-tile rounds: whatever the
-  // caller's memory held there could pass for a launch number no launch ever reaches (the products
-  // would still be right, on the fixed assignment of sub-tiles), so it starts from zero
-  if (steps > 0 && gws_bytes >= 256 && launch_zero_words(w + l.total - 256, 32, hs)) return FM_ERR_LAUNCH;
   const bool tall = rows > cols;
   const bool padded = l.padded && steps > 0;
   const int M = padded ? l.M : (tall ? cols : rows), K = padded ? l.K : (tall ? rows : cols);
@@ -389,12 +469,16 @@ int fm_newtonschulz_batched_bf16(const void* const* G, int dtype, int batch, int
   bf16_t* X = reinterpret_cast<bf16_t*>(w + l.x[0]);
   bf16_t* XT = reinterpret_cast<bf16_t*>(w + l.xt[0]);
   {
-    // Frobenius norms, then the scaled bf16 cast in both orientations: one launch each for the batch
-    float* sumsq = reinterpret_cast<float*>(w + l.sumsq);
-    float* partials = reinterpret_cast<float*>(w + l.partials);
-    for (int i = 0; i < batch; ++i)
-      if (misaligned(G[i], dtype_size(dtype))) return FM_ERR_ALIGN;
-    if (launch_sumsq_batched(G, batch, dtype, rows, cols, ldg, sumsq, 64, partials, hs)) return FM_ERR_LAUNCH;
+    // Frobenius norms (partial sums), then the scaled bf16 cast in both orientations: one launch each for the
+    // batch.  The last 256 bytes of the GEMM scratch hold the ticket word of the sub-tile rounds: whatever
+    // the caller's memory held there could pass for a launch number no launch ever reaches (the products
+    // would still be right, on the fixed assignment of sub-tiles), so it starts from zero.
+    float* sumsq = reinterpret_cast<float*>(w + l.partials);
+    const int parts = sumsq_parts((int64_t)rows * cols);
+    const bool word = steps > 0 && gws_bytes >= 256;
+    if (launch_sumsq_parts_batched(G, batch, dtype, rows, cols, ldg, sumsq, hs,
+                                   word ? reinterpret_cast<unsigned*>(w + l.total - 256) : nullptr, word ? 64 : 0))
+      return FM_ERR_LAUNCH;
     bf16_t* d[kMaxBatch];
     bf16_t* t[kMaxBatch];
     for (int i = 0; i < batch; ++i) {
@@ -404,7 +488,7 @@ int fm_newtonschulz_batched_bf16(const void* const* G, int dtype, int batch, int
     }
     const int64_t ldd = steps == 0 ? ldout : (!tall ? K : M), ldt = !tall ? M : K;
     // with padding: G's orientation is (tall ? K x M : M x K) there, and what lies beyond G is zeroed
-    if (launch_scale_cast_batched(G, batch, dtype, rows, cols, ldg, sumsq, 64, eps, d, ldd,
+    if (launch_scale_cast_batched(G, batch, dtype, rows, cols, ldg, sumsq, parts, eps, d, ldd,
                                   steps == 0 ? nullptr : t, ldt, hs, padded ? (tall ? K : M) : rows,
                                   padded ? (tall ? M : K) : cols))
       return FM_ERR_LAUNCH;

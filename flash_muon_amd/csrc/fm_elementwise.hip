@@ -51,13 +51,17 @@ __device__ __forceinline__ float block_sum(float v, float* red /* NT/64 floats o
 // ---- sum of squares -----------------------------------------------------------------------------
 // blockIdx.y is the matrix of a batch: its pointer comes from the list, its partial sums go to its
 // own run of gridDim.x floats
+// `zero`: n_zero words that the kernels behind this one want cleared (counters of the caller's workspace), done
+// here by the blocks of the first matrix rather than by a launch of its own
 template <int DT, bool FLAT_VEC>
 __global__ __launch_bounds__(256) void sumsq_partial_kernel(PtrList Gl, int rows, int cols,
-                                                            int64_t ldg, float* partials) {
+                                                            int64_t ldg, float* partials, unsigned* zero, int n_zero) {
   typedef typename Elem<DT>::raw raw;
   __shared__ float red[4];
   const void* Gv = Gl.p[blockIdx.y];
   partials += (size_t)blockIdx.y * gridDim.x;
+  if (blockIdx.y == 0)
+    for (int i = (int)blockIdx.x * 256 + (int)threadIdx.x; i < n_zero; i += (int)gridDim.x * 256) zero[i] = 0u;
   const raw* G = reinterpret_cast<const raw*>(Gv);
   const int64_t n = (int64_t)rows * cols;
   float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
@@ -99,8 +103,14 @@ __global__ __launch_bounds__(256) void sumsq_final_kernel(const float* partials,
   if (threadIdx.x == 0) out[0] = s;
 }
 
-int launch_sumsq_batched(const void* const* G, int batch, int dtype, int rows, int cols, int64_t ldg,
-                         float* out, int out_stride, float* partials, hipStream_t stream) {
+// Blocks, and so partial sums, per matrix: about 2048 elements each, kSumsqBlocks at most.
+int sumsq_parts(int64_t n) {
+  const int64_t b = (n + 2047) / 2048;
+  return b < 1 ? 1 : b > kSumsqBlocks ? kSumsqBlocks : (int)b;
+}
+
+int launch_sumsq_parts_batched(const void* const* G, int batch, int dtype, int rows, int cols, int64_t ldg,
+                               float* partials, hipStream_t stream, unsigned* zero, int n_zero) {
   const int64_t n = (int64_t)rows * cols;
   const int esz = dtype == 2 ? 4 : 2;
   bool flat = (ldg == cols) && (n % (16 / esz) == 0);
@@ -109,22 +119,24 @@ int launch_sumsq_batched(const void* const* G, int batch, int dtype, int rows, i
     gl.p[i] = const_cast<void*>(G[i]);
     flat = flat && ((reinterpret_cast<uintptr_t>(G[i]) & 15) == 0);
   }
-  dim3 grid(kSumsqBlocks, (unsigned)batch), block(256);
+  dim3 grid((unsigned)sumsq_parts(n), (unsigned)batch), block(256);
 #define FM_SUMSQ(DT)                                                                               \
   if (flat) hipLaunchKernelGGL((sumsq_partial_kernel<DT, true>), grid, block, 0, stream, gl, rows, \
-                               cols, ldg, partials);                                               \
+                               cols, ldg, partials, zero, n_zero);                                 \
   else hipLaunchKernelGGL((sumsq_partial_kernel<DT, false>), grid, block, 0, stream, gl, rows,     \
-                          cols, ldg, partials);
+                          cols, ldg, partials, zero, n_zero);
   if (dtype == 0) { FM_SUMSQ(0) } else if (dtype == 1) { FM_SUMSQ(1) } else { FM_SUMSQ(2) }
 #undef FM_SUMSQ
-  hipLaunchKernelGGL(sumsq_final_kernel, dim3((unsigned)batch), dim3(256), 0, stream,
-                     (const float*)partials, kSumsqBlocks, out, out_stride);
   return (int)hipGetLastError();
 }
 
 int launch_sumsq(const void* G, int dtype, int rows, int cols, int64_t ldg, float* out,
                  float* partials, hipStream_t stream) {
-  return launch_sumsq_batched(&G, 1, dtype, rows, cols, ldg, out, 0, partials, stream);
+  const int rc = launch_sumsq_parts_batched(&G, 1, dtype, rows, cols, ldg, partials, stream, nullptr, 0);
+  if (rc) return rc;
+  hipLaunchKernelGGL(sumsq_final_kernel, dim3(1), dim3(256), 0, stream, (const float*)partials,
+                     sumsq_parts((int64_t)rows * cols), out, 0);
+  return (int)hipGetLastError();
 }
 
 // 16-byte accesses of data that is touched once per call: marked non-temporal, so that the stream
@@ -143,10 +155,18 @@ __device__ __forceinline__ void st_stream(void* p, uint4 v) {
 // One 64x64 tile of G per block: D gets the tile in place, T gets it transposed through LDS.
 // D is rows_p x cols_p and T cols_p x rows_p with rows_p >= rows, cols_p >= cols: what lies beyond
 // G in them is written as zero.
-// blockIdx.z is the matrix of a batch (pointers from the lists, sums of squares sumsq_stride apart).
+// blockIdx.z is the matrix of a batch (pointers from the lists, its `parts` partial sums of squares at
+// sumsq + parts blockIdx.z: every block adds them up itself, which takes less time than a launch in between).
+__device__ __forceinline__ float sum_of_squares(const float* sumsq, int parts, float* red) {
+  if (parts == 1) return sumsq[blockIdx.z];
+  float s = 0.0f;
+  for (int i = threadIdx.x; i < parts; i += 256) s += sumsq[(size_t)blockIdx.z * parts + i];
+  return block_sum<256>(s, red);
+}
+
 template <int DT>
 __global__ __launch_bounds__(256) void scale_cast_kernel(PtrList Gl, int rows, int cols, int rows_p, int cols_p,
-                                                         int64_t ldg, const float* sumsq, int sumsq_stride,
+                                                         int64_t ldg, const float* sumsq, int parts,
                                                          float eps, PtrList Dl, int64_t ldd,
                                                          PtrList Tl, int64_t ldt,
                                                          int g_vec, int d_vec, int t_vec) {
@@ -156,7 +176,8 @@ __global__ __launch_bounds__(256) void scale_cast_kernel(PtrList Gl, int rows, i
   const raw* G = reinterpret_cast<const raw*>(Gl.p[blockIdx.z]);
   unsigned short* D = reinterpret_cast<unsigned short*>(Dl.p[blockIdx.z]);
   unsigned short* T = reinterpret_cast<unsigned short*>(Tl.p[blockIdx.z]);
-  const float denom = __builtin_sqrtf(sumsq[(size_t)blockIdx.z * sumsq_stride]) + eps;
+  __shared__ float red[4];
+  const float denom = __builtin_sqrtf(sum_of_squares(sumsq, parts, red)) + eps;
   const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
   const int tid = threadIdx.x;
   const int ch = tid & 7;   // 8-element chunk along the contiguous dimension
@@ -227,16 +248,17 @@ __global__ __launch_bounds__(256) void scale_cast_kernel(PtrList Gl, int rows, i
 // in 16-byte reads: word p of column c sits at word p ^ 4 (c / 8 % 16) of the column's 64, which
 // keeps both the writes of a wave (16 column chunks x 4 row pairs) and its reads (16 consecutive
 // groups of a column) on 64 different banks.
-template <int DT>
+// HAS_D: D is wanted too, and not T alone.
+template <int DT, bool HAS_D>
 __global__ __launch_bounds__(256) void scale_cast_tile128_kernel(PtrList Gl, int64_t ldg, const float* sumsq,
-                                                                 int sumsq_stride, float eps, PtrList Dl, int64_t ldd,
+                                                                 int parts, float eps, PtrList Dl, int64_t ldd,
                                                                  PtrList Tl, int64_t ldt) {
   typedef typename Elem<DT>::raw raw;
   __shared__ __align__(16) uint32_t tile[128 * 64];
   const raw* G = reinterpret_cast<const raw*>(Gl.p[blockIdx.z]) + (int64_t)blockIdx.y * 128 * ldg + blockIdx.x * 128;
-  unsigned short* D = reinterpret_cast<unsigned short*>(Dl.p[blockIdx.z]) + (int64_t)blockIdx.y * 128 * ldd + blockIdx.x * 128;
+  unsigned short* D = HAS_D ? reinterpret_cast<unsigned short*>(Dl.p[blockIdx.z]) + (int64_t)blockIdx.y * 128 * ldd + blockIdx.x * 128 : nullptr;
   unsigned short* T = reinterpret_cast<unsigned short*>(Tl.p[blockIdx.z]) + (int64_t)blockIdx.x * 128 * ldt + blockIdx.y * 128;
-  const float denom = __builtin_sqrtf(sumsq[(size_t)blockIdx.z * sumsq_stride]) + eps;
+  __shared__ float red[4];
   const int tid = threadIdx.x;
   const int ch = tid & 15;   // 8-element chunk along the contiguous dimension
   constexpr int NV = sizeof(raw) / 2;   // 16-byte loads per 8 elements
@@ -251,6 +273,7 @@ __global__ __launch_bounds__(256) void scale_cast_tile128_kernel(PtrList Gl, int
 #pragma unroll
       for (int q = 0; q < NV; ++q) in[pass][h].v[q] = reinterpret_cast<const uint4*>(src)[q];
     }
+  const float denom = __builtin_sqrtf(sum_of_squares(sumsq, parts, red)) + eps;   // while the tile is on its way
 #pragma unroll
   for (int pass = 0; pass < 4; ++pass) {
     const int rp = pass * 16 + (tid >> 4);   // rows 2 rp and 2 rp + 1 of the tile
@@ -259,7 +282,7 @@ __global__ __launch_bounds__(256) void scale_cast_tile128_kernel(PtrList Gl, int
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[h].h[e] = Elem<0>::st(as_bf16_value<DT>(in[pass][h].e[e]) / denom);
-      *reinterpret_cast<uint4*>(D + (int64_t)(2 * rp + h) * ldd + ch * 8) = o[h].v;
+      if constexpr (HAS_D) *reinterpret_cast<uint4*>(D + (int64_t)(2 * rp + h) * ldd + ch * 8) = o[h].v;
     }
     uint32_t* const col = tile + (ch * 8) * 64 + (rp ^ (4 * ch));   // columns 8 ch .. + 7 share ch = column / 8 % 16
 #pragma unroll
@@ -277,8 +300,43 @@ __global__ __launch_bounds__(256) void scale_cast_tile128_kernel(PtrList Gl, int
   }
 }
 
+// D alone, of matrices whose rows allow 16-byte accesses: 8 elements per lane, blockIdx.y strides over the rows
+// of D, which is rows_p x cols_p with zeros beyond G.
+template <int DT>
+__global__ __launch_bounds__(256) void scale_cast_rows_kernel(PtrList Gl, int rows, int cols, int rows_p, int cols_p,
+                                                              int64_t ldg, const float* sumsq, int parts, float eps,
+                                                              PtrList Dl, int64_t ldd) {
+  typedef typename Elem<DT>::raw raw;
+  __shared__ float red[4];
+  const raw* G = reinterpret_cast<const raw*>(Gl.p[blockIdx.z]);
+  unsigned short* D = reinterpret_cast<unsigned short*>(Dl.p[blockIdx.z]);
+  const float denom = __builtin_sqrtf(sum_of_squares(sumsq, parts, red)) + eps;
+  const int chunks = cols_p / 8, total = chunks * rows_p;
+  for (int i = (int)blockIdx.x * 256 + (int)threadIdx.x; i < total; i += (int)gridDim.x * 256) {
+    const int r = i / chunks, c = (i - r * chunks) * 8;
+    union { uint4 v; unsigned short h[8]; } o;
+    o.v = uint4{0u, 0u, 0u, 0u};
+    if (r < rows) {
+      const raw* src = G + (int64_t)r * ldg + c;
+      if (c + 8 <= cols) {
+        union { uint4 v[sizeof(raw) / 2]; raw e[8]; } u;
+#pragma unroll
+        for (int q = 0; q < (int)sizeof(raw) / 2; ++q) u.v[q] = reinterpret_cast<const uint4*>(src)[q];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o.h[e] = Elem<0>::st(as_bf16_value<DT>(u.e[e]) / denom);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (c + e < cols) o.h[e] = Elem<0>::st(as_bf16_value<DT>(src[e]) / denom);
+      }
+    }
+    *reinterpret_cast<uint4*>(D + (int64_t)r * ldd + c) = o.v;
+  }
+}
+
+// `parts` partial sums of squares per matrix at `sumsq`, one matrix after the other.  D or T may be absent.
 int launch_scale_cast_batched(const void* const* G, int batch, int dtype, int rows, int cols, int64_t ldg,
-                              const float* sumsq, int sumsq_stride, float eps, bf16_t* const* D, int64_t ldd,
+                              const float* sumsq, int parts, float eps, bf16_t* const* D, int64_t ldd,
                               bf16_t* const* T, int64_t ldt, hipStream_t stream, int rows_p, int cols_p) {
   if (rows_p < rows) rows_p = rows;
   if (cols_p < cols) cols_p = cols;
@@ -291,19 +349,31 @@ int launch_scale_cast_batched(const void* const* G, int batch, int dtype, int ro
     if (D) { dl.p[i] = D[i]; dv = dv && (reinterpret_cast<uintptr_t>(D[i]) & 15) == 0; }
     if (T) { tl.p[i] = T[i]; tv = tv && (reinterpret_cast<uintptr_t>(T[i]) & 15) == 0; }
   }
-  if (D && T && gv && dv && tv && rows_p == rows && cols_p == cols && rows % 128 == 0 && cols % 128 == 0) {
+  if (D && !T && gv && dv && cols_p % 8 == 0 && (int64_t)rows_p * cols_p / 8 < (1LL << 31)) {
+    // 8 chunks per thread at most, so that a block's sum of the partial sums is paid for
+    const int64_t blocks = ((int64_t)rows_p * (cols_p / 8) + 1023) / 1024;
+    dim3 gridr((unsigned)blocks, 1, (unsigned)batch);
+#define FM_SCALE_ROWS(DT) hipLaunchKernelGGL(scale_cast_rows_kernel<DT>, gridr, dim3(256), 0, stream, gl, rows, cols, rows_p, cols_p, \
+                                             ldg, sumsq, parts, eps, dl, ldd)
+    if (dtype == 0) FM_SCALE_ROWS(0);
+    else if (dtype == 1) FM_SCALE_ROWS(1);
+    else FM_SCALE_ROWS(2);
+#undef FM_SCALE_ROWS
+    return (int)hipGetLastError();
+  }
+  if (T && gv && (dv || !D) && tv && rows_p == rows && cols_p == cols && rows % 128 == 0 && cols % 128 == 0) {
     dim3 grid128((unsigned)(cols / 128), (unsigned)(rows / 128), (unsigned)batch);
-#define FM_SCALE128(DT) hipLaunchKernelGGL(scale_cast_tile128_kernel<DT>, grid128, dim3(256), 0, stream, gl, ldg, sumsq, \
-                                           sumsq_stride, eps, dl, ldd, tl, ldt)
-    if (dtype == 0) FM_SCALE128(0);
-    else if (dtype == 1) FM_SCALE128(1);
-    else FM_SCALE128(2);
+#define FM_SCALE128(DT, HAS_D) hipLaunchKernelGGL((scale_cast_tile128_kernel<DT, HAS_D>), grid128, dim3(256), 0, stream, gl, ldg, \
+                                                  sumsq, parts, eps, dl, ldd, tl, ldt)
+    if (dtype == 0) { if (D) FM_SCALE128(0, true); else FM_SCALE128(0, false); }
+    else if (dtype == 1) { if (D) FM_SCALE128(1, true); else FM_SCALE128(1, false); }
+    else { if (D) FM_SCALE128(2, true); else FM_SCALE128(2, false); }
 #undef FM_SCALE128
     return (int)hipGetLastError();
   }
   dim3 grid((unsigned)((cols_p + 63) / 64), (unsigned)((rows_p + 63) / 64), (unsigned)batch), block(256);
 #define FM_SCALE(DT) hipLaunchKernelGGL(scale_cast_kernel<DT>, grid, block, 0, stream, gl, rows, cols, rows_p, cols_p, ldg, \
-                                        sumsq, sumsq_stride, eps, dl, ldd, tl, ldt, gv, dv, tv)
+                                        sumsq, parts, eps, dl, ldd, tl, ldt, gv, dv, tv)
   if (dtype == 0) FM_SCALE(0);
   else if (dtype == 1) FM_SCALE(1);
   else FM_SCALE(2);
@@ -314,16 +384,17 @@ int launch_scale_cast_batched(const void* const* G, int batch, int dtype, int ro
 int launch_scale_cast(const void* G, int dtype, int rows, int cols, int64_t ldg,
                       const float* sumsq, float eps, bf16_t* D, int64_t ldd, bf16_t* T, int64_t ldt,
                       hipStream_t stream) {
-  return launch_scale_cast_batched(&G, 1, dtype, rows, cols, ldg, sumsq, 0, eps, D ? &D : nullptr, ldd,
+  return launch_scale_cast_batched(&G, 1, dtype, rows, cols, ldg, sumsq, 1, eps, D ? &D : nullptr, ldd,
                                    T ? &T : nullptr, ldt, stream, rows, cols);
 }
 
-// ---- a few zero words (a fill launch rather than hipMemsetAsync, so that callers can be captured) ---
-__global__ void zero_words_kernel(unsigned long long* p, int n) {
-  if ((int)threadIdx.x < n) p[threadIdx.x] = 0ull;
+// ---- zero words (a fill launch rather than hipMemsetAsync, so that callers can be captured) ----------
+__global__ __launch_bounds__(256) void zero_words_kernel(unsigned* p, int n) {
+  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (i < n) p[i] = 0u;
 }
-int launch_zero_words(void* p, int n, hipStream_t stream) {
-  hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(64), 0, stream, static_cast<unsigned long long*>(p), n < 64 ? n : 64);
+int launch_zero_words(unsigned* p, int n, hipStream_t stream) {
+  hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, p, n);
   return (int)hipGetLastError();
 }
 

@@ -50,31 +50,6 @@ __device__ __forceinline__ void copy_f32(const float* src, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" :: "v"(src), "s"(lds) : "memory", "m0");
 }
 
-// Position -> tile (ti, tj), ti <= tj: bands of 8 tile rows, column by column inside a band, so that
-// the 64 tiles the workgroups of one XCD hold at a time lie on about 8 + 8 operand panels.
-__device__ __forceinline__ void f32_tile_at(int pos, int T, int& ti, int& tj) {
-  int r0 = 0, rows = T < 8 ? T : 8;
-  for (;;) {
-    const int head = rows * (rows + 1) / 2, cnt = head + (T - r0 - rows) * rows;
-    if (pos < cnt) {
-      if (pos < head) {           // column c of the band's triangle holds c + 1 tiles
-        int c = 0;
-        while (pos > c) { pos -= c + 1; ++c; }
-        ti = r0 + pos; tj = r0 + c;
-      } else {
-        pos -= head;
-        const int c = pos / rows;
-        ti = r0 + (pos - c * rows); tj = r0 + rows + c;
-      }
-      return;
-    }
-    pos -= cnt;
-    r0 += 8;
-    rows = T - r0 < 8 ? T - r0 : 8;
-    if (rows <= 0) { ti = tj = 0; return; }   // not reached for pos < T (T + 1) / 2
-  }
-}
-
 // One wave's 32x32 block at (row0, col0) of Y and its mirror image, from the accumulators: register
 // 4 q + e of lane l is row 8 q + 4 (l / 32) + e, column l % 32.  Both copies come from the same register;
 // on a diagonal tile only what lies on or above the diagonal counts.
@@ -210,7 +185,7 @@ __global__ __launch_bounds__(256) void syrk_f32_kernel(F32Args p) {
   int ti, tj;
   for (int r = 0; r < p.rounds + (p.piece == 0 ? 1 : 0); ++r) {
     if (r == p.rounds && w >= p.rem) break;
-    f32_tile_at(r * G + w, p.T, ti, tj);
+    band_tri_decode(r * G + w, p.T, ti, tj);
     run(ti, tj, 0, p.nk, acc);
     f32_write_block(p, acc, ti == tj, ti * T32 + wm * 32, tj * T32 + wn * 32, lane);
   }
@@ -220,7 +195,7 @@ __global__ __launch_bounds__(256) void syrk_f32_kernel(F32Args p) {
   for (int slot = 0; s < end; ++slot) {   // at most two tiles: piece <= nk
     const int t = s / p.nk, kb = s - t * p.nk;
     const int ke = kb + (end - s) < p.nk ? kb + (end - s) : p.nk;
-    f32_tile_at(p.rounds * G + t, p.T, ti, tj);
+    band_tri_decode(p.rounds * G + t, p.T, ti, tj);
     run(ti, tj, kb, ke, acc);
     float* const dst = p.parts + (int64_t)(2 * w + slot) * kPartFloats32 + wave * 1024 + lane * 4;
 #pragma unroll
@@ -235,7 +210,7 @@ __global__ __launch_bounds__(64) void syrk_f32_reduce_kernel(F32Args p, int main
   const int lane = threadIdx.x;
   const int t = (int)(blockIdx.x >> 2), blk = (int)(blockIdx.x & 3);
   int ti, tj;
-  f32_tile_at(p.rounds * main_grid + t, p.T, ti, tj);
+  band_tri_decode(p.rounds * main_grid + t, p.T, ti, tj);
   const int s0 = t * p.nk, w0 = s0 / p.piece, w1 = (s0 + p.nk - 1) / p.piece;
   f32x16_t acc;
 #pragma unroll

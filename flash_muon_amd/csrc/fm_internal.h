@@ -46,6 +46,31 @@ __device__ __forceinline__ void tri_decode(int t, int T, int& i, int& j) {
   j = ii + (t - (ii * T - (ii * (ii - 1)) / 2));
 }
 
+// Position -> tile (ti, tj), ti <= tj, of a T x T upper triangle: bands of 8 tile rows, column by column
+// inside a band, so that a run of 64 positions lies on about 8 + 8 operand panels.
+__device__ __forceinline__ void band_tri_decode(int pos, int T, int& ti, int& tj) {
+  int r0 = 0, rows = T < 8 ? T : 8;
+  for (;;) {
+    const int head = rows * (rows + 1) / 2, cnt = head + (T - r0 - rows) * rows;
+    if (pos < cnt) {
+      if (pos < head) {           // column c of the band's triangle holds c + 1 tiles
+        int c = 0;
+        while (pos > c) { pos -= c + 1; ++c; }
+        ti = r0 + pos; tj = r0 + c;
+      } else {
+        pos -= head;
+        const int c = pos / rows;
+        ti = r0 + (pos - c * rows); tj = r0 + rows + c;
+      }
+      return;
+    }
+    pos -= cnt;
+    r0 += 8;
+    rows = T - r0 < 8 ? T - r0 : 8;
+    if (rows <= 0) { ti = tj = 0; return; }   // not reached for pos < T (T + 1) / 2
+  }
+}
+
 // The GEMM kernels exist for two 16-bit element types with the same memory layout; pointers are
 // typed bf16_t in both cases and F16 says what the bits mean.
 template <bool F16>
@@ -136,12 +161,14 @@ int launch_gemm_mid(GemmArgs args, void* ws, size_t ws_bytes, hipStream_t stream
 // up to kMaxBatch device pointers, passed to a kernel by value
 struct PtrList { void* p[kMaxBatch]; };
 
-// the batched forms take HOST arrays of `batch` device pointers; matrix i reads / writes its own
-// slot of the strided arrays (out and sumsq: stride in floats; partials: kSumsqBlocks floats)
-int launch_sumsq_batched(const void* const* G, int batch, int dtype, int rows, int cols, int64_t ldg,
-                         float* out, int out_stride, float* partials, hipStream_t stream);
+// The batched forms take HOST arrays of `batch` device pointers.  Sums of squares come as sumsq_parts(n)
+// partial sums per matrix of n elements, one matrix after the other; n_zero words at `zero` are cleared on
+// the way.
+int sumsq_parts(int64_t n);
+int launch_sumsq_parts_batched(const void* const* G, int batch, int dtype, int rows, int cols, int64_t ldg,
+                               float* partials, hipStream_t stream, unsigned* zero, int n_zero);
 int launch_scale_cast_batched(const void* const* G, int batch, int dtype, int rows, int cols, int64_t ldg,
-                              const float* sumsq, int sumsq_stride, float eps, bf16_t* const* D, int64_t ldd,
+                              const float* sumsq, int parts, float eps, bf16_t* const* D, int64_t ldd,
                               bf16_t* const* T, int64_t ldt, hipStream_t stream, int rows_p = 0, int cols_p = 0);
 int launch_sumsq(const void* G, int dtype, int rows, int cols, int64_t ldg, float* out,
                  float* partials, hipStream_t stream);
@@ -159,9 +186,24 @@ int launch_momentum_nesterov(void* g, void* buf, int dtype, int64_t n, float w_b
 int launch_weight_update(void* p, int p_dtype, const bf16_t* u, int64_t n, float decay_mul,
                          float alpha, hipStream_t stream);
 
-// n (at most 64) 64-bit words at p set to zero by a one-block launch
-int launch_zero_words(void* p, int n, hipStream_t stream);
+// The Newton-Schulz iteration of a batch in one launch (fm_flow.hip).  M and K are whole multiples of the edges; X
+// holds step 0's iterate and room for `steps` of them, A, P and pdiag for as many.
+struct FlowProblem {
+  bf16_t* X; int64_t x_step;
+  bf16_t* A; bf16_t* P; int64_t a_step;
+  float* pdiag; int64_t d_step, d_mat;
+  int M, K, batch, steps;
+  int edge_s, edge_x;                 // tiles of the symmetric products and of X': 64 and 64, 64 and 128, or 128 and 128
+  float a, b, c;
+  unsigned* counters;                 // flow_counter_words of them, zero
+  void* const* out; int64_t ldout;    // rows x cols, X' of the last step or (tall) its transpose
+  int rows, cols, tall;
+};
+int flow_counter_words(int batch, int steps);
+int launch_ns_flow(const FlowProblem& f, hipStream_t stream);
 
-constexpr int kSumsqBlocks = 1024;   // partial sums written by the first reduction stage
+int launch_zero_words(unsigned* p, int n, hipStream_t stream);
+
+constexpr int kSumsqBlocks = 1024;   // partial sums per matrix, at most
 
 }  // namespace fm

@@ -212,10 +212,13 @@ FM_API int fm_scale_cast_bf16(const void* G, int dtype, int rows, int cols, int6
 
 /* ---------------------------------------------------------------------------------------------
  * The whole quintic Newton-Schulz orthogonalisation of one matrix: G is rows x cols of `dtype`
- * (row stride ldg), out is rows x cols bf16 (row stride ldout).  Runs fm_sumsq,
- * fm_scale_cast_bf16 and `steps` x (fm_syrk_bf16, fm_syrk_poly_bf16, fm_gemm_axpby_bf16) on
- * `stream`, iterating on the wide orientation (M = min(rows, cols)).  steps == 0 returns the
- * normalised input.  out must not overlap G.  A matrix whose sides are not whole multiples of 128
+ * (row stride ldg), out is rows x cols bf16 (row stride ldout).  Runs the sum of squares, the scaled
+ * cast and `steps` x (fm_syrk_bf16, fm_syrk_poly_bf16, fm_gemm_axpby_bf16) on
+ * `stream`, iterating on the wide orientation (M = min(rows, cols)).  Matrices of up to 512 to 1280 rows
+ * (by size, shape and number) run all products of up to five steps as one launch, whose workgroups wait
+ * for each other inside it but need not be resident together; their workspace holds every step's
+ * iterate and squares (6 M K + 10 M^2 bf16 per matrix, against 4 M K + 2 M^2 otherwise).
+ * steps == 0 returns the normalised input.  out must not overlap G.  A matrix whose sides are not whole multiples of 128
  * (of 256 where whole 256x256 tiles are estimated to pay for the padding) is iterated on zero-padded to whole tiles inside the workspace (zero rows and columns stay zero
  * through every step) and the rows x cols part is copied out at the end.
  * Replaces fast_newtonschulz: flash_muon/muon.py:6-33.
