@@ -49,12 +49,6 @@ constexpr int kFlowSteps = 5;   // steps per launch of the one-launch iteration
 // 2816 x 7168 26).  The long side alone goes to a multiple of 256 where the short one is one already
 // (32 of 2048 x 5504 15.4 ms, of 2048 x 5632 11.9; one matrix 0.72 and 0.59; below 1536 rows a single
 // matrix gains nothing).
-constexpr int kPad256From = 2944;       // the stand-alone product: there the copies have to be paid for
-static int ns_pad(int n) {
-  int p = (n + 127) / 128 * 128;
-  if (p >= kPad256From && p % 256 != 0) p += 128;
-  return p;
-}
 // Which matrices iterate in one launch (fm_flow.hip), and on which tiles: M x K with M <= K, `batch` of them.
 // Five steps in us, one launch / launches per product: 256^2 91 / 109, 512 x 2048 133 / 154, 768^2 121 / 146,
 // 1024^2 137 / 158, 24 of 768^2 360 / 393, 8 of 1024 x 2816 593 / 705, 16 of 768 x 3072 649 / 967.  The launches per
@@ -178,16 +172,40 @@ size_t fm_gemm_workspace_bytes(int rows_out, int cols_out) {
 
 int fm_set_knob(int which, long long value) { return set_knob(which, value) == 0 ? FM_OK : FM_ERR_SHAPE; }
 
-// X * X^T of a matrix whose sides are not whole 128-tiles, through zero-padded copies: X padded in
-// the workspace, the product of that on the tiled paths into a padded Y beside it, and the M x M
-// part copied out.  Taken from 65536 elements of X on (below that the general path's single launch
-// wins); 16-bit elements only.  The tiled paths need whole 128-row tiles and whole 64-wide k stages,
-// so a shape that has both is left alone and k is padded to a multiple of 64 only.
+// X * X^T in 16 bits of sides that the 256-tiles of launch_gemm_nt do not fit: in place (fm_gemm_ragged.hip), or behind
+// a copy of X with rows of whole stages, where 16-byte copies cannot take the rows or too many of them would cross a line.
+//   Sides that are no whole 128-tiles, from 65536 elements of X on (below that the general path's single launch wins).
+// us, zero-padded copies of both X and Y around the tiled paths before, now: 600^2 17.3 -> 10.7, 1000^2 16.7 -> 11.0, 2000^2 32 ->
+// 23, 3000 x 1000 33 -> 24, 3000 x 5000 79 -> 70, 3900 x 8000 140 -> 104, 600 x 8000 32 -> 22, 6500^2 356 -> 294.
+//   Odd numbers of 128-tiles, rows on 128-byte lines (in launch_gemm_nt's 128-tiles, or its 256-tiles with a half at the edge):
+// 1408^2 14.2 -> 12.4, 2944^2 46.7 -> 38.2, 4224^2 96 -> 78, 5504 x 2048 81 -> 62, 8064 x 1024 114 -> 70; but 2176^2 (153 tiles) 20.7 and
+// 21.8, 2688^2 26.3 and 26.9: between 121 and 256 tiles of a workgroup each the older path stays.
+struct SyrkRagged { int Kp; size_t slots, x, total; };
+constexpr int64_t kSyrkRaggedMinElems = 256 * 256;
+static bool whole_tiles(int M, int K) { return M % 128 == 0 && K % 64 == 0; }
+static bool syrk_ragged_layout(int M, int K, SyrkRagged* p) {
+  if (M <= 0 || K <= 0 || (int64_t)M * K < kSyrkRaggedMinElems || K >= (1 << 22)) return false;
+  if (whole_tiles(M, K)) {
+    const int64_t T = M / 128, tiles = T * (T + 1) / 2;
+    if (M % 256 == 0 || (tiles > 120 && tiles <= 256)) return false;
+  }
+  p->Kp = (K + 63) / 64 * 64;
+  p->slots = syrk_ragged_workspace_bytes(M, K);
+  p->x = align_up(p->slots, 256);   // (a copy has as many stages, and so the same pieces)
+  // the last 256 bytes of a workspace are left alone: the tickets of the 256-tiles' last rounds are counted there
+  p->total = p->x + (whole_tiles(M, K) ? 0 : align_up((size_t)M * p->Kp * 2, 256)) + 256;
+  return true;
+}
+// Both X and Y as copies padded to whole 256-tiles, for a matrix that has to be copied anyway: where the 256-tiles just
+// fill a round of half tiles (16 tile rows) or leave few workgroups idle (20 and 31: 210 and 496 tiles) while the
+// 128-tiles begin another round: 4000^2 77 us and 85 behind one copy, 4000 x 2000 51 and 55, 5000 x 3000 92 and 98, 7776^2 400 and
+// 448; but 3500^2 83 and 65, 5500^2 194 and 184 (22 tile rows), 7200^2 377 and 372 (29), 7500 x 4000 281 and 219 (30).
 struct SyrkPad { int Mp, Kp; size_t x, y, gemm, total; };
-constexpr int64_t kSyrkPadMinElems = 256 * 256;
 static bool syrk_pad_layout(int M, int K, SyrkPad* p) {
-  if (M <= 0 || K <= 0 || (M % 128 == 0 && K % 64 == 0) || (int64_t)M * K < kSyrkPadMinElems) return false;
-  p->Mp = ns_pad(M);
+  if (whole_tiles(M, K) || M <= 3968 || K < 1500) return false;
+  const int64_t T = (M + 255) / 256;
+  if (T != 16 && T != 20 && T != 31) return false;
+  p->Mp = (int)T * 256;
   p->Kp = (K + 63) / 64 * 64;
   p->x = 0;
   p->y = align_up((size_t)p->Mp * p->Kp * 2, 256);
@@ -198,16 +216,23 @@ static bool syrk_pad_layout(int M, int K, SyrkPad* p) {
 
 size_t fm_syrk_workspace_bytes(int M, int K) {
   if (M <= 0) return 0;
-  const size_t plain = gemm_fast_workspace_bytes(M, M, 1);
+  size_t need = gemm_fast_workspace_bytes(M, M, 1);
+  SyrkRagged r;
+  if (!syrk_ragged_layout(M, K, &r)) return need;
+  if (r.total > need) need = r.total;
   SyrkPad p;
-  if (!syrk_pad_layout(M, K, &p)) return plain;
-  return p.total > plain ? p.total : plain;
+  if (syrk_pad_layout(M, K, &p) && p.total > need) need = p.total;
+  if (!whole_tiles(M, K)) {   // what the interface promises room for, whichever way is taken: X and Y padded to 128-tiles
+    const size_t Mp = (size_t)(M + 127) / 128 * 128, both = Mp * (r.Kp + Mp) * 2;
+    if (both > need) need = both;
+  }
+  return need;
 }
 
 size_t fm_syrk_f32_workspace_bytes(int M, int K) { return M <= 0 || K <= 0 ? 0 : syrk_f32_workspace_bytes(M, K); }
 
 static int syrk_impl(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64_t ldy_col, int M, int K,
-                     void* ws, size_t ws_bytes, fm_stream_t stream, int elem, bool may_pad = true) {
+                     void* ws, size_t ws_bytes, fm_stream_t stream, int elem, bool may_copy = true) {
   if (M < 0 || K < 0) return FM_ERR_SHAPE;
   if (M == 0) return FM_OK;
   if (!X && K > 0) return FM_ERR_NULL;
@@ -238,23 +263,38 @@ static int syrk_impl(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64
   GemmArgs a = {};
   a.E = nullptr; a.lde = 0;
   a.alpha = 0.0f; a.beta = 1.0f; a.symmetric = 1; a.elem = elem;
-  SyrkPad p;
-  // Y is symmetric, so a unit stride in either direction makes its lines rows for the copy out
+  // Y is symmetric, so a unit stride in either direction makes its lines rows for the write-out
   const int64_t ldy = ldy_col == 1 ? ldy_row : ldy_row == 1 ? ldy_col : 0;
-  if (may_pad && ldy >= M && usable_ws(ws) && syrk_pad_layout(M, K, &p) && ws_bytes >= p.total &&
-      !overlaps(mat_range(X, M, K, ldx, es), Range{reinterpret_cast<uintptr_t>(ws), reinterpret_cast<uintptr_t>(ws) + p.total}) &&
-      !overlaps(mat_range(Y, M, M, ldy, es), Range{reinterpret_cast<uintptr_t>(ws), reinterpret_cast<uintptr_t>(ws) + p.total})) {
-    unsigned char* w = static_cast<unsigned char*>(ws);
-    bf16_t* Xp = reinterpret_cast<bf16_t*>(w + p.x);
-    bf16_t* Yp = reinterpret_cast<bf16_t*>(w + p.y);
-    bf16_t* xl[1] = {Xp};
-    bf16_t* yl[1] = {static_cast<bf16_t*>(Y)};
-    if (launch_copy2d_batched(static_cast<const bf16_t*>(X), ldx, 0, xl, p.Kp, 1, M, K, p.Mp, p.Kp, hs)) return FM_ERR_LAUNCH;
-    a.A = a.B = Xp; a.lda = a.ldb = p.Kp;
-    a.C = a.C2 = Yp; a.c_rs = a.c2_rs = p.Mp; a.c_cs = a.c2_cs = 1;
-    a.Ma = a.Nb = p.Mp; a.Kc = p.Kp;
-    if (launch_gemm_nt(a, w + p.gemm, ws_bytes - p.gemm, hs)) return FM_ERR_LAUNCH;
-    return hip_status(launch_copy2d_batched(Yp, p.Mp, 0, yl, ldy, 1, M, M, M, M, hs));
+  const uintptr_t w0 = reinterpret_cast<uintptr_t>(ws);
+  auto room = [&](size_t need) {   // a workspace of that size which is nobody's operand
+    const Range w = {w0, w0 + need};
+    return need == 0 || (usable_ws(ws) && ws_bytes >= need && !overlaps(mat_range(X, M, K, ldx, es), w) && !overlaps(mat_range(Y, M, M, ldy, es), w));
+  };
+  SyrkRagged r;
+  if (ldy >= M && syrk_ragged_layout(M, K, &r)) {
+    const bf16_t* const x = static_cast<const bf16_t*>(X);
+    bf16_t* const y = static_cast<bf16_t*>(Y);
+    const int how = syrk_ragged_reads(x, ldx, M, K);
+    SyrkPad p;
+    const bool pad = may_copy && how != kReadsLines && syrk_pad_layout(M, K, &p) && room(p.total);
+    if (!pad && (how == kReadsLines || (how == kReadsRows && !whole_tiles(M, K))) && room(r.slots ? r.slots + 256 : 0))
+      return hip_status(launch_syrk_ragged(x, ldx, y, ldy, M, K, elem == kElemF16, ws, r.slots, hs));
+    if (pad) {
+      unsigned char* w = static_cast<unsigned char*>(ws);
+      bf16_t* Xp = reinterpret_cast<bf16_t*>(w + p.x);
+      bf16_t* Yp = reinterpret_cast<bf16_t*>(w + p.y);
+      if (launch_copy2d_batched(x, ldx, 0, &Xp, p.Kp, 1, M, K, p.Mp, p.Kp, hs)) return FM_ERR_LAUNCH;
+      a.A = a.B = Xp; a.lda = a.ldb = p.Kp;
+      a.C = a.C2 = Yp; a.c_rs = a.c2_rs = p.Mp; a.c_cs = a.c2_cs = 1;
+      a.Ma = a.Nb = p.Mp; a.Kc = p.Kp;
+      if (launch_gemm_nt(a, w + p.gemm, ws_bytes - p.gemm, hs)) return FM_ERR_LAUNCH;
+      return hip_status(launch_copy2d_batched(Yp, p.Mp, 0, &y, ldy, 1, M, M, M, M, hs));
+    }
+    if (may_copy && !whole_tiles(M, K) && room(r.total)) {
+      bf16_t* copy = reinterpret_cast<bf16_t*>(static_cast<unsigned char*>(ws) + r.x);
+      if (launch_copy2d_batched(x, ldx, 0, &copy, r.Kp, 1, M, K, M, r.Kp, hs)) return FM_ERR_LAUNCH;
+      return hip_status(launch_syrk_ragged(copy, r.Kp, y, ldy, M, r.Kp, elem == kElemF16, ws, r.slots, hs));
+    }
   }
   a.A = a.B = static_cast<const bf16_t*>(X); a.lda = a.ldb = ldx;
   a.C = a.C2 = static_cast<bf16_t*>(Y);

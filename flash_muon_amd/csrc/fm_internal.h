@@ -149,6 +149,15 @@ int launch_gemm_general(GemmArgs args, hipStream_t stream);
 size_t syrk_f32_workspace_bytes(int M, int K);
 int launch_syrk_f32(const float* X, int64_t ldx, float* Y, int64_t rs, int64_t cs, int M, int K, void* ws,
                     size_t ws_bytes, hipStream_t stream);
+// Y = X X^T in 16 bits of any M and K, read and written in place (fm_gemm_ragged.hip), for rows of X that 16-byte copies
+// can take, Y's lines of unit stride ldy apart; without a workspace of syrk_ragged_workspace_bytes the tiles stay whole.
+// How such a matrix is read best: by its rows as they lie on 128-byte lines, by its rows although they do not,
+// or not at all before it has been copied.
+constexpr int kReadsLines = 0, kReadsRows = 1, kReadsCopy = 2;
+int syrk_ragged_reads(const bf16_t* X, int64_t ldx, int M, int K);
+size_t syrk_ragged_workspace_bytes(int M, int K);
+int launch_syrk_ragged(const bf16_t* X, int64_t ldx, bf16_t* Y, int64_t ldy, int M, int K, bool f16, void* ws, size_t ws_bytes,
+                       hipStream_t stream);
 bool gemm_fast_eligible(const GemmArgs& a);
 // bytes of fp32 partial tiles the 256x256 path can need for `batch` Ma x Nb outputs, whatever k is
 // (0 when no schedule of this shape cuts a tile)

@@ -99,21 +99,19 @@ __device__ __forceinline__ void stage(f32x4_t (&acc)[4][4], Frag& f0, Frag& f1, 
   substep<F16, AS, BS, 1>(acc, f1, f0, smem, L, voB, nB);
 }
 
-// n k stages (n >= 1) from (gA, gB) on.  `count`, where a thread has one, is counted up once the first stage has
-// landed everywhere: by then the stores that every wave issued before this call have completed too (one
-// counter tracks both, in order).  voA, voB: byte offsets of this lane's four copies per operand.  On
-// return no copy is in flight and nobody reads the ring.
-template <bool F16>
-__device__ __forceinline__ void main_loop(f32x4_t (&acc)[4][4], int n, const unsigned char* smem, const Lane& L,
-                                          const uint32_t (&voA)[4], const uint32_t (&voB)[4], const bf16_t* gA, const bf16_t* gB,
-                                          unsigned* count) {
-  // stages past the end are the last stage again (into slots nobody reads), so that the number of copies
-  // in flight is the same at every wait
-  const int last = n - 1, k1 = last < 1 ? last : 1;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) copy16(voA[q], gA, L.ldsw, q * 4096);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) copy16(voB[q], gB, L.ldsw, B_OFF + q * 4096);
+// n k stages (n >= 1).  `first` issues the 8 copies of stage 0 and `landed` is called when this wave's have landed, in
+// front of the barrier that says so for everybody; stage s >= 1 is at (gA, gB) + s BK, as stage 0 is if `lo` is 0.
+// voA, voB: byte offsets of this lane's four copies per operand.  `count`, where a thread has one, is counted up once
+// the first stage has landed everywhere: by then the stores that every wave issued before this call have completed
+// too (one counter tracks both, in order).  On return no copy is in flight and nobody reads the ring.
+template <bool F16, class First, class Landed>
+__device__ __forceinline__ void main_loop_from(f32x4_t (&acc)[4][4], int n, const unsigned char* smem, const Lane& L,
+                                               const uint32_t (&voA)[4], const uint32_t (&voB)[4], const bf16_t* gA, const bf16_t* gB,
+                                               unsigned* count, int lo, const First& first, const Landed& landed) {
+  // stages past the end are the last stage again, or stage `lo` (into slots nobody reads), so that the number of
+  // copies in flight is the same at every wait
+  const int last = n - 1, fill = last < lo ? lo : last, k1 = last < 1 ? fill : 1;
+  first();
 #pragma unroll
   for (int q = 0; q < 4; ++q) copy16(voA[q], gA + k1 * BK, L.ldsw, OPER + q * 4096);
 #pragma unroll
@@ -122,7 +120,9 @@ __device__ __forceinline__ void main_loop(f32x4_t (&acc)[4][4], int n, const uns
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+  landed();
+  asm volatile("s_barrier" ::: "memory");
   if (count) __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   Frag f0, f1;
 #pragma unroll
@@ -131,7 +131,7 @@ __device__ __forceinline__ void main_loop(f32x4_t (&acc)[4][4], int n, const uns
   for (int i = 0; i < 4; ++i) f0.b[i] = *reinterpret_cast<const bf16x8_t*>(smem + L.fb[0] + i * 2048);
 #define FM_T128_STAGE(AS, BS, S)                                                                  \
   {                                                                                               \
-    const int kn = (S) + 2 < last ? (S) + 2 : last;                                               \
+    const int kn = (S) + 2 < last ? (S) + 2 : fill;                                               \
     stage<F16, AS, BS>(acc, f0, f1, smem, L, voA, voB, gA + kn * BK, gB + kn * BK);               \
     if ((S) + 1 >= n) break;                                                                      \
   }
@@ -145,6 +145,19 @@ __device__ __forceinline__ void main_loop(f32x4_t (&acc)[4][4], int n, const uns
   }
 #undef FM_T128_STAGE
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// ... all of them from (gA, gB) on
+template <bool F16>
+__device__ __forceinline__ void main_loop(f32x4_t (&acc)[4][4], int n, const unsigned char* smem, const Lane& L,
+                                          const uint32_t (&voA)[4], const uint32_t (&voB)[4], const bf16_t* gA, const bf16_t* gB,
+                                          unsigned* count) {
+  main_loop_from<F16>(acc, n, smem, L, voA, voB, gA, gB, count, 0, [&]() {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) copy16(voA[q], gA, L.ldsw, q * 4096);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) copy16(voB[q], gB, L.ldsw, B_OFF + q * 4096);
+  }, []() {});
 }
 
 // ---- the same with both operands k-major --------------------------------------------------------
@@ -286,11 +299,12 @@ __device__ __forceinline__ void copy_offsets(uint32_t (&voA)[4], uint32_t (&voB)
 // consecutive rows of a column per 16-byte load, which is what a lane holds of that column.
 struct Out {
   const bf16_t* ET; int ldet;     // nullptr: no operand E
-  bf16_t* C; int c_rs;            // nullptr: no such output
-  bf16_t* C2; int c2_rs;
+  bf16_t* C; int64_t c_rs;        // nullptr: no such output
+  bf16_t* C2; int64_t c2_rs;
   float alpha, beta;
   const float* row_alpha;
   float* diag_out;                // fp32 diagonal split off (blocks on the diagonal of a symmetric product)
+  int limit;                      // EDGE: rows and columns of the output that exist
 };
 
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -308,8 +322,25 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
   }
 }
 
-// AUX: cache policy of the stores (0, or 16: written through to memory, for readers on other XCDs)
-template <bool F16, int AUX>
+// One lane's 16 bytes of a row of a square output of `limit` rows: columns c .. c + 7 of row r, at any alignment of the
+// element type
+__device__ __forceinline__ void store_edge(bf16_t* C, int64_t ld, int r, int c, int limit, uint4 d) {
+  if (r >= limit) return;
+  bf16_t* const dst = C + r * ld + c;
+  if (c + 8 <= limit) {
+    __builtin_memcpy(dst, &d, 16);
+  } else {
+    union { uint4 v; unsigned short h[8]; } u;
+    u.v = d;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (c + e < limit) reinterpret_cast<unsigned short*>(dst)[e] = u.h[e];
+  }
+}
+
+// AUX: cache policy of the stores (0, or 16: written through to memory, for readers on other XCDs).  EDGE: blocks may
+// reach beyond the output, whose rows may start at any element.
+template <bool F16, int AUX, bool EDGE = false>
 __device__ __forceinline__ void write_block(const Out& o, bool diag, const f32x4_t (&acc)[4][4], unsigned char* T, int row0,
                                             int col0, int lane) {
   asm volatile("" : "+v"(lane));   // offsets derived anew for every tile, not kept across the main loop
@@ -400,7 +431,7 @@ __device__ __forceinline__ void write_block(const Out& o, bool diag, const f32x4
   const int lr = lane >> 3, ch = lane & 7;
   if (direct) {
     const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc(o.C + (int64_t)row0 * o.c_rs + col0, 0, 0xffffffff, 0x00020000);
-    const uint32_t vo = (uint32_t)(lr * o.c_rs + ch * 8) * 2u;
+    const uint32_t vo = (uint32_t)(lr * (int)o.c_rs + ch * 8) * 2u;
     uint4 d[8];
 #pragma unroll
     for (int it = 0; it < 8; ++it) {
@@ -408,12 +439,14 @@ __device__ __forceinline__ void write_block(const Out& o, bool diag, const f32x4
       d[it] = *reinterpret_cast<const uint4*>(T + ((R ^ (gg >> 1)) * 128) + (((ch >> 2) ^ (gg & 1)) * 64) + (ch & 3) * 16);
     }
 #pragma unroll
-    for (int it = 0; it < 8; ++it)
-      __builtin_amdgcn_raw_buffer_store_b128(v4i{(int)d[it].x, (int)d[it].y, (int)d[it].z, (int)d[it].w}, buf, (int)vo, it * 16 * o.c_rs, AUX);
+    for (int it = 0; it < 8; ++it) {
+      if constexpr (EDGE) store_edge(o.C, o.c_rs, row0 + 8 * it + lr, col0 + 8 * ch, o.limit, d[it]);
+      else __builtin_amdgcn_raw_buffer_store_b128(v4i{(int)d[it].x, (int)d[it].y, (int)d[it].z, (int)d[it].w}, buf, (int)vo, it * 16 * (int)o.c_rs, AUX);
+    }
   }
   if (mirror) {
     const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc(o.C2 + (int64_t)col0 * o.c2_rs + row0, 0, 0xffffffff, 0x00020000);
-    const uint32_t vo = (uint32_t)(lr * o.c2_rs + ch * 8) * 2u;
+    const uint32_t vo = (uint32_t)(lr * (int)o.c2_rs + ch * 8) * 2u;
     uint4 d[8];
 #pragma unroll
     for (int it = 0; it < 8; ++it) {
@@ -421,8 +454,10 @@ __device__ __forceinline__ void write_block(const Out& o, bool diag, const f32x4
       d[it] = *reinterpret_cast<const uint4*>(T2 + ((c ^ ((c >> 4) & 1)) * 128) + ((ch ^ ((c >> 1) & 7)) << 4));
     }
 #pragma unroll
-    for (int it = 0; it < 8; ++it)
-      __builtin_amdgcn_raw_buffer_store_b128(v4i{(int)d[it].x, (int)d[it].y, (int)d[it].z, (int)d[it].w}, buf, (int)vo, it * 16 * o.c2_rs, AUX);
+    for (int it = 0; it < 8; ++it) {
+      if constexpr (EDGE) store_edge(o.C2, o.c2_rs, col0 + 8 * it + lr, row0 + 8 * ch, o.limit, d[it]);
+      else __builtin_amdgcn_raw_buffer_store_b128(v4i{(int)d[it].x, (int)d[it].y, (int)d[it].z, (int)d[it].w}, buf, (int)vo, it * 16 * (int)o.c2_rs, AUX);
+    }
   }
 }
 

@@ -112,9 +112,10 @@ FM_API int fm_syrk_bf16(const void* X, int64_t ldx, void* Y, int64_t ldy_row, in
                  int M, int K, void* ws, size_t ws_bytes, fm_stream_t stream);
 
 /* Scratch for fm_syrk_bf16 and fm_syrk_f16 by the shape of X: fm_gemm_workspace_bytes(M, M), and for
- * an X whose sides are not whole multiples of 128 also room for a zero-padded copy of X and the padded
- * product, so that such shapes run on the tiled schedules too (copied in, multiplied, the M x M part
- * copied out: three launches) instead of the general one.  With less than this the calls still run,
+ * an X whose sides are not whole multiples of 128 at least room for a zero-padded copy of X and the padded
+ * product.  Such shapes are read and written in place (rows that 16-byte copies can take), or read from
+ * a copy of X, or multiplied as padded copies, whichever is faster; what is left of a last round of tiles is cut
+ * along k and its fp32 sums lie here too.  With less than this the calls still run,
  * on the schedule that the scratch they get allows.  No counterpart in the reference, whose masked
  * loads and stores take any shape (flash_muon/matmul_transpose_triton.py:48-52, 70-75).
  */
@@ -127,8 +128,8 @@ FM_API size_t fm_syrk_workspace_bytes(int M, int K);
  * that the library holds in the device memory of every GPU it is used on, from the first use until
  * the process ends.  (Outputs of few tiles with a long k, which fm_syrk_bf16 cuts deeper along k when
  * it is given the up to 192 MiB of fm_gemm_workspace_bytes, are cut as far as 256 slots allow; their
- * fp32 sums then run in another order.  Sides that are not whole tiles run on the general schedule,
- * without padded copies.)  Nothing is allocated, freed or synchronised; the first call on
+ * fp32 sums then run in another order.  Sides that are not whole tiles run in place
+ * where 16-byte copies can take the rows of X, and on the general schedule otherwise: no copies.)  Nothing is allocated, freed or synchronised; the first call on
  * a device looks the array's address up (do that once outside a graph capture).
  * Limits: M <= FM_STATIC_MAX_M and K <= FM_STATIC_MAX_K, otherwise FM_ERR_SHAPE.  All calls on one
  * GPU share the array, which keeps the last call's contents (nothing in it has to start at zero:

@@ -1,0 +1,58 @@
+"""Symmetric products of 16-bit matrices that are read and written in place: sides around a 128-tile, the part of k
+that a stage of 64 leaves, tiles in rounds, whole and in pieces along k, odd numbers of whole tiles, and inputs that are
+copied first.  Integer inputs: every sum is exact in fp32 (and fp64), so the result is the exactly rounded one."""
+import pytest
+import torch
+
+from flash_muon_amd import matmul_transpose_assign
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _ints(M, K, seed, dtype):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randint(-3, 4, (M, K), generator=g).to(dtype)
+
+
+def _run(X, pitch_x, pitch_y, offset_y=0):
+    """X in rows of pitch_x whose rest is NaN, into rows of pitch_y of an output that starts at an odd place."""
+    M, K = X.shape
+    x = torch.full((M, pitch_x), float("nan"), dtype=X.dtype, device=DEV)
+    x[:, :K] = X.to(DEV)
+    flat = torch.full((M * pitch_y + offset_y + 64,), 7.0, dtype=X.dtype, device=DEV)
+    y = flat[offset_y:offset_y + M * pitch_y].view(M, pitch_y)
+    matmul_transpose_assign(x[:, :K], y[:, :M])
+    assert bool((y[:, M:] == 7.0).all()) and bool((flat[:offset_y] == 7.0).all()) and bool((flat[offset_y + M * pitch_y:] == 7.0).all())
+    return y[:, :M].cpu()
+
+
+# (M, K): sides one around whole tiles, tails of 8 and 56, K of one stage and a tail; 300 tiles, whole and (copied, in two
+# pieces per CU) partly cut; 45 and 15 tiles in pieces, more than one round of tiles and a cut rest behind it; copied inputs (K
+# odd, K below one stage, both sides padded); odd numbers of whole tiles, uncut and cut; 153 of them (the older path)
+@pytest.mark.parametrize("M,K", [(1024, 72), (1023, 120), (1025, 128), (129, 520), (2999, 200), (4200, 136), (1100, 4088), (3000, 5000),
+                                 (4100, 4104), (513, 8184), (700, 333), (1500, 57), (1, 65544), (1030, 64), (4000, 1504), (1408, 256),
+                                 (4224, 128), (1152, 4096), (2176, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_integers_bit_exact(M, K, dtype):
+    X = _ints(M, K, M + K, dtype)
+    want = (X.double() @ X.double().T).to(dtype)
+    got = _run(X, K, M)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("pitch_x,pitch_y,offset_y", [(400, 777, 0), (408, 784, 8), (401, 776, 0), (400, 778, 3), (392, 777, 1)])
+def test_pitches_and_alignment(pitch_x, pitch_y, offset_y):
+    X = _ints(776, 392, 5, torch.bfloat16)
+    want = (X.double() @ X.double().T).bfloat16()
+    assert torch.equal(_run(X, pitch_x, pitch_y, offset_y), want)
+
+
+def test_infinities_beside_the_rows():
+    """What lies beyond a row's end takes no part, also where it is the next row's infinities."""
+    X = torch.ones(600, 200, dtype=torch.bfloat16)
+    X[:, :8] = 2.0
+    X[300, 0] = float("inf")
+    got = _run(X, 200, 600)
+    want = (X.double() @ X.double().T).to(torch.bfloat16)
+    assert torch.equal(got, want)
