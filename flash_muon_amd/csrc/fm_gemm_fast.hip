@@ -12,7 +12,7 @@
 // workgroup, which go to memory as fp32 and are added in part order by a second, small kernel that
 // also runs the epilogue.  A product whose 128x256 half tiles fit into one round runs on those, and
 // one of at most 16 tiles may run on sub-tiles altogether.
-#include "fm_internal.h"
+#include "fm_tile128.h"
 
 #include <type_traits>
 #include <cstdlib>
@@ -1847,6 +1847,40 @@ __global__ __launch_bounds__(256) void gemm_nt_mid_kernel(GemmArgs gb, MidSplit 
   epilogue_quarter<F16>(g, diag, F, e_buf, RA, 0, row0, col0, lane, 0, 8, 3);
 }
 
+// The same tiles by workgroups that share a CU in pairs (fm_tile128.h), for more whole tiles than CUs: one workgroup's
+// start, first stages and write-out lie under the other's multiplications, where the kernel above leaves them bare
+// between its tiles.  X' of 1664 x 6400 (650 tiles of 26 stages) 60 -> 46 us, fast_newtonschulz(5) of it 596 -> 527, of 1408 x 5632
+// 436 -> 377, 2 of 1600^2 393 -> 345.  Bound by the copies into the LDS (fm_gemm_ragged.hip): 0.43 us a stage, tile and CU.
+template <bool F16>
+__global__ __launch_bounds__(256, 2) void gemm_nt_pair_kernel(GemmArgs gb) {
+  __shared__ __align__(1024) unsigned char smem[t128::SMEM];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // workgroups are dealt round-robin to the 8 XCDs: give each XCD a contiguous run of tiles
+  int w = (int)blockIdx.x;
+  {
+    const int chunk = (int)gridDim.x >> 3;
+    if (w < chunk * 8) w = (w & 7) * chunk + (w >> 3);
+  }
+  int bi, ti, tj;
+  tile_at(gb, w, bi, ti, tj);
+  const GemmArgs g = batch_view(gb, bi);
+  uint32_t voA[4], voB[4];
+  t128::copy_offsets(voA, voB, (int)g.lda, (int)g.ldb, lane, wave);
+  f32x4_t acc[4][4];
+  const t128::Lane L = t128::lane_setup(smem, lane, wave);
+  t128::main_loop<F16>(acc, g.Kc / BKF, smem, L, voA, voB, g.A + (int64_t)ti * MID_T * g.lda, g.B + (int64_t)tj * MID_T * g.ldb, nullptr);
+  t128::Out o;
+  o.ET = g.E ? g.ET : nullptr;
+  o.ldet = (int)g.ldet;
+  o.C = g.C; o.c_rs = g.c_rs;
+  o.C2 = g.C2; o.c2_rs = g.c2_rs;
+  o.alpha = g.alpha; o.beta = g.beta;
+  o.row_alpha = g.row_alpha;
+  o.diag_out = g.diag_out;
+  t128::write_block<F16, 0>(o, g.symmetric && ti == tj, acc, smem + wave * 16384, ti * MID_T + (wave >> 1) * 64, tj * MID_T + (wave & 1) * 64, lane);
+}
+
 // Second kernel of the cut 128x128 tiles: one workgroup per (tile, quarter).  Its four waves add
 // the quarter's parts in k order, so the bits do not depend on which workgroup finished when, and
 // share the iterations of its epilogue.
@@ -2086,6 +2120,12 @@ bool gemm_fast_eligible(const GemmArgs& a) {
 
 bool gemm_mid_eligible(const GemmArgs& a) { return tiled_dma_eligible(a, MID_T); }
 
+// (with up to one tile per CU the deeper ring of gemm_nt_mid_kernel is as fast or faster: 2048^2 19.2 us, 20.2 in pairs)
+// what gemm_nt_pair_kernel asks for besides: E through its transpose
+static bool pair_eligible(const GemmArgs& a) {
+  return !a.E || (a.ET && a.ldet % 8 == 0 && a.ldet < (1 << 21) && (reinterpret_cast<uintptr_t>(a.ET) & 15) == 0 && (a.batch < 2 || a.bs_et % 8 == 0));
+}
+
 int launch_gemm_mid(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) {
   a.tiles_m = a.Ma / MID_T;
   a.tiles_n = a.Nb / MID_T;
@@ -2097,6 +2137,11 @@ int launch_gemm_mid(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) {
   // without room for the parts the tiles stay whole
   if (sp.ksplit > 1 && (!ws || (size_t)a.num_tiles * sp.ksplit * MID_PART_FLOATS * sizeof(float) > ws_bytes)) sp.ksplit = 1;
   const unsigned grid = (unsigned)(a.num_tiles * sp.ksplit);
+  if (sp.ksplit == 1 && a.num_tiles > cu_count() && pair_eligible(a)) {
+    if (a.elem == kElemF16) hipLaunchKernelGGL(gemm_nt_pair_kernel<true>, dim3(grid), dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL(gemm_nt_pair_kernel<false>, dim3(grid), dim3(256), 0, stream, a);
+    return (int)hipGetLastError();
+  }
   if (a.elem == kElemF16) hipLaunchKernelGGL(gemm_nt_mid_kernel<true>, dim3(grid), dim3(256), 0, stream, a, sp);
   else hipLaunchKernelGGL(gemm_nt_mid_kernel<false>, dim3(grid), dim3(256), 0, stream, a, sp);
   if (sp.ksplit > 1) {
