@@ -431,10 +431,11 @@ size_t fm_newtonschulz_workspace_bytes(int rows, int cols) {
   return fm_newtonschulz_batched_workspace_bytes(1, rows, cols);
 }
 
-int fm_newtonschulz_batched_bf16(const void* const* G, int dtype, int batch, int rows, int cols,
-                                 int64_t ldg, void* const* out, int64_t ldout, int steps, float a,
-                                 float b, float c, float eps, void* ws, size_t ws_bytes,
-                                 fm_stream_t stream) {
+// the momentum update that comes before: of g and buf, one of which is G
+struct NsMomentum { void* const* g; void* const* buf; float w_buf, w_nes; int nesterov; };
+
+static int ns_impl(const void* const* G, int dtype, int batch, int rows, int cols, int64_t ldg, void* const* out, int64_t ldout, int steps,
+                   float a, float b, float c, float eps, void* ws, size_t ws_bytes, fm_stream_t stream, const NsMomentum* mom) {
   if (bad_dtype(dtype)) return FM_ERR_DTYPE;
   if (rows < 0 || cols < 0 || steps < 0 || batch < 0 || batch > kMaxBatch) return FM_ERR_SHAPE;
   if (rows == 0 || cols == 0 || batch == 0) return FM_OK;
@@ -462,6 +463,19 @@ int fm_newtonschulz_batched_bf16(const void* const* G, int dtype, int batch, int
         return FM_ERR_ALIAS;
   }
 
+  // sums of squares of G, behind its momentum update or with it
+  auto squares = [&](float* partials, unsigned* zero, int n_zero) -> int {
+    hipStream_t hs = static_cast<hipStream_t>(stream);
+    const int64_t n = (int64_t)rows * cols;
+    int rc = 0;
+    if (mom) {
+      if (launch_momentum_sumsq_batched(mom->g, mom->buf, batch, dtype, n, mom->w_buf, mom->w_nes, mom->nesterov, partials, hs, zero, n_zero, &rc))
+        return rc;
+      rc = launch_momentum_nesterov_batched(mom->g, mom->buf, batch, dtype, n, mom->w_buf, mom->w_nes, mom->nesterov, hs);
+      if (rc) return rc;
+    }
+    return launch_sumsq_parts_batched(G, batch, dtype, rows, cols, ldg, partials, hs, zero, n_zero);
+  };
   unsigned char* w = static_cast<unsigned char*>(ws);
   if (l.flow && steps > 0) {
     hipStream_t hs = static_cast<hipStream_t>(stream);
@@ -472,7 +486,7 @@ int fm_newtonschulz_batched_bf16(const void* const* G, int dtype, int batch, int
     const int n_counters = flow_counter_words(batch, steps < kFlowSteps ? steps : kFlowSteps);
     const int64_t mk = (int64_t)l.M * l.K;
     bf16_t* X = reinterpret_cast<bf16_t*>(w + l.x[0]);
-    if (launch_sumsq_parts_batched(G, batch, dtype, rows, cols, ldg, sumsq, hs, counters, n_counters)) return FM_ERR_LAUNCH;
+    if (squares(sumsq, counters, n_counters)) return FM_ERR_LAUNCH;
     bf16_t* x[kMaxBatch];
     for (int i = 0; i < batch; ++i) x[i] = X + i * mk;
     if (launch_scale_cast_batched(G, batch, dtype, rows, cols, ldg, sumsq, parts, eps, tall ? nullptr : x, l.K, tall ? x : nullptr, l.K,
@@ -522,9 +536,7 @@ int fm_newtonschulz_batched_bf16(const void* const* G, int dtype, int batch, int
     float* sumsq = reinterpret_cast<float*>(w + l.partials);
     const int parts = sumsq_parts((int64_t)rows * cols);
     const bool word = steps > 0 && gws_bytes >= 256;
-    if (launch_sumsq_parts_batched(G, batch, dtype, rows, cols, ldg, sumsq, hs,
-                                   word ? reinterpret_cast<unsigned*>(w + l.total - 256) : nullptr, word ? 64 : 0))
-      return FM_ERR_LAUNCH;
+    if (squares(sumsq, word ? reinterpret_cast<unsigned*>(w + l.total - 256) : nullptr, word ? 64 : 0)) return FM_ERR_LAUNCH;
     bf16_t* d[kMaxBatch];
     bf16_t* t[kMaxBatch];
     for (int i = 0; i < batch; ++i) {
@@ -596,6 +608,13 @@ int fm_newtonschulz_batched_bf16(const void* const* G, int dtype, int batch, int
   return FM_OK;
 }
 
+int fm_newtonschulz_batched_bf16(const void* const* G, int dtype, int batch, int rows, int cols,
+                                 int64_t ldg, void* const* out, int64_t ldout, int steps, float a,
+                                 float b, float c, float eps, void* ws, size_t ws_bytes,
+                                 fm_stream_t stream) {
+  return ns_impl(G, dtype, batch, rows, cols, ldg, out, ldout, steps, a, b, c, eps, ws, ws_bytes, stream, nullptr);
+}
+
 int fm_newtonschulz_bf16(const void* G, int dtype, int rows, int cols, int64_t ldg, void* out,
                          int64_t ldout, int steps, float a, float b, float c, float eps, void* ws,
                          size_t ws_bytes, fm_stream_t stream) {
@@ -619,11 +638,7 @@ int fm_momentum_nesterov(void* g, void* buf, int dtype, int64_t n, float w_buf, 
                                              static_cast<hipStream_t>(stream)));
 }
 
-int fm_momentum_nesterov_batched(void* const* g, void* const* buf, int batch, int dtype, int64_t n,
-                                 float w_buf, float w_nes, int nesterov, fm_stream_t stream) {
-  if (bad_dtype(dtype)) return FM_ERR_DTYPE;
-  if (n < 0 || batch < 0 || batch > kMaxBatch) return FM_ERR_SHAPE;
-  if (n == 0 || batch == 0) return FM_OK;
+static int momentum_checks(void* const* g, void* const* buf, int batch, int dtype, int64_t n) {
   if (!g || !buf) return FM_ERR_NULL;
   const int esz = dtype_size(dtype);
   for (int i = 0; i < batch; ++i) {
@@ -636,8 +651,41 @@ int fm_momentum_nesterov_batched(void* const* g, void* const* buf, int batch, in
         return FM_ERR_ALIAS;
     }
   }
+  return FM_OK;
+}
+
+int fm_momentum_nesterov_batched(void* const* g, void* const* buf, int batch, int dtype, int64_t n,
+                                 float w_buf, float w_nes, int nesterov, fm_stream_t stream) {
+  if (bad_dtype(dtype)) return FM_ERR_DTYPE;
+  if (n < 0 || batch < 0 || batch > kMaxBatch) return FM_ERR_SHAPE;
+  if (n == 0 || batch == 0) return FM_OK;
+  const int rc = momentum_checks(g, buf, batch, dtype, n);
+  if (rc != FM_OK) return rc;
   return hip_status(launch_momentum_nesterov_batched(g, buf, batch, dtype, n, w_buf, w_nes, nesterov,
                                                      static_cast<hipStream_t>(stream)));
+}
+
+int fm_momentum_newtonschulz_batched(void* const* g, void* const* buf, int dtype, int batch, int rows, int cols, float w_buf,
+                                     float w_nes, int nesterov, void* const* out, int64_t ldout, int steps, float a, float b,
+                                     float c, float eps, void* ws, size_t ws_bytes, fm_stream_t stream) {
+  if (bad_dtype(dtype)) return FM_ERR_DTYPE;
+  if (rows < 0 || cols < 0 || batch < 0 || batch > kMaxBatch) return FM_ERR_SHAPE;
+  if (rows == 0 || cols == 0 || batch == 0) return FM_OK;
+  const int64_t n = (int64_t)rows * cols;
+  const int rc = momentum_checks(g, buf, batch, dtype, n);
+  if (rc != FM_OK) return rc;
+  if (!out) return FM_ERR_NULL;
+  // what is not orthogonalised is written too: neither outputs nor scratch may lie on it
+  void* const* const other = nesterov ? buf : g;
+  const Range w = {reinterpret_cast<uintptr_t>(ws), reinterpret_cast<uintptr_t>(ws) + ws_bytes};
+  for (int i = 0; i < batch; ++i) {
+    const Range r = mat_range(other[i], rows, cols, cols, dtype_size(dtype));
+    if (overlaps(r, w)) return FM_ERR_ALIAS;
+    for (int j = 0; j < batch; ++j)
+      if (overlaps(r, mat_range(out[j], rows, cols, ldout, 2))) return FM_ERR_ALIAS;
+  }
+  const NsMomentum mom = {g, buf, w_buf, w_nes, nesterov};
+  return ns_impl(nesterov ? g : buf, dtype, batch, rows, cols, cols, out, ldout, steps, a, b, c, eps, ws, ws_bytes, stream, &mom);
 }
 
 int fm_weight_update_batched(void* const* p, int p_dtype, const void* const* u_bf16, int batch, int64_t n,

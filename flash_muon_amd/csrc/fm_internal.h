@@ -184,6 +184,8 @@ int launch_sumsq(const void* G, int dtype, int rows, int cols, int64_t ldg, floa
 int launch_scale_cast(const void* G, int dtype, int rows, int cols, int64_t ldg,
                       const float* sumsq, float eps, bf16_t* D, int64_t ldd, bf16_t* T, int64_t ldt,
                       hipStream_t stream);
+bool launch_momentum_sumsq_batched(void* const* g, void* const* buf, int batch, int dtype, int64_t n, float w_buf, float w_nes, int nesterov,
+                                   float* partials, hipStream_t stream, unsigned* zero, int n_zero, int* rc);
 int launch_momentum_nesterov_batched(void* const* g, void* const* buf, int batch, int dtype, int64_t n,
                                      float w_buf, float w_nes, int nesterov, hipStream_t stream);
 int launch_weight_update_batched(void* const* p, const bf16_t* const* u, int batch, int p_dtype, int64_t n,

@@ -211,27 +211,27 @@ class Muon(torch.optim.Optimizer):
                             buf = state["momentum_buffer"] = buf.contiguous()
                         gcs.append(g if g.is_contiguous() else g.contiguous())
                         bufs.append(buf)
-                    # buf.lerp_(g, 1 - mu); g.lerp_(buf, mu) in place on p.grad (muon.py:99-100),
-                    # one launch for the chunk
+                    shape = gcs[0].shape
+                    if len(shape) == 4:   # conv filters (muon.py:101-102)
+                        shape = (shape[0], gcs[0].numel() // shape[0] if shape[0] else 0)
+                    assert len(shape) == 2, "Input `d_in` must be a 2D tensor"
+                    # buf.lerp_(g, 1 - mu); g.lerp_(buf, mu) in place on p.grad (muon.py:99-100), and the
+                    # orthogonalisation (muon.py:103) of g or buf into rows of the staging buffer
+                    rows, cols = shape
+                    a, b, c = NS_COEFFS
                     with _lib.on_device(dev):
-                        st = lib.fm_momentum_nesterov_batched(
+                        ws, ws_bytes = _lib.workspace(lib.fm_newtonschulz_batched_workspace_bytes(n, rows, cols), dev)
+                        st = lib.fm_momentum_newtonschulz_batched(
                             (ctypes.c_void_p * n)(*[t.data_ptr() for t in gcs]),
                             (ctypes.c_void_p * n)(*[t.data_ptr() for t in bufs]),
-                            n, _lib.dtype_code(gcs[0].dtype), gcs[0].numel(), 1 - mu, mu,
-                            1 if nesterov else 0, stream)
-                    _lib.check("fm_momentum_nesterov_batched", st)
-                    srcs = []
-                    for p, gc, buf in zip(chunk, gcs, bufs):
-                        if gc is not p.grad and nesterov:
-                            p.grad.copy_(gc)
-                        src = gc if nesterov else buf
-                        if src.ndim == 4:   # conv filters (muon.py:101-102)
-                            src = src.view(len(src), -1)
-                        assert src.ndim == 2, "Input `d_in` must be a 2D tensor"
-                        srcs.append(src)
-                    # orthogonalise (muon.py:103) into rows of the staging buffer
-                    outs = [staging[i].view(srcs[i].shape) for i in range(n)]
-                    _newtonschulz_into(srcs, outs, group["ns_steps"])
+                            _lib.dtype_code(gcs[0].dtype), n, rows, cols, 1 - mu, mu, 1 if nesterov else 0,
+                            (ctypes.c_void_p * n)(*[staging[i].data_ptr() for i in range(n)]), cols,
+                            group["ns_steps"], a, b, c, NS_EPS, ws.data_ptr() if ws is not None else None, ws_bytes, stream)
+                    _lib.check("fm_momentum_newtonschulz_batched", st)
+                    if nesterov:
+                        for p, gc in zip(chunk, gcs):
+                            if gc is not p.grad:
+                                p.grad.copy_(gc)
                     # p *= 1 - lr*wd ; p += -lr*sqrt(max(1, rows/cols)) * update (muon.py:87-89),
                     # one launch for the chunk (same shape, so the same scale)
                     pcs = [p if p.is_contiguous() else p.contiguous() for p in chunk]

@@ -264,6 +264,14 @@ FM_API int fm_momentum_nesterov(void* g, void* buf, int dtype, int64_t n, float 
 FM_API int fm_weight_update(void* p, int p_dtype, const void* u_bf16, int64_t n, float decay_mul,
                      float alpha, fm_stream_t stream);
 
+/* fm_momentum_nesterov_batched of `batch` dense rows x cols tensors, then fm_newtonschulz_batched_bf16 of g (nesterov) or
+ * buf: the same results, bit for bit, in one call that reads the updated tensors once less.  `ws` as for the latter,
+ * fm_newtonschulz_batched_workspace_bytes(batch, rows, cols).  Neither g, buf, out nor ws may overlap another.
+ * flash_muon/muon.py:99-103. */
+FM_API int fm_momentum_newtonschulz_batched(void* const* g, void* const* buf, int dtype, int batch, int rows, int cols, float w_buf,
+                                            float w_nes, int nesterov, void* const* out, int64_t ldout, int steps, float a, float b,
+                                            float c, float eps, void* ws, size_t ws_bytes, fm_stream_t stream);
+
 /* ---------------------------------------------------------------------------------------------
  * The two updates above for `batch` (1..32) tensors of n elements each in one launch: g, buf, p and
  * u_bf16 are HOST arrays of `batch` device pointers; tensor i gets exactly what the single-tensor
