@@ -252,7 +252,7 @@ __global__ __launch_bounds__(256) void scale_cast_kernel(PtrList Gl, int rows, i
   }
 }
 
-// The same for whole 128x128 tiles of 16-byte aligned matrices with nothing to pad: a lane moves 8
+// The same for whole 128x128 tiles of 16-byte aligned matrices, and whole tiles of padding: a lane moves 8
 // columns of two rows at a time (256 contiguous bytes of G, D and T per 16 lanes), and the tile
 // goes through LDS as 32-bit words (rows 2 p and 2 p + 1 of one column), so that a row of T leaves
 // in 16-byte reads: word p of column c sits at word p ^ 4 (c / 8 % 16) of the column's 64, which
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(256) void scale_cast_kernel(PtrList Gl, int rows, i
 template <int DT, bool HAS_D>
 __global__ __launch_bounds__(256) void scale_cast_tile128_kernel(PtrList Gl, int64_t ldg, const float* sumsq,
                                                                  int parts, float eps, PtrList Dl, int64_t ldd,
-                                                                 PtrList Tl, int64_t ldt) {
+                                                                 PtrList Tl, int64_t ldt, int tiles_r, int tiles_c) {
   typedef typename Elem<DT>::raw raw;
   __shared__ __align__(16) uint32_t tile[128 * 64];
   const raw* G = reinterpret_cast<const raw*>(Gl.p[blockIdx.z]) + (int64_t)blockIdx.y * 128 * ldg + blockIdx.x * 128;
@@ -275,10 +275,16 @@ __global__ __launch_bounds__(256) void scale_cast_tile128_kernel(PtrList Gl, int
 
   union In { uint4 v[NV]; raw e[8]; };
   In in[4][2];
+  const bool there = (int)blockIdx.y < tiles_r && (int)blockIdx.x < tiles_c;   // a tile of G, and not of the padding
 #pragma unroll
   for (int pass = 0; pass < 4; ++pass)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
+      if (!there) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) in[pass][h].v[q] = uint4{0u, 0u, 0u, 0u};
+        continue;
+      }
       const raw* src = G + (int64_t)(2 * (pass * 16 + (tid >> 4)) + h) * ldg + ch * 8;
 #pragma unroll
       for (int q = 0; q < NV; ++q) in[pass][h].v[q] = reinterpret_cast<const uint4*>(src)[q];
@@ -291,7 +297,7 @@ __global__ __launch_bounds__(256) void scale_cast_tile128_kernel(PtrList Gl, int
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[h].h[e] = Elem<0>::st(as_bf16_value<DT>(in[pass][h].e[e]) / denom);
+      for (int e = 0; e < 8; ++e) o[h].h[e] = there ? Elem<0>::st(as_bf16_value<DT>(in[pass][h].e[e]) / denom) : (unsigned short)0;
       if constexpr (HAS_D) *reinterpret_cast<uint4*>(D + (int64_t)(2 * rp + h) * ldd + ch * 8) = o[h].v;
     }
     uint32_t* const col = tile + (ch * 8) * 64 + (rp ^ (4 * ch));   // columns 8 ch .. + 7 share ch = column / 8 % 16
@@ -371,10 +377,10 @@ int launch_scale_cast_batched(const void* const* G, int batch, int dtype, int ro
 #undef FM_SCALE_ROWS
     return (int)hipGetLastError();
   }
-  if (T && gv && (dv || !D) && tv && rows_p == rows && cols_p == cols && rows % 128 == 0 && cols % 128 == 0) {
-    dim3 grid128((unsigned)(cols / 128), (unsigned)(rows / 128), (unsigned)batch);
+  if (T && gv && (dv || !D) && tv && rows_p % 128 == 0 && cols_p % 128 == 0 && rows % 128 == 0 && cols % 128 == 0) {
+    dim3 grid128((unsigned)(cols_p / 128), (unsigned)(rows_p / 128), (unsigned)batch);
 #define FM_SCALE128(DT, HAS_D) hipLaunchKernelGGL((scale_cast_tile128_kernel<DT, HAS_D>), grid128, dim3(256), 0, stream, gl, ldg, \
-                                                  sumsq, parts, eps, dl, ldd, tl, ldt)
+                                                  sumsq, parts, eps, dl, ldd, tl, ldt, rows / 128, cols / 128)
     if (dtype == 0) { if (D) FM_SCALE128(0, true); else FM_SCALE128(0, false); }
     else if (dtype == 1) { if (D) FM_SCALE128(1, true); else FM_SCALE128(1, false); }
     else { if (D) FM_SCALE128(2, true); else FM_SCALE128(2, false); }

@@ -213,6 +213,7 @@ static int launch_cfg(GemmArgs a, bool aligned, hipStream_t stream) {
 }
 
 int launch_gemm_general(GemmArgs a, hipStream_t stream) {
+  if (a.rows_v) { a.Ma = a.rows_v; a.Nb = a.cols_v; }   // any shape will do here
   const bool aligned = (a.lda % 8 == 0) && (a.ldb % 8 == 0) && (a.Kc % 8 == 0) &&
                        ((reinterpret_cast<uintptr_t>(a.A) & 15) == 0) &&
                        ((reinterpret_cast<uintptr_t>(a.B) & 15) == 0);

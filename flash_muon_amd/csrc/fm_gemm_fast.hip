@@ -457,6 +457,7 @@ template <bool F16>
 __device__ __forceinline__ void epilogue_quarter(const GemmArgs& g, bool diag, float* F, const unsigned char* Eb,
                                                  const float* RA, int ra_off, int row_base, int col_base,
                                                  int lane, int it_begin, int it_end, int passes) {
+  if (!block_written(g, row_base, col_base)) return;
   if constexpr (!F16) {   // fp16 problems carry no operand E
     if (g.E) {
       if (diag) epilogue_quarter_t<false, true, true>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
@@ -752,8 +753,9 @@ __device__ __forceinline__ void epilogue_regs16(const GemmArgs& g, bool diag, in
   asm volatile("" : "+v"(lane));
   constexpr bool has_e = !F16 && MODE != 0;
   const int n = lane & 15, grp = lane >> 4;
-  const bool direct = g.C != nullptr;
-  const bool mirror = g.C2 != nullptr && !diag;
+  const bool written = block_written(g, row0, col0);
+  const bool direct = g.C != nullptr && written;
+  const bool mirror = g.C2 != nullptr && !diag && written;
   const bool dout = diag && g.diag_out != nullptr;
   const float alpha = g.alpha, beta = g.beta;
   float* const RA = reinterpret_cast<float*>(T + QT_BYTES);
@@ -1277,7 +1279,8 @@ __device__ __forceinline__ void sub64_tile(const GemmArgs& g, int ti, int tj, in
   // hold each other's, bit for bit): such a sub-tile is written once, by the direct pass
   const bool bdiag = tdiag && si == sj;
   const bool use_e = !F16 && g.E != nullptr;
-  const bool mirror = !bdiag && g.C2 != nullptr;
+  const bool written = block_written(g, m0, n0);
+  const bool mirror = !bdiag && g.C2 != nullptr && written;
   {
     const int r = lane >> 1, c0 = (lane & 1) * 16;
     const int row = row0 + r, col = col0 + c0;
@@ -1310,7 +1313,7 @@ __device__ __forceinline__ void sub64_tile(const GemmArgs& g, int ti, int tj, in
       o.h[k] = f32_to_elem<F16>(v[k]);
       if (mirror) F[(c0 + k) * SUB_F_PITCH + r] = elem_to_f32<F16>(o.h[k]);
     }
-    if (g.C) {
+    if (g.C && written) {
       uint4* dst = reinterpret_cast<uint4*>(reinterpret_cast<unsigned short*>(g.C) + (int64_t)row * g.c_rs + col);
       dst[0] = o.q[0];
       dst[1] = o.q[1];
@@ -1870,6 +1873,7 @@ __global__ __launch_bounds__(256, 2) void gemm_nt_pair_kernel(GemmArgs gb) {
   f32x4_t acc[4][4];
   const t128::Lane L = t128::lane_setup(smem, lane, wave);
   t128::main_loop<F16>(acc, g.Kc / BKF, smem, L, voA, voB, g.A + (int64_t)ti * MID_T * g.lda, g.B + (int64_t)tj * MID_T * g.ldb, nullptr);
+  if (!block_written(g, ti * MID_T, tj * MID_T)) return;
   t128::Out o;
   o.ET = g.E ? g.ET : nullptr;
   o.ldet = (int)g.ldet;

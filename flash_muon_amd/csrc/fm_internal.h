@@ -109,6 +109,7 @@ struct GemmArgs {
   float alpha, beta;
   const float* row_alpha;   // optional per-row addition to alpha
   float* diag_out;          // optional fp32 copy of the diagonal, which is then stored as zero
+  int rows_v, cols_v;       // of C (columns and rows of C2), whole multiples of 128: what lies beyond is not written; 0: all of it
   int symmetric;
   int elem;                 // element type of A, B, C, C2: kElemBf16 or kElemF16
   // `batch` independent problems of the same shape in one launch: matrix b of an operand starts
@@ -123,6 +124,9 @@ struct GemmArgs {
   int num_tiles;          // tiles actually computed, over the whole batch
   int diag_last;          // 256x256 schedule, one symmetric matrix: its last `diag_last` diagonal tiles end the tile order
 };
+
+// whether the block of C at (row, col), of at most 128x128 and on a multiple of its size, is written
+__host__ __device__ inline bool block_written(const GemmArgs& g, int row, int col) { return g.rows_v == 0 || (row < g.rows_v && col < g.cols_v); }
 
 // the arguments of matrix b of a batch, as a single-matrix problem
 __host__ __device__ inline GemmArgs batch_view(const GemmArgs& g, int b) {
