@@ -85,7 +85,15 @@ __global__ __launch_bounds__(256) void sumsq_partial_kernel(PtrList Gl, int rows
     const int64_t nv = n / V, per = units_per_block(nv, (int)gridDim.x), i0 = blockIdx.x * per;
     const int64_t i1 = i0 + per < nv ? i0 + per : nv;
     const uint4* G4 = reinterpret_cast<const uint4*>(Gv);
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += 256) {
+    int64_t i = i0 + threadIdx.x;
+    for (; i + 768 < i1; i += 1024) {   // four loads on their way at a time
+      union { uint4 v; raw e[V]; } u[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) u[k].v = G4[i + 256 * k];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) add_squares<DT>(s4, u[k].e);
+    }
+    for (; i < i1; i += 256) {
       union { uint4 v; raw e[V]; } u;
       u.v = G4[i];
       add_squares<DT>(s4, u.e);
@@ -500,14 +508,26 @@ __global__ __launch_bounds__(256) void momentum_sumsq_kernel(PtrList gl, PtrList
     for (int i = (int)blockIdx.x * 256 + (int)threadIdx.x; i < n_zero; i += (int)gridDim.x * 256) zero[i] = 0u;
   const int64_t per = units_per_block(nv, (int)gridDim.x), i0 = blockIdx.x * per, i1 = i0 + per < nv ? i0 + per : nv;
   float s4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int64_t i = i0 + threadIdx.x; i < i1; i += 256) {
-    union { uint4 v; raw e[V]; } ug, ub;
-    ug.v = ld_stream(g4 + i); ub.v = ld_stream(b4 + i);
+  union Unit { uint4 v; raw e[V]; };
+  auto update = [&](int64_t i, Unit& ug, Unit& ub) {
 #pragma unroll
     for (int e = 0; e < V; ++e) momentum_one<DT>(ug.e[e], ub.e[e], w_buf, w_nes, nesterov);
     st_stream(b4 + i, ub.v);
     if (nesterov) st_stream(g4 + i, ug.v);
     add_squares<DT>(s4, nesterov ? ug.e : ub.e);
+  };
+  int64_t i = i0 + threadIdx.x;
+  for (; i + 256 < i1; i += 512) {   // two units' loads on their way at a time
+    Unit ug[2], ub[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) { ug[k].v = ld_stream(g4 + i + 256 * k); ub[k].v = ld_stream(b4 + i + 256 * k); }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) update(i + 256 * k, ug[k], ub[k]);
+  }
+  if (i < i1) {
+    Unit ug, ub;
+    ug.v = ld_stream(g4 + i); ub.v = ld_stream(b4 + i);
+    update(i, ug, ub);
   }
   const float s = block_sum<256>((s4[0] + s4[1]) + (s4[2] + s4[3]), red);
   if (threadIdx.x == 0) partials[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = s;
