@@ -43,8 +43,8 @@ constexpr int kFlowSteps = 5;   // steps per launch of the one-launch iteration
 // zero-padded to whole tiles instead: zero rows and columns stay zero through every step, and the
 // tiled paths run.  Whole 256x256 tiles pay for up to 128 more rows and columns, also where the
 // sides are whole multiples of 128 already, once the 256x256 path has enough of them: for a single
-// matrix from a short side of 2816 on (five steps at 3200^2 0.86 ms, padded to 3328^2 0.79; 3200 x 8000 1.66 and 1.55;
-// but 2176^2 0.407 and 0.422, 2688^2 0.509 and 0.539), for a batch as
+// matrix from a short side of 2176 on, of a square one of 2816 (five steps at 3200^2 0.86 ms, padded to 3328^2 0.79; 3200 x
+// 8000 1.66 and 1.55; 2176 x 4400 0.58 and 0.55; but 2176^2 0.407 and 0.422, 2688^2 0.509 and 0.539), for a batch as
 // soon as its 256x256 tiles fill the GPU (32 of 1664^2 4.6 ms, of 1792^2 4.2; 2688 x 7168 36 and
 // 2816 x 7168 26).  The long side alone goes to a multiple of 256 where the short one is one already
 // (32 of 2048 x 5504 15.4 ms, of 2048 x 5632 11.9; one matrix 0.72 and 0.59; below 1536 rows a single
@@ -105,7 +105,8 @@ NsLayout ns_layout(int batch, int rows, int cols) {
   l.K = (k + 127) / 128 * 128;
   {
     const int64_t t = (l.M + 255) / 256;
-    const bool both = l.M >= (batch == 1 ? 2816 : 2176) || (l.M >= 1152 && (int64_t)batch * t * (t + 1) / 2 >= 120);
+    const bool near_square = k < m + m / 5;
+    const bool both = l.M >= (batch == 1 && near_square ? 2816 : 2176) || (l.M >= 1152 && (int64_t)batch * t * (t + 1) / 2 >= 120);
     if (both) l.M = (int)t * 256;
     if (l.M % 256 == 0 && (both || l.M >= 1536 || (batch >= 4 && l.M >= 768))) l.K = (k + 255) / 256 * 256;
   }

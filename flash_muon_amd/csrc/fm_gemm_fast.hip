@@ -457,7 +457,7 @@ template <bool F16>
 __device__ __forceinline__ void epilogue_quarter(const GemmArgs& g, bool diag, float* F, const unsigned char* Eb,
                                                  const float* RA, int ra_off, int row_base, int col_base,
                                                  int lane, int it_begin, int it_end, int passes) {
-  if (!block_written(g, row_base, col_base)) return;
+  if (g.E && !block_written(g, row_base, col_base)) return;   // (only products with E leave blocks out)
   if constexpr (!F16) {   // fp16 problems carry no operand E
     if (g.E) {
       if (diag) epilogue_quarter_t<false, true, true>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
@@ -753,7 +753,7 @@ __device__ __forceinline__ void epilogue_regs16(const GemmArgs& g, bool diag, in
   asm volatile("" : "+v"(lane));
   constexpr bool has_e = !F16 && MODE != 0;
   const int n = lane & 15, grp = lane >> 4;
-  const bool written = block_written(g, row0, col0);
+  const bool written = !has_e || block_written(g, row0, col0);   // (only products with E leave blocks out)
   const bool direct = g.C != nullptr && written;
   const bool mirror = g.C2 != nullptr && !diag && written;
   const bool dout = diag && g.diag_out != nullptr;
@@ -1279,7 +1279,7 @@ __device__ __forceinline__ void sub64_tile(const GemmArgs& g, int ti, int tj, in
   // hold each other's, bit for bit): such a sub-tile is written once, by the direct pass
   const bool bdiag = tdiag && si == sj;
   const bool use_e = !F16 && g.E != nullptr;
-  const bool written = block_written(g, m0, n0);
+  const bool written = !use_e || block_written(g, m0, n0);   // (only products with E leave blocks out)
   const bool mirror = !bdiag && g.C2 != nullptr && written;
   {
     const int r = lane >> 1, c0 = (lane & 1) * 16;
@@ -1873,7 +1873,7 @@ __global__ __launch_bounds__(256, 2) void gemm_nt_pair_kernel(GemmArgs gb) {
   f32x4_t acc[4][4];
   const t128::Lane L = t128::lane_setup(smem, lane, wave);
   t128::main_loop<F16>(acc, g.Kc / BKF, smem, L, voA, voB, g.A + (int64_t)ti * MID_T * g.lda, g.B + (int64_t)tj * MID_T * g.ldb, nullptr);
-  if (!block_written(g, ti * MID_T, tj * MID_T)) return;
+  if (g.E && !block_written(g, ti * MID_T, tj * MID_T)) return;
   t128::Out o;
   o.ET = g.E ? g.ET : nullptr;
   o.ldet = (int)g.ldet;

@@ -109,7 +109,6 @@ struct GemmArgs {
   float alpha, beta;
   const float* row_alpha;   // optional per-row addition to alpha
   float* diag_out;          // optional fp32 copy of the diagonal, which is then stored as zero
-  int rows_v, cols_v;       // of C (columns and rows of C2), whole multiples of 128: what lies beyond is not written; 0: all of it
   int symmetric;
   int elem;                 // element type of A, B, C, C2: kElemBf16 or kElemF16
   // `batch` independent problems of the same shape in one launch: matrix b of an operand starts
@@ -123,6 +122,8 @@ struct GemmArgs {
   int tiles_m, tiles_n;   // number of block tiles along each output dimension of one matrix
   int num_tiles;          // tiles actually computed, over the whole batch
   int diag_last;          // 256x256 schedule, one symmetric matrix: its last `diag_last` diagonal tiles end the tile order
+  // with E: the rows and columns of C (columns and rows of C2) that are written, whole multiples of 128; 0: all of them
+  int rows_v, cols_v;
 };
 
 // whether the block of C at (row, col), of at most 128x128 and on a multiple of its size, is written
