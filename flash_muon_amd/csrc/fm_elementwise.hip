@@ -2,6 +2,7 @@
 // momentum / Nesterov update and the decayed weight update.  All are streaming kernels with
 // 16-byte accesses per lane on the aligned path and a scalar path for everything else.
 #include "fm_internal.h"
+#include "fm_routes.h"
 
 namespace fm {
 
@@ -373,10 +374,10 @@ int launch_scale_cast_batched(const void* const* G, int batch, int dtype, int ro
     if (D) { dl.p[i] = D[i]; dv = dv && (reinterpret_cast<uintptr_t>(D[i]) & 15) == 0; }
     if (T) { tl.p[i] = T[i]; tv = tv && (reinterpret_cast<uintptr_t>(T[i]) & 15) == 0; }
   }
-  if (D && !T && gv && dv && cols_p % 8 == 0 && (int64_t)rows_p * cols_p / 8 < (1LL << 31)) {
-    // 8 chunks per thread at most, so that a block's sum of the partial sums is paid for
-    const int64_t blocks = ((int64_t)rows_p * (cols_p / 8) + 1023) / 1024;
-    dim3 gridr((unsigned)blocks, 1, (unsigned)batch);
+  const int64_t row_blocks = D && !T && gv && dv && cols_p % 8 == 0 ? scale_cast_rows_blocks(rows_p, cols_p) : 0;
+  if (row_blocks > 0) {
+    // (4 chunks per thread, so that a block's sum of the partial sums is paid for)
+    dim3 gridr((unsigned)row_blocks, 1, (unsigned)batch);
 #define FM_SCALE_ROWS(DT) hipLaunchKernelGGL(scale_cast_rows_kernel<DT>, gridr, dim3(256), 0, stream, gl, rows, cols, rows_p, cols_p, \
                                              ldg, sumsq, parts, eps, dl, ldd)
     if (dtype == 0) FM_SCALE_ROWS(0);
