@@ -2,6 +2,7 @@
 // Newton-Schulz composition.  No torch types, no allocation, no synchronisation.
 #include "../../include/flashmuon.h"
 #include "fm_internal.h"
+#include "fm_routes.h"
 #include <atomic>
 
 using namespace fm;
@@ -49,26 +50,6 @@ constexpr int kFlowSteps = 5;   // steps per launch of the one-launch iteration
 // 2816 x 7168 26).  The long side alone goes to a multiple of 256 where the short one is one already
 // (32 of 2048 x 5504 15.4 ms, of 2048 x 5632 11.9; one matrix 0.72 and 0.59; below 1536 rows a single
 // matrix gains nothing).
-// Which matrices iterate in one launch (fm_flow.hip), and on which tiles: M x K with M <= K, `batch` of them.
-// Five steps in us, one launch / launches per product.  One or two matrices, whose products are chains of short launches:
-// 256^2 91 / 109, 1024^2 137 / 158, 1408^2 185 / 233, 1024 x 4096 209 / 234, 1408 x 2816 225 / 302, 2 of 640 x 2560 156 / 245, 2 of 1408^2 249 /
-// 285; but 1536^2 258 / 254, 1280 x 5120 383 / 304 (its first product is cut along k there), 2 of 768 x 3072 236 / 223.  More of
-// them, with an odd number of 128-tiles (padded to 256-tiles, or on tiles of 128 in launches): 12 of 1152^2 532 / 817, 16
-// of 1408^2 1009 / 1669, 6 of 1408 x 3872 976 / 1224, 12 of 1664^2 1253 / 1821, 32 of 1920^2 5273 / 5411; an even one, as long as the 256-tiles
-// do not fill the GPU by themselves: 24 of 768^2 360 / 393, 16 of 768 x 3072 672 / 972, 16 of 1280^2 817 / 911, 6 of 1280 x 3520 774 / 844, 24 of
-// 1536^2 2046 / 2102; but 6 of 768 x 3072 407 / 366, 6 of 1024 x 2048 424 / 377, 6 of 1280^2 451 / 423, 24 of 2048^2 4600 / 4200.
-bool ns_flow_chosen(int batch, int m, int k) {
-  const double r = (double)k / m;
-  if (k >= (1 << 21)) return false;   // in-tile byte offsets stay below 2^31
-  if (m <= 512) return true;
-  if (batch == 1) return m <= 1024 || (m <= 1408 && r <= 2.25);
-  if (batch == 2) return m <= 640 || (m <= 1408 && r <= 2.75);
-  const int T = (m + 127) / 128;
-  if (T & 1) return batch >= 4 ? m <= 1920 : m <= 1408 && r <= 2.75;
-  if (m <= 1024) return r <= 1.5 || batch >= 8 || (m > 768 && r > 3);
-  if (m <= 1280) return r <= 3.5 && (batch >= 12 || (batch >= 4 && r > 2.5));
-  return m <= 1536 && batch >= 16 && r <= 1.5;
-}
 // 64x64 tiles for X' as long as every CU gets at most one, and for the symmetric products as long as they are
 // about one round (a longer K makes the 64-tiles of A = X X^T pay a little further): 512^2 104 us on 64x64
 // tiles, 115 with X' on 128x128, 144 all on 128x128; 8 of 384 x 768 152, 111 and 133; 24 of 768^2 520, 423 and 360.

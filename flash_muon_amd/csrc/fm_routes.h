@@ -13,4 +13,47 @@ inline int64_t scale_cast_rows_blocks(int64_t rows_p, int64_t cols_p) {
   return chunks + blocks * 256 <= INT32_MAX ? blocks : 0;
 }
 
+// Which matrices iterate in one launch (fm_flow.hip): M x K with M <= K, `batch` of them.
+// Five steps in us, one launch / launches per product.  One or two matrices, whose products are chains of short launches:
+// 256^2 91 / 109, 1024^2 137 / 158, 1408^2 185 / 233, 1024 x 4096 209 / 234, 1408 x 2816 225 / 302, 2 of 640 x 2560 156 / 245, 2 of 1408^2 249 /
+// 285; but 1536^2 258 / 254, 1280 x 5120 383 / 304 (its first product is cut along k there), 2 of 768 x 3072 236 / 223.  More of
+// them, with an odd number of 128-tiles (padded to 256-tiles, or on tiles of 128 in launches): 12 of 1152^2 532 / 817, 16
+// of 1408^2 1009 / 1669, 6 of 1408 x 3872 976 / 1224, 12 of 1664^2 1253 / 1821, 32 of 1920^2 5273 / 5411; an even one, as long as the 256-tiles
+// do not fill the GPU by themselves: 24 of 768^2 360 / 393, 16 of 768 x 3072 672 / 972, 16 of 1280^2 817 / 911, 6 of 1280 x 3520 774 / 844, 24 of
+// 1536^2 2046 / 2102; but 6 of 768 x 3072 407 / 366, 6 of 1024 x 2048 424 / 377, 6 of 1280^2 451 / 423, 24 of 2048^2 4600 / 4200.
+inline bool ns_flow_pays(int batch, int m, int k) {
+  const double r = (double)k / m;
+  if (m <= 512) return true;
+  if (batch == 1) return m <= 1024 || (m <= 1408 && r <= 2.25);
+  if (batch == 2) return m <= 640 || (m <= 1408 && r <= 2.75);
+  const int T = (m + 127) / 128;
+  if (T & 1) return batch >= 4 ? m <= 1920 : m <= 1408 && r <= 2.75;
+  if (m <= 1024) return r <= 1.5 || batch >= 8 || (m > 768 && r > 3);
+  if (m <= 1280) return r <= 3.5 && (batch >= 12 || (batch >= 4 && r > 2.5));
+  return m <= 1536 && batch >= 16 && r <= 1.5;
+}
+// A long K: A = X X^T is whole tiles there, a chain of K / 64 stages (0.2 us each on a 64-tile), where a launch of its own is cut
+// along k; and X' is 128-tiles, where a launch of its own has 256-tiles once there are enough of them.  With x the 128-tiles of X':
+//   x about the CUs: up to K 8192.  512 x 8192 221 / 235 but x 10240 306 / 247, x 16384 398 / 275, x 65536 1268 / 629; 128 x 8192 166 / 179, x 16384
+//   264 / 198; 1024 x 4096 212 / 242 but x 5120 (320 tiles) 314 / 277, x 16384 562 / 445; 2 of 512 x 4096 168 / 228 but x 8192 302 / 263; 4 of 256 x
+//   8192 247 / 262;
+//   an odd number of tile rows, which the 256-tiles do not fit, and enough matrices: up to 32768.  16 of 640 x 12288 1959 / 2383, 8 of 896 x 16384
+//   2265 / 2464, 12 of 384 x 32768 2112 / 2281, but 4 of 576 x 131072 7547 / 6641;
+//   eight matrices or more: up to 8192 below 1024 tiles, then 16384, 32768 for 24 of them (8 of 256 x 16384 509 / 531, 24 of 512 x 24576
+//   4135 / 4206; but 8 of 128 x 16384 341 / 293, 8 of 512 x 24576 1682 / 1587, 16 of 256 x 24576 1353 / 1273), of more than 768 rows only while x <= 5000
+//   (12 of 1024 x 6144 1568 / 1759 but 16 of it 2031 / 1978, 12 of 1024 x 12288 3081 / 2910);
+//   fewer: one round of 256-tiles at most (x < 1024) up to K 4096 or 5120 (4 of 384 x 4096 206 / 245; but 2 of 512 x 5120 239 / 234, 3 of 512 x 6144
+//   318 / 287, 6 of 256 x 8192 307 / 267; not above 768 rows: 4 of 960 x 3072 441 / 379), and beyond it where the 256-tiles' last round is a fifth
+//   empty or more (4 of 1024 x 6144 679 / 822, 4 of 512 x 12288 481 / 631; but 4 of 1024 x 8192 921 / 817, 6 of 512 x 10240 633 / 585).
+inline bool ns_flow_short_enough(int batch, int m, int k) {
+  if (k <= 2048) return true;
+  const int64_t T = (m + 127) / 128, x = batch * T * ((k + 127) / 128);
+  if (x <= 280 || (m <= 256 && x <= 512)) return k <= 8192;
+  if ((T & 1) && T > 1 && batch * T >= 18) return k <= 32768;
+  if (batch >= 8) return k <= (x <= 1024 ? 8192 : batch < 24 ? 16384 : 32768) && (m <= 768 || k <= 4 * m || x <= 5000);
+  if (x < 1024) return (m <= 768 || 4 * (int64_t)k <= 11 * (int64_t)m) && k <= (batch <= 4 ? 4096 : 5120);
+  return k <= 12288 && x <= (x + 1023) / 1024 * 820;
+}
+inline bool ns_flow_chosen(int batch, int m, int k) { return ns_flow_pays(batch, m, k) && ns_flow_short_enough(batch, m, k); }
+
 }  // namespace fm

@@ -65,3 +65,13 @@ def test_concurrent_streams():
     torch.cuda.synchronize()
     for i, y in enumerate(got):
         assert torch.equal(y, want[i % len(Gs)])
+
+
+# a K of up to 8192 in one launch, the next one in launches per product, which cut the first product along k; more matrices, up to 16384 and beyond
+@pytest.mark.parametrize("rows,cols,batch", [(128, 8192, 1), (128, 8193, 1), (8200, 500, 1), (384, 9000, 8), (16400, 250, 8)])
+def test_long_rows_on_both_sides_of_the_rule(rows, cols, batch):
+    Gs = torch.stack([synthetic.gradient_like_bf16(rows, cols, 8, 30 + i % 2) for i in range(min(batch, 2))])
+    got = fast_newtonschulz(Gs.to(DEV)[torch.arange(batch) % len(Gs)] if batch > 1 else Gs[0].to(DEV), 5).view(batch, rows, cols)
+    for i in range(2, batch):
+        assert torch.equal(got[i], got[i % 2])
+    _check(got[0].cpu(), Gs[0], 5)

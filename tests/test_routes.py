@@ -12,6 +12,7 @@ HOST = """
 #include "fm_routes.h"
 extern "C" {
 long long scale_cast_rows_blocks(long long r, long long c) { return fm::scale_cast_rows_blocks(r, c); }
+int ns_flow_chosen(int batch, int m, int k) { return fm::ns_flow_chosen(batch, m, k); }
 }
 """
 
@@ -43,3 +44,22 @@ def test_the_walk_over_rows_stays_below_two_to_the_31(routes, rows, cols):
         assert max(beyond) <= INT32_MAX
     else:   # what is left to the kernel of 64x64 tiles is only what would not fit
         assert chunks + chunks // 4 > INT32_MAX - 1024
+
+
+# (batch, M, K, us in one launch, us in launches per product), measured; the first ones are ordinary ratios
+NS_TIMES = [(1, 1024, 4096, 212, 242), (2, 640, 2560, 156, 245), (6, 1408, 3872, 976, 1224), (16, 768, 3072, 672, 972), (4, 960, 3072, 441, 379),
+            (1, 512, 8192, 221, 235), (1, 512, 10240, 306, 247), (1, 512, 16384, 398, 275), (1, 512, 65536, 1268, 629), (1, 512, 32768, 386, 274),
+            (1, 128, 8192, 166, 179), (1, 128, 16384, 264, 198), (1, 1024, 5120, 314, 277), (1, 1024, 16384, 562, 445), (1, 768, 9216, 311, 265),
+            (2, 512, 4096, 168, 228), (2, 512, 8192, 302, 263), (4, 256, 8192, 247, 262), (6, 256, 8192, 307, 267), (4, 512, 12288, 481, 631),
+            (16, 640, 12288, 1959, 2383), (12, 384, 32768, 2112, 2281), (4, 576, 131072, 7547, 6641), (8, 256, 16384, 509, 531),
+            (8, 512, 24576, 1682, 1587), (8, 128, 16384, 341, 293), (12, 1024, 6144, 1568, 1759), (4, 1024, 6144, 679, 822), (4, 1024, 8192, 921, 817)]
+
+
+@pytest.mark.parametrize("batch,m,k,one,launches", NS_TIMES)
+def test_one_launch_newtonschulz_where_it_measured_faster(routes, lib, batch, m, k, one, launches):
+    assert bool(routes.ns_flow_chosen(batch, m, k)) == (one < launches)
+    # one launch keeps every step's iterate and squares, in either orientation of the matrices
+    if one < launches:
+        need = lib.fm_newtonschulz_batched_workspace_bytes(batch, m, k)
+        assert need >= batch * (6 * m * k + 10 * m * m) * 2
+        assert need == lib.fm_newtonschulz_batched_workspace_bytes(batch, k, m)
