@@ -184,22 +184,17 @@ static bool syrk_ragged_layout(int M, int K, SyrkRagged* p) {
   p->total = p->x + (whole_tiles(M, K) ? 0 : align_up((size_t)M * p->Kp * 2, 256)) + 256;
   return true;
 }
-// Both X and Y as copies padded to whole 256-tiles, for a matrix that has to be copied anyway: where the 256-tiles just
-// fill a round of half tiles (16 tile rows) or leave few workgroups idle (20 and 31: 210 and 496 tiles) while the
-// 128-tiles begin another round: 4000^2 77 us and 85 behind one copy, 4000 x 2000 51 and 55, 5000 x 3000 92 and 98, 7776^2 400 and
-// 448; but 3500^2 83 and 65, 5500^2 194 and 184 (22 tile rows), 7200^2 377 and 372 (29), 7500 x 4000 281 and 219 (30).
+// Both X and Y as copies padded to whole 256-tiles, where that is estimated to be faster (syrk_padded_pays).
 struct SyrkPad { int Mp, Kp; size_t x, y, gemm, total; };
-static bool syrk_pad_layout(int M, int K, SyrkPad* p) {
-  if (whole_tiles(M, K) || M <= 3968 || K < 1500) return false;
-  const int64_t T = (M + 255) / 256;
-  if (T != 16 && T != 20 && T != 31) return false;
-  p->Mp = (int)T * 256;
-  p->Kp = (K + 63) / 64 * 64;
-  p->x = 0;
-  p->y = align_up((size_t)p->Mp * p->Kp * 2, 256);
-  p->gemm = p->y + align_up((size_t)p->Mp * p->Mp * 2, 256);
-  p->total = p->gemm + gemm_fast_workspace_bytes(p->Mp, p->Mp, 1);
-  return true;
+static SyrkPad syrk_pad_layout(int M, int K) {
+  SyrkPad p;
+  p.Mp = (M + 255) / 256 * 256;
+  p.Kp = (K + 63) / 64 * 64;
+  p.x = 0;
+  p.y = align_up((size_t)p.Mp * p.Kp * 2, 256);
+  p.gemm = p.y + align_up((size_t)p.Mp * p.Mp * 2, 256);
+  p.total = p.gemm + gemm_fast_workspace_bytes(p.Mp, p.Mp, 1);
+  return p;
 }
 
 size_t fm_syrk_workspace_bytes(int M, int K) {
@@ -208,8 +203,11 @@ size_t fm_syrk_workspace_bytes(int M, int K) {
   SyrkRagged r;
   if (!syrk_ragged_layout(M, K, &r)) return need;
   if (r.total > need) need = r.total;
-  SyrkPad p;
-  if (syrk_pad_layout(M, K, &p) && p.total > need) need = p.total;
+  // (rows may lie on lines or not, and Y's rows allow 16-byte stores or not)
+  if ((K % 64 == 0 && syrk_padded_pays(M, K, true, true)) || (!whole_tiles(M, K) && syrk_padded_pays(M, K, false, true))) {
+    const SyrkPad p = syrk_pad_layout(M, K);
+    if (p.total > need) need = p.total;
+  }
   if (!whole_tiles(M, K)) {   // what the interface promises room for, whichever way is taken: X and Y padded to 128-tiles
     const size_t Mp = (size_t)(M + 127) / 128 * 128, both = Mp * (r.Kp + Mp) * 2;
     if (both > need) need = both;
@@ -263,8 +261,9 @@ static int syrk_impl(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64
     const bf16_t* const x = static_cast<const bf16_t*>(X);
     bf16_t* const y = static_cast<bf16_t*>(Y);
     const int how = syrk_ragged_reads(x, ldx, M, K);
-    SyrkPad p;
-    const bool pad = may_copy && how != kReadsLines && syrk_pad_layout(M, K, &p) && room(p.total);
+    const SyrkPad p = syrk_pad_layout(M, K);
+    const bool aligned = ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;
+    const bool pad = may_copy && (how == kReadsLines || !whole_tiles(M, K)) && syrk_padded_pays(M, K, how == kReadsLines, aligned) && room(p.total);
     if (!pad && (how == kReadsLines || (how == kReadsRows && !whole_tiles(M, K))) && room(r.slots ? r.slots + 256 : 0))
       return hip_status(launch_syrk_ragged(x, ldx, y, ldy, M, K, elem == kElemF16, ws, r.slots, hs));
     if (pad) {

@@ -13,15 +13,15 @@
 //
 // Bound by the copies into the LDS: 0.43 us per 64-wide k stage, tile and CU with two workgroups (copies alone 0.36, 90 bytes
 // per ns and CU), 0.53 with one.  Behind a copy of X 3000 x 5000 takes 53 us of 70, the copy 10.6, the second kernel 6.
+#include "fm_routes.h"
 #include "fm_tile128.h"
 
 namespace fm {
 
 namespace {
 
-constexpr int kGrid = 512;                        // workgroups: two per CU
+constexpr int kGrid = kRaggedGrid;
 constexpr int kPartFloats = 128 * 128;
-constexpr int kMinPiece = 8, kMaxParts = 16;      // stages a piece of a left-over tile has at least, pieces of one
 
 struct RaggedArgs {
   const bf16_t* X; int64_t ldx;
@@ -148,34 +148,19 @@ __global__ __launch_bounds__(64) void syrk_ragged_reduce_kernel(RaggedArgs p, in
   write_out<F16>(p, ti, tj, acc, smem, lane, blk);
 }
 
-void ragged_schedule(int M, int K, RaggedArgs& p) {
+void set_schedule(int M, int K, RaggedArgs& p) {
+  const RaggedSchedule s = ragged_schedule(M, K);
   p.M = M;
   p.tail = K % t128::BK;
-  p.nk = (K + t128::BK - 1) / t128::BK;
-  p.T = (M + 127) / 128;
-  const int64_t tiles = (int64_t)p.T * (p.T + 1) / 2;
-  p.rounds = (int)(tiles / kGrid);
-  const int rem = (int)(tiles % kGrid);
-  p.whole = rem; p.cut = 0; p.parts = 1;
-  if (rem > 256) {
-    int n = 256 / (rem - 256);
-    if (n > kMaxParts) n = kMaxParts;
-    if (n > p.nk / kMinPiece) n = p.nk / kMinPiece;
-    if (n > 1 && p.nk - p.nk / n >= 40) { p.whole = 256; p.cut = rem - 256; p.parts = n; }
-  } else if (rem > 0) {
-    int n = 256 / rem;
-    if (n > kMaxParts) n = kMaxParts;
-    if (n > p.nk / kMinPiece) n = p.nk / kMinPiece;
-    if (n > 1 && p.nk - p.nk / n >= (p.rounds > 0 ? 45 : 25)) { p.whole = 0; p.cut = rem; p.parts = n; }
-  }
+  p.nk = s.nk; p.T = s.T;
+  p.rounds = s.rounds; p.whole = s.whole; p.cut = s.cut; p.parts = s.parts;
 }
 
 }  // namespace
 
 size_t syrk_ragged_workspace_bytes(int M, int K) {
-  RaggedArgs p = {};
-  ragged_schedule(M, K, p);
-  return (size_t)p.cut * p.parts * kPartFloats * sizeof(float);
+  const RaggedSchedule s = ragged_schedule(M, K);
+  return (size_t)s.cut * s.parts * kPartFloats * sizeof(float);
 }
 
 // A 128-byte piece of a row that does not start on a line makes two requests of one: 3000 x 5000 (10000-byte rows) 75 us
@@ -190,7 +175,7 @@ int syrk_ragged_reads(const bf16_t* X, int64_t ldx, int M, int K) {
 
 int launch_syrk_ragged(const bf16_t* X, int64_t ldx, bf16_t* Y, int64_t ldy, int M, int K, bool f16, void* ws, size_t ws_bytes, hipStream_t stream) {
   RaggedArgs p = {};
-  ragged_schedule(M, K, p);
+  set_schedule(M, K, p);
   p.X = X; p.ldx = ldx; p.Y = Y; p.ldy = ldy;
   p.slots = static_cast<float*>(ws);
   if (!ws || ws_bytes < (size_t)p.cut * p.parts * kPartFloats * sizeof(float)) { p.whole += p.cut; p.cut = 0; p.parts = 1; }

@@ -56,4 +56,68 @@ inline bool ns_flow_short_enough(int batch, int m, int k) {
 }
 inline bool ns_flow_chosen(int batch, int m, int k) { return ns_flow_pays(batch, m, k) && ns_flow_short_enough(batch, m, k); }
 
+// ---- X X^T in 16 bits of sides that the 256-tiles do not fit -------------------------------------
+// The in-place kernel's schedule (fm_gemm_ragged.hip): 128x128 tiles in full rounds of 512 workgroups; of those left over `whole` in one
+// piece and `cut` in `parts` pieces along k each.
+constexpr int kRaggedGrid = 512;                        // workgroups: two per CU
+constexpr int kRaggedMinPiece = 8, kRaggedMaxParts = 16;   // stages a piece has at least, pieces of a tile
+struct RaggedSchedule { int T, nk, rounds, whole, cut, parts; };
+inline RaggedSchedule ragged_schedule(int M, int K) {
+  RaggedSchedule s;
+  s.nk = (K + 63) / 64;
+  s.T = (M + 127) / 128;
+  const int64_t tiles = (int64_t)s.T * (s.T + 1) / 2;
+  s.rounds = (int)(tiles / kRaggedGrid);
+  const int rem = (int)(tiles % kRaggedGrid);
+  s.whole = rem; s.cut = 0; s.parts = 1;
+  if (rem > 256) {
+    int n = 256 / (rem - 256);
+    if (n > kRaggedMaxParts) n = kRaggedMaxParts;
+    if (n > s.nk / kRaggedMinPiece) n = s.nk / kRaggedMinPiece;
+    if (n > 1 && s.nk - s.nk / n >= 40) { s.whole = 256; s.cut = rem - 256; s.parts = n; }
+  } else if (rem > 0) {
+    int n = 256 / rem;
+    if (n > kRaggedMaxParts) n = kRaggedMaxParts;
+    if (n > s.nk / kRaggedMinPiece) n = s.nk / kRaggedMinPiece;
+    if (n > 1 && s.nk - s.nk / n >= (s.rounds > 0 ? 45 : 25)) { s.whole = 0; s.cut = rem; s.parts = n; }
+  }
+  return s;
+}
+
+// Its time in us, in place or (`lines` false) behind a copy of X, and that of both X and Y as copies padded to whole 256-tiles
+// (a round of 256 of them, the rest cut along k; `aligned`: rows of Y that 16-byte stores can take).  Constants: least squares over 400 sizes
+// of 2900 to 28000 rows and K of 200 to 16000, 4 % rms each.  A stage of a tile slows down once X and what is written beside it outgrow the 256 MB
+// of the memory-side cache, on 128-tiles (twice the operand bytes per flop) from about 100 MB of X on.
+inline double syrk_ragged_us(int M, int K, bool lines) {
+  const RaggedSchedule s = ragged_schedule(M, K);
+  const double mk = (double)M * K, mm = (double)M * M, mb = 2e-6 * mk;
+  double t = s.rounds * (0.77 * s.nk - 4.8) + 6.8e-7 * mm;
+  if (s.cut) t += s.whole ? 0.62 * s.nk - 3.6 : 0.37 * s.nk / s.parts + 11.2;
+  else if (s.whole) t += s.whole <= 256 ? 0.37 * s.nk + 0.5 : 0.66 * s.nk - 0.6;
+  double slow = 1.0 + (lines ? 0.0045 * (mb - 105.0) : 0.005 * (mb - 100.0));
+  slow = slow < 1.0 ? 1.0 : slow > 1.5 ? 1.5 : slow;
+  return t * slow + (lines ? 3.5 : 7.5 + 6.8e-7 * mk);
+}
+inline double syrk_padded_us(int M, int K, bool aligned) {
+  const int64_t T = (M + 255) / 256, tiles = T * (T + 1) / 2, rounds = tiles / 256, rem = tiles % 256;
+  const double nk = (K + 63) / 64, mk = (double)M * K, out = (aligned ? 7.1e-7 : 15.4e-7) * M * M;
+  if (T == 16)   // 256 half tiles, one round
+    return 12.4 + 6.8e-7 * mk + out + (mk < 7e7 ? 0.71 : 0.85) * nk;
+  double t = 4.4 + 1.9e-6 * mk + out + rounds * (1.07 * nk + 19.6);
+  const int64_t parts = rem ? 256 / rem : 1;
+  if (rem && parts < 16) t += 0.753 * nk / parts + (parts == 1 ? 8.0 : 11.4);   // (up to 16 of them run as sub-tiles beside the rounds)
+  return t;
+}
+// Whether it is padded, for matrices that may be (the copies cost memory: not for a gain of under 4 % of the estimates).  us, in place
+// or behind a copy of X / padded: 4000^2 86 / 78, 3936 x 4000 69 / 77, 5280 x 6000 183 / 167, 5536 x 4000 127 / 130, 7776 x 4000 242 / 248, 8096 x 8040 509 / 453,
+// 8008 x 4000 246 / 263, 8008 x 16000 1102 / 821, 10000 x 8000 887 / 700, 16008 x 2000 544 / 646, x 4000 1159 / 974, x 8000 2576 / 1684, 24000 x 4000 3036 / 2152; of whole
+// tiles 7552 x 4096 195 / 253, x 16384 898 / 781, 10112 x 8192 1007 / 711, 16256 x 8192 2783 / 1722.
+// Below 16 tile rows of 256 only a matrix that has to be copied in any case and does not fit the cache: 2980 x 24000 (143 MB) 220 / 319, x 60000 (358 MB) 768 / 531,
+// 1956 x 60000 562 / 298; of fewer than 8 (1000 x 262144) none.
+inline bool syrk_padded_pays(int M, int K, bool lines, bool aligned) {
+  if (K < 1500 || K > (1 << 21) - 128) return false;   // (4056 x 1248 38 / 43; what the 256-tiles' byte offsets allow)
+  if (M <= 15 * 256) return !lines && M > 7 * 256 && 2e-6 * M * K > 200.0;
+  return 0.96 * syrk_padded_us(M, K, aligned) < syrk_ragged_us(M, K, lines);
+}
+
 }  // namespace fm

@@ -56,3 +56,13 @@ def test_infinities_beside_the_rows():
     got = _run(X, 200, 600)
     want = (X.double() @ X.double().T).to(torch.bfloat16)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("M,K", [(5248, 12288), (5280, 6000), (1800, 56008)])
+def test_what_outgrows_the_cache_is_padded(M, K):
+    """An odd number of whole tiles, sides of neither, and few tile rows whose rows lie on no lines.  (Sums below 2^24: any fp32 product is exact.)"""
+    X = _ints(M, K, 3, torch.bfloat16)
+    x = X.to(DEV).float()
+    want = (x @ x.T).bfloat16().cpu()
+    assert torch.equal(_run(X, K, M), want)
+    assert torch.equal(_run(X, K, M + 5, 3), want)

@@ -12,6 +12,7 @@ HOST = """
 #include "fm_routes.h"
 extern "C" {
 long long scale_cast_rows_blocks(long long r, long long c) { return fm::scale_cast_rows_blocks(r, c); }
+int syrk_padded_pays(int M, int K, int lines, int aligned) { return fm::syrk_padded_pays(M, K, lines, aligned); }
 int ns_flow_chosen(int batch, int m, int k) { return fm::ns_flow_chosen(batch, m, k); }
 }
 """
@@ -63,3 +64,22 @@ def test_one_launch_newtonschulz_where_it_measured_faster(routes, lib, batch, m,
         need = lib.fm_newtonschulz_batched_workspace_bytes(batch, m, k)
         assert need >= batch * (6 * m * k + 10 * m * m) * 2
         assert need == lib.fm_newtonschulz_batched_workspace_bytes(batch, k, m)
+
+
+# (M, K, us on 128x128 tiles - in place where the rows lie on lines, else behind a copy -, us padded to 256-tiles), measured
+PADDED_TIMES = [(2980, 60000, 768, 531), (1956, 60000, 562, 298), (2980, 24000, 220, 319), (3936, 4000, 69.4, 77.4), (4056, 1248, 37.6, 42.8), (4000, 4000, 85.9, 77.7), (3000, 5000, 70.1, 75.7),
+                (5280, 6000, 183, 167), (5792, 4000, 150, 193), (6048, 2000, 91, 122), (7776, 2000, 133, 161), (7580, 8040, 469, 429), (8096, 8040, 509, 453),
+                (8008, 4000, 246, 263), (8008, 16000, 1102, 821), (10000, 8000, 887, 700), (10000, 4000, 402, 429), (11000, 16000, 2106, 1577), (12000, 8000, 1291, 959),
+                (16008, 2000, 544, 646), (16008, 4000, 1159, 974), (16008, 8000, 2576, 1684), (20000, 2000, 782, 1017), (24000, 4000, 3036, 2152), (28000, 2000, 1727, 1920),
+                (7552, 4096, 195, 253), (7552, 16384, 898, 781), (10112, 8192, 1007, 711), (12160, 2048, 276, 396), (12928, 8192, 1685, 1088), (16256, 8192, 2783, 1722)]
+
+
+@pytest.mark.parametrize("M,K,tiles128,padded", PADDED_TIMES)
+def test_large_products_of_ragged_sides_are_padded_where_it_measured_faster(routes, lib, M, K, tiles128, padded):
+    pays = bool(routes.syrk_padded_pays(M, K, K % 64 == 0, M % 8 == 0))
+    assert pays == (padded < tiles128)
+    Mp, Kp = (M + 255) // 256 * 256, (K + 63) // 64 * 64
+    if pays:   # room for both copies and the product's own scratch
+        assert lib.fm_syrk_workspace_bytes(M, K) >= 2 * Mp * (Mp + Kp) + lib.fm_gemm_workspace_bytes(Mp, Mp)
+    elif M % 128 == 0 and K % 64 == 0:   # whole tiles that are multiplied in place: the parts of left-over tiles at most
+        assert lib.fm_syrk_workspace_bytes(M, K) <= (16 << 20) + 512
