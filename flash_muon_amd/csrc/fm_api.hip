@@ -165,18 +165,13 @@ int fm_set_knob(int which, long long value) { return set_knob(which, value) == 0
 //   Sides that are no whole 128-tiles, from 65536 elements of X on (below that the general path's single launch wins).
 // us, zero-padded copies of both X and Y around the tiled paths before, now: 600^2 17.3 -> 10.7, 1000^2 16.7 -> 11.0, 2000^2 32 ->
 // 23, 3000 x 1000 33 -> 24, 3000 x 5000 79 -> 70, 3900 x 8000 140 -> 104, 600 x 8000 32 -> 22, 6500^2 356 -> 294.
-//   Odd numbers of 128-tiles, rows on 128-byte lines (in launch_gemm_nt's 128-tiles, or its 256-tiles with a half at the edge):
-// 1408^2 14.2 -> 12.4, 2944^2 46.7 -> 38.2, 4224^2 96 -> 78, 5504 x 2048 81 -> 62, 8064 x 1024 114 -> 70; but 2176^2 (153 tiles) 20.7 and
-// 21.8, 2688^2 26.3 and 26.9: between 121 and 256 tiles of a workgroup each the older path stays.
+//   Odd numbers of whole 128-tiles with rows on 128-byte lines, by syrk_whole_in_place.
 struct SyrkRagged { int Kp; size_t slots, x, total; };
 constexpr int64_t kSyrkRaggedMinElems = 256 * 256;
 static bool whole_tiles(int M, int K) { return M % 128 == 0 && K % 64 == 0; }
 static bool syrk_ragged_layout(int M, int K, SyrkRagged* p) {
   if (M <= 0 || K <= 0 || (int64_t)M * K < kSyrkRaggedMinElems || K >= (1 << 22)) return false;
-  if (whole_tiles(M, K)) {
-    const int64_t T = M / 128, tiles = T * (T + 1) / 2;
-    if (M % 256 == 0 || (tiles > 120 && tiles <= 256)) return false;
-  }
+  if (whole_tiles(M, K) && (M % 256 == 0 || !syrk_whole_in_place(M, K, cu_count()))) return false;
   p->Kp = (K + 63) / 64 * 64;
   p->slots = syrk_ragged_workspace_bytes(M, K);
   p->x = align_up(p->slots, 256);   // (a copy has as many stages, and so the same pieces)

@@ -12,6 +12,7 @@
 // workgroup, which go to memory as fp32 and are added in part order by a second, small kernel that
 // also runs the epilogue.  A product whose 128x256 half tiles fit into one round runs on those, and
 // one of at most 16 tiles may run on sub-tiles altogether.
+#include "fm_routes.h"
 #include "fm_tile128.h"
 
 #include <type_traits>
@@ -2005,40 +2006,15 @@ static bool tiled_dma_eligible(const GemmArgs& a, int tile) {
   return true;
 }
 
-// Parts per 128x128 tile along k, by estimate in microseconds (measured: 0.36 per stage, 4.5 for a
-// tile's start and write-out; cut, 11 for the fp32 round trip and the second launch and 0.035 per
-// part for their traffic).  At most as many parts as fill the chip, of at least 8 stages each; the
-// tiles stay whole unless the cut saves a tenth.
-static double estimate_mid_cut(long long tiles, int nk, int s) {
-  return (double)((nk + s - 1) / s) * 0.36 + 11.0 + 0.035 * (double)(tiles * s);
-}
 static int mid_ksplit(long long tiles, int nk, int grid) {
   const long long k = knob(kKnobKsplit);
   if (k >= 1) {
     const int s = (int)(k > kMaxParts ? kMaxParts : k);
     return s > nk ? nk : s;
   }
-  if (tiles * 2 > grid || nk < 16) return 1;
-  int smax = (int)(grid / tiles);
-  if (smax > nk / 8) smax = nk / 8;
-  if (smax > 16) smax = 16;
-  int best = 1;
-  double t_best = 0.9 * (nk * 0.36 + 4.5);
-  for (int s = 2; s <= smax; ++s) {
-    const double t = estimate_mid_cut(tiles, nk, s);
-    if (t < t_best) { t_best = t; best = s; }
-  }
-  return best;
+  return mid_parts(tiles, nk, grid);
 }
-// (a stage costs 0.36 us while about half the CUs work and 0.52 when all do; a write-out with an
-// operand E costs 5 more)
-static double estimate_mid(long long tiles, int nk, int grid, bool with_e) {
-  const int s = mid_ksplit(tiles, nk, grid);
-  if (s > 1) return estimate_mid_cut(tiles, nk, s) + (with_e ? 5.0 : 0.0);
-  const double occ = tiles >= grid ? 1.0 : (double)tiles / grid;
-  const double stage = 0.36 + 0.36 * (occ > 0.55 ? occ - 0.55 : 0.0);
-  return (double)((tiles + grid - 1) / grid) * (nk * stage + (with_e ? 11.0 : 6.0));
-}
+static double estimate_mid(long long tiles, int nk, int grid, bool with_e) { return mid_us(tiles, nk, grid, mid_ksplit(tiles, nk, grid), with_e); }
 
 // Estimates in microseconds, from measured costs of a k stage and of a tile's start and write-out.
 // The clock the power cap allows falls as the chip fills, so a stage costs more the more CUs work.

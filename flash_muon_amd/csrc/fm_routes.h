@@ -120,4 +120,49 @@ inline bool syrk_padded_pays(int M, int K, bool lines, bool aligned) {
   return 0.96 * syrk_padded_us(M, K, aligned) < syrk_ragged_us(M, K, lines);
 }
 
+// ---- 128x128 tiles of whole, aligned matrices, one per CU (launch_gemm_mid) ------------------------
+// Parts per tile along k, by estimate in microseconds (measured: 0.36 per stage, 4.5 for a
+// tile's start and write-out; cut, 11 for the fp32 round trip and the second launch and 0.035 per
+// part for their traffic).  At most as many parts as fill the chip, of at least 8 stages each; the
+// tiles stay whole unless the cut saves a tenth.
+inline double mid_cut_us(long long tiles, int nk, int s) { return (double)((nk + s - 1) / s) * 0.36 + 11.0 + 0.035 * (double)(tiles * s); }
+inline int mid_parts(long long tiles, int nk, int grid) {
+  if (tiles * 2 > grid || nk < 16) return 1;
+  int smax = (int)(grid / tiles);
+  if (smax > nk / 8) smax = nk / 8;
+  if (smax > 16) smax = 16;
+  int best = 1;
+  double t_best = 0.9 * (nk * 0.36 + 4.5);
+  for (int s = 2; s <= smax; ++s) {
+    const double t = mid_cut_us(tiles, nk, s);
+    if (t < t_best) { t_best = t; best = s; }
+  }
+  return best;
+}
+// (a stage costs 0.36 us while about half the CUs work and 0.52 when all do; a write-out with an
+// operand E costs 5 more)
+inline double mid_us(long long tiles, int nk, int grid, int parts, bool with_e) {
+  if (parts > 1) return mid_cut_us(tiles, nk, parts) + (with_e ? 5.0 : 0.0);
+  const double occ = tiles >= grid ? 1.0 : (double)tiles / grid;
+  const double stage = 0.36 + 0.36 * (occ > 0.55 ? occ - 0.55 : 0.0);
+  return (double)((tiles + grid - 1) / grid) * (nk * stage + (with_e ? 11.0 : 6.0));
+}
+
+// X X^T of an odd number of whole 128-tiles, rows on lines: in place on tiles that share a CU in pairs (fm_gemm_ragged.hip), or on the
+// tiles above.  us, above / in place: more tiles than CUs 2944^2 46.7 / 38.2, 4224^2 96 / 78, 5504 x 2048 81 / 62, 8064 x 1024 114 / 70; 121 to
+// 256 of them 2176^2 20.7 / 21.8, 2688^2 26.3 / 26.9.  Fewer: the deeper ring above starts later (4 us) and takes 0.36 us a stage where
+// this one takes 0.53, which is why a long k, cut or not, is better off there: 1408 x 1024 11.5 / 9.5, x 2048 16.9 / 18.8, x 4096 27.4 / 21.5 (cut in
+// place alone), x 8192 31.8 / 31.4, x 16384 48.1 / 51.3, x 32768 80 / 94; 1920 x 3072 23.3 / 26.9, x 6144 40.0 / 34.7, x 32768 125 / 144; 640 x 32768 31.3 / 28.1.
+// (estimates within 10 % of these; a near tie stays in place)
+inline bool syrk_whole_in_place(int M, int K, int cus) {
+  const int64_t T = M / 128, tiles = T * (T + 1) / 2;
+  if (tiles > 256) return true;
+  if (tiles > 120) return false;
+  const RaggedSchedule s = ragged_schedule(M, K);
+  const double load = tiles < 66 ? tiles / 66.0 : 1.0, pieces = (double)s.cut * s.parts;
+  const double t = s.cut ? 9.0 + 0.015 * pieces + (0.36 + 0.12 * (pieces < 180.0 ? pieces / 180.0 : 1.0)) * ((s.nk + s.parts - 1) / s.parts)
+                         : 2.2 + (0.33 + 0.19 * load * load) * s.nk;
+  return 0.97 * t <= mid_us(tiles, s.nk, cus, mid_parts(tiles, s.nk, cus), false);
+}
+
 }  // namespace fm

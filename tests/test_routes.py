@@ -13,6 +13,7 @@ HOST = """
 extern "C" {
 long long scale_cast_rows_blocks(long long r, long long c) { return fm::scale_cast_rows_blocks(r, c); }
 int syrk_padded_pays(int M, int K, int lines, int aligned) { return fm::syrk_padded_pays(M, K, lines, aligned); }
+int syrk_whole_in_place(int M, int K) { return fm::syrk_whole_in_place(M, K, 256); }
 int ns_flow_chosen(int batch, int m, int k) { return fm::ns_flow_chosen(batch, m, k); }
 }
 """
@@ -83,3 +84,16 @@ def test_large_products_of_ragged_sides_are_padded_where_it_measured_faster(rout
         assert lib.fm_syrk_workspace_bytes(M, K) >= 2 * Mp * (Mp + Kp) + lib.fm_gemm_workspace_bytes(Mp, Mp)
     elif M % 128 == 0 and K % 64 == 0:   # whole tiles that are multiplied in place: the parts of left-over tiles at most
         assert lib.fm_syrk_workspace_bytes(M, K) <= (16 << 20) + 512
+
+
+# (M, K, us on tiles of their own CU, us in place): odd numbers of whole 128-tiles
+WHOLE_TIMES = [(128, 2048, 14.7, 12.0), (128, 65536, 34.5, 28.6), (384, 32768, 27.4, 23.5), (640, 2048, 16.1, 13.5), (640, 32768, 31.3, 28.1), (1152, 1536, 13.8, 11.5),
+               (1152, 4096, 23.5, 20.0), (1152, 32768, 57.0, 61.3), (1408, 1024, 11.5, 9.6), (1408, 2048, 16.9, 18.8), (1408, 4096, 27.4, 21.5), (1408, 16384, 47.8, 51.3),
+               (1408, 32768, 80.1, 93.9), (1664, 1024, 11.7, 10.0), (1664, 2048, 17.2, 19.2), (1664, 3072, 23.0, 26.8), (1664, 4096, 27.4, 25.6), (1664, 12288, 50.9, 55.8),
+               (1664, 32768, 108.5, 132.4), (1920, 1024, 12.0, 10.4), (1920, 2048, 17.5, 19.3), (1920, 3072, 23.4, 26.9), (1920, 6144, 39.9, 34.7), (1920, 32768, 125.3, 144.5),
+               (2176, 2176, 20.7, 21.8), (2688, 2688, 26.3, 26.9), (2944, 2944, 46.7, 38.2), (8064, 1024, 114, 70)]
+
+
+@pytest.mark.parametrize("M,K,apart,in_place", WHOLE_TIMES)
+def test_odd_numbers_of_whole_tiles_are_multiplied_in_place_where_it_measured_faster(routes, M, K, apart, in_place):
+    assert bool(routes.syrk_whole_in_place(M, K)) == (in_place < apart)
