@@ -163,14 +163,10 @@ size_t syrk_ragged_workspace_bytes(int M, int K) {
   return (size_t)s.cut * s.parts * kPartFloats * sizeof(float);
 }
 
-// A 128-byte piece of a row that does not start on a line makes two requests of one: 3000 x 5000 (10000-byte rows) 75 us
-// in place and 70 behind a copy of X, 7000 x 2000 129 and 110; but 2000^2 23 and 30, 4000 x 1000 33 and 37, where a launch
-// and 8 bytes of traffic per element cost more than what they save in 16384 stages of tiles or less.
 int syrk_ragged_reads(const bf16_t* X, int64_t ldx, int M, int K) {
   if (K < t128::BK || K % 8 != 0 || ldx % 8 != 0 || ldx >= (1 << 23) || (reinterpret_cast<uintptr_t>(X) & 15) != 0) return kReadsCopy;
   if (ldx % 64 == 0 && (reinterpret_cast<uintptr_t>(X) & 127) == 0) return kReadsLines;
-  const int64_t T = (M + 127) / 128, nk = (K + t128::BK - 1) / t128::BK;
-  return T * (T + 1) / 2 * nk < 16384 ? kReadsRows : kReadsCopy;
+  return syrk_copy_pays(M, K) ? kReadsCopy : kReadsRows;
 }
 
 int launch_syrk_ragged(const bf16_t* X, int64_t ldx, bf16_t* Y, int64_t ldy, int M, int K, bool f16, void* ws, size_t ws_bytes, hipStream_t stream) {

@@ -108,6 +108,15 @@ inline double syrk_padded_us(int M, int K, bool aligned) {
   if (rem && parts < 16) t += 0.753 * nk / parts + (parts == 1 ? 8.0 : 11.4);   // (up to 16 of them run as sub-tiles beside the rounds)
   return t;
 }
+// Whether rows that 16-byte copies can take but that do not lie on 128-byte lines are copied first: a 128-byte piece of such a row makes two requests
+// of one.  us, in place / behind a copy of X: 3000 x 5000 75 / 70, 7000 x 2000 129 / 110; but 2000^2 23 / 30, 4000 x 1000 33 / 37, where a launch and 8
+// bytes of traffic per element cost more than they save in 16384 stages of tiles or less; and with at most a tile per CU, whose stages the requests do
+// not hold up, 1956 x 12000 94 / 104, 2724 x 12000 110 / 120, 1920 x 65544 349 / 385, 1000 x 65544 106 / 126.
+inline bool syrk_copy_pays(int M, int K) {
+  const RaggedSchedule s = ragged_schedule(M, K);
+  const int64_t tiles = (int64_t)s.T * (s.T + 1) / 2;
+  return tiles > 256 && tiles * s.nk >= 16384;
+}
 // Whether it is padded, for matrices that may be (the copies cost memory: not for a gain of under 4 % of the estimates).  us, in place
 // or behind a copy of X / padded: 4000^2 86 / 78, 3936 x 4000 69 / 77, 5280 x 6000 183 / 167, 5536 x 4000 127 / 130, 7776 x 4000 242 / 248, 8096 x 8040 509 / 453,
 // 8008 x 4000 246 / 263, 8008 x 16000 1102 / 821, 10000 x 8000 887 / 700, 16008 x 2000 544 / 646, x 4000 1159 / 974, x 8000 2576 / 1684, 24000 x 4000 3036 / 2152; of whole

@@ -14,6 +14,7 @@ extern "C" {
 long long scale_cast_rows_blocks(long long r, long long c) { return fm::scale_cast_rows_blocks(r, c); }
 int syrk_padded_pays(int M, int K, int lines, int aligned) { return fm::syrk_padded_pays(M, K, lines, aligned); }
 int syrk_whole_in_place(int M, int K) { return fm::syrk_whole_in_place(M, K, 256); }
+int syrk_copy_pays(int M, int K) { return fm::syrk_copy_pays(M, K); }
 int ns_flow_chosen(int batch, int m, int k) { return fm::ns_flow_chosen(batch, m, k); }
 }
 """
@@ -97,3 +98,13 @@ WHOLE_TIMES = [(128, 2048, 14.7, 12.0), (128, 65536, 34.5, 28.6), (384, 32768, 2
 @pytest.mark.parametrize("M,K,apart,in_place", WHOLE_TIMES)
 def test_odd_numbers_of_whole_tiles_are_multiplied_in_place_where_it_measured_faster(routes, M, K, apart, in_place):
     assert bool(routes.syrk_whole_in_place(M, K)) == (in_place < apart)
+
+
+# (M, K, us in place, us behind a copy of X): rows that 16-byte copies can take and that lie on no lines
+COPY_TIMES = [(3000, 5000, 75, 70), (7000, 2000, 129, 110), (2000, 2000, 23, 30), (4000, 1000, 33, 37), (1956, 12000, 93.6, 103.7), (2468, 12000, 99.6, 112.3),
+              (2724, 12000, 110, 120), (1000, 65544, 106, 126), (1920, 65544, 349, 385), (3492, 6000, 117, 90), (4004, 4000, 88.2, 84.5), (5028, 6000, 183, 161)]
+
+
+@pytest.mark.parametrize("M,K,in_place,copied", COPY_TIMES)
+def test_rows_off_lines_are_copied_where_it_measured_faster(routes, M, K, in_place, copied):
+    assert bool(routes.syrk_copy_pays(M, K)) == (copied < in_place)
