@@ -199,7 +199,7 @@ size_t fm_syrk_workspace_bytes(int M, int K) {
   if (!syrk_ragged_layout(M, K, &r)) return need;
   if (r.total > need) need = r.total;
   // (rows may lie on lines or not, and Y's rows allow 16-byte stores or not)
-  if ((K % 64 == 0 && syrk_padded_pays(M, K, true, true)) || (!whole_tiles(M, K) && syrk_padded_pays(M, K, false, true))) {
+  if ((K % 64 == 0 && syrk_padded_pays(M, K, kRowsLines, true)) || (!whole_tiles(M, K) && syrk_padded_pays(M, K, kRowsAny, true))) {
     const SyrkPad p = syrk_pad_layout(M, K);
     if (p.total > need) need = p.total;
   }
@@ -258,7 +258,8 @@ static int syrk_impl(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64
     const int how = syrk_ragged_reads(x, ldx, M, K);
     const SyrkPad p = syrk_pad_layout(M, K);
     const bool aligned = ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;
-    const bool pad = may_copy && (how == kReadsLines || !whole_tiles(M, K)) && syrk_padded_pays(M, K, how == kReadsLines, aligned) && room(p.total);
+    const int rows = how == kReadsLines ? kRowsLines : ldx % 32 == 0 ? kRowsHalfLines : kRowsAny;
+    const bool pad = may_copy && (how == kReadsLines || !whole_tiles(M, K)) && syrk_padded_pays(M, K, rows, aligned) && room(p.total);
     if (!pad && (how == kReadsLines || (how == kReadsRows && !whole_tiles(M, K))) && room(r.slots ? r.slots + 256 : 0))
       return hip_status(launch_syrk_ragged(x, ldx, y, ldy, M, K, elem == kElemF16, ws, r.slots, hs));
     if (pad) {

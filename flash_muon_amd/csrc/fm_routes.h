@@ -110,23 +110,28 @@ inline double syrk_padded_us(int M, int K, bool aligned) {
 }
 // Whether rows that 16-byte copies can take but that do not lie on 128-byte lines are copied first: a 128-byte piece of such a row makes two requests
 // of one.  us, in place / behind a copy of X: 3000 x 5000 75 / 70, 7000 x 2000 129 / 110; but 2000^2 23 / 30, 4000 x 1000 33 / 37, where a launch and 8
-// bytes of traffic per element cost more than they save in 16384 stages of tiles or less; and with at most a tile per CU, whose stages the requests do
-// not hold up, 1956 x 12000 94 / 104, 2724 x 12000 110 / 120, 1920 x 65544 349 / 385, 1000 x 65544 106 / 126.
+// bytes of traffic per element cost more than they save in 16384 stages of tiles or less; and with a tile on four fifths of the CUs at most, whose stages
+// the requests do not hold up, 1956 x 12000 94 / 104, 2468 x 12000 100 / 112, 1920 x 65544 349 / 385, 1000 x 65544 106 / 126 (253 tiles: 2768 x 9784 107 / 101).
 inline bool syrk_copy_pays(int M, int K) {
   const RaggedSchedule s = ragged_schedule(M, K);
   const int64_t tiles = (int64_t)s.T * (s.T + 1) / 2;
-  return tiles > 256 && tiles * s.nk >= 16384;
+  return tiles > 210 && tiles * s.nk >= 16384;
 }
 // Whether it is padded, for matrices that may be (the copies cost memory: not for a gain of under 4 % of the estimates).  us, in place
 // or behind a copy of X / padded: 4000^2 86 / 78, 3936 x 4000 69 / 77, 5280 x 6000 183 / 167, 5536 x 4000 127 / 130, 7776 x 4000 242 / 248, 8096 x 8040 509 / 453,
 // 8008 x 4000 246 / 263, 8008 x 16000 1102 / 821, 10000 x 8000 887 / 700, 16008 x 2000 544 / 646, x 4000 1159 / 974, x 8000 2576 / 1684, 24000 x 4000 3036 / 2152; of whole
 // tiles 7552 x 4096 195 / 253, x 16384 898 / 781, 10112 x 8192 1007 / 711, 16256 x 8192 2783 / 1722.
-// Below 16 tile rows of 256 only a matrix that has to be copied in any case and does not fit the cache: 2980 x 24000 (143 MB) 220 / 319, x 60000 (358 MB) 768 / 531,
-// 1956 x 60000 562 / 298; of fewer than 8 (1000 x 262144) none.
-inline bool syrk_padded_pays(int M, int K, bool lines, bool aligned) {
-  if (K < 1500 || K > (1 << 21) - 128) return false;   // (4056 x 1248 38 / 43; what the 256-tiles' byte offsets allow)
-  if (M <= 15 * 256) return !lines && M > 7 * 256 && 2e-6 * M * K > 200.0;
-  return 0.96 * syrk_padded_us(M, K, aligned) < syrk_ragged_us(M, K, lines);
+// Below 16 tile rows of 256, where the padded product is cut along k over all CUs: of 8 to 10, whose 120 to 210 tiles of 128 leave CUs idle, by the time of
+// a stage in place (rows on lines, on half lines, neither) against a linear fit of the padded way: 2043 x 7496 74 / 67, 1956 x 12000 94 / 93, 2468 x 12000 100 / 116,
+// 2560 x 30416 289 / 223, x 24000 on lines 180 / 191, 2200 x 72576 on lines 581 / 416; of more only a matrix that does not fit the cache: 2980 x 24000 (143 MB) 220
+// / 319, 3200 x 32768 on lines (210 MB) 317 / 406, 2980 x 60000 (358 MB) 768 / 531; of fewer (1000 x 262144 340 / 497) none.
+constexpr int kRowsLines = 0, kRowsHalfLines = 1, kRowsAny = 2;
+inline bool syrk_padded_pays(int M, int K, int rows, bool aligned) {
+  if (K < 1500 || K > (1 << 21) - 128 || M <= 7 * 256) return false;   // (4056 x 1248 38 / 43; what the 256-tiles' byte offsets allow)
+  const int T = (M + 255) / 256, nk = (K + 63) / 64;
+  if (T <= 10) return 0.96 * (3.6 * T + (0.144 + 0.026 * T) * nk) < 2.0 + (rows == kRowsLines ? 0.47 : rows == kRowsHalfLines ? 0.51 : 0.60) * nk;
+  if (T < 16) return 2e-6 * M * K > (rows == kRowsLines ? 260.0 : 200.0);
+  return 0.96 * syrk_padded_us(M, K, aligned) < syrk_ragged_us(M, K, rows == kRowsLines);
 }
 
 // ---- 128x128 tiles of whole, aligned matrices, one per CU (launch_gemm_mid) ------------------------
@@ -168,8 +173,8 @@ inline bool syrk_whole_in_place(int M, int K, int cus) {
   if (tiles > 256) return true;
   if (tiles > 120) return false;
   const RaggedSchedule s = ragged_schedule(M, K);
-  const double load = tiles < 66 ? tiles / 66.0 : 1.0, pieces = (double)s.cut * s.parts;
-  const double t = s.cut ? 9.0 + 0.015 * pieces + (0.36 + 0.12 * (pieces < 180.0 ? pieces / 180.0 : 1.0)) * ((s.nk + s.parts - 1) / s.parts)
+  const double load = tiles < 66 ? tiles / 66.0 : 1.0, busy = tiles < 28 ? tiles / 28.0 : 1.0;
+  const double t = s.cut ? 9.0 + 0.015 * s.cut * s.parts + (0.36 + 0.12 * busy * busy) * ((s.nk + s.parts - 1) / s.parts)
                          : 2.2 + (0.33 + 0.19 * load * load) * s.nk;
   return 0.97 * t <= mid_us(tiles, s.nk, cus, mid_parts(tiles, s.nk, cus), false);
 }

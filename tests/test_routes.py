@@ -12,7 +12,7 @@ HOST = """
 #include "fm_routes.h"
 extern "C" {
 long long scale_cast_rows_blocks(long long r, long long c) { return fm::scale_cast_rows_blocks(r, c); }
-int syrk_padded_pays(int M, int K, int lines, int aligned) { return fm::syrk_padded_pays(M, K, lines, aligned); }
+int syrk_padded_pays(int M, int K, int rows, int aligned) { return fm::syrk_padded_pays(M, K, rows, aligned); }
 int syrk_whole_in_place(int M, int K) { return fm::syrk_whole_in_place(M, K, 256); }
 int syrk_copy_pays(int M, int K) { return fm::syrk_copy_pays(M, K); }
 int ns_flow_chosen(int batch, int m, int k) { return fm::ns_flow_chosen(batch, m, k); }
@@ -69,7 +69,8 @@ def test_one_launch_newtonschulz_where_it_measured_faster(routes, lib, batch, m,
 
 
 # (M, K, us on 128x128 tiles - in place where the rows lie on lines, else behind a copy -, us padded to 256-tiles), measured
-PADDED_TIMES = [(2980, 60000, 768, 531), (1956, 60000, 562, 298), (2980, 24000, 220, 319), (3936, 4000, 69.4, 77.4), (4056, 1248, 37.6, 42.8), (4000, 4000, 85.9, 77.7), (3000, 5000, 70.1, 75.7),
+PADDED_TIMES = [(1956, 6000, 54.4, 55.5), (1960, 6896, 63.4, 58.5), (2043, 7496, 74, 67), (2468, 12000, 99.6, 115.9), (2560, 30416, 289, 223), (2468, 24000, 180, 191),
+                (2212, 24000, 175.1, 172), (2200, 72576, 581, 416), (1000, 262144, 340, 497), (3200, 32768, 316.8, 405), (2980, 60000, 768, 531), (1956, 60000, 562, 298), (2980, 24000, 220, 319), (3936, 4000, 69.4, 77.4), (4056, 1248, 37.6, 42.8), (4000, 4000, 85.9, 77.7), (3000, 5000, 70.1, 75.7),
                 (5280, 6000, 183, 167), (5792, 4000, 150, 193), (6048, 2000, 91, 122), (7776, 2000, 133, 161), (7580, 8040, 469, 429), (8096, 8040, 509, 453),
                 (8008, 4000, 246, 263), (8008, 16000, 1102, 821), (10000, 8000, 887, 700), (10000, 4000, 402, 429), (11000, 16000, 2106, 1577), (12000, 8000, 1291, 959),
                 (16008, 2000, 544, 646), (16008, 4000, 1159, 974), (16008, 8000, 2576, 1684), (20000, 2000, 782, 1017), (24000, 4000, 3036, 2152), (28000, 2000, 1727, 1920),
@@ -78,7 +79,7 @@ PADDED_TIMES = [(2980, 60000, 768, 531), (1956, 60000, 562, 298), (2980, 24000, 
 
 @pytest.mark.parametrize("M,K,tiles128,padded", PADDED_TIMES)
 def test_large_products_of_ragged_sides_are_padded_where_it_measured_faster(routes, lib, M, K, tiles128, padded):
-    pays = bool(routes.syrk_padded_pays(M, K, K % 64 == 0, M % 8 == 0))
+    pays = bool(routes.syrk_padded_pays(M, K, 0 if K % 64 == 0 else 1 if K % 32 == 0 else 2, M % 8 == 0))
     assert pays == (padded < tiles128)
     Mp, Kp = (M + 255) // 256 * 256, (K + 63) // 64 * 64
     if pays:   # room for both copies and the product's own scratch
@@ -88,7 +89,7 @@ def test_large_products_of_ragged_sides_are_padded_where_it_measured_faster(rout
 
 
 # (M, K, us on tiles of their own CU, us in place): odd numbers of whole 128-tiles
-WHOLE_TIMES = [(128, 2048, 14.7, 12.0), (128, 65536, 34.5, 28.6), (384, 32768, 27.4, 23.5), (640, 2048, 16.1, 13.5), (640, 32768, 31.3, 28.1), (1152, 1536, 13.8, 11.5),
+WHOLE_TIMES = [(128, 2048, 14.7, 12.0), (128, 65536, 34.5, 28.6), (384, 32768, 27.4, 23.5), (640, 2048, 16.1, 13.5), (640, 32768, 31.3, 28.1), (640, 85696, 53, 48.9), (1152, 1536, 13.8, 11.5),
                (1152, 4096, 23.5, 20.0), (1152, 32768, 57.0, 61.3), (1408, 1024, 11.5, 9.6), (1408, 2048, 16.9, 18.8), (1408, 4096, 27.4, 21.5), (1408, 16384, 47.8, 51.3),
                (1408, 32768, 80.1, 93.9), (1664, 1024, 11.7, 10.0), (1664, 2048, 17.2, 19.2), (1664, 3072, 23.0, 26.8), (1664, 4096, 27.4, 25.6), (1664, 12288, 50.9, 55.8),
                (1664, 32768, 108.5, 132.4), (1920, 1024, 12.0, 10.4), (1920, 2048, 17.5, 19.3), (1920, 3072, 23.4, 26.9), (1920, 6144, 39.9, 34.7), (1920, 32768, 125.3, 144.5),
@@ -102,7 +103,7 @@ def test_odd_numbers_of_whole_tiles_are_multiplied_in_place_where_it_measured_fa
 
 # (M, K, us in place, us behind a copy of X): rows that 16-byte copies can take and that lie on no lines
 COPY_TIMES = [(3000, 5000, 75, 70), (7000, 2000, 129, 110), (2000, 2000, 23, 30), (4000, 1000, 33, 37), (1956, 12000, 93.6, 103.7), (2468, 12000, 99.6, 112.3),
-              (2724, 12000, 110, 120), (1000, 65544, 106, 126), (1920, 65544, 349, 385), (3492, 6000, 117, 90), (4004, 4000, 88.2, 84.5), (5028, 6000, 183, 161)]
+              (2768, 9784, 106.9, 100.8), (1000, 65544, 106, 126), (1920, 65544, 349, 385), (3492, 6000, 117, 90), (4004, 4000, 88.2, 84.5), (5028, 6000, 183, 161)]
 
 
 @pytest.mark.parametrize("M,K,in_place,copied", COPY_TIMES)
