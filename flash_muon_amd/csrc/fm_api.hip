@@ -255,14 +255,14 @@ static int syrk_impl(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64
   if (ldy >= M && syrk_ragged_layout(M, K, &r)) {
     const bf16_t* const x = static_cast<const bf16_t*>(X);
     bf16_t* const y = static_cast<bf16_t*>(Y);
-    const int how = syrk_ragged_reads(x, ldx, M, K);
+    const int how = syrk_ragged_reads(x, ldx, K);
     const SyrkPad p = syrk_pad_layout(M, K);
     const bool aligned = ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;
     const int rows = how == kReadsLines ? kRowsLines : ldx % 32 == 0 ? kRowsHalfLines : kRowsAny;
-    const bool pad = may_copy && (how == kReadsLines || !whole_tiles(M, K)) && syrk_padded_pays(M, K, rows, aligned) && room(p.total);
-    if (!pad && (how == kReadsLines || (how == kReadsRows && !whole_tiles(M, K))) && room(r.slots ? r.slots + 256 : 0))
-      return hip_status(launch_syrk_ragged(x, ldx, y, ldy, M, K, elem == kElemF16, ws, r.slots, hs));
-    if (pad) {
+    // an odd number of whole tiles off the lines is left to launch_gemm_nt
+    const bool in_place = how == kReadsLines || (how == kReadsRows && !whole_tiles(M, K));
+    const bool slots = room(r.slots ? r.slots + 256 : 0);
+    if (may_copy && (how == kReadsLines || !whole_tiles(M, K)) && syrk_padded_pays(M, K, rows, aligned) && room(p.total)) {
       unsigned char* w = static_cast<unsigned char*>(ws);
       bf16_t* Xp = reinterpret_cast<bf16_t*>(w + p.x);
       bf16_t* Yp = reinterpret_cast<bf16_t*>(w + p.y);
@@ -273,11 +273,18 @@ static int syrk_impl(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64
       if (launch_gemm_nt(a, w + p.gemm, ws_bytes - p.gemm, hs)) return FM_ERR_LAUNCH;
       return hip_status(launch_copy2d_batched(Yp, p.Mp, 0, &y, ldy, 1, M, M, M, M, hs));
     }
+    const bool copy_wanted = how == kReadsNot || (how == kReadsRows && syrk_copy_pays(M, K));
+    if (in_place && slots && !copy_wanted)
+      return hip_status(launch_syrk_ragged(x, ldx, y, ldy, M, K, elem == kElemF16, ws, r.slots, hs));
     if (may_copy && !whole_tiles(M, K) && room(r.total)) {
       bf16_t* copy = reinterpret_cast<bf16_t*>(static_cast<unsigned char*>(ws) + r.x);
       if (launch_copy2d_batched(x, ldx, 0, &copy, r.Kp, 1, M, K, M, r.Kp, hs)) return FM_ERR_LAUNCH;
       return hip_status(launch_syrk_ragged(copy, r.Kp, y, ldy, M, r.Kp, elem == kElemF16, ws, r.slots, hs));
     }
+    // no room for a copy, or none allowed: in place where the rows can be read, with whole tiles if there is no room for parts either
+    // (3000 x 5000 75 us, the general schedule 99)
+    if (in_place && !whole_tiles(M, K))
+      return hip_status(launch_syrk_ragged(x, ldx, y, ldy, M, K, elem == kElemF16, slots ? ws : nullptr, slots ? r.slots : 0, hs));
   }
   a.A = a.B = static_cast<const bf16_t*>(X); a.lda = a.ldb = ldx;
   a.C = a.C2 = static_cast<bf16_t*>(Y);

@@ -163,10 +163,9 @@ size_t syrk_ragged_workspace_bytes(int M, int K) {
   return (size_t)s.cut * s.parts * kPartFloats * sizeof(float);
 }
 
-int syrk_ragged_reads(const bf16_t* X, int64_t ldx, int M, int K) {
-  if (K < t128::BK || K % 8 != 0 || ldx % 8 != 0 || ldx >= (1 << 23) || (reinterpret_cast<uintptr_t>(X) & 15) != 0) return kReadsCopy;
-  if (ldx % 64 == 0 && (reinterpret_cast<uintptr_t>(X) & 127) == 0) return kReadsLines;
-  return syrk_copy_pays(M, K) ? kReadsCopy : kReadsRows;
+int syrk_ragged_reads(const bf16_t* X, int64_t ldx, int K) {
+  if (K < t128::BK || K % 8 != 0 || ldx % 8 != 0 || ldx >= (1 << 23) || (reinterpret_cast<uintptr_t>(X) & 15) != 0) return kReadsNot;
+  return ldx % 64 == 0 && (reinterpret_cast<uintptr_t>(X) & 127) == 0 ? kReadsLines : kReadsRows;
 }
 
 int launch_syrk_ragged(const bf16_t* X, int64_t ldx, bf16_t* Y, int64_t ldy, int M, int K, bool f16, void* ws, size_t ws_bytes, hipStream_t stream) {

@@ -156,10 +156,9 @@ int launch_syrk_f32(const float* X, int64_t ldx, float* Y, int64_t rs, int64_t c
                     size_t ws_bytes, hipStream_t stream);
 // Y = X X^T in 16 bits of any M and K, read and written in place (fm_gemm_ragged.hip), for rows of X that 16-byte copies
 // can take, Y's lines of unit stride ldy apart; without a workspace of syrk_ragged_workspace_bytes the tiles stay whole.
-// How such a matrix is read best: by its rows as they lie on 128-byte lines, by its rows although they do not,
-// or not at all before it has been copied.
-constexpr int kReadsLines = 0, kReadsRows = 1, kReadsCopy = 2;
-int syrk_ragged_reads(const bf16_t* X, int64_t ldx, int M, int K);
+// How such a matrix can be read: by its rows, which lie on 128-byte lines or do not, or not before it has been copied.
+constexpr int kReadsLines = 0, kReadsRows = 1, kReadsNot = 2;
+int syrk_ragged_reads(const bf16_t* X, int64_t ldx, int K);
 size_t syrk_ragged_workspace_bytes(int M, int K);
 int launch_syrk_ragged(const bf16_t* X, int64_t ldx, bf16_t* Y, int64_t ldy, int M, int K, bool f16, void* ws, size_t ws_bytes,
                        hipStream_t stream);

@@ -4,7 +4,7 @@ copied first.  Integer inputs: every sum is exact in fp32 (and fp64), so the res
 import pytest
 import torch
 
-from flash_muon_amd import matmul_transpose_assign
+from flash_muon_amd import _lib, matmul_transpose_assign
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -66,3 +66,28 @@ def test_what_outgrows_the_cache_is_padded(M, K):
     want = (x @ x.T).bfloat16().cpu()
     assert torch.equal(_run(X, K, M), want)
     assert torch.equal(_run(X, K, M + 5, 3), want)
+
+
+def test_rows_that_can_be_read_are_read_in_place_where_there_is_no_room_for_a_copy(lib):
+    """3000 x 4992 in rows off the lines is copied first, given the room; without it the same tiles and pieces run in place (the bits of the
+    copied call; the general schedule adds in another order), and with no workspace at all the tiles stay whole."""
+    M, K, pitch = 3000, 4992, 5000
+    X = torch.randn(M, pitch, generator=torch.Generator().manual_seed(1)).bfloat16().to(DEV)
+    full = lib.fm_syrk_workspace_bytes(M, K)
+    ws = torch.full((full,), 255, dtype=torch.uint8, device=DEV)
+
+    def call(ws_bytes):
+        y = torch.empty(M, M, dtype=torch.bfloat16, device=DEV)
+        _lib.check("fm_syrk_bf16", lib.fm_syrk_bf16(X.data_ptr(), pitch, y.data_ptr(), M, 1, M, K, ws.data_ptr(), ws_bytes, _lib.stream_ptr(X.device)))
+        return y
+
+    copied = call(full)
+    assert torch.equal(call(16 << 20), copied)   # room for the parts alone
+    y = torch.empty(M, M, dtype=torch.bfloat16, device=DEV)
+    _lib.check("fm_syrk_bf16_static", lib.fm_syrk_bf16_static(X.data_ptr(), pitch, y.data_ptr(), M, 1, M, K, _lib.stream_ptr(X.device)))
+    assert torch.equal(y, copied)
+    whole = call(0)
+    assert torch.equal(whole, whole.T)
+    # tiles that nothing cuts: the first 4 rows of tiles, in the order they are kept whole in
+    assert torch.equal(whole[:512, :512], copied[:512, :512])
+    assert float((whole.float() - copied.float()).norm() / copied.float().norm()) < 1e-3
