@@ -62,7 +62,7 @@ NsLayout ns_layout(int batch, int rows, int cols) {
   const int m = rows < cols ? rows : cols, k = rows < cols ? cols : rows;
   const size_t B = (size_t)batch;
   NsLayout l = {};
-  if (ns_flow_chosen(batch, m, k)) {
+  if (!any_knob_set() && ns_flow_chosen(batch, m, k)) {
     l.flow = true;
     ns_flow_edges(batch, m, k, &l.edge_s, &l.edge_x);
     l.M = (m + l.edge_x - 1) / l.edge_x * l.edge_x;
@@ -171,7 +171,7 @@ constexpr int64_t kSyrkRaggedMinElems = 256 * 256;
 static bool whole_tiles(int M, int K) { return M % 128 == 0 && K % 64 == 0; }
 static bool syrk_ragged_layout(int M, int K, SyrkRagged* p) {
   if (M <= 0 || K <= 0 || (int64_t)M * K < kSyrkRaggedMinElems || K >= (1 << 22)) return false;
-  if (whole_tiles(M, K) && (M % 256 == 0 || !syrk_whole_in_place(M, K, cu_count()))) return false;
+  if (whole_tiles(M, K) && (M % 256 == 0 || any_knob_set() || !syrk_whole_in_place(M, K, cu_count()))) return false;
   p->Kp = (K + 63) / 64 * 64;
   p->slots = syrk_ragged_workspace_bytes(M, K);
   p->x = align_up(p->slots, 256);   // (a copy has as many stages, and so the same pieces)
@@ -179,11 +179,13 @@ static bool syrk_ragged_layout(int M, int K, SyrkRagged* p) {
   p->total = p->x + (whole_tiles(M, K) ? 0 : align_up((size_t)M * p->Kp * 2, 256)) + 256;
   return true;
 }
-// Both X and Y as copies padded to whole 256-tiles, where that is estimated to be faster (syrk_padded_pays).
+// Both X and Y as copies padded to whole 256-tiles, where that is estimated to be faster (syrk_padded_pays), or, with a knob set,
+// to the 128- or 256-tiles of the schedules that it speaks of.
 struct SyrkPad { int Mp, Kp; size_t x, y, gemm, total; };
 static SyrkPad syrk_pad_layout(int M, int K) {
   SyrkPad p;
-  p.Mp = (M + 255) / 256 * 256;
+  const int edge = any_knob_set() && M <= 2816 ? 128 : 256;
+  p.Mp = (M + edge - 1) / edge * edge;
   p.Kp = (K + 63) / 64 * 64;
   p.x = 0;
   p.y = align_up((size_t)p.Mp * p.Kp * 2, 256);
@@ -199,7 +201,7 @@ size_t fm_syrk_workspace_bytes(int M, int K) {
   if (!syrk_ragged_layout(M, K, &r)) return need;
   if (r.total > need) need = r.total;
   // (rows may lie on lines or not, and Y's rows allow 16-byte stores or not)
-  if ((K % 64 == 0 && syrk_padded_pays(M, K, kRowsLines, true)) || (!whole_tiles(M, K) && syrk_padded_pays(M, K, kRowsAny, true))) {
+  if ((any_knob_set() && !whole_tiles(M, K)) || (K % 64 == 0 && syrk_padded_pays(M, K, kRowsLines, true)) || (!whole_tiles(M, K) && syrk_padded_pays(M, K, kRowsAny, true))) {
     const SyrkPad p = syrk_pad_layout(M, K);
     if (p.total > need) need = p.total;
   }
@@ -261,8 +263,8 @@ static int syrk_impl(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64
     const int rows = how == kReadsLines ? kRowsLines : ldx % 32 == 0 ? kRowsHalfLines : kRowsAny;
     // an odd number of whole tiles off the lines is left to launch_gemm_nt
     const bool in_place = how == kReadsLines || (how == kReadsRows && !whole_tiles(M, K));
-    const bool slots = room(r.slots ? r.slots + 256 : 0);
-    if (may_copy && (how == kReadsLines || !whole_tiles(M, K)) && syrk_padded_pays(M, K, rows, aligned) && room(p.total)) {
+    const bool slots = room(r.slots ? r.slots + 256 : 0), forced = any_knob_set();   // (a knob has left whole tiles to launch_gemm_nt)
+    if (may_copy && (how == kReadsLines || !whole_tiles(M, K)) && (forced || syrk_padded_pays(M, K, rows, aligned)) && room(p.total)) {
       unsigned char* w = static_cast<unsigned char*>(ws);
       bf16_t* Xp = reinterpret_cast<bf16_t*>(w + p.x);
       bf16_t* Yp = reinterpret_cast<bf16_t*>(w + p.y);
@@ -274,16 +276,16 @@ static int syrk_impl(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64
       return hip_status(launch_copy2d_batched(Yp, p.Mp, 0, &y, ldy, 1, M, M, M, M, hs));
     }
     const bool copy_wanted = how == kReadsNot || (how == kReadsRows && syrk_copy_pays(M, K));
-    if (in_place && slots && !copy_wanted)
+    if (!forced && in_place && slots && !copy_wanted)
       return hip_status(launch_syrk_ragged(x, ldx, y, ldy, M, K, elem == kElemF16, ws, r.slots, hs));
-    if (may_copy && !whole_tiles(M, K) && room(r.total)) {
+    if (!forced && may_copy && !whole_tiles(M, K) && room(r.total)) {
       bf16_t* copy = reinterpret_cast<bf16_t*>(static_cast<unsigned char*>(ws) + r.x);
       if (launch_copy2d_batched(x, ldx, 0, &copy, r.Kp, 1, M, K, M, r.Kp, hs)) return FM_ERR_LAUNCH;
       return hip_status(launch_syrk_ragged(copy, r.Kp, y, ldy, M, r.Kp, elem == kElemF16, ws, r.slots, hs));
     }
     // no room for a copy, or none allowed: in place where the rows can be read, with whole tiles if there is no room for parts either
     // (3000 x 5000 75 us, the general schedule 99)
-    if (in_place && !whole_tiles(M, K))
+    if (!forced && in_place && !whole_tiles(M, K))
       return hip_status(launch_syrk_ragged(x, ldx, y, ldy, M, K, elem == kElemF16, slots ? ws : nullptr, slots ? r.slots : 0, hs));
   }
   a.A = a.B = static_cast<const bf16_t*>(X); a.lda = a.ldb = ldx;

@@ -260,6 +260,12 @@ int set_knob(int which, long long value) {
   return 0;
 }
 
+bool any_knob_set() {
+  for (int i = 0; i < kKnobCount; ++i)
+    if (knob(i) >= 0) return true;
+  return false;
+}
+
 int cu_count() {
   constexpr int kMaxDev = 64;
   static std::atomic<int> cached[kMaxDev];

@@ -24,6 +24,9 @@ constexpr int kErrWorkspace = -2;     // the schedule needs more partial-tile sl
 constexpr int kKnobGrid = 0, kKnobKsplit = 1, kKnobFastMinUnits = 2, kKnobNoMid = 3, kKnobNoSub64 = 4, kKnobHalf = 5, kKnobDiagLast = 6, kKnobNoTickets = 7, kKnobCount = 8;
 long long knob(int which);
 int set_knob(int which, long long value);
+// The knobs speak of the schedules of launch_gemm_nt: while one is set, every product runs there, and not on the kernels that
+// have none of their own (fm_flow.hip, fm_gemm_ragged.hip).
+bool any_knob_set();
 // compute units of the current device (queried once per device)
 int cu_count();
 

@@ -57,7 +57,9 @@ FM_API const char* fm_status_string(int status);
 FM_API const char* fm_version(void);
 
 /* Tuning knobs, for experiments and for tests that have to reach a particular schedule.  A
- * negative value gives the decision back to the library.  The environment variables
+ * negative value gives the decision back to the library.  While a knob is set, Newton-Schulz runs a launch per product
+ * and products of sides that are no whole 256-tiles run on the schedules below too (copied to whole tiles first, with
+ * fm_syrk_workspace_bytes asked for while it is set), not on kernels of their own.  The environment variables
  * FLASHMUON_GRID, FLASHMUON_KSPLIT, FLASHMUON_FAST_MIN_UNITS, FLASHMUON_NO_MID, FLASHMUON_NO_SUB64, FLASHMUON_HALF,
  * FLASHMUON_DIAG_LAST and FLASHMUON_NO_TICKETS set the initial
  * values; they are read once, when the library is first used, never per call.  No counterpart in

@@ -155,3 +155,19 @@ def test_batched_newtonschulz_with_tiles_cut_along_k(lib, knobs, no_256_path):
     knobs("FLASHMUON_KSPLIT", 1)
     whole = fast_newtonschulz(G, steps=5)
     assert float((cut.float() - whole.float()).norm() / whole.float().norm()) < 2e-2
+
+
+@pytest.mark.parametrize("what", ["odd_tiles", "ragged", "newtonschulz"])
+def test_the_cut_reaches_products_that_other_kernels_take_by_themselves(lib, knobs, no_256_path, what):
+    """An odd number of whole tiles and ragged sides (multiplied in place otherwise) and a small Newton-Schulz (one launch otherwise): on
+    Gaussian input two parts along k round some sums differently from one."""
+    from flash_muon_amd import fast_newtonschulz
+    X = torch.randn(*{"odd_tiles": (640, 2048), "ragged": (600, 2040), "newtonschulz": (384, 1280)}[what],
+                    generator=torch.Generator().manual_seed(3)).bfloat16().to(DEV)
+    run = fast_newtonschulz if what == "newtonschulz" else matmul_transpose
+    knobs("FLASHMUON_KSPLIT", 2)
+    cut = run(X)
+    knobs("FLASHMUON_KSPLIT", 1)
+    whole = run(X)
+    assert not torch.equal(cut, whole)
+    assert float((cut.float() - whole.float()).norm() / whole.float().norm()) < (2e-2 if what == "newtonschulz" else 3e-3)

@@ -109,3 +109,15 @@ COPY_TIMES = [(3000, 5000, 75, 70), (7000, 2000, 129, 110), (2000, 2000, 23, 30)
 @pytest.mark.parametrize("M,K,in_place,copied", COPY_TIMES)
 def test_rows_off_lines_are_copied_where_it_measured_faster(routes, M, K, in_place, copied):
     assert bool(routes.syrk_copy_pays(M, K)) == (copied < in_place)
+
+
+@pytest.mark.parametrize("name,value", [("FLASHMUON_KSPLIT", 2), ("FLASHMUON_NO_MID", 1), ("FLASHMUON_FAST_MIN_UNITS", 0), ("FLASHMUON_HALF", 0)])
+def test_a_knob_leads_every_product_to_the_schedules_it_speaks_of(lib, knobs, name, value):
+    """The workspaces are those of launches per product, and of copies padded to whole tiles with the product's own scratch."""
+    per_product = lambda b, m, k: b * (4 * m * k + 2 * m * m) * 2
+    assert lib.fm_newtonschulz_batched_workspace_bytes(12, 1152, 1152) > 12 * (6 + 10) * 1152 * 1152 * 2      # one launch
+    knobs(name, value)
+    need = lib.fm_newtonschulz_batched_workspace_bytes(12, 1152, 1152)                                          # padded to 1280
+    assert per_product(12, 1280, 1280) < need < per_product(12, 1280, 1280) + lib.fm_gemm_workspace_bytes(1280, 1280) + (1 << 20)
+    assert lib.fm_syrk_workspace_bytes(1000, 2000) >= 2 * 1024 * (2048 + 1024) + lib.fm_gemm_workspace_bytes(1024, 1024)
+    assert lib.fm_syrk_workspace_bytes(1152, 4096) == lib.fm_gemm_workspace_bytes(1152, 1152)
