@@ -58,11 +58,12 @@ void ns_flow_edges(int batch, int m, int k, int* es, int* ex) {
   *ex = rect <= 256 ? 64 : 128;
   *es = rect <= 256 || sym <= 256 || (sym <= 440 && k >= 2 * m) ? 64 : 128;
 }
-NsLayout ns_layout(int batch, int rows, int cols) {
+// `flow`: one launch where that is the faster one
+NsLayout ns_layout(int batch, int rows, int cols, bool flow) {
   const int m = rows < cols ? rows : cols, k = rows < cols ? cols : rows;
   const size_t B = (size_t)batch;
   NsLayout l = {};
-  if (!any_knob_set() && ns_flow_chosen(batch, m, k)) {
+  if (flow && !any_knob_set() && ns_flow_chosen(batch, m, k)) {
     l.flow = true;
     ns_flow_edges(batch, m, k, &l.edge_s, &l.edge_x);
     l.M = (m + l.edge_x - 1) / l.edge_x * l.edge_x;
@@ -410,7 +411,13 @@ int fm_scale_cast_bf16(const void* G, int dtype, int rows, int cols, int64_t ldg
 
 size_t fm_newtonschulz_batched_workspace_bytes(int batch, int rows, int cols) {
   if (batch <= 0 || rows <= 0 || cols <= 0) return 0;
-  return ns_layout(batch, rows, cols).total;
+  return ns_layout(batch, rows, cols, true).total;
+}
+
+size_t fm_newtonschulz_batched_min_workspace_bytes(int batch, int rows, int cols) {
+  if (batch <= 0 || rows <= 0 || cols <= 0) return 0;
+  const size_t best = ns_layout(batch, rows, cols, true).total, launches = ns_layout(batch, rows, cols, false).total;
+  return best < launches ? best : launches;
 }
 
 size_t fm_newtonschulz_workspace_bytes(int rows, int cols) {
@@ -436,7 +443,8 @@ static int ns_impl(const void* const* G, int dtype, int batch, int rows, int col
       if (j != i && overlaps(mat_range(out[j], rows, cols, ldout, 2), oi)) return FM_ERR_ALIAS;
     }
   }
-  const NsLayout l = ns_layout(batch, rows, cols);
+  NsLayout l = ns_layout(batch, rows, cols, true);
+  if (l.flow && ws_bytes < l.total) l = ns_layout(batch, rows, cols, false);   // which keeps two iterates, not one for every step
   if (!ws || ws_bytes < l.total) return FM_ERR_WORKSPACE;
   if (reinterpret_cast<uintptr_t>(ws) % 256 != 0) return FM_ERR_ALIGN;
   {

@@ -29,6 +29,19 @@ def _rows_unit_stride(G):
 MAX_BATCH = 32  # kMaxBatch of the library: matrices per batched launch
 
 
+def _ns_workspace(lib, n, rows, cols, device):
+    """Scratch of one Newton-Schulz call.  Where memory is short for that of the one-launch iteration (every step's
+    iterate), that of a launch per product does."""
+    need = lib.fm_newtonschulz_batched_workspace_bytes(n, rows, cols)
+    try:
+        return _lib.workspace(need, device)
+    except torch.cuda.OutOfMemoryError:
+        least = lib.fm_newtonschulz_batched_min_workspace_bytes(n, rows, cols)
+        if least >= need:
+            raise
+    return _lib.workspace(least, device)
+
+
 def _newtonschulz_into(Gs, outs, steps):
     """Orthogonalise the 2-D matrices Gs (one shape, dtype and row pitch; bf16/fp16/fp32, rows
     unit-stride) into `outs` (bf16, same shape, one row pitch), every stage one launch for all."""
@@ -41,7 +54,7 @@ def _newtonschulz_into(Gs, outs, steps):
     g_ptrs = (ctypes.c_void_p * n)(*[g.data_ptr() for g in Gs])
     o_ptrs = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
     with _lib.on_device(G0.device):
-        ws, ws_bytes = _lib.workspace(lib.fm_newtonschulz_batched_workspace_bytes(n, rows, cols), G0.device)
+        ws, ws_bytes = _ns_workspace(lib, n, rows, cols, G0.device)
         st = lib.fm_newtonschulz_batched_bf16(g_ptrs, _lib.dtype_code(G0.dtype), n, rows, cols, ldg,
                                               o_ptrs, ldo, steps, a, b, c, NS_EPS,
                                               ws.data_ptr(), ws_bytes, _lib.stream_ptr(G0.device))
@@ -220,7 +233,7 @@ class Muon(torch.optim.Optimizer):
                     rows, cols = shape
                     a, b, c = NS_COEFFS
                     with _lib.on_device(dev):
-                        ws, ws_bytes = _lib.workspace(lib.fm_newtonschulz_batched_workspace_bytes(n, rows, cols), dev)
+                        ws, ws_bytes = _ns_workspace(lib, n, rows, cols, dev)
                         st = lib.fm_momentum_newtonschulz_batched(
                             (ctypes.c_void_p * n)(*[t.data_ptr() for t in gcs]),
                             (ctypes.c_void_p * n)(*[t.data_ptr() for t in bufs]),

@@ -237,6 +237,12 @@ FM_API size_t fm_newtonschulz_workspace_bytes(int rows, int cols);
  * flash_muon/muon.py:90-103 is meant to call the path.
  */
 FM_API size_t fm_newtonschulz_batched_workspace_bytes(int batch, int rows, int cols);
+
+/* The least scratch that fm_newtonschulz_batched_bf16 and fm_momentum_newtonschulz_batched run with: that of a launch per product where
+ * fm_newtonschulz_batched_workspace_bytes is that of the one launch and larger (up to 2.4 times).  With less than the latter the products are
+ * launches of their own: slower, and rounded in another order here and there.
+ */
+FM_API size_t fm_newtonschulz_batched_min_workspace_bytes(int batch, int rows, int cols);
 FM_API int fm_newtonschulz_batched_bf16(const void* const* G, int dtype, int batch, int rows, int cols,
                                         int64_t ldg, void* const* out, int64_t ldout, int steps,
                                         float a, float b, float c, float eps,

@@ -6,10 +6,13 @@ Tolerance: 1e-2 Frobenius-relative per five steps from 256 rows on, as for every
 rows the rounding of the iterate to bf16 averages out less (1.2e-2 for 64 x 64, whatever computes it), so
 there the bound is the error that rounding after every operation, as the reference does, makes on the same
 input: this path rounds in a third of those places."""
+import ctypes
+
 import pytest
 import torch
 
-from flash_muon_amd import fast_newtonschulz, synthetic
+from flash_muon_amd import _lib, fast_newtonschulz, synthetic
+from flash_muon_amd.muon import NS_COEFFS, NS_EPS
 from oracle import oracle
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +78,41 @@ def test_long_rows_on_both_sides_of_the_rule(rows, cols, batch):
     for i in range(2, batch):
         assert torch.equal(got[i], got[i % 2])
     _check(got[0].cpu(), Gs[0], 5)
+
+
+def test_the_scratch_of_launches_per_product_is_enough(lib):
+    """Every step's iterate, in one launch, takes more memory than calls had to bring before: what fits them still runs, a byte less does not."""
+    n, rows, cols = 12, 1152, 1500
+    full, least = lib.fm_newtonschulz_batched_workspace_bytes(n, rows, cols), lib.fm_newtonschulz_batched_min_workspace_bytes(n, rows, cols)
+    assert least < 0.8 * full
+    assert lib.fm_newtonschulz_batched_min_workspace_bytes(1, 64, 64) == lib.fm_newtonschulz_batched_workspace_bytes(1, 64, 64)
+    Gs = torch.stack([synthetic.gradient_like_bf16(rows, cols, 8, 7)] * n).to(DEV)
+    outs = torch.empty_like(Gs)
+    ws = torch.full((full,), 255, dtype=torch.uint8, device=DEV)
+    ptrs = lambda t: (ctypes.c_void_p * n)(*[t[i].data_ptr() for i in range(n)])
+
+    def call(ws_bytes):
+        return lib.fm_newtonschulz_batched_bf16(ptrs(Gs), _lib.FM_BF16, n, rows, cols, cols, ptrs(outs), cols, 5, *NS_COEFFS, NS_EPS, ws.data_ptr(),
+                                                ws_bytes, _lib.stream_ptr(Gs.device))
+
+    for ws_bytes in (full, full - 1, least):
+        outs.fill_(7.0)
+        assert call(ws_bytes) == 0
+        _check(outs[n - 1].cpu(), Gs[0].cpu(), 5)
+    assert call(least - 1) == 6   # FM_ERR_WORKSPACE
+
+
+def test_short_of_memory():
+    """A stack that fitted with the smaller scratch still does (the allocator's limit set for the length of the test)."""
+    G = synthetic.gradient_like_bf16(1920, 1920, 8, 5).to(DEV).expand(32, 1920, 1920).contiguous()
+    want = fast_newtonschulz(G[:1], 5)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 2.3e9) / total)
+        got = fast_newtonschulz(G, 5)   # 0.24 GB of result and 1.7 GB of scratch, where the one launch takes 3.8
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert float(oracle.rel_fro(got[31].cpu(), want[0].float().cpu())) < 1e-2
