@@ -149,7 +149,10 @@ def gemm_workspace(nbytes, device, stream=None):
     if ws is None or ws.numel() < nbytes:
         # zeroed once: its last 256 bytes hold the word the library counts sub-tile tickets in, which
         # the library keeps in order from then on (garbage there costs speed, never correctness)
-        ws = _gemm_ws[key] = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+        try:
+            ws = _gemm_ws[key] = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+        except torch.cuda.OutOfMemoryError:   # the calls run with less, or with none, on slower schedules
+            return (ws, ws.numel()) if ws is not None else (None, 0)
     return ws, ws.numel()
 
 

@@ -91,3 +91,23 @@ def test_rows_that_can_be_read_are_read_in_place_where_there_is_no_room_for_a_co
     # tiles that nothing cuts: the first 4 rows of tiles, in the order they are kept whole in
     assert torch.equal(whole[:512, :512], copied[:512, :512])
     assert float((whole.float() - copied.float()).norm() / copied.float().norm()) < 1e-3
+
+
+def test_padded_copies_that_find_no_memory():
+    """5248 x 12288 is padded, in 0.25 GB of scratch; where that cannot be had the product runs in place, as it did with 16 MiB."""
+    _lib.release_workspaces()
+    X = _ints(5248, 12288, 4, torch.bfloat16).to(DEV)
+    x = X.float()
+    want = (x @ x.T).bfloat16()
+    y = torch.empty_like(want)
+    del x
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 64e6) / total)
+        matmul_transpose_assign(X, y)
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(y, want)
