@@ -190,3 +190,30 @@ def test_the_main_loops_move_no_sums_between_registers(assembly):
         with_e = "ILb0ELi1E" in k or "ILb0ELi2E" in k
         assert c["mfma"] >= c["loop"], (k, c)
         assert c["moves"] <= (0 if with_e else 200), (k, c)
+
+
+def test_the_loads_of_a_scaled_tile_are_on_their_way_together(tmp_path):
+    """scale_cast_tile128_kernel reads its tile in 8 (16-bit) or 16 (fp32) loads per lane before it needs the first: with a branch
+    around each of them the compiler waits for every load by itself."""
+    if shutil.which(build.HIPCC) is None and not os.path.exists(build.HIPCC):
+        pytest.skip("no hipcc here")
+    out = tmp_path / "fm_elementwise.s"
+    cmd = [build.HIPCC, *[f for f in build.FLAGS if f != "-fPIC"], "-S", "--cuda-device-only", os.path.join(build.CSRC, "fm_elementwise.hip"), "-o", str(out)]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    kernel, run, longest = None, 0, {}
+    for line in out.read_text().split("\n"):
+        m = re.match(r"^(_Z\w*scale_cast_tile128_kernelILi(\d)\w*):", line)
+        if re.match(r"^_Z\w+:", line):
+            kernel, run = (m.group(1), int(m.group(2))) if m else None, 0
+        t = line.strip()
+        if kernel is None:
+            continue
+        if t.startswith("global_load_dwordx4"):
+            run += 1
+            longest[kernel] = max(longest.get(kernel, 0), run)
+        elif t.startswith("s_waitcnt") and "vmcnt" in t:
+            run = 0
+    assert len(longest) == 6
+    for (name, dtype), n in longest.items():
+        assert n == (16 if dtype == 2 else 8), (name, n)
