@@ -277,7 +277,6 @@ __global__ __launch_bounds__(256) void scale_cast_tile128_kernel(PtrList Gl, int
   const raw* G = reinterpret_cast<const raw*>(Gl.p[blockIdx.z]) + (int64_t)blockIdx.y * 128 * ldg + blockIdx.x * 128;
   unsigned short* D = HAS_D ? reinterpret_cast<unsigned short*>(Dl.p[blockIdx.z]) + (int64_t)blockIdx.y * 128 * ldd + blockIdx.x * 128 : nullptr;
   unsigned short* T = reinterpret_cast<unsigned short*>(Tl.p[blockIdx.z]) + (int64_t)blockIdx.x * 128 * ldt + blockIdx.y * 128;
-  __shared__ float red[4];
   const int tid = threadIdx.x;
   const int ch = tid & 15;   // 8-element chunk along the contiguous dimension
   constexpr int NV = sizeof(raw) / 2;   // 16-byte loads per 8 elements
@@ -302,7 +301,8 @@ __global__ __launch_bounds__(256) void scale_cast_tile128_kernel(PtrList Gl, int
 #pragma unroll
       for (int q = 0; q < NV; ++q) in[pass][h].v[q] = reinterpret_cast<const uint4*>(src)[q];
     }
-  const float denom = __builtin_sqrtf(sum_of_squares(sumsq, parts, red)) + eps;   // while the tile is on its way
+  // while the tile is on its way, and in its LDS: 16 bytes more would leave room for four blocks per CU instead of five
+  const float denom = __builtin_sqrtf(sum_of_squares(sumsq, parts, reinterpret_cast<float*>(tile))) + eps;
 #pragma unroll
   for (int pass = 0; pass < 4; ++pass) {
     const int rp = pass * 16 + (tid >> 4);   // rows 2 rp and 2 rp + 1 of the tile

@@ -192,17 +192,22 @@ def test_the_main_loops_move_no_sums_between_registers(assembly):
         assert c["moves"] <= (0 if with_e else 200), (k, c)
 
 
-def test_the_loads_of_a_scaled_tile_are_on_their_way_together(tmp_path):
-    """scale_cast_tile128_kernel reads its tile in 8 (16-bit) or 16 (fp32) loads per lane before it needs the first: with a branch
-    around each of them the compiler waits for every load by itself."""
+@pytest.fixture(scope="module")
+def elementwise(tmp_path_factory):
     if shutil.which(build.HIPCC) is None and not os.path.exists(build.HIPCC):
         pytest.skip("no hipcc here")
-    out = tmp_path / "fm_elementwise.s"
+    out = tmp_path_factory.mktemp("asm") / "fm_elementwise.s"
     cmd = [build.HIPCC, *[f for f in build.FLAGS if f != "-fPIC"], "-S", "--cuda-device-only", os.path.join(build.CSRC, "fm_elementwise.hip"), "-o", str(out)]
     r = subprocess.run(cmd, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-2000:]
+    return out.read_text().split("\n")
+
+
+def test_the_loads_of_a_scaled_tile_are_on_their_way_together(elementwise):
+    """scale_cast_tile128_kernel reads its tile in 8 (16-bit) or 16 (fp32) loads per lane before it needs the first: with a branch
+    around each of them the compiler waits for every load by itself."""
     kernel, run, longest = None, 0, {}
-    for line in out.read_text().split("\n"):
+    for line in elementwise:
         m = re.match(r"^(_Z\w*scale_cast_tile128_kernelILi(\d)\w*):", line)
         if re.match(r"^_Z\w+:", line):
             kernel, run = (m.group(1), int(m.group(2))) if m else None, 0
@@ -217,3 +222,16 @@ def test_the_loads_of_a_scaled_tile_are_on_their_way_together(tmp_path):
     assert len(longest) == 6
     for (name, dtype), n in longest.items():
         assert n == (16 if dtype == 2 else 8), (name, n)
+
+
+def test_five_blocks_of_a_scaled_tile_fit_a_cu(elementwise):
+    """160 KB of LDS are five blocks of the 32 KB that a 128x128 tile takes, and four of a byte more."""
+    kernel, sizes = None, {}
+    for line in elementwise:
+        m = re.match(r"^\s*\.amdhsa_kernel (\S+)", line)
+        if m:
+            kernel = m.group(1)
+        m = re.match(r"^\s*\.amdhsa_group_segment_fixed_size (\d+)", line)
+        if m and "scale_cast_tile128_kernel" in kernel:
+            sizes[kernel] = int(m.group(1))
+    assert len(sizes) == 6 and all(5 * n <= 160 * 1024 for n in sizes.values()), sizes
