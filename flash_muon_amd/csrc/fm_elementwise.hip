@@ -267,8 +267,8 @@ __global__ __launch_bounds__(256) void scale_cast_kernel(PtrList Gl, int rows, i
 // in 16-byte reads: word p of column c sits at word p ^ 4 (c / 8 % 16) of the column's 64, which
 // keeps both the writes of a wave (16 column chunks x 4 row pairs) and its reads (16 consecutive
 // groups of a column) on 64 different banks.
-// HAS_D: D is wanted too, and not T alone.
-template <int DT, bool HAS_D>
+// HAS_D: D is wanted too, and not T alone.  ONE: the sum of squares is there as one number (as an argument it costs 0.2 to 1 us of 5 to 13).
+template <int DT, bool HAS_D, bool ONE>
 __global__ __launch_bounds__(256) void scale_cast_tile128_kernel(PtrList Gl, int64_t ldg, const float* sumsq,
                                                                  int parts, float eps, PtrList Dl, int64_t ldd,
                                                                  PtrList Tl, int64_t ldt, int tiles_r, int tiles_c) {
@@ -291,6 +291,7 @@ __global__ __launch_bounds__(256) void scale_cast_tile128_kernel(PtrList Gl, int
     }
     return;
   }
+  float denom = ONE ? __builtin_sqrtf(sumsq[blockIdx.z]) + eps : 0.0f;
   union In { uint4 v[NV]; raw e[8]; };
   In in[4][2];
 #pragma unroll
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(256) void scale_cast_tile128_kernel(PtrList Gl, int
       for (int q = 0; q < NV; ++q) in[pass][h].v[q] = reinterpret_cast<const uint4*>(src)[q];
     }
   // while the tile is on its way, and in its LDS: 16 bytes more would leave room for four blocks per CU instead of five
-  const float denom = __builtin_sqrtf(sum_of_squares(sumsq, parts, reinterpret_cast<float*>(tile))) + eps;
+  if constexpr (!ONE) denom = __builtin_sqrtf(sum_of_squares(sumsq, parts, reinterpret_cast<float*>(tile))) + eps;
 #pragma unroll
   for (int pass = 0; pass < 4; ++pass) {
     const int rp = pass * 16 + (tid >> 4);   // rows 2 rp and 2 rp + 1 of the tile
@@ -392,11 +393,19 @@ int launch_scale_cast_batched(const void* const* G, int batch, int dtype, int ro
   }
   if (T && gv && (dv || !D) && tv && rows_p % 128 == 0 && cols_p % 128 == 0 && rows % 128 == 0 && cols % 128 == 0) {
     dim3 grid128((unsigned)(cols_p / 128), (unsigned)(rows_p / 128), (unsigned)batch);
-#define FM_SCALE128(DT, HAS_D) hipLaunchKernelGGL((scale_cast_tile128_kernel<DT, HAS_D>), grid128, dim3(256), 0, stream, gl, ldg, \
-                                                  sumsq, parts, eps, dl, ldd, tl, ldt, rows / 128, cols / 128)
-    if (dtype == 0) { if (D) FM_SCALE128(0, true); else FM_SCALE128(0, false); }
-    else if (dtype == 1) { if (D) FM_SCALE128(1, true); else FM_SCALE128(1, false); }
-    else { if (D) FM_SCALE128(2, true); else FM_SCALE128(2, false); }
+#define FM_SCALE128_(DT, HAS_D, ONE) hipLaunchKernelGGL((scale_cast_tile128_kernel<DT, HAS_D, ONE>), grid128, dim3(256), 0, stream, gl, ldg, \
+                                                        sumsq, parts, eps, dl, ldd, tl, ldt, rows / 128, cols / 128)
+#define FM_SCALE128(DT)                                                                  \
+  do {                                                                                   \
+    if (D && parts == 1) FM_SCALE128_(DT, true, true);                                   \
+    else if (D) FM_SCALE128_(DT, true, false);                                           \
+    else if (parts == 1) FM_SCALE128_(DT, false, true);                                  \
+    else FM_SCALE128_(DT, false, false);                                                 \
+  } while (0)
+    if (dtype == 0) FM_SCALE128(0);
+    else if (dtype == 1) FM_SCALE128(1);
+    else FM_SCALE128(2);
+#undef FM_SCALE128_
 #undef FM_SCALE128
     return (int)hipGetLastError();
   }

@@ -219,7 +219,7 @@ def test_the_loads_of_a_scaled_tile_are_on_their_way_together(elementwise):
             longest[kernel] = max(longest.get(kernel, 0), run)
         elif t.startswith("s_waitcnt") and "vmcnt" in t:
             run = 0
-    assert len(longest) == 6
+    assert len(longest) == 12
     for (name, dtype), n in longest.items():
         assert n == (16 if dtype == 2 else 8), (name, n)
 
@@ -234,4 +234,4 @@ def test_five_blocks_of_a_scaled_tile_fit_a_cu(elementwise):
         m = re.match(r"^\s*\.amdhsa_group_segment_fixed_size (\d+)", line)
         if m and "scale_cast_tile128_kernel" in kernel:
             sizes[kernel] = int(m.group(1))
-    assert len(sizes) == 6 and all(5 * n <= 160 * 1024 for n in sizes.values()), sizes
+    assert len(sizes) == 12 and all(5 * n <= 160 * 1024 for n in sizes.values()), sizes
