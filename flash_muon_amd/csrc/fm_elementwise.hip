@@ -391,7 +391,8 @@ int launch_scale_cast_batched(const void* const* G, int batch, int dtype, int ro
 #undef FM_SCALE_ROWS
     return (int)hipGetLastError();
   }
-  if (T && gv && (dv || !D) && tv && rows_p % 128 == 0 && cols_p % 128 == 0 && rows % 128 == 0 && cols % 128 == 0) {
+  if (T && gv && (dv || !D) && tv && rows_p % 128 == 0 && cols_p % 128 == 0 && rows % 128 == 0 && cols % 128 == 0 &&
+      (D || parts > 1 || scale_cast_t_on_128((int64_t)(rows_p / 128) * (cols_p / 128) * batch))) {
     dim3 grid128((unsigned)(cols_p / 128), (unsigned)(rows_p / 128), (unsigned)batch);
 #define FM_SCALE128_(DT, HAS_D, ONE) hipLaunchKernelGGL((scale_cast_tile128_kernel<DT, HAS_D, ONE>), grid128, dim3(256), 0, stream, gl, ldg, \
                                                         sumsq, parts, eps, dl, ldd, tl, ldt, rows / 128, cols / 128)

@@ -13,6 +13,10 @@ inline int64_t scale_cast_rows_blocks(int64_t rows_p, int64_t cols_p) {
   return chunks + blocks * 256 <= INT32_MAX ? blocks : 0;
 }
 
+// T alone, of whole 128-tiles and a given sum of squares, on the kernel of 128x128 tiles rather than that of 64x64: from about half as many of them as
+// CUs on.  us, 64 / 128: 768^2 3.9 / 4.3, 1024^2 4.1 / 4.3 (64 tiles; fp32 4.1 / 4.6), 1536^2 4.8 / 4.8, 2048^2 6.4 / 5.4, 4096^2 15.9 / 13.0.
+inline bool scale_cast_t_on_128(int64_t tiles) { return tiles >= 128; }
+
 // Which matrices iterate in one launch (fm_flow.hip): M x K with M <= K, `batch` of them.
 // Five steps in us, one launch / launches per product.  One or two matrices, whose products are chains of short launches:
 // 256^2 91 / 109, 1024^2 137 / 158, 1408^2 185 / 233, 1024 x 4096 209 / 234, 1408 x 2816 225 / 302, 2 of 640 x 2560 156 / 245, 2 of 1408^2 249 /

@@ -15,6 +15,7 @@ long long scale_cast_rows_blocks(long long r, long long c) { return fm::scale_ca
 int syrk_padded_pays(int M, int K, int rows, int aligned) { return fm::syrk_padded_pays(M, K, rows, aligned); }
 int syrk_whole_in_place(int M, int K) { return fm::syrk_whole_in_place(M, K, 256); }
 int syrk_copy_pays(int M, int K) { return fm::syrk_copy_pays(M, K); }
+int scale_cast_t_on_128(long long tiles) { return fm::scale_cast_t_on_128(tiles); }
 int ns_flow_chosen(int batch, int m, int k) { return fm::ns_flow_chosen(batch, m, k); }
 }
 """
@@ -47,6 +48,11 @@ def test_the_walk_over_rows_stays_below_two_to_the_31(routes, rows, cols):
         assert max(beyond) <= INT32_MAX
     else:   # what is left to the kernel of 64x64 tiles is only what would not fit
         assert chunks + chunks // 4 > INT32_MAX - 1024
+
+
+@pytest.mark.parametrize("side,on64,on128", [(768, 3.9, 4.3), (1024, 4.1, 4.3), (2048, 6.4, 5.4), (4096, 15.9, 13.0)])
+def test_a_lone_transpose_is_cast_on_the_tiles_that_measured_faster(routes, side, on64, on128):
+    assert bool(routes.scale_cast_t_on_128(ctypes.c_longlong((side // 128) ** 2))) == (on128 < on64)
 
 
 # (batch, M, K, us in one launch, us in launches per product), measured; the first ones are ordinary ratios
