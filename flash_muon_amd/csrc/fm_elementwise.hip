@@ -379,7 +379,8 @@ int launch_scale_cast_batched(const void* const* G, int batch, int dtype, int ro
     if (D) { dl.p[i] = D[i]; dv = dv && (reinterpret_cast<uintptr_t>(D[i]) & 15) == 0; }
     if (T) { tl.p[i] = T[i]; tv = tv && (reinterpret_cast<uintptr_t>(T[i]) & 15) == 0; }
   }
-  const int64_t row_blocks = D && !T && gv && dv && cols_p % 8 == 0 ? scale_cast_rows_blocks(rows_p, cols_p) : 0;
+  const bool on_tiles = parts == 1 && scale_cast_d_on_tiles(rows_p, cols_p);
+  const int64_t row_blocks = D && !T && !on_tiles && gv && dv && cols_p % 8 == 0 ? scale_cast_rows_blocks(rows_p, cols_p) : 0;
   if (row_blocks > 0) {
     // (4 chunks per thread, so that a block's sum of the partial sums is paid for)
     dim3 gridr((unsigned)row_blocks, 1, (unsigned)batch);

@@ -13,6 +13,11 @@ inline int64_t scale_cast_rows_blocks(int64_t rows_p, int64_t cols_p) {
   return chunks + blocks * 256 <= INT32_MAX ? blocks : 0;
 }
 
+// D alone with a given sum of squares: on the kernel of 64x64 tiles where those are whole, up to 2^25 elements, rather than on the walk over rows.  us, tiles /
+// rows: 1024^2 4.0 / 4.1, 1536^2 4.1 / 4.9, 2560^2 6.4 / 7.3, 2048 x 5504 9.2 / 10.2, 4096^2 12.4 / 12.8; but 4096 x 11008 30.7 / 28.1, 8192^2 41.7 / 41.0, and
+// 3000^2 11.0 / 8.5, 3 x 1000000 9.0 / 5.3, 1000000 x 8 33 / 7.6.
+inline bool scale_cast_d_on_tiles(int64_t rows, int64_t cols) { return rows % 64 == 0 && cols % 64 == 0 && rows * cols <= (1 << 25); }
+
 // T alone, of whole 128-tiles and a given sum of squares, on the kernel of 128x128 tiles rather than that of 64x64: from about half as many of them as
 // CUs on.  us, 64 / 128: 768^2 3.9 / 4.3, 1024^2 4.1 / 4.3 (64 tiles; fp32 4.1 / 4.6), 1536^2 4.8 / 4.8, 2048^2 6.4 / 5.4, 4096^2 15.9 / 13.0.
 inline bool scale_cast_t_on_128(int64_t tiles) { return tiles >= 128; }

@@ -15,6 +15,7 @@ long long scale_cast_rows_blocks(long long r, long long c) { return fm::scale_ca
 int syrk_padded_pays(int M, int K, int rows, int aligned) { return fm::syrk_padded_pays(M, K, rows, aligned); }
 int syrk_whole_in_place(int M, int K) { return fm::syrk_whole_in_place(M, K, 256); }
 int syrk_copy_pays(int M, int K) { return fm::syrk_copy_pays(M, K); }
+int scale_cast_d_on_tiles(long long r, long long c) { return fm::scale_cast_d_on_tiles(r, c); }
 int scale_cast_t_on_128(long long tiles) { return fm::scale_cast_t_on_128(tiles); }
 int ns_flow_chosen(int batch, int m, int k) { return fm::ns_flow_chosen(batch, m, k); }
 }
@@ -53,6 +54,12 @@ def test_the_walk_over_rows_stays_below_two_to_the_31(routes, rows, cols):
 @pytest.mark.parametrize("side,on64,on128", [(768, 3.9, 4.3), (1024, 4.1, 4.3), (2048, 6.4, 5.4), (4096, 15.9, 13.0)])
 def test_a_lone_transpose_is_cast_on_the_tiles_that_measured_faster(routes, side, on64, on128):
     assert bool(routes.scale_cast_t_on_128(ctypes.c_longlong((side // 128) ** 2))) == (on128 < on64)
+
+
+@pytest.mark.parametrize("rows,cols,tiles,walk", [(1536, 1536, 4.1, 4.9), (2560, 2560, 6.4, 7.3), (2048, 5504, 9.2, 10.2), (4096, 4096, 12.4, 12.8),
+                                                  (4096, 11008, 30.7, 28.1), (3000, 3000, 11.0, 8.5), (3, 1000000, 9.0, 5.3), (1000000, 8, 33.3, 7.6)])
+def test_a_lone_cast_takes_the_kernel_that_measured_faster(routes, rows, cols, tiles, walk):
+    assert bool(routes.scale_cast_d_on_tiles(ctypes.c_longlong(rows), ctypes.c_longlong(cols))) == (tiles < walk)
 
 
 # (batch, M, K, us in one launch, us in launches per product), measured; the first ones are ordinary ratios
