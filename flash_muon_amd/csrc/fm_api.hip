@@ -202,7 +202,7 @@ size_t fm_syrk_workspace_bytes(int M, int K) {
   if (!syrk_ragged_layout(M, K, &r)) return need;
   if (r.total > need) need = r.total;
   // (rows may lie on lines or not, and Y's rows allow 16-byte stores or not)
-  if ((any_knob_set() && !whole_tiles(M, K)) || (K % 64 == 0 && syrk_padded_pays(M, K, kRowsLines, true)) || (!whole_tiles(M, K) && syrk_padded_pays(M, K, kRowsAny, true))) {
+  if ((any_knob_set() && !whole_tiles(M, K)) || (K % 64 == 0 && syrk_padded_pays(M, K, kRowsLines, true)) || ((!whole_tiles(M, K) || M > 15 * 256) && syrk_padded_pays(M, K, kRowsAny, true))) {
     const SyrkPad p = syrk_pad_layout(M, K);
     if (p.total > need) need = p.total;
   }
@@ -265,7 +265,8 @@ static int syrk_impl(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64
     // an odd number of whole tiles off the lines is left to launch_gemm_nt
     const bool in_place = how == kReadsLines || (how == kReadsRows && !whole_tiles(M, K));
     const bool slots = room(r.slots ? r.slots + 256 : 0), forced = any_knob_set();   // (a knob has left whole tiles to launch_gemm_nt)
-    if (may_copy && (how == kReadsLines || !whole_tiles(M, K)) && (forced || syrk_padded_pays(M, K, rows, aligned)) && room(p.total)) {
+    // (whole tiles off the lines: 10112 x 8192 1025 us before the pairs of workgroups of launch_gemm_nt, 1082 with them, 686 padded; few of them stay there)
+    if (may_copy && (how == kReadsLines || !whole_tiles(M, K) || M > 15 * 256) && (forced || syrk_padded_pays(M, K, rows, aligned)) && room(p.total)) {
       unsigned char* w = static_cast<unsigned char*>(ws);
       bf16_t* Xp = reinterpret_cast<bf16_t*>(w + p.x);
       bf16_t* Yp = reinterpret_cast<bf16_t*>(w + p.y);
