@@ -62,10 +62,12 @@ def test_refuses_what_the_two_calls_refuse(lib):
     g, b = _tensors(1, 64, 64, torch.float32, 1.0, 1, 0), _tensors(1, 64, 64, torch.float32, 1.0, 2, 0)
     ws = torch.empty(lib.fm_newtonschulz_batched_workspace_bytes(1, 64, 64), dtype=torch.uint8, device=DEV)
     out = [torch.empty(64, 64, dtype=torch.bfloat16, device=DEV)]
+    before = [t.clone() for t in g + b]
     assert _fused(lib, g, g, out, 1, ws) == _lib.FM_ERR_ALIAS
     assert _fused(lib, g, b, g, 1, ws) == _lib.FM_ERR_ALIAS
     assert _fused(lib, g, b, b, 1, ws) == _lib.FM_ERR_ALIAS
     assert _fused(lib, g, b, out, 1, ws[:256]) == 6          # FM_ERR_WORKSPACE
     assert _fused(lib, g, b, out, 1, ws, steps=-1) == 2      # FM_ERR_SHAPE
-    before = g[0].clone()
-    assert torch.equal(g[0], before)
+    # and the momentum update of a refused call has not been made
+    for t, was in zip(g + b, before):
+        assert torch.equal(t, was)

@@ -1,7 +1,7 @@
-"""GPU parity of the symmetric product on matrices whose sides are not whole 128-tiles, which run
-through zero-padded copies in the workspace when it has fm_syrk_workspace_bytes(M, K): bit-exact
-against the integer CPU oracle, bit-exact symmetry, the same bits as the general schedule on integer
-inputs, nothing written outside the M x M result, and within one bf16 rounding of the fp32 oracle on
+"""GPU parity of the symmetric product on matrices whose sides are not whole 128-tiles, which are read in place, or behind a
+copy of X or as zero-padded copies in a workspace of fm_syrk_workspace_bytes(M, K): bit-exact
+against the integer CPU oracle, bit-exact symmetry, the same bits as the general schedule (outputs without a unit
+stride) on integer inputs, nothing written outside the M x M result, and within one bf16 rounding of the fp32 oracle on
 Gaussian inputs."""
 import pytest
 import torch
@@ -31,7 +31,7 @@ def _call(lib, entry, X, Y, ws_bytes):
 
 
 def test_workspace_sizes(lib):
-    # whole tiles and small matrices need what the product itself needs; ragged ones room for the copies
+    # whole tiles and small matrices need what the product itself needs; ragged ones have room for copies of X and Y
     assert lib.fm_syrk_workspace_bytes(1024, 2048) == lib.fm_gemm_workspace_bytes(1024, 1024)
     assert lib.fm_syrk_workspace_bytes(100, 37) == lib.fm_gemm_workspace_bytes(100, 100)
     assert lib.fm_syrk_workspace_bytes(1000, 1000) >= 2 * 1024 * 1024 * 2
@@ -44,13 +44,14 @@ def test_integer_inputs_bit_exact_on_both_schedules(lib, M, K):
     X = _int_matrix(M, K, 300 + M + K)
     want = oracle.xxt_int64(X).float().bfloat16()
     Xd = X.to(DEV)
-    padded = _call(lib, "fm_syrk_bf16", Xd, torch.empty(M, M, dtype=torch.bfloat16, device=DEV),
-                   lib.fm_syrk_workspace_bytes(M, K))
-    general = _call(lib, "fm_syrk_bf16", Xd, torch.empty(M, M, dtype=torch.bfloat16, device=DEV),
-                    lib.fm_gemm_workspace_bytes(M, M))
-    assert torch.equal(padded.cpu(), want)
+    tiled = _call(lib, "fm_syrk_bf16", Xd, torch.empty(M, M, dtype=torch.bfloat16, device=DEV),
+                  lib.fm_syrk_workspace_bytes(M, K))
+    # an output with no unit stride takes the general schedule, whatever the workspace
+    general = _call(lib, "fm_syrk_bf16", Xd, torch.empty(M, 2 * M, dtype=torch.bfloat16, device=DEV)[:, ::2],
+                    lib.fm_syrk_workspace_bytes(M, K))
+    assert torch.equal(tiled.cpu(), want)
     assert torch.equal(general.cpu(), want)
-    assert torch.equal(padded, padded.T)
+    assert torch.equal(tiled, tiled.T)
     assert torch.equal(matmul_transpose(Xd).cpu(), want)
 
 
@@ -115,7 +116,7 @@ def test_too_little_workspace_takes_the_general_schedule(lib):
 
 
 def test_repeated_calls_of_changing_shapes_share_the_workspace():
-    # the shared workspace keeps the last call's contents: the padding has to be rewritten every time
+    # the shared workspace keeps the last call's contents: a copy's padding and the parts of cut tiles have to be rewritten every time
     a = _int_matrix(1000, 900, 17).to(DEV)
     b = _int_matrix(600, 1500, 18).to(DEV)
     wa = oracle.xxt_int64(a.cpu()).float().bfloat16()
