@@ -10,8 +10,10 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-# whole tiles, and sides that are not (zero-padded copies in the workspace)
-@pytest.mark.parametrize("gshape,xshape", [((512, 1536), (768, 1024)), ((500, 1500), (700, 1000))])
+# whole tiles, and sides that are not: Newton-Schulz in one launch and in launches per product (padded), products in place with cut tiles, behind a
+# copy of the operand and as padded copies
+@pytest.mark.parametrize("gshape,xshape", [((512, 1536), (768, 1024)), ((500, 1500), (700, 1000)), ((1600, 2500), (3000, 5000)), ((700, 6000), (4000, 3000)),
+                                           ((1100, 5000), (1100, 4088))])
 def test_graph_replays_match_eager(gshape, xshape):
     G = synthetic.gradient_like_bf16(gshape[0], gshape[1], 8, 41).to(DEV)
     X = synthetic.gaussian_bf16(xshape[0], xshape[1], 42).to(DEV)

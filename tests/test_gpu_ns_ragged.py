@@ -1,5 +1,6 @@
 """GPU parity of fast_newtonschulz on matrices whose sides are not whole 128-tiles: the library keeps
-the iterates zero-padded to whole tiles in its workspace and copies the caller's part out.
+the iterates zero-padded to whole tiles in its workspace, in one launch (which writes the caller's part itself) for the
+smaller ones and in launches per product with a copy out for the others.
 
 Tolerance: Frobenius-relative error <= 1e-2 against the fp32 CPU oracle after five free-running
 steps (below 128 rows 2e-2, or 1.2 times the error of the reference's own bf16 rounding order where
@@ -33,6 +34,13 @@ def test_five_steps_against_the_oracle(rows, cols, rank, seed):
     # has noise directions that five steps amplify in any bf16 run, so there only that holds
     assert err < 1.2 * eager
     assert err < (TOL if min(rows, cols) >= 128 else max(TOL_SMALL, 1.2 * eager))
+
+
+@pytest.mark.parametrize("rows,cols,rank,seed", SHAPES)
+def test_launches_per_product(lib, knobs, rows, cols, rank, seed):
+    """What runs by itself in one launch, as launches per product (with a knob set, or little scratch): the same bound."""
+    knobs("FLASHMUON_NO_TICKETS", 0)
+    test_five_steps_against_the_oracle(rows, cols, rank, seed)
 
 
 @pytest.mark.parametrize("steps", [1, 2, 3])
@@ -96,7 +104,7 @@ def test_batched_matches_single_and_leaves_strided_output_alone(lib, rows, cols)
 
 def test_batch_padded_to_256_tiles_where_a_single_matrix_is_not():
     # eight matrices of 1280 x 1408 fill the GPU with 256x256 tiles, so the batch runs on 1280 x 1536;
-    # a single one stays on 128x128 tiles of 1280 x 1408: same results within the oracle's tolerance
+    # a single one runs unpadded, in one launch on 128x128 tiles: same results within the oracle's tolerance
     G = torch.stack([synthetic.gradient_like_bf16(1280, 1408, 8, 60 + i) for i in range(8)]).to(DEV)
     got = fast_newtonschulz(G, 5)
     assert got.shape == G.shape
