@@ -249,6 +249,8 @@ void f32_schedule(int M, int K, F32Args& p) {
 
 }  // namespace
 
+// (The last slot is never written - the last piece lies in the last tile alone, as piece <= nk - so that the ticket word that a workspace
+// shared with 16-bit products holds in its last 256 bytes stays as it is.)
 size_t syrk_f32_workspace_bytes(int M, int K) {
   F32Args p = {};
   f32_schedule(M, K, p);
