@@ -158,7 +158,8 @@ def gemm_workspace(nbytes, device, stream=None):
 
 def release_workspaces():
     """Give the cached scratch of the single GEMM-shaped calls back to torch's allocator.  One
-    tensor per (device, stream) is kept and only ever grows (up to about 256 MiB each); call this after
+    tensor per (device, stream) is kept and only ever grows (up to about 256 MiB each, or copies of operand and result for
+    large sides that are no whole tiles); call this after
     the last matmul_transpose on streams that will not be used again, or to drop a block that a call
     under graph capture took from the graph's private pool.  Not while such calls are in flight."""
     _gemm_ws.clear()

@@ -39,6 +39,14 @@ struct NsLayout {
   size_t counters;
 };
 constexpr int kFlowSteps = 5;   // steps per launch of the one-launch iteration
+// 64x64 tiles for X' as long as every CU gets at most one, and for the symmetric products as long as they are
+// about one round (a longer K makes the 64-tiles of A = X X^T pay a little further): 512^2 104 us on 64x64
+// tiles, 115 with X' on 128x128, 144 all on 128x128; 8 of 384 x 768 152, 111 and 133; 24 of 768^2 520, 423 and 360.
+void ns_flow_edges(int batch, int m, int k, int* es, int* ex) {
+  const int64_t t = (m + 63) / 64, sym = t * (t + 1) / 2 * batch, rect = t * ((k + 63) / 64) * batch;
+  *ex = rect <= 256 ? 64 : 128;
+  *es = rect <= 256 || sym <= 256 || (sym <= 440 && k >= 2 * m) ? 64 : 128;
+}
 // A matrix whose sides are not whole 128-tiles would take the general GEMM path in every stage
 // (0.5-0.8 times the vendor GEMMs).  Its iterates live in the workspace anyway, so they are kept
 // zero-padded to whole tiles instead: zero rows and columns stay zero through every step, and the
@@ -50,15 +58,7 @@ constexpr int kFlowSteps = 5;   // steps per launch of the one-launch iteration
 // 2816 x 7168 26).  The long side alone goes to a multiple of 256 where the short one is one already
 // (32 of 2048 x 5504 15.4 ms, of 2048 x 5632 11.9; one matrix 0.72 and 0.59; below 1536 rows a single
 // matrix gains nothing).
-// 64x64 tiles for X' as long as every CU gets at most one, and for the symmetric products as long as they are
-// about one round (a longer K makes the 64-tiles of A = X X^T pay a little further): 512^2 104 us on 64x64
-// tiles, 115 with X' on 128x128, 144 all on 128x128; 8 of 384 x 768 152, 111 and 133; 24 of 768^2 520, 423 and 360.
-void ns_flow_edges(int batch, int m, int k, int* es, int* ex) {
-  const int64_t t = (m + 63) / 64, sym = t * (t + 1) / 2 * batch, rect = t * ((k + 63) / 64) * batch;
-  *ex = rect <= 256 ? 64 : 128;
-  *es = rect <= 256 || sym <= 256 || (sym <= 440 && k >= 2 * m) ? 64 : 128;
-}
-// `flow`: one launch where that is the faster one
+// `flow`: one launch where that is the faster one (ns_flow_chosen).
 NsLayout ns_layout(int batch, int rows, int cols, bool flow) {
   const int m = rows < cols ? rows : cols, k = rows < cols ? cols : rows;
   const size_t B = (size_t)batch;
@@ -202,7 +202,8 @@ size_t fm_syrk_workspace_bytes(int M, int K) {
   if (!syrk_ragged_layout(M, K, &r)) return need;
   if (r.total > need) need = r.total;
   // (rows may lie on lines or not, and Y's rows allow 16-byte stores or not)
-  if ((any_knob_set() && !whole_tiles(M, K)) || (K % 64 == 0 && syrk_padded_pays(M, K, kRowsLines, true)) || ((!whole_tiles(M, K) || M > 15 * 256) && syrk_padded_pays(M, K, kRowsAny, true))) {
+  if ((any_knob_set() && !whole_tiles(M, K)) || (K % 64 == 0 && syrk_padded_pays(M, K, kRowsLines, true)) ||
+      ((!whole_tiles(M, K) || M > 15 * 256) && syrk_padded_pays(M, K, kRowsAny, true))) {
     const SyrkPad p = syrk_pad_layout(M, K);
     if (p.total > need) need = p.total;
   }
@@ -262,10 +263,10 @@ static int syrk_impl(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64
     const SyrkPad p = syrk_pad_layout(M, K);
     const bool aligned = ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;
     const int rows = how == kReadsLines ? kRowsLines : ldx % 32 == 0 ? kRowsHalfLines : kRowsAny;
-    // an odd number of whole tiles off the lines is left to launch_gemm_nt
+    // (an odd number of whole tiles off the lines is left to launch_gemm_nt)
     const bool in_place = how == kReadsLines || (how == kReadsRows && !whole_tiles(M, K));
     const bool slots = room(r.slots ? r.slots + 256 : 0), forced = any_knob_set();   // (a knob has left whole tiles to launch_gemm_nt)
-    // (whole tiles off the lines: 10112 x 8192 1025 us before the pairs of workgroups of launch_gemm_nt, 1082 with them, 686 padded; few of them stay there)
+    // (whole tiles off the lines, padded or by the pairs of workgroups of launch_gemm_nt: 10112 x 8192 686 us / 1082; few of them stay there)
     if (may_copy && (how == kReadsLines || !whole_tiles(M, K) || M > 15 * 256) && (forced || syrk_padded_pays(M, K, rows, aligned)) && room(p.total)) {
       unsigned char* w = static_cast<unsigned char*>(ws);
       bf16_t* Xp = reinterpret_cast<bf16_t*>(w + p.x);

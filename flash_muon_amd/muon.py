@@ -111,8 +111,8 @@ class Muon(torch.optim.Optimizer):
         rank, world_size: required, as in the reference; only (0, 1) is implemented.
         batch: (not in the reference) how many same-shape matrices are orthogonalised per launch,
             1..32; default 32.  Memory: the Newton-Schulz scratch of a launch (four padded copies of
-            the iterate, two squares; six and ten for matrices of up to about 1920 rows) is about 4.8 to 16
-            times the bytes of its bf16 matrices, 0.44 GB per 4096 x 11008 matrix and 14 GB for 32 of them (the reference holds about 0.3 GB, one
+            the iterate, two squares; six and ten for matrices of up to about 1920 rows, unless
+            memory is short) is about 4.8 to 16 times the bytes of its bf16 matrices, 0.44 GB per 4096 x 11008 matrix and 14 GB for 32 of them (the reference holds about 0.3 GB, one
             matrix at a time), taken from torch's caching allocator per call; a [batch, numel] bf16
             staging buffer per group stays with the optimizer (2.9 GB at the default for that
             shape).  A smaller batch shrinks both in proportion.

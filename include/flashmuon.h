@@ -114,11 +114,11 @@ FM_API int fm_syrk_bf16(const void* X, int64_t ldx, void* Y, int64_t ldy_row, in
                  int M, int K, void* ws, size_t ws_bytes, fm_stream_t stream);
 
 /* Scratch for fm_syrk_bf16 and fm_syrk_f16 by the shape of X: fm_gemm_workspace_bytes(M, M), and for
- * an X whose sides are not whole multiples of 128 at least room for a zero-padded copy of X and the padded
- * product.  Such shapes are read and written in place (rows that 16-byte copies can take), or read from
- * a copy of X, or multiplied as padded copies, whichever is faster; what is left of a last round of tiles is cut
- * along k and its fp32 sums lie here too.  With less than this the calls still run,
- * on the schedule that the scratch they get allows.  No counterpart in the reference, whose masked
+ * an X whose sides are not whole multiples of 128, or an odd number of them beyond what stays in the memory-side cache, at least
+ * room for a zero-padded copy of X and the padded product.  Such shapes are read and written in place (rows that 16-byte copies can
+ * take), or read from a copy of X, or multiplied as padded copies, whichever is estimated to be faster; what is left of a last
+ * round of tiles is cut along k and its fp32 sums lie here too.  With less than this the calls still run, on the schedule that the
+ * scratch they get allows: in place, with whole tiles if need be, wherever 16-byte copies can take the rows.  No counterpart in the reference, whose masked
  * loads and stores take any shape (flash_muon/matmul_transpose_triton.py:48-52, 70-75).
  */
 FM_API size_t fm_syrk_workspace_bytes(int M, int K);
@@ -179,8 +179,8 @@ FM_API int fm_syrk_poly_bf16(const void* A, int64_t lda, void* P, int64_t ldp, i
  * Xout = a*X + P*X for P (M x M, row stride ldp) and X (M x K, row stride ldx).  The
  * contraction runs over the rows of X, so the kernel reads X through its transpose
  * XT (K x M, row stride ldxt), which the caller supplies (fm_scale_cast_bf16 and this function
- * both produce it).  X and XT must hold the same values: on the 256x256 schedule the term a*X is
- * read through XT as well, on the other schedules through X.  Either output may be NULL, not both:
+ * both produce it).  X and XT must hold the same values: on the 256x256 schedule, and on 128x128 tiles where
+ * there are more of them than CUs, the term a*X is read through XT as well, on the other schedules through X.  Either output may be NULL, not both:
  * Xout is M x K (row stride ldo), XoutT is its transpose K x M (row stride ldot), written from the
  * same registers.
  * If row_alpha is not NULL (M floats), row i uses a + row_alpha[i] in place of a, i.e. the
@@ -217,13 +217,15 @@ FM_API int fm_scale_cast_bf16(const void* G, int dtype, int rows, int cols, int6
  * The whole quintic Newton-Schulz orthogonalisation of one matrix: G is rows x cols of `dtype`
  * (row stride ldg), out is rows x cols bf16 (row stride ldout).  Runs the sum of squares, the scaled
  * cast and `steps` x (fm_syrk_bf16, fm_syrk_poly_bf16, fm_gemm_axpby_bf16) on
- * `stream`, iterating on the wide orientation (M = min(rows, cols)).  Matrices of up to 512 to 1280 rows
- * (by size, shape and number) run all products of up to five steps as one launch, whose workgroups wait
+ * `stream`, iterating on the wide orientation (M = min(rows, cols)).  Matrices of up to 512 to 1920 rows
+ * (by size, shape and number; not with a long K) run all products of up to five steps as one launch, whose workgroups wait
  * for each other inside it but need not be resident together; their workspace holds every step's
- * iterate and squares (6 M K + 10 M^2 bf16 per matrix, against 4 M K + 2 M^2 otherwise).
+ * iterate and squares (6 M K + 10 M^2 bf16 per matrix, against 4 M K + 2 M^2 otherwise), and with less they run
+ * a launch per product (fm_newtonschulz_batched_min_workspace_bytes).
  * steps == 0 returns the normalised input.  out must not overlap G.  A matrix whose sides are not whole multiples of 128
  * (of 256 where whole 256x256 tiles are estimated to pay for the padding) is iterated on zero-padded to whole tiles inside the workspace (zero rows and columns stay zero
- * through every step) and the rows x cols part is copied out at the end.
+ * through every step); the last product writes the rows x cols part itself (one launch; whole multiples of 128 padded to 256), or it is
+ * copied out at the end.
  * Replaces fast_newtonschulz: flash_muon/muon.py:6-33.
  */
 FM_API size_t fm_newtonschulz_workspace_bytes(int rows, int cols);
