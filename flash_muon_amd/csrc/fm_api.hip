@@ -278,7 +278,7 @@ static int syrk_impl(const void* X, int64_t ldx, void* Y, int64_t ldy_row, int64
       if (launch_gemm_nt(a, w + p.gemm, ws_bytes - p.gemm, hs)) return FM_ERR_LAUNCH;
       return hip_status(launch_copy2d_batched(Yp, p.Mp, 0, &y, ldy, 1, M, M, M, M, hs));
     }
-    const bool copy_wanted = how == kReadsNot || (how == kReadsRows && syrk_copy_pays(M, K));
+    const bool copy_wanted = how == kReadsNot || (how == kReadsRows && syrk_copy_pays(M, K, rows == kRowsHalfLines));
     if (!forced && in_place && slots && !copy_wanted)
       return hip_status(launch_syrk_ragged(x, ldx, y, ldy, M, K, elem == kElemF16, ws, r.slots, hs));
     if (!forced && may_copy && !whole_tiles(M, K) && room(r.total)) {

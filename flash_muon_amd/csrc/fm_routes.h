@@ -117,14 +117,15 @@ inline double syrk_padded_us(int M, int K, bool aligned) {
   if (rem && parts < 16) t += 0.753 * nk / parts + (parts == 1 ? 8.0 : 11.4);   // (up to 16 of them run as sub-tiles beside the rounds)
   return t;
 }
-// Whether rows that 16-byte copies can take but that do not lie on 128-byte lines are copied first: a 128-byte piece of such a row makes two requests
-// of one.  us, in place / behind a copy of X: 3000 x 5000 75 / 70, 7000 x 2000 129 / 110; but 2000^2 23 / 30, 4000 x 1000 33 / 37, where a launch and 8
-// bytes of traffic per element cost more than they save in 16384 stages of tiles or less; and with a tile on four fifths of the CUs at most, whose stages
-// the requests do not hold up, 1956 x 12000 94 / 104, 2468 x 12000 100 / 112, 1920 x 65544 349 / 385, 1000 x 65544 106 / 126 (253 tiles: 2768 x 9784 107 / 101).
-inline bool syrk_copy_pays(int M, int K) {
+// Whether rows that 16-byte copies can take but that do not lie on 128-byte lines (`half`: on halves of them) are copied first: a 128-byte piece of such a
+// row makes two requests of one.  us, in place / behind a copy of X: 3000 x 5000 75 / 70, 7000 x 2000 129 / 110; but 2000^2 23 / 30, 4000 x 1000 33 / 37,
+// where a launch and 8 bytes of traffic per element cost more than they save in 16384 stages of tiles or less; and with a tile on half of the CUs (on half
+// lines four fifths), whose stages the requests do not hold up, 1000 x 65544 106 / 126, 1920 x 65544 349 / 385, half lines 1956 x 12000 94 / 104, 2468 x
+// 12000 100 / 112 (but 2432 x 9304, 190 tiles, 92 / 88, 2768 x 9784, 253 tiles, 107 / 101).
+inline bool syrk_copy_pays(int M, int K, bool half) {
   const RaggedSchedule s = ragged_schedule(M, K);
   const int64_t tiles = (int64_t)s.T * (s.T + 1) / 2;
-  return tiles > 210 && tiles * s.nk >= 16384;
+  return tiles > (half ? 210 : 136) && tiles * s.nk >= 16384;
 }
 // Whether it is padded, for matrices that may be (the copies cost memory: not for a gain of under 4 % of the estimates).  us, in place
 // or behind a copy of X / padded: 4000^2 86 / 78, 3936 x 4000 69 / 77, 5280 x 6000 183 / 167, 5536 x 4000 127 / 130, 7776 x 4000 242 / 248, 8096 x 8040 509 / 453,
