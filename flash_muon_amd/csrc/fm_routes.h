@@ -134,13 +134,13 @@ inline bool syrk_copy_pays(int M, int K, bool half) {
 // Below 16 tile rows of 256, where the padded product is cut along k over all CUs: of 8 to 10, whose 120 to 210 tiles of 128 leave CUs idle, by the time of
 // a stage in place (rows on lines, on half lines, neither) against a linear fit of the padded way: 2043 x 7496 74 / 67, 1956 x 12000 94 / 93, 2468 x 12000 100 / 116,
 // 2560 x 30416 289 / 223, x 24000 on lines 180 / 191, 2200 x 72576 on lines 581 / 416; of more only a matrix that does not fit the cache: 2980 x 24000 (143 MB) 220
-// / 319, 3200 x 32768 on lines (210 MB) 317 / 406, 2980 x 60000 (358 MB) 768 / 531; of fewer (1000 x 262144 340 / 497) none.
+// / 319, 3664 x 24072 off them (176 MB) 391 / 340, 3200 x 32768 on lines (210 MB) 317 / 406, 2980 x 60000 (358 MB) 768 / 531; of fewer (1000 x 262144 340 / 497) none.
 constexpr int kRowsLines = 0, kRowsHalfLines = 1, kRowsAny = 2;
 inline bool syrk_padded_pays(int M, int K, int rows, bool aligned) {
   if (K < 1500 || K > (1 << 21) - 128 || M <= 7 * 256) return false;   // (4056 x 1248 38 / 43; what the 256-tiles' byte offsets allow)
   const int T = (M + 255) / 256, nk = (K + 63) / 64;
   if (T <= 10) return 0.96 * (3.6 * T + (0.144 + 0.026 * T) * nk) < 2.0 + (rows == kRowsLines ? 0.47 : rows == kRowsHalfLines ? 0.51 : 0.60) * nk;
-  if (T < 16) return 2e-6 * M * K > (rows == kRowsLines ? 260.0 : 200.0);
+  if (T < 16) return 2e-6 * M * K > (rows == kRowsLines ? 260.0 : T >= 14 ? 130.0 : 200.0);
   return 0.96 * syrk_padded_us(M, K, aligned) < syrk_ragged_us(M, K, rows == kRowsLines);
 }
 

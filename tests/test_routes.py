@@ -82,7 +82,7 @@ def test_one_launch_newtonschulz_where_it_measured_faster(routes, lib, batch, m,
 
 
 # (M, K, us on 128x128 tiles - in place where the rows lie on lines, else behind a copy -, us padded to 256-tiles), measured
-PADDED_TIMES = [(1956, 6000, 54.4, 55.5), (1960, 6896, 63.4, 58.5), (2043, 7496, 74, 67), (2468, 12000, 99.6, 115.9), (2560, 30416, 289, 223), (2468, 24000, 180, 191),
+PADDED_TIMES = [(3664, 24072, 391, 340), (3748, 12000, 177.6, 187.1), (1956, 6000, 54.4, 55.5), (1960, 6896, 63.4, 58.5), (2043, 7496, 74, 67), (2468, 12000, 99.6, 115.9), (2560, 30416, 289, 223), (2468, 24000, 180, 191),
                 (2212, 24000, 175.1, 172), (2200, 72576, 581, 416), (1000, 262144, 340, 497), (3200, 32768, 316.8, 405), (2980, 60000, 768, 531), (1956, 60000, 562, 298), (2980, 24000, 220, 319), (3936, 4000, 69.4, 77.4), (4056, 1248, 37.6, 42.8), (4000, 4000, 85.9, 77.7), (3000, 5000, 70.1, 75.7),
                 (5280, 6000, 183, 167), (5792, 4000, 150, 193), (6048, 2000, 91, 122), (7776, 2000, 133, 161), (7580, 8040, 469, 429), (8096, 8040, 509, 453),
                 (8008, 4000, 246, 263), (8008, 16000, 1102, 821), (10000, 8000, 887, 700), (10000, 4000, 402, 429), (11000, 16000, 2106, 1577), (12000, 8000, 1291, 959),
