@@ -27,18 +27,40 @@ inline bool scale_cast_t_on_128(int64_t tiles) { return tiles >= 128; }
 // 256^2 91 / 109, 1024^2 137 / 158, 1408^2 185 / 233, 1024 x 4096 209 / 234, 1408 x 2816 225 / 302, 2 of 640 x 2560 156 / 245, 2 of 1408^2 249 /
 // 285; but 1536^2 258 / 254, 1280 x 5120 383 / 304 (its first product is cut along k there), 2 of 768 x 3072 236 / 223.  More of
 // them, with an odd number of 128-tiles (padded to 256-tiles, or on tiles of 128 in launches): 12 of 1152^2 532 / 817, 16
-// of 1408^2 1009 / 1669, 6 of 1408 x 3872 976 / 1224, 12 of 1664^2 1253 / 1821, 32 of 1920^2 5273 / 5411; an even one, as long as the 256-tiles
+// of 1408^2 1009 / 1669, 6 of 1408 x 3872 976 / 1224, 12 of 1664^2 1253 / 1821; an even one, as long as the 256-tiles
 // do not fill the GPU by themselves: 24 of 768^2 360 / 393, 16 of 768 x 3072 672 / 972, 16 of 1280^2 817 / 911, 6 of 1280 x 3520 774 / 844, 24 of
 // 1536^2 2046 / 2102; but 6 of 768 x 3072 407 / 366, 6 of 1024 x 2048 424 / 377, 6 of 1280^2 451 / 423, 24 of 2048^2 4600 / 4200.
+// So up to 768 rows of more than 1.5 : 1, and a few of 1280, only once X' would be more than about one round of 256-tiles (x, its 128-tiles, over 1000
+// and 1050): 12 of 744 x 1992 433 / 571 and 8 of 768 x 3072 431 / 559, but 8 of 696 x 1864 344 / 321 (x = 720) and 10 of 768 x 1760 361 / 352; 4 of
+// 1272 x 3416 586 / 678, but 4 of 1160 x 3112 550 / 517.  Three to seven of 1024 gain only where X' is about 256 or 512 tiles, one or two a CU (4 of
+// 1024^2 199 / 234, 7 of 1024 x 1152 312 / 346, but 6 of 1024^2 280 / 274, 3 of 1024 x 1536 272 / 260, 6 of 960 x 1440 368 / 339), or long.  30 and more
+// of 1280 fill the 256-tiles when long: 32 of 1280 x 3440 3693 / 3684, of 1216 x 4256 4466 / 4275.
+// An odd number of 128-tiles, 11 and more: the larger it is, the less the padding costs, and the longer the matrices and the more of them, the
+// better the 256-tiles are filled.  11: 16 of 1408 x 7744 4596 / 4974, but x 11264 6681 / 6581, 2 of 1408 x 2112 364 / 332, 3 of 1408 x 2816 520 / 440.
+// 13: 12 of 1664 x 5488 3428 / 3757, 32 of 1608 x 3216 5870 / 6173, but 28 of 1608 x 6432 9348 / 8948, 5 of 1664^2 605 / 577.  15: 8 of 1920 x 3840
+// 2152 / 2376, 24 of 1856 x 2784 5090 / 5280, but 12 of 1920 x 5160 4318 / 4216, 32 of 1920 x 7680 16558 / 14446.  Three of 9: 1088^2 212 / 235, but
+// 1088 x 2176 339 / 307.
+inline bool ns_flow_odd(int batch, int T, double r) {
+  if (batch == 3) return T <= 7 ? r <= 2.75 : T == 9 && r <= 1.125;
+  if (T <= 9) return true;
+  if (T == 11) return r <= (batch <= 5 ? 12 : batch <= 8 ? 9 : 6);
+  if (T == 13) return batch <= 5 ? r > 1.125 && r <= 6 : r <= (batch == 6 ? 4.5 : batch <= 8 ? 3.5 : batch <= 12 ? 4.1 : batch <= 16 ? 3.5 :
+                                                                    batch < 28 ? 3 : 2.5);
+  if (T == 15) return batch == 4 ? r > 1.125 && r <= 6 : r <= (batch == 5 ? 3 : batch <= 7 ? 2.25 : batch <= 10 ? 2.75 : batch <= 16 ? 2.1 :
+                                                                    batch <= 24 ? 1.5 : 1.25);
+  return false;
+}
 inline bool ns_flow_pays(int batch, int m, int k) {
   const double r = (double)k / m;
   if (m <= 512) return true;
   if (batch == 1) return m <= 1024 || (m <= 1408 && r <= 2.25);
-  if (batch == 2) return m <= 640 || (m <= 1408 && r <= 2.75);
+  if (batch == 2) return m <= 640 || (m <= 1280 && r <= 2.75) || (m <= 1408 && r <= 1.125);
   const int T = (m + 127) / 128;
-  if (T & 1) return batch >= 4 ? m <= 1920 : m <= 1408 && r <= 2.75;
-  if (m <= 1024) return r <= 1.5 || batch >= 8 || (m > 768 && r > 3);
-  if (m <= 1280) return r <= 3.5 && (batch >= 12 || (batch >= 4 && r > 2.5));
+  const int64_t x = (int64_t)batch * T * (((int64_t)k + 127) / 128);
+  if (T & 1) return ns_flow_odd(batch, T, r);
+  if (m <= 768) return r <= 1.5 || (batch >= 8 && x > 1000);
+  if (m <= 1024) return batch >= 8 || r > 3 || (x > 480 && x <= 512) || r <= (batch == 3 ? 1.4 : batch == 4 ? 1.125 : 0);
+  if (m <= 1280) return r <= (batch < 30 ? 3.5 : 2.7) && (batch >= 12 || (batch >= 4 && r > 2.5 && x > 1050));
   return m <= 1536 && batch >= 16 && r <= 1.5;
 }
 // A long K: A = X X^T is whole tiles there, a chain of K / 64 stages (0.2 us each on a 64-tile), where a launch of its own is cut

@@ -68,7 +68,15 @@ NS_TIMES = [(1, 1024, 4096, 212, 242), (2, 640, 2560, 156, 245), (6, 1408, 3872,
             (1, 128, 8192, 166, 179), (1, 128, 16384, 264, 198), (1, 1024, 5120, 314, 277), (1, 1024, 16384, 562, 445), (1, 768, 9216, 311, 265),
             (2, 512, 4096, 168, 228), (2, 512, 8192, 302, 263), (4, 256, 8192, 247, 262), (6, 256, 8192, 307, 267), (4, 512, 12288, 481, 631),
             (16, 640, 12288, 1959, 2383), (12, 384, 32768, 2112, 2281), (4, 576, 131072, 7547, 6641), (8, 256, 16384, 509, 531),
-            (8, 512, 24576, 1682, 1587), (8, 128, 16384, 341, 293), (12, 1024, 6144, 1568, 1759), (4, 1024, 6144, 679, 822), (4, 1024, 8192, 921, 817)]
+            (8, 512, 24576, 1682, 1587), (8, 128, 16384, 341, 293), (12, 1024, 6144, 1568, 1759), (4, 1024, 6144, 679, 822), (4, 1024, 8192, 921, 817),
+            # sides of 11, 13 and 15 tiles of 128, from square to long; then 6, 9 and 10 of them
+            (16, 1408, 7744, 4596, 4974), (16, 1408, 11264, 6681, 6581), (2, 1408, 2112, 364, 332), (3, 1408, 2816, 520, 440), (2, 1408, 1408, 249, 285),
+            (12, 1664, 5488, 3428, 3757), (32, 1608, 3216, 5870, 6173), (28, 1608, 6432, 9348, 8948), (5, 1664, 1664, 605, 577), (12, 1664, 1664, 1253, 1821),
+            (8, 1920, 3840, 2152, 2376), (24, 1856, 2784, 5090, 5280), (12, 1920, 5160, 4318, 4216), (32, 1920, 7680, 16558, 14446),
+            (5, 1856, 5568, 1919, 2086), (7, 1920, 5760, 2766, 2531), (4, 1856, 7424, 1823, 1940), (4, 1856, 1856, 681, 674),
+            (12, 744, 1992, 433, 571), (8, 768, 3072, 431, 559), (8, 696, 1864, 344, 321), (10, 768, 1760, 361, 352), (3, 1088, 1088, 212, 235),
+            (3, 1088, 2176, 339, 307), (4, 1272, 3416, 586, 678), (4, 1160, 3112, 550, 517), (32, 1216, 4256, 4466, 4275),
+            (3, 1024, 1280, 209, 240), (3, 1024, 1536, 272, 260), (4, 1024, 1024, 199, 234), (6, 960, 1440, 368, 339), (6, 1408, 11264, 2461, 2655)]
 
 
 @pytest.mark.parametrize("batch,m,k,one,launches", NS_TIMES)
