@@ -251,6 +251,14 @@ __device__ __forceinline__ void dstage(f32x16_t (&acc)[3][4], DFrag& f0, DFrag& 
   dsubstep<F16, TRI, ANEXT, 0, 0, AFREE, false>(acc, f1, f0, smem, fa, 0, vo, nP, ldsw);
 }
 
+// ---- the forms of GemmArgs ----------------------------------------------------------------------
+// FORM below is GemmArgs::form where a kernel is built for one of them, and 0 for the products that have none: what
+// the elements of the output are, and whether the product is scaled on the way.
+__host__ __device__ constexpr bool out_f16(bool f16, int form) { return form == kFormScaledF16 || (f16 && form != kFormScaledBf16); }
+__host__ __device__ constexpr bool form_scales(int form) { return form == kFormScaledF16 || form == kFormScaledBf16; }
+// of a kernel with the write-out MODE (below), which is the form where there is one
+__host__ __device__ constexpr int mode_form(bool f16, int mode) { return form_scales(mode) || (f16 && mode == kFormPoly) ? mode : 0; }
+
 // ---- the part of a tile after the main loop -----------------------------------------------------
 // Each wave finishes its 128x128 block a quarter (32 rows x 128 columns, one row of MFMA tiles) at
 // a time, in its own LDS region:
@@ -390,7 +398,7 @@ __device__ __forceinline__ void direct_e_batch(const GemmArgs& g, float* F, cons
   }
 }
 
-template <bool F16, bool HAS_E, bool DIAG>
+template <bool F16, bool HAS_E, bool DIAG, int FORM = 0>
 __device__ __forceinline__ void epilogue_quarter_t(const GemmArgs& g, float* F, const unsigned char* Eb,
                                                    const float* RA, int ra_off, int row_base, int col_base,
                                                    int lane, int it_begin, int it_end, int passes) {
@@ -420,7 +428,14 @@ __device__ __forceinline__ void epilogue_quarter_t(const GemmArgs& g, float* F, 
 #pragma unroll
         for (int k = 0; k < 8; ++k) v[k] = __builtin_fmaf(al, elem_to_f32<F16>(e.s[k]), beta * v[k]);
       }
-      if (DIAG) {                                       // selects only: no branch per element
+      if constexpr (form_scales(FORM)) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] *= beta;
+      }
+      if constexpr (DIAG && FORM == kFormPoly) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] += row - col == k ? g.diag_add : 0.0f;
+      } else if (DIAG) {                                // selects only: no branch per element
         const int kd = row - col;                       // the diagonal element of this row, if 0..7
         float dv = 0.0f;
 #pragma unroll
@@ -432,7 +447,7 @@ __device__ __forceinline__ void epilogue_quarter_t(const GemmArgs& g, float* F, 
         if (dout && (unsigned)kd < 8u) g.diag_out[row] = dv;
       }
 #pragma unroll
-      for (int k = 0; k < 8; ++k) o.s[k] = f32_to_elem<F16>(v[k]);
+      for (int k = 0; k < 8; ++k) o.s[k] = f32_to_elem<out_f16(F16, FORM)>(v[k]);
       if (g.C) *reinterpret_cast<uint4*>(C + (int64_t)row * g.c_rs + col) = o.v;
     }
   }
@@ -448,26 +463,26 @@ __device__ __forceinline__ void epilogue_quarter_t(const GemmArgs& g, float* F, 
       const float a[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       union { uint4 v; unsigned short s[8]; } o;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) o.s[k] = f32_to_elem<F16>(a[k]);
+      for (int k = 0; k < 8; ++k) o.s[k] = f32_to_elem<out_f16(F16, FORM)>(form_scales(FORM) ? beta * a[k] : a[k]);
       *reinterpret_cast<uint4*>(C2 + (int64_t)col * g.c2_rs + row) = o.v;
     }
   }
 }
 
-template <bool F16>
+template <bool F16, int FORM = 0>
 __device__ __forceinline__ void epilogue_quarter(const GemmArgs& g, bool diag, float* F, const unsigned char* Eb,
                                                  const float* RA, int ra_off, int row_base, int col_base,
                                                  int lane, int it_begin, int it_end, int passes) {
   if (g.E && !block_written(g, row_base, col_base)) return;   // (only products with E leave blocks out)
-  if constexpr (!F16) {   // fp16 problems carry no operand E
+  if constexpr (!F16 || FORM == kFormPoly) {   // other fp16 problems carry no operand E
     if (g.E) {
-      if (diag) epilogue_quarter_t<false, true, true>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
-      else epilogue_quarter_t<false, true, false>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
+      if (diag) epilogue_quarter_t<F16, true, true, FORM>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
+      else epilogue_quarter_t<F16, true, false, FORM>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
       return;
     }
   }
-  if (diag) epilogue_quarter_t<F16, false, true>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
-  else epilogue_quarter_t<F16, false, false>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
+  if (diag) epilogue_quarter_t<F16, false, true, FORM>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
+  else epilogue_quarter_t<F16, false, false, FORM>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
 }
 
 // ---- write-out of a whole tile from the accumulators --------------------------------------------
@@ -525,7 +540,7 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
 }
 
 // MODE: 0 without the operand E, 1 with it and beta == 1 (the product is added as it is), 2 with it
-// and any beta.  A kernel holds one instance only: of identical element reads in several branches
+// and any beta; kFormPoly in fp16 and the scaled forms.  A kernel holds one instance only: of identical element reads in several branches
 // the optimizer makes one read of all 256 accumulators ahead of the branch, and they do not fit
 // into the vector registers.
 // The wave's block is 32 NI rows x 128 columns at (row0, col0).  `diag`: the block has no mirror
@@ -554,11 +569,13 @@ __device__ __forceinline__ void epilogue_regs(const GemmArgs& g, bool diag, int 
   // what follows is derived from `lane` anew for every tile: kept in registers across the main
   // loop instead, the per-lane offsets of the write-out would crowd out the loop's own
   asm volatile("" : "+v"(lane));
-  constexpr bool has_e = !F16 && MODE != 0;
+  constexpr bool has_e = MODE == 1 || MODE == 2;
+  constexpr int FORM = mode_form(F16, MODE);
+  constexpr bool OF16 = out_f16(F16, FORM);
   const int lc = lane & 31, lh = lane >> 5, par = lane & 1;
   const bool direct = g.C != nullptr;
   const bool mirror = g.C2 != nullptr && !diag;
-  const bool dout = (KIND == 1 || (KIND == 0 && diag)) && g.diag_out != nullptr;
+  const bool dout = (KIND == 1 || (KIND == 0 && diag)) && (FORM == kFormPoly || g.diag_out != nullptr);
   const float alpha = g.alpha, beta = g.beta;
   const uint32_t sel = par ? 0x03020706u : 0x05040100u;   // odd lanes keep the high halves, even lanes the low ones
   float* const RA = reinterpret_cast<float*>(T + QT_BYTES);
@@ -642,7 +659,14 @@ __device__ __forceinline__ void epilogue_regs(const GemmArgs& g, bool diag, int 
           v[r] = __builtin_fmaf(al[r >> 2][r & 3], ef, v[r]);
         }
       }
-      if constexpr (DOUT) {
+      if constexpr (form_scales(FORM)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] *= beta;
+      }
+      if constexpr (DOUT && FORM == kFormPoly) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] += lc == 8 * (r >> 2) + 4 * lh + (r & 3) ? g.diag_add : 0.0f;
+      } else if constexpr (DOUT) {
         float dv = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -656,7 +680,7 @@ __device__ __forceinline__ void epilogue_regs(const GemmArgs& g, bool diag, int 
 #pragma unroll
       for (int qq = 0; qq < 4; ++qq)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) P[qq][h] = pack2<F16>(v[4 * qq + 2 * h], v[4 * qq + 2 * h + 1]);
+        for (int h = 0; h < 2; ++h) P[qq][h] = pack2<OF16>(v[4 * qq + 2 * h], v[4 * qq + 2 * h + 1]);
       if (direct) {   // stage the column of the quarter for the direct output
 #pragma unroll
         for (int qq = 0; qq < 4; ++qq)
@@ -752,12 +776,14 @@ __device__ __forceinline__ void epilogue_regs16(const GemmArgs& g, bool diag, in
   constexpr int NQ = NA / 2;   // quarters: groups of 32 rows
   // derived from `lane` anew for every tile (see epilogue_regs)
   asm volatile("" : "+v"(lane));
-  constexpr bool has_e = !F16 && MODE != 0;
+  constexpr bool has_e = MODE == 1 || MODE == 2;
+  constexpr int FORM = mode_form(F16, MODE);
+  constexpr bool OF16 = out_f16(F16, FORM);
   const int n = lane & 15, grp = lane >> 4;
   const bool written = !has_e || block_written(g, row0, col0);   // (only products with E leave blocks out)
   const bool direct = g.C != nullptr && written;
   const bool mirror = g.C2 != nullptr && !diag && written;
-  const bool dout = diag && g.diag_out != nullptr;
+  const bool dout = diag && (FORM == kFormPoly || g.diag_out != nullptr);
   const float alpha = g.alpha, beta = g.beta;
   float* const RA = reinterpret_cast<float*>(T + QT_BYTES);
   // direct staging: this lane writes rows 8 grp + 4 a + r, the 4 bytes of columns 32 J + 2 n .. + 1, at
@@ -831,7 +857,22 @@ __device__ __forceinline__ void epilogue_regs16(const GemmArgs& g, bool diag, in
               }
           }
         }
-        if constexpr (DOUT) {
+        if constexpr (form_scales(FORM)) {
+#pragma unroll
+          for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) v[a][b][r] *= beta;
+        }
+        if constexpr (DOUT && FORM == kFormPoly) {
+#pragma unroll
+          for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) v[a][b][r] += 2 * n + b == 8 * grp + 4 * a + r ? g.diag_add : 0.0f;
+        } else if constexpr (DOUT) {
           // row 8 grp + 4 a + r meets column 2 n + b: the lanes with n / 4 == grp hold two elements of the
           // diagonal, rows 2 n and 2 n + 1 of the sub-block; they are split off in fp32 and stored as zero
           float dv[2] = {0.0f, 0.0f};
@@ -855,7 +896,7 @@ __device__ __forceinline__ void epilogue_regs16(const GemmArgs& g, bool diag, in
           for (int a = 0; a < 2; ++a)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-              *reinterpret_cast<uint32_t*>(tw + (4 * a + r) * QD_PITCH + 64 * (J ^ grp)) = pack2<F16>(v[a][0][r], v[a][1][r]);
+              *reinterpret_cast<uint32_t*>(tw + (4 * a + r) * QD_PITCH + 64 * (J ^ grp)) = pack2<OF16>(v[a][0][r], v[a][1][r]);
         }
         if (mirror) {
 #pragma unroll
@@ -863,7 +904,7 @@ __device__ __forceinline__ void epilogue_regs16(const GemmArgs& g, bool diag, in
 #pragma unroll
             for (int a = 0; a < 2; ++a)
               *reinterpret_cast<uint2*>(mw + (32 * J + b) * QM_PITCH + 64 * (I & 1) + 8 * a) =
-                  uint2{pack2<F16>(v[a][b][0], v[a][b][1]), pack2<F16>(v[a][b][2], v[a][b][3])};
+                  uint2{pack2<OF16>(v[a][b][0], v[a][b][1]), pack2<OF16>(v[a][b][2], v[a][b][3])};
         }
       };
       if (dout && J == I + dshift) block(std::true_type{});
@@ -1003,10 +1044,12 @@ __device__ __forceinline__ void tile_at(const GemmArgs& g, int pos, int& b, int&
 // Position in the half-tile schedule -> tile and half.  A product that is not symmetric has two
 // items per tile, the upper (h = 0) and the lower 128 rows.  A symmetric one has its diagonal tiles
 // as one item each (`whole_diag`), so a matrix of T x T tiles makes T (T - 1) + T = T^2 items; the
-// order is that of tile_at, the two halves of a tile next to each other.
+// order is that of tile_at, the two halves of a tile next to each other.  MIXED: of two different operands, whose
+// diagonal tiles are two items like the others.
+template <bool MIXED>
 __device__ __forceinline__ void half_item_at(const GemmArgs& g, int e, int& b, int& ti, int& tj, int& h, bool& whole_diag) {
   whole_diag = false;
-  if (!g.symmetric) {
+  if (!g.symmetric || (MIXED && g.A != g.B)) {
     h = e & 1;
     tile_at(g, e >> 1, b, ti, tj);
     return;
@@ -1171,7 +1214,7 @@ constexpr int SUB_STAGE = 2 * SUB_OPER;
 constexpr int SUB_DEPTH = 8;
 constexpr int SUB_F_PITCH = 36;               // floats per staged column: 32 rows + 4 of padding
 
-template <bool F16>
+template <bool F16, int FORM = 0>
 __device__ __forceinline__ void sub64_tile(const GemmArgs& g, int ti, int tj, int si, int sj, int nk,
                                            unsigned char* smem, int lane, int wave) {
   const bool tdiag = g.symmetric && ti == tj;
@@ -1279,7 +1322,7 @@ __device__ __forceinline__ void sub64_tile(const GemmArgs& g, int ti, int tj, in
   // a block of a diagonal sub-tile holds its own mirror image (or is one of a pair of blocks that
   // hold each other's, bit for bit): such a sub-tile is written once, by the direct pass
   const bool bdiag = tdiag && si == sj;
-  const bool use_e = !F16 && g.E != nullptr;
+  const bool use_e = FORM == kFormPoly || (!F16 && FORM == 0 && g.E != nullptr);
   const bool written = !use_e || block_written(g, m0, n0);   // (only products with E leave blocks out)
   const bool mirror = !bdiag && g.C2 != nullptr && written;
   {
@@ -1297,7 +1340,14 @@ __device__ __forceinline__ void sub64_tile(const GemmArgs& g, int ti, int tj, in
 #pragma unroll
       for (int k = 0; k < 16; ++k) v[k] = __builtin_fmaf(al, elem_to_f32<F16>(e.h[k]), g.beta * v[k]);
     }
-    if (bdiag && wm == wn && g.diag_out != nullptr) {   // this block lies on the diagonal of the product
+    if constexpr (form_scales(FORM)) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) v[k] *= g.beta;
+    }
+    if constexpr (FORM == kFormPoly) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) v[k] += bdiag && wm == wn && r - c0 == k ? g.diag_add : 0.0f;
+    } else if (bdiag && wm == wn && g.diag_out != nullptr) {   // this block lies on the diagonal of the product
       const int kd = r - c0;                            // the diagonal element of this row, if 0..15
       float dv = 0.0f;
 #pragma unroll
@@ -1311,8 +1361,8 @@ __device__ __forceinline__ void sub64_tile(const GemmArgs& g, int ti, int tj, in
     union { uint4 q[2]; unsigned short h[16]; } o;
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
-      o.h[k] = f32_to_elem<F16>(v[k]);
-      if (mirror) F[(c0 + k) * SUB_F_PITCH + r] = elem_to_f32<F16>(o.h[k]);
+      o.h[k] = f32_to_elem<out_f16(F16, FORM)>(v[k]);
+      if (mirror) F[(c0 + k) * SUB_F_PITCH + r] = elem_to_f32<out_f16(F16, FORM)>(o.h[k]);
     }
     if (g.C && written) {
       uint4* dst = reinterpret_cast<uint4*>(reinterpret_cast<unsigned short*>(g.C) + (int64_t)row * g.c_rs + col);
@@ -1324,7 +1374,7 @@ __device__ __forceinline__ void sub64_tile(const GemmArgs& g, int ti, int tj, in
     const int c = lane >> 1, r0 = (lane & 1) * 16;
     union { uint4 q[2]; unsigned short h[16]; } o;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) o.h[k] = f32_to_elem<F16>(F[c * SUB_F_PITCH + r0 + k]);
+    for (int k = 0; k < 16; ++k) o.h[k] = f32_to_elem<out_f16(F16, FORM)>(F[c * SUB_F_PITCH + r0 + k]);
     uint4* dst = reinterpret_cast<uint4*>(reinterpret_cast<unsigned short*>(g.C2) + (int64_t)(col0 + c) * g.c2_rs + row0 + r0);
     dst[0] = o.q[0];
     dst[1] = o.q[1];
@@ -1384,7 +1434,7 @@ __device__ __forceinline__ void whole_tile16(const GemmArgs& g, bool diag, int n
       stage16<F16, NA, AS, BS, FIRST>(acc, f0, f1, smem, fa, voA, voB, gA + kn * BKF, gB + kn * BKF, ldsw);  \
     }
 #define FM_STAGE(AS, BS, S) FM_STAGE_T(AS, BS, S, false)
-    if constexpr (MODE == 0) {
+    if constexpr (MODE != 1 && MODE != 2) {
       // the first stage stands apart: its first MFMAs start the sums from zero
       FM_STAGE_T(0, 0, 0, true)
       int s = 1;
@@ -1479,13 +1529,12 @@ __device__ __forceinline__ void whole_tile16(const GemmArgs& g, bool diag, int n
   }
 }
 
-// MODE: how whole tiles are written out (see epilogue_regs); chosen by the host from E and beta
+// MODE: how whole tiles are written out (see epilogue_regs); chosen by the host from E and beta.
+// smem: the operand ring during the main loop (five slots of 32 KiB: A0 A1 B0 B1 A2), the staging of
+// the four waves' write-out afterwards
 template <bool F16, int MODE, int NI>
-__global__ __launch_bounds__(256) void gemm_nt_rounds_kernel(FastArgs p) {
-  // the operand ring during the main loop (five slots of 32 KiB: A0 A1 B0 B1 A2), the staging of
-  // the four waves' write-out afterwards
-  __shared__ __align__(1024) unsigned char smem[SMEM_BYTES];
-
+__device__ __forceinline__ void rounds(const FastArgs& p, unsigned char* smem) {
+  constexpr int FORM = mode_form(F16, MODE);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
@@ -1536,7 +1585,7 @@ __global__ __launch_bounds__(256) void gemm_nt_rounds_kernel(FastArgs p) {
         int sbi, sti, stj;
         tile_at(p.g, p.rounds * p.grid + (w >> 4), sbi, sti, stj);
         const GemmArgs sg = batch_view(p.g, sbi);
-        sub64_tile<F16>(sg, sti, stj, (w >> 2) & 3, w & 3, p.nk, smem, lane, wave);
+        sub64_tile<F16, FORM>(sg, sti, stj, (w >> 2) & 3, w & 3, p.nk, smem, lane, wave);
         break;
       }
       // The workgroups do not leave the last full round together: the XCDs of one chip differ by
@@ -1566,7 +1615,7 @@ __global__ __launch_bounds__(256) void gemm_nt_rounds_kernel(FastArgs p) {
         int sbi, sti, stj;
         tile_at(p.g, p.rounds * p.grid + tile, sbi, sti, stj);
         const GemmArgs sg = batch_view(p.g, sbi);
-        sub64_tile<F16>(sg, sti, stj, si, sj, p.nk, smem, lane, wave);
+        sub64_tile<F16, FORM>(sg, sti, stj, si, sj, p.nk, smem, lane, wave);
         if (t == kNoTickets) break;
       }
       break;
@@ -1580,7 +1629,7 @@ __global__ __launch_bounds__(256) void gemm_nt_rounds_kernel(FastArgs p) {
     const int n = ke - kb;
     int bi, ti, tj, half = 0;
     bool ditem = false;   // NI == 2: a whole diagonal tile of a symmetric product
-    if constexpr (NI == 2) half_item_at(p.g, item, bi, ti, tj, half, ditem);
+    if constexpr (NI == 2) half_item_at<form_scales(FORM)>(p.g, item, bi, ti, tj, half, ditem);
     else tile_at(p.g, p.ksplit > 1 ? item / p.ksplit : item, bi, ti, tj);
     const GemmArgs g = batch_view(p.g, bi);
     const int m0 = ti * BM + half * 128, n0 = tj * BN;
@@ -1617,7 +1666,7 @@ __global__ __launch_bounds__(256) void gemm_nt_rounds_kernel(FastArgs p) {
     }
 
     {   // a whole tile, a part of one along k, or a half tile (never on the diagonal of a symmetric product)
-      const bool diag = NI == 4 && g.symmetric && ti == tj;
+      const bool diag = (NI == 4 || form_scales(FORM)) && g.symmetric && ti == tj;
       float* const slot = NI == 4 && n != p.nk ? p.partials + (size_t)slot_id * PART_FLOATS : nullptr;
       const bool draws = NI == 4 && p.sub64 && p.tickets != nullptr && round == p.rounds - 1 && tickets_live;
       whole_tile16<F16, MODE, 2 * NI>(g, diag, n, slot, smem, fa16, voA, voB, gA, gB, ldsw, m0 + wm * (32 * NI), n0 + wn * 128,
@@ -1628,11 +1677,23 @@ __global__ __launch_bounds__(256) void gemm_nt_rounds_kernel(FastArgs p) {
   }
 }
 
+template <bool F16, int MODE, int NI>
+__global__ __launch_bounds__(256) void gemm_nt_rounds_kernel(FastArgs p) {
+  __shared__ __align__(1024) unsigned char smem[SMEM_BYTES];
+  rounds<F16, MODE, NI>(p, smem);
+}
+// the same for the forms of GemmArgs
+template <bool F16, int FORM, int NI>
+__global__ __launch_bounds__(256) void gemm_nt_form_kernel(FastArgs p) {
+  __shared__ __align__(1024) unsigned char smem[SMEM_BYTES];
+  rounds<F16, FORM, NI>(p, smem);
+}
+
 // Second kernel, for the tiles that were not computed whole: one workgroup per (tile, 128x128
 // block, quarter).  Its four waves add the tile's parts in k order, so the bits do not depend on
 // which workgroup finished when, into one staging buffer, and then share the iterations of the
 // same epilogue the main kernel runs.
-template <bool F16>
+template <bool F16, int FORM>
 __global__ __launch_bounds__(256) void gemm_nt_reduce_kernel(FastArgs p) {
   __shared__ __align__(1024) unsigned char smem[EPI_WAVE_BYTES];
   __shared__ int s_slot[kMaxParts];
@@ -1671,9 +1732,9 @@ __global__ __launch_bounds__(256) void gemm_nt_reduce_kernel(FastArgs p) {
   __syncthreads();
   const bool diag = g.symmetric && ti == tj;
   // direct pass, then (after everybody has put its rounded values back) the transposed pass
-  epilogue_quarter<F16>(g, diag, L.F, L.E[0], L.RA, 32 * q, row0 + 32 * q, col0, lane, wave * 2, wave * 2 + 2, 1);
+  epilogue_quarter<F16, FORM>(g, diag, L.F, L.E[0], L.RA, 32 * q, row0 + 32 * q, col0, lane, wave * 2, wave * 2 + 2, 1);
   __syncthreads();
-  epilogue_quarter<F16>(g, diag, L.F, L.E[0], L.RA, 32 * q, row0 + 32 * q, col0, lane, wave * 2, wave * 2 + 2, 2);
+  epilogue_quarter<F16, FORM>(g, diag, L.F, L.E[0], L.RA, 32 * q, row0 + 32 * q, col0, lane, wave * 2, wave * 2 + 2, 2);
 }
 
 // ---- 128x128 tiles, one per workgroup, for problems too small for the rounds above --------------
@@ -1700,7 +1761,7 @@ struct MidSplit {
 };
 constexpr int MID_PART_FLOATS = MID_T * MID_T;   // one fp32 partial tile: 64 KiB
 
-template <bool F16>
+template <bool F16, int FORM>
 __global__ __launch_bounds__(256) void gemm_nt_mid_kernel(GemmArgs gb, MidSplit sp) {
   __shared__ __align__(1024) unsigned char smem[MID_SMEM];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1724,7 +1785,7 @@ __global__ __launch_bounds__(256) void gemm_nt_mid_kernel(GemmArgs gb, MidSplit 
   const int row0 = m0 + wave * 32, col0 = n0;
 
   // the epilogue operand and the per-row additions first: they are long there when needed
-  const bool use_e = !F16 && g.E != nullptr && sp.ksplit == 1;
+  const bool use_e = (!F16 || FORM == kFormPoly) && g.E != nullptr && sp.ksplit == 1;
   unsigned char* const e_buf = smem + MID_RING + wave * QE_BYTES;
   float ra = 0.0f;
   if (use_e) {
@@ -1848,14 +1909,14 @@ __global__ __launch_bounds__(256) void gemm_nt_mid_kernel(GemmArgs gb, MidSplit 
     return;
   }
   const bool diag = g.symmetric && ti == tj;
-  epilogue_quarter<F16>(g, diag, F, e_buf, RA, 0, row0, col0, lane, 0, 8, 3);
+  epilogue_quarter<F16, FORM>(g, diag, F, e_buf, RA, 0, row0, col0, lane, 0, 8, 3);
 }
 
 // The same tiles by workgroups that share a CU in pairs (fm_tile128.h), for more whole tiles than CUs: one workgroup's
 // start, first stages and write-out lie under the other's multiplications, where the kernel above leaves them bare
 // between its tiles.  X' of 1664 x 6400 (650 tiles of 26 stages) 60 -> 46 us, fast_newtonschulz(5) of it 596 -> 527, of 1408 x 5632
 // 436 -> 377, 2 of 1600^2 393 -> 345.  Bound by the copies into the LDS (fm_gemm_ragged.hip): 0.43 us a stage, tile and CU.
-template <bool F16>
+template <bool F16, int FORM>
 __global__ __launch_bounds__(256, 2) void gemm_nt_pair_kernel(GemmArgs gb) {
   __shared__ __align__(1024) unsigned char smem[t128::SMEM];
   const int lane = threadIdx.x & 63;
@@ -1883,13 +1944,14 @@ __global__ __launch_bounds__(256, 2) void gemm_nt_pair_kernel(GemmArgs gb) {
   o.alpha = g.alpha; o.beta = g.beta;
   o.row_alpha = g.row_alpha;
   o.diag_out = g.diag_out;
-  t128::write_block<F16, 0>(o, g.symmetric && ti == tj, acc, smem + wave * 16384, ti * MID_T + (wave >> 1) * 64, tj * MID_T + (wave & 1) * 64, lane);
+  if constexpr (FORM == kFormPoly) o.diag_add = g.diag_add;
+  t128::write_block<F16, 0, false, FORM>(o, g.symmetric && ti == tj, acc, smem + wave * 16384, ti * MID_T + (wave >> 1) * 64, tj * MID_T + (wave & 1) * 64, lane);
 }
 
 // Second kernel of the cut 128x128 tiles: one workgroup per (tile, quarter).  Its four waves add
 // the quarter's parts in k order, so the bits do not depend on which workgroup finished when, and
 // share the iterations of its epilogue.
-template <bool F16>
+template <bool F16, int FORM>
 __global__ __launch_bounds__(256) void gemm_nt_mid_reduce_kernel(GemmArgs gb, MidSplit sp) {
   __shared__ __align__(1024) unsigned char smem[EPI_WAVE_BYTES];
   __shared__ int s_slot[kMaxParts];
@@ -1912,9 +1974,9 @@ __global__ __launch_bounds__(256) void gemm_nt_mid_reduce_kernel(GemmArgs gb, Mi
   __syncthreads();
   const bool diag = g.symmetric && ti == tj;
   // direct pass, then (after everybody has put its rounded values back) the transposed pass
-  epilogue_quarter<F16>(g, diag, L.F, L.E[0], L.RA, 0, row0, col0, lane, wave * 2, wave * 2 + 2, 1);
+  epilogue_quarter<F16, FORM>(g, diag, L.F, L.E[0], L.RA, 0, row0, col0, lane, wave * 2, wave * 2 + 2, 1);
   __syncthreads();
-  epilogue_quarter<F16>(g, diag, L.F, L.E[0], L.RA, 0, row0, col0, lane, wave * 2, wave * 2 + 2, 2);
+  epilogue_quarter<F16, FORM>(g, diag, L.F, L.E[0], L.RA, 0, row0, col0, lane, wave * 2, wave * 2 + 2, 2);
 }
 
 }  // namespace
@@ -1984,7 +2046,7 @@ static void fast_schedule(int num_tiles, int nk, long long max_slots, FastArgs& 
 // what both tile shapes ask of a problem: whole tiles of edge `tile`, whole k stages, 16-byte
 // accesses everywhere
 static bool tiled_dma_eligible(const GemmArgs& a, int tile) {
-  if (a.elem == kElemF16 && a.E) return false;
+  if (a.elem == kElemF16 && a.E && a.form == 0) return false;
   if (a.Kc < BKF || a.Kc % BKF != 0) return false;
   if (a.lda % 8 != 0 || a.ldb % 8 != 0) return false;
   if ((reinterpret_cast<uintptr_t>(a.A) & 15) || (reinterpret_cast<uintptr_t>(a.B) & 15)) return false;
@@ -2031,6 +2093,12 @@ static double estimate_half_round(long long half_items, int nk, int grid) {
   return nk * (0.50 + 0.78 * (occ > 0.6 ? occ - 0.6 : 0.0)) + 13.0;
 }
 
+// half items of all matrices: a diagonal tile of A A^T is one, of the product of two matrices two
+static long long half_item_count(const GemmArgs& a) {
+  const long long tm = a.Ma / BM, tn = a.Nb / BN, nb = a.batch < 1 ? 1 : a.batch;
+  return (!a.symmetric ? 2 * tm * tn : a.A == a.B ? tm * tm : tm * (tm + 1)) * nb;
+}
+
 // The half-tile schedule (128x256 items, a diagonal tile of a symmetric product as one item) is
 // taken when all its items fit into one round and that round is estimated to be shorter than the
 // round of whole tiles: those would leave about half of the CUs idle, and half items are never
@@ -2064,7 +2132,7 @@ static bool sub64_schedule_chosen(const GemmArgs& a, long long tiles, int nk, in
   const int ksplit = auto_ksplit(tiles, nk, grid);
   const double t_large = (nk / ksplit) * 1.45 + 15.0 + (ksplit > 1 ? 25.0 : 0.0);
   if (t_large < t_best) t_best = t_large;
-  const long long half_items = (a.symmetric ? tm * tm : 2 * tm * tn) * nb;
+  const long long half_items = half_item_count(a);
   if (half_schedule_chosen(half_items, tiles, nk, grid)) {
     const double t_half = estimate_half_round(half_items, nk, grid);
     if (t_half < t_best) t_best = t_half;
@@ -2092,7 +2160,7 @@ bool gemm_fast_eligible(const GemmArgs& a) {
   const double t_large = (nk / ksplit) * 1.45 + 15.0 + (ksplit > 1 ? 25.0 : 0.0);
   const long long small_tiles = (a.symmetric ? 2 * tm * (2 * tm + 1) / 2 : 4 * tm * tn) * (a.batch < 1 ? 1 : a.batch);
   const double t_small = estimate_mid(small_tiles, nk, cus, a.E != nullptr);
-  const long long half_items = (a.symmetric ? tm * tm : 2 * tm * tn) * (a.batch < 1 ? 1 : a.batch);
+  const long long half_items = half_item_count(a);
   // (the 128x128 tiles keep the benefit of the doubt against half tiles)
   if (half_schedule_chosen(half_items, tiles, nk, cus) && estimate_half_round(half_items, nk, cus) < 0.9 * t_small) return true;
   return t_large < t_small;
@@ -2116,18 +2184,28 @@ int launch_gemm_mid(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) {
   sp.partials = static_cast<float*>(ws);
   // without room for the parts the tiles stay whole
   if (sp.ksplit > 1 && (!ws || (size_t)a.num_tiles * sp.ksplit * MID_PART_FLOATS * sizeof(float) > ws_bytes)) sp.ksplit = 1;
+  // (the products of two M x M matrices are never cut: where they have few tiles their k is short)
+  if (a.form && a.elem == kElemF16) sp.ksplit = 1;
   const unsigned grid = (unsigned)(a.num_tiles * sp.ksplit);
-  if (sp.ksplit == 1 && a.num_tiles > cu_count() && pair_eligible(a)) {
-    if (a.elem == kElemF16) hipLaunchKernelGGL(gemm_nt_pair_kernel<true>, dim3(grid), dim3(256), 0, stream, a);
-    else hipLaunchKernelGGL(gemm_nt_pair_kernel<false>, dim3(grid), dim3(256), 0, stream, a);
-    return (int)hipGetLastError();
-  }
-  if (a.elem == kElemF16) hipLaunchKernelGGL(gemm_nt_mid_kernel<true>, dim3(grid), dim3(256), 0, stream, a, sp);
-  else hipLaunchKernelGGL(gemm_nt_mid_kernel<false>, dim3(grid), dim3(256), 0, stream, a, sp);
-  if (sp.ksplit > 1) {
-    if (a.elem == kElemF16) hipLaunchKernelGGL(gemm_nt_mid_reduce_kernel<true>, dim3(a.num_tiles * 4), dim3(256), 0, stream, a, sp);
-    else hipLaunchKernelGGL(gemm_nt_mid_reduce_kernel<false>, dim3(a.num_tiles * 4), dim3(256), 0, stream, a, sp);
-  }
+  const bool pairs = sp.ksplit == 1 && a.num_tiles > cu_count() && pair_eligible(a);
+#define FM_MID(F16, FORM)                                                                                                          \
+  do {                                                                                                                             \
+    if (pairs) {                                                                                                                   \
+      hipLaunchKernelGGL((gemm_nt_pair_kernel<F16, FORM>), dim3(grid), dim3(256), 0, stream, a);                                    \
+      break;                                                                                                                       \
+    }                                                                                                                              \
+    hipLaunchKernelGGL((gemm_nt_mid_kernel<F16, FORM>), dim3(grid), dim3(256), 0, stream, a, sp);                                   \
+    if constexpr (!F16 || FORM == 0) {                                                                                              \
+      if (sp.ksplit > 1) hipLaunchKernelGGL((gemm_nt_mid_reduce_kernel<F16, FORM>), dim3(a.num_tiles * 4), dim3(256), 0, stream, a, sp); \
+    }                                                                                                                              \
+  } while (0)
+  if (a.form == kFormPoly) FM_MID(true, kFormPoly);
+  else if (a.form == kFormScaledBf16) FM_MID(true, kFormScaledBf16);
+  else if (a.form == kFormScaledF16 && a.elem == kElemF16) FM_MID(true, kFormScaledF16);
+  else if (a.form == kFormScaledF16) FM_MID(false, kFormScaledF16);
+  else if (a.elem == kElemF16) FM_MID(true, 0);
+  else FM_MID(false, 0);
+#undef FM_MID
   return (int)hipGetLastError();
 }
 
@@ -2179,7 +2257,7 @@ int launch_gemm_fast(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) 
   int grid = cu_count() < kMaxGrid ? cu_count() : kMaxGrid;
   const long long kg = knob(kKnobGrid);
   if (kg > 0 && kg < grid) grid = (int)kg;
-  const long long half_items = a.symmetric ? (long long)a.tiles_m * a.tiles_m * a.batch : 2LL * a.num_tiles;   // a diagonal tile is one item
+  const long long half_items = half_item_count(a);
   if (sub64_schedule_chosen(a, a.num_tiles, f.nk, grid)) {   // every tile as 16 sub-tiles of 64x64, one workgroup each
     f.grid = a.num_tiles * 16;
     f.ksplit = 1;
@@ -2221,27 +2299,27 @@ int launch_gemm_fast(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) 
     if (f.epoch != 0)
       f.tickets = reinterpret_cast<unsigned long long*>(static_cast<unsigned char*>(ws) + (ws_bytes / kTicketBytes - 1) * kTicketBytes);
   }
-  if (f.half) {
-    if (a.elem == kElemF16) hipLaunchKernelGGL((gemm_nt_rounds_kernel<true, 0, 2>), dim3(f.grid), dim3(256), 0, stream, f);
-    else if (!a.E) hipLaunchKernelGGL((gemm_nt_rounds_kernel<false, 0, 2>), dim3(f.grid), dim3(256), 0, stream, f);
-    else if (a.beta == 1.0f) hipLaunchKernelGGL((gemm_nt_rounds_kernel<false, 1, 2>), dim3(f.grid), dim3(256), 0, stream, f);
-    else hipLaunchKernelGGL((gemm_nt_rounds_kernel<false, 2, 2>), dim3(f.grid), dim3(256), 0, stream, f);
-    return (int)hipGetLastError();
-  }
   const int slots = f.tail_slot0 + f.rem * f.split;
   const int reduce_tiles = a.num_tiles - f.reduce_tile0;
-  if (reduce_tiles > 0 && (slots > have || f.ksplit * f.split > kMaxParts)) return kErrWorkspace;
-  if (a.elem == kElemF16) {
-    hipLaunchKernelGGL((gemm_nt_rounds_kernel<true, 0, 4>), dim3(f.grid), dim3(256), 0, stream, f);
-    if (reduce_tiles > 0)
-      hipLaunchKernelGGL(gemm_nt_reduce_kernel<true>, dim3(reduce_tiles * 16), dim3(256), 0, stream, f);
-  } else {
-    if (!a.E) hipLaunchKernelGGL((gemm_nt_rounds_kernel<false, 0, 4>), dim3(f.grid), dim3(256), 0, stream, f);
-    else if (a.beta == 1.0f) hipLaunchKernelGGL((gemm_nt_rounds_kernel<false, 1, 4>), dim3(f.grid), dim3(256), 0, stream, f);
-    else hipLaunchKernelGGL((gemm_nt_rounds_kernel<false, 2, 4>), dim3(f.grid), dim3(256), 0, stream, f);
-    if (reduce_tiles > 0)
-      hipLaunchKernelGGL(gemm_nt_reduce_kernel<false>, dim3(reduce_tiles * 16), dim3(256), 0, stream, f);
-  }
+  if (!f.half && reduce_tiles > 0 && (slots > have || f.ksplit * f.split > kMaxParts)) return kErrWorkspace;
+#define FM_ROUNDS(KERNEL, F16, MODE, FORM)                                                                             \
+  do {                                                                                                                 \
+    if (f.half) {                                                                                                      \
+      hipLaunchKernelGGL((KERNEL<F16, MODE, 2>), dim3(f.grid), dim3(256), 0, stream, f);                                \
+      break;                                                                                                           \
+    }                                                                                                                  \
+    hipLaunchKernelGGL((KERNEL<F16, MODE, 4>), dim3(f.grid), dim3(256), 0, stream, f);                                  \
+    if (reduce_tiles > 0) hipLaunchKernelGGL((gemm_nt_reduce_kernel<F16, FORM>), dim3(reduce_tiles * 16), dim3(256), 0, stream, f); \
+  } while (0)
+  if (a.form == kFormPoly) FM_ROUNDS(gemm_nt_form_kernel, true, kFormPoly, kFormPoly);
+  else if (a.form == kFormScaledBf16) FM_ROUNDS(gemm_nt_form_kernel, true, kFormScaledBf16, kFormScaledBf16);
+  else if (a.form == kFormScaledF16 && a.elem == kElemF16) FM_ROUNDS(gemm_nt_form_kernel, true, kFormScaledF16, kFormScaledF16);
+  else if (a.form == kFormScaledF16) FM_ROUNDS(gemm_nt_form_kernel, false, kFormScaledF16, kFormScaledF16);
+  else if (a.elem == kElemF16) FM_ROUNDS(gemm_nt_rounds_kernel, true, 0, 0);
+  else if (!a.E) FM_ROUNDS(gemm_nt_rounds_kernel, false, 0, 0);
+  else if (a.beta == 1.0f) FM_ROUNDS(gemm_nt_rounds_kernel, false, 1, 0);
+  else FM_ROUNDS(gemm_nt_rounds_kernel, false, 2, 0);
+#undef FM_ROUNDS
   return (int)hipGetLastError();
 }
 

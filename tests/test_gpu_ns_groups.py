@@ -1,0 +1,118 @@
+"""Newton-Schulz steps in groups on the Gram matrix (long matrices, five steps or more): every schedule that its products of
+M x M matrices run on, padded and transposed inputs, step counts and coefficients.
+
+Tolerance: the groups round fewer things and finer than the steps one by one do (fp16 instead of bf16 for the M x M
+matrices, two iterates instead of five), so the result may be no further from the iteration in 64 bits than the
+steps one by one with the roundings of their kernels: A, P without its diagonal, and X to bf16, sums in fp32.  (What runs
+one by one itself differs from that by the order of its sums, which turns some roundings: a hundredth of the bound.)"""
+import ctypes
+
+import pytest
+import torch
+
+from flash_muon_amd import _lib, fast_newtonschulz
+from flash_muon_amd.muon import NS_COEFFS, NS_EPS
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _inputs(rows, cols, dtype, seed):
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    u, v = torch.randn(rows, 32, generator=gen, device=DEV), torch.randn(32, cols, generator=gen, device=DEV)
+    return (torch.randn(rows, cols, generator=gen, device=DEV) + 0.1 * u @ v).to(dtype)
+
+
+def _one_by_one(X, steps, coeffs):
+    a, b, c = coeffs
+    X = X.bfloat16().float()
+    for _ in range(steps):
+        A = (X @ X.T).bfloat16().float()
+        P = b * A + c * (A @ A)
+        d = a + P.diagonal().clone()
+        P = P.bfloat16().float().fill_diagonal_(0)
+        X = (d[:, None] * X + P @ X).bfloat16().float()
+    return X
+
+
+def _check(got, G, steps, coeffs=NS_COEFFS):
+    X = G.bfloat16().double()
+    X = X.T.contiguous() if X.shape[0] > X.shape[1] else X
+    got = got.double().T if got.shape[0] > got.shape[1] else got.double()
+    X = X / (X.norm() + NS_EPS)
+    want, by_one = X, _one_by_one(X.float(), steps, coeffs).double()
+    for _ in range(steps):
+        want = oracle.ns_step(want, coeffs)
+    err, limit = (float((y - want).norm() / want.norm()) for y in (got, by_one))
+    assert err <= 1.01 * limit and limit < 2e-2, (err, limit)
+
+
+def _library_call(Gs, steps, coeffs=NS_COEFFS):
+    """Through the C ABI with the least scratch, which keeps matrices of any size on launches per product."""
+    lib = _lib.load()
+    n, rows, cols = len(Gs), *Gs[0].shape
+    outs = [torch.empty(rows, cols, dtype=torch.bfloat16, device=DEV) for _ in Gs]
+    need = lib.fm_newtonschulz_batched_min_workspace_bytes(n, rows, cols)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    st = lib.fm_newtonschulz_batched_bf16((ctypes.c_void_p * n)(*[g.data_ptr() for g in Gs]), _lib.dtype_code(Gs[0].dtype), n, rows, cols, cols,
+                                          (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs]), cols, steps, *coeffs, NS_EPS,
+                                          ws.data_ptr(), need, _lib.stream_ptr(Gs[0].device))
+    _lib.check("fm_newtonschulz_batched_bf16", st)
+    return outs
+
+
+# 64x64 sub-tiles alone; 128-tiles, one per CU; the same with A = X X^T cut along k; in pairs; half tiles; whole 256-tiles in one round;
+# rounds with sub-tiles behind them, handed out by ticket, and with their last tiles cut along k; diagonal tiles last
+@pytest.mark.parametrize("rows,cols,batch", [(512, 1024, 1), (1664, 3328, 1), (640, 10240, 1), (1664, 3328, 4), (3072, 6144, 1), (4096, 8192, 1),
+                                             (4096, 8192, 2), (2816, 5632, 5), (8192, 16384, 1)])
+def test_every_schedule_of_the_chain(rows, cols, batch):
+    Gs = [_inputs(rows, cols, torch.bfloat16, 7 + i) for i in range(batch)]
+    outs = _library_call(Gs, 5)
+    for i in {0, batch - 1}:
+        _check(outs[i], Gs[i], 5)
+
+
+# padded to 128- and 256-tiles, tall, fp32, into the output without a copy (5504 x 2048), K at and below twice M
+@pytest.mark.parametrize("rows,cols,batch,dtype", [(2700, 1150, 1, torch.float32), (1150, 2700, 1, torch.float16), (5504, 2048, 3, torch.bfloat16),
+                                                   (1600, 6401, 1, torch.float32), (1536, 3072, 8, torch.bfloat16), (1536, 3071, 1, torch.bfloat16),
+                                                   (1664, 3328, 8, torch.bfloat16), (3200, 6400, 1, torch.bfloat16)])
+def test_padded_and_transposed(rows, cols, batch, dtype):
+    G = torch.stack([_inputs(rows, cols, dtype, 40 + i) for i in range(batch)])
+    got = fast_newtonschulz(G if batch > 1 else G[0], 5).view(G.shape)
+    for i in {0, batch - 1}:
+        _check(got[i], G[i], 5)
+
+
+@pytest.mark.parametrize("steps", [4, 5, 6, 7, 8])
+def test_step_counts(steps):
+    G = _inputs(1664, 4000, torch.bfloat16, 3)
+    _check(fast_newtonschulz(G, steps), G, steps)
+
+
+# the last two would leave fp16's range and run one by one
+@pytest.mark.parametrize("coeffs", [(1.5, -0.5, 0.0), (1.875, -1.25, 0.375), (3.0, -3.2, 1.2), (4.0, -6.0, 3.0), (2.0, 0.0, 0.0)])
+def test_other_coefficients(coeffs):
+    G = _inputs(1664, 4000, torch.bfloat16, 4)
+    _check(_library_call([G], 5, coeffs)[0], G, 5, coeffs)
+
+
+def test_scales_of_the_input():
+    """Rows over six decades: what is small beside the rest keeps its direction in fp16 as in bf16."""
+    G = _inputs(1664, 4000, torch.float32, 5) * torch.logspace(0, -6, 1664, device=DEV)[:, None]
+    got = fast_newtonschulz(G, 5)
+    _check(got, G, 5)
+    X = G.bfloat16().double()
+    X = X / X.norm()
+    for _ in range(5):
+        X = oracle.ns_step(X)
+    by_row = (got.double() - X).norm(dim=1) / X.norm(dim=1)
+    by_one = (_one_by_one((G.bfloat16().float() / G.bfloat16().float().norm()), 5, NS_COEFFS).double() - X).norm(dim=1) / X.norm(dim=1)
+    assert bool((by_row <= by_one.max()).all())
+
+
+def test_nan_and_zero():
+    G = _inputs(1664, 4000, torch.bfloat16, 6)
+    G[3, 5] = float("nan")
+    assert bool(fast_newtonschulz(G, 5).isnan().all())
+    assert float(fast_newtonschulz(torch.zeros_like(G), 5).float().abs().max()) == 0.0
