@@ -84,10 +84,57 @@ def test_padded_and_transposed(rows, cols, batch, dtype):
         _check(got[i], G[i], 5)
 
 
-@pytest.mark.parametrize("steps", [4, 5, 6, 7, 8])
-def test_step_counts(steps):
-    G = _inputs(1664, 4000, torch.bfloat16, 3)
-    _check(fast_newtonschulz(G, steps), G, steps)
+# in one launch: whole and ragged tiles, tall, the fewest rows and columns, outputs that 16-byte stores cannot take
+@pytest.mark.parametrize("rows,cols,batch,dtype", [(512, 1408, 16, torch.bfloat16), (3072, 768, 16, torch.float32), (1000, 2816, 8, torch.bfloat16),
+                                                   (1921, 901, 12, torch.float16), (1408, 2820, 5, torch.bfloat16), (1150, 2301, 5, torch.float32)])
+def test_in_one_launch(rows, cols, batch, dtype):
+    G = torch.stack([_inputs(rows, cols, dtype, 60 + i) for i in range(batch)])
+    got = fast_newtonschulz(G, 5)
+    for i in {0, batch // 2, batch - 1}:
+        _check(got[i], G[i], 5)
+    again = fast_newtonschulz(G[:1].expand(batch, rows, cols).contiguous(), 5)
+    assert all(torch.equal(again[i], got[0]) for i in range(batch))   # whatever workgroup draws what and when
+
+
+@pytest.mark.parametrize("steps", [4, 5, 6, 7, 8, 11])
+@pytest.mark.parametrize("batch", [1, 8])   # in launches per product, in one launch per two groups
+def test_step_counts(steps, batch):
+    G = _inputs(1300, 2700, torch.bfloat16, 3)
+    got = fast_newtonschulz(G.expand(batch, *G.shape).contiguous() if batch > 1 else G, steps).view(batch, *G.shape)
+    _check(got[0], G, steps)
+    assert all(torch.equal(got[0], g) for g in got)
+
+
+def test_streams_at_once():
+    Gs = [torch.stack([_inputs(r, c, torch.bfloat16, 80 + i) for i in range(b)]) for r, c, b in [(768, 2064, 8), (640, 1720, 16), (2816, 1024, 8)]]
+    want = [fast_newtonschulz(G, 5) for G in Gs]
+    streams = [torch.cuda.Stream() for _ in Gs]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        got = []
+        for s, G in zip(streams, Gs):
+            with torch.cuda.stream(s):
+                got.append(fast_newtonschulz(G, 5))
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("rows,cols,batch", [(768, 3072, 8), (1664, 4000, 1)])
+def test_in_a_graph(rows, cols, batch):
+    G = torch.stack([_inputs(rows, cols, torch.bfloat16, 90 + i) for i in range(batch)])
+    for _ in range(2):
+        want = fast_newtonschulz(G, 5)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = fast_newtonschulz(G, 5)
+    for i in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        G.mul_(2.0)                          # the iterate, and with powers of two its bits, do not depend on the scale
+        assert torch.equal(fast_newtonschulz(G, 5), want)
 
 
 # the last two would leave fp16's range and run one by one
