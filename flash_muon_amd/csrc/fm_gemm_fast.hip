@@ -194,12 +194,20 @@ __device__ __forceinline__ void stage16(f32x4_t (&acc)[NA][8], Frag16<NA>& f0, F
 // fragments, read once more rather than picked from the six at the cost of vector instructions
 // among the MFMAs).  Both operands are the one 256-row panel, which goes round the three A slots
 // (8 copies per wave and stage, issued two stages ahead); the B slots are idle.
+// MIXED: of the product of two matrices, which has a row panel and a column panel.  The row panel goes round
+// the A slots as above, the column panel round the B slots, its copies for the stage two ahead behind the
+// barrier of a stage (0.9 of a stage to land); a triangle wave reads 4 + 4 fragments.  4096^2, one matrix: 256
+// items in one round take 71 us, 136 whole tiles on as many CUs 96.
 struct DFrag { bf16x8_t f[8]; };   // triangle waves: rows 32q of their square; the others: 2 row, 4 column fragments and the ninth tile's two
 struct DFragAddr { uint32_t lo[8][4], hi[8][4]; };   // A slots 0 and 1 / A slot 2
 
-template <int ASLOT>
+// whether fragment q of a MIXED item comes from the column panel
+__host__ __device__ constexpr bool d_col(bool tri, int q) { return tri ? q >= 4 : (q >= 2 && q != 6); }
+
+template <int ASLOT, int BSLOT, bool COL>
 __device__ __forceinline__ bf16x8_t read_d(const unsigned char* smem, const DFragAddr& fa, int q, int ks) {
-  if constexpr (ASLOT == 2) return *reinterpret_cast<const bf16x8_t*>(smem + fa.hi[q][ks]);
+  if constexpr (COL) return *reinterpret_cast<const bf16x8_t*>(smem + fa.lo[q][ks] + BSLOT * OPER_BYTES);
+  else if constexpr (ASLOT == 2) return *reinterpret_cast<const bf16x8_t*>(smem + fa.hi[q][ks]);
   else return *reinterpret_cast<const bf16x8_t*>(smem + fa.lo[q][ks] + ASLOT * OPER_BYTES);
 }
 
@@ -210,23 +218,30 @@ __host__ __device__ constexpr int tri_c(int i, int j) { return i < 3 ? j : (j < 
 __host__ __device__ constexpr int tri_i(int q) { return q < 2 ? q : q < 5 ? 2 : 3; }
 __host__ __device__ constexpr int tri_j(int q) { return q < 2 ? q : q < 5 ? q - 2 : q - 5; }
 
-// the 9 MFMAs of one substep, with the fragment reads of `ks_next` of slot RSLOT riding on the
-// first ones and copies Q0 .. Q1-1 of the panel two stages ahead on the later ones.
-template <bool F16, bool TRI, int RSLOT, int Q0, int Q1, int CSLOT, bool FIRST>
+// the 9 MFMAs of one substep, with the fragment reads of `ks_next` of slots RSLOT, BSLOT riding on the
+// first ones and copies Q0 .. Q1-1 of the panel two stages ahead on the later ones, or (COPYB) all 8 of the
+// column panel.
+template <bool F16, bool TRI, bool MIXED, int RSLOT, int BSLOT, int Q0, int Q1, int CSLOT, bool COPYB, bool FIRST>
 __device__ __forceinline__ void dsubstep(f32x16_t (&acc)[3][4], const DFrag& cur, DFrag& nxt, const unsigned char* smem,
                                          const DFragAddr& fa, int ks_next, const uint32_t (&vo)[8], const bf16_t* gP,
                                          uint32_t ldsw) {
-  constexpr int NM = 9, NRD = TRI ? 4 : 8;
+  constexpr int NM = 9, NRD = TRI && !MIXED ? 4 : 8;
   constexpr int C0 = 5, CSTEP = 1;   // copies after MFMA 5, 6, 7
 #pragma unroll
   for (int q = 0; q < NM; ++q) {
-    if (q < NRD) nxt.f[q] = read_d<RSLOT>(smem, fa, q, ks_next);
-    if (q >= C0 && (q - C0) % CSTEP == 0 && Q0 + (q - C0) / CSTEP < Q1)
+    if (q < NRD) {
+      if (MIXED && d_col(TRI, q)) nxt.f[q] = read_d<RSLOT, BSLOT, true>(smem, fa, q, ks_next);
+      else nxt.f[q] = read_d<RSLOT, BSLOT, false>(smem, fa, q, ks_next);
+    }
+    if constexpr (COPYB) {
+      if (q > 0) dma16o(vo[q > 0 ? q - 1 : 0], gP, ldsw, b_slot_off(CSLOT) + (q - 1) * 4096);
+    } else if (q >= C0 && (q - C0) % CSTEP == 0 && Q0 + (q - C0) / CSTEP < Q1) {
       dma16o(vo[Q0 + (q - C0) / CSTEP], gP, ldsw, a_slot_off(CSLOT) + (Q0 + (q - C0) / CSTEP) * 4096);
+    }
     const f32x16_t zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     if constexpr (TRI) {
       f32x16_t& c = acc[tri_r(tri_i(q), tri_j(q))][tri_c(tri_i(q), tri_j(q))];
-      c = mfma_32x32x16<F16>(cur.f[tri_i(q)], cur.f[tri_j(q)], FIRST ? zero : c);
+      c = mfma_32x32x16<F16>(cur.f[tri_i(q)], cur.f[tri_j(q) + (MIXED ? 4 : 0)], FIRST ? zero : c);
     } else if (q < 8) {
       f32x16_t& c = acc[q >> 2][q & 3];
       c = mfma_32x32x16<F16>(cur.f[q >> 2], cur.f[2 + (q & 3)], FIRST ? zero : c);
@@ -237,18 +252,20 @@ __device__ __forceinline__ void dsubstep(f32x16_t (&acc)[3][4], const DFrag& cur
   }
 }
 
-// one k stage of the panel in A slot ASLOT
-template <bool F16, bool TRI, int ASLOT, bool FIRST>
+// one k stage of the panel in A slot ASLOT (and of the column panel in B slot BSLOT)
+template <bool F16, bool TRI, bool MIXED, int ASLOT, int BSLOT, bool FIRST>
 __device__ __forceinline__ void dstage(f32x16_t (&acc)[3][4], DFrag& f0, DFrag& f1, const unsigned char* smem,
-                                       const DFragAddr& fa, const uint32_t (&vo)[8], const bf16_t* nP, uint32_t ldsw) {
+                                       const DFragAddr& fa, const uint32_t (&vo)[8], const uint32_t (&voB)[8], const bf16_t* nP,
+                                       const bf16_t* nB, uint32_t ldsw) {
   constexpr int AFREE = (ASLOT + 2) % 3, ANEXT = (ASLOT + 1) % 3;
-  dsubstep<F16, TRI, ASLOT, 0, 3, AFREE, FIRST>(acc, f0, f1, smem, fa, 1, vo, nP, ldsw);
-  dsubstep<F16, TRI, ASLOT, 3, 6, AFREE, false>(acc, f1, f0, smem, fa, 2, vo, nP, ldsw);
-  dsubstep<F16, TRI, ASLOT, 6, 8, AFREE, false>(acc, f0, f1, smem, fa, 3, vo, nP, ldsw);
+  dsubstep<F16, TRI, MIXED, ASLOT, BSLOT, 0, 3, AFREE, false, FIRST>(acc, f0, f1, smem, fa, 1, vo, nP, ldsw);
+  dsubstep<F16, TRI, MIXED, ASLOT, BSLOT, 3, 6, AFREE, false, false>(acc, f1, f0, smem, fa, 2, vo, nP, ldsw);
+  dsubstep<F16, TRI, MIXED, ASLOT, BSLOT, 6, 8, AFREE, false, false>(acc, f0, f1, smem, fa, 3, vo, nP, ldsw);
   // everybody's copies of the next stage have landed (all but the 8 newest, of the stage after),
-  // and nobody reads the slot that the next stage's copies go to
+  // and nobody reads the slots that the next copies go to
   asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  dsubstep<F16, TRI, ANEXT, 0, 0, AFREE, false>(acc, f1, f0, smem, fa, 0, vo, nP, ldsw);
+  if constexpr (MIXED) dsubstep<F16, TRI, MIXED, ANEXT, BSLOT ^ 1, 0, 0, BSLOT, true, false>(acc, f1, f0, smem, fa, 0, voB, nB, ldsw);
+  else dsubstep<F16, TRI, MIXED, ANEXT, 0, 0, 0, AFREE, false, false>(acc, f1, f0, smem, fa, 0, vo, nP, ldsw);
 }
 
 // ---- the forms of GemmArgs ----------------------------------------------------------------------
@@ -1044,12 +1061,10 @@ __device__ __forceinline__ void tile_at(const GemmArgs& g, int pos, int& b, int&
 // Position in the half-tile schedule -> tile and half.  A product that is not symmetric has two
 // items per tile, the upper (h = 0) and the lower 128 rows.  A symmetric one has its diagonal tiles
 // as one item each (`whole_diag`), so a matrix of T x T tiles makes T (T - 1) + T = T^2 items; the
-// order is that of tile_at, the two halves of a tile next to each other.  MIXED: of two different operands, whose
-// diagonal tiles are two items like the others.
-template <bool MIXED>
+// order is that of tile_at, the two halves of a tile next to each other.
 __device__ __forceinline__ void half_item_at(const GemmArgs& g, int e, int& b, int& ti, int& tj, int& h, bool& whole_diag) {
   whole_diag = false;
-  if (!g.symmetric || (MIXED && g.A != g.B)) {
+  if (!g.symmetric) {
     h = e & 1;
     tile_at(g, e >> 1, b, ti, tj);
     return;
@@ -1095,40 +1110,61 @@ __device__ __forceinline__ void half_item_at(const GemmArgs& g, int e, int& b, i
 
 // The k loop of a diagonal item for one kind of wave; the copies of the first two stages are in
 // flight and stage 0 has landed everywhere.
-template <bool F16, bool TRI>
+template <bool F16, bool TRI, bool MIXED>
 __device__ __forceinline__ void diag_item_loop(f32x16_t (&acc)[3][4], const unsigned char* smem, const DFragAddr& dfa,
-                                               const uint32_t (&vo)[8], const bf16_t* gP, int n, uint32_t ldsw) {
+                                               const uint32_t (&vo)[8], const uint32_t (&voB)[8], const bf16_t* gP, const bf16_t* gB, int n,
+                                               uint32_t ldsw) {
   const int last = n - 1;
   DFrag f0, f1;
 #pragma unroll
-  for (int q = 0; q < (TRI ? 4 : 8); ++q) f0.f[q] = read_d<0>(smem, dfa, q, 0);
+  for (int q = 0; q < (TRI && !MIXED ? 4 : 8); ++q) {
+    if (MIXED && d_col(TRI, q)) f0.f[q] = read_d<0, 0, true>(smem, dfa, q, 0);
+    else f0.f[q] = read_d<0, 0, false>(smem, dfa, q, 0);
+  }
   // stages past the end are the last stage again (into slots nobody reads), so that the number of
   // copies in flight is the same at every wait
-#define FM_DSTAGE(AS, S, FIRST)                                                                \
-  {                                                                                            \
-    const int kn = (S) + 2 < last ? (S) + 2 : last;                                            \
-    dstage<F16, TRI, AS, FIRST>(acc, f0, f1, smem, dfa, vo, gP + kn * BKF, ldsw);              \
+#define FM_DSTAGE(AS, BS, S, FIRST)                                                                          \
+  {                                                                                                          \
+    const int kn = (S) + 2 < last ? (S) + 2 : last;                                                          \
+    dstage<F16, TRI, MIXED, AS, BS, FIRST>(acc, f0, f1, smem, dfa, vo, voB, gP + kn * BKF, gB + kn * BKF, ldsw); \
   }
-  FM_DSTAGE(0, 0, true)
+  FM_DSTAGE(0, 0, 0, true)
   int s = 1;
-  for (; s + 3 <= n; s += 3) {
-    FM_DSTAGE(1, s, false)
-    FM_DSTAGE(2, s + 1, false)
-    FM_DSTAGE(0, s + 2, false)
-  }
-  if (s < n) {
-    FM_DSTAGE(1, s, false)
-    if (s + 1 < n) FM_DSTAGE(2, s + 1, false)
+  if constexpr (MIXED) {   // the pair of slots comes round every 6 stages
+    for (; s < n; s += 6) {
+      FM_DSTAGE(1, 1, s, false)
+      if (s + 1 >= n) break;
+      FM_DSTAGE(2, 0, s + 1, false)
+      if (s + 2 >= n) break;
+      FM_DSTAGE(0, 1, s + 2, false)
+      if (s + 3 >= n) break;
+      FM_DSTAGE(1, 0, s + 3, false)
+      if (s + 4 >= n) break;
+      FM_DSTAGE(2, 1, s + 4, false)
+      if (s + 5 >= n) break;
+      FM_DSTAGE(0, 0, s + 5, false)
+    }
+  } else {
+    for (; s + 3 <= n; s += 3) {
+      FM_DSTAGE(1, 0, s, false)
+      FM_DSTAGE(2, 0, s + 1, false)
+      FM_DSTAGE(0, 0, s + 2, false)
+    }
+    if (s < n) {
+      FM_DSTAGE(1, 0, s, false)
+      if (s + 1 < n) FM_DSTAGE(2, 0, s + 1, false)
+    }
   }
 #undef FM_DSTAGE
   wait_vmcnt<0>();
   __syncthreads();   // no copy in flight and no wave still reading: LDS is free again
 }
 
-// A diagonal tile (at m0 on the diagonal) of a symmetric product, over n k stages from gP on.
+// A diagonal tile (at m0 on the diagonal) of a symmetric product, over n k stages from gP (and gB) on.
 template <bool F16, int MODE>
 __device__ __forceinline__ void diag_item(const GemmArgs& g, int m0, int n, unsigned char* smem, const uint32_t (&vo)[8],
-                                          const bf16_t* gP, uint32_t ldsw, int lane, int wave) {
+                                          const uint32_t (&voB)[8], const bf16_t* gP, const bf16_t* gB, uint32_t ldsw, int lane, int wave) {
+  constexpr bool MIXED = F16 && form_scales(mode_form(F16, MODE));
   const bool tri = wave < 2;
   DFragAddr dfa;
   int dlane = lane;   // derived anew for every such item instead of being kept across the others
@@ -1140,31 +1176,40 @@ __device__ __forceinline__ void diag_item(const GemmArgs& g, int m0, int n, unsi
                        : (q < 2 ? 64 * (wave - 2) + 32 * q : q < 6 ? 128 + 32 * (q - 2) : 128 * (wave - 2) + 32 * (7 - q));
     const int r = r0 + (dlane & 31);
     const uint32_t o = (uint32_t)(r * ROWB + (((dlane >> 5) ^ swz(r)) << 4));
+    const uint32_t slot0 = MIXED && d_col(tri, q) ? b_slot_off(0) : 0;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
-      dfa.lo[q][ks] = o ^ (ks << 5);
+      dfa.lo[q][ks] = (o ^ (ks << 5)) + slot0;
       dfa.hi[q][ks] = (o ^ (ks << 5)) + a_slot_off(2);
     }
   }
   const int k1 = n - 1 < 1 ? n - 1 : 1;
 #pragma unroll
   for (int q = 0; q < 8; ++q) dma16o(vo[q], gP, ldsw, a_slot_off(0) + q * 4096);
+  if constexpr (MIXED) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) dma16o(voB[q], gB, ldsw, b_slot_off(0) + q * 4096);
+  }
 #pragma unroll
   for (int q = 0; q < 8; ++q) dma16o(vo[q], gP + k1 * BKF, ldsw, a_slot_off(1) + q * 4096);
-  wait_vmcnt<8>();
+  if constexpr (MIXED) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) dma16o(voB[q], gB + k1 * BKF, ldsw, b_slot_off(1) + q * 4096);
+  }
+  wait_vmcnt<MIXED ? 16 : 8>();
   __syncthreads();
   unsigned char* const wave_lds = smem + wave * EPI_WAVE_BYTES;
   // (each kind of wave has accumulators of its own, pinned to their registers before the write-out)
   if (tri) {
     f32x16_t acc[3][4];
-    diag_item_loop<F16, true>(acc, smem, dfa, vo, gP, n, ldsw);
+    diag_item_loop<F16, true, MIXED>(acc, smem, dfa, vo, voB, gP, gB, n, ldsw);
 #pragma unroll
     for (int q = 0; q < 9; ++q) asm volatile("" : "+a"(acc[tri_r(tri_i(q), tri_j(q))][tri_c(tri_i(q), tri_j(q))]));
     const int sq = m0 + 128 * wave;
     epilogue_regs<F16, MODE, 2, 1>(g, false, 0, acc, wave_lds, sq, sq, lane);
   } else {
     f32x16_t acc[3][4];
-    diag_item_loop<F16, false>(acc, smem, dfa, vo, gP, n, ldsw);
+    diag_item_loop<F16, false, MIXED>(acc, smem, dfa, vo, voB, gP, gB, n, ldsw);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1629,7 +1674,7 @@ __device__ __forceinline__ void rounds(const FastArgs& p, unsigned char* smem) {
     const int n = ke - kb;
     int bi, ti, tj, half = 0;
     bool ditem = false;   // NI == 2: a whole diagonal tile of a symmetric product
-    if constexpr (NI == 2) half_item_at<form_scales(FORM)>(p.g, item, bi, ti, tj, half, ditem);
+    if constexpr (NI == 2) half_item_at(p.g, item, bi, ti, tj, half, ditem);
     else tile_at(p.g, p.ksplit > 1 ? item / p.ksplit : item, bi, ti, tj);
     const GemmArgs g = batch_view(p.g, bi);
     const int m0 = ti * BM + half * 128, n0 = tj * BN;
@@ -1638,14 +1683,15 @@ __device__ __forceinline__ void rounds(const FastArgs& p, unsigned char* smem) {
     const bf16_t* gB = g.B + (int64_t)n0 * g.ldb + (int64_t)kb * BKF;
 
     if constexpr (NI == 2) {
-      if (ditem) {   // a diagonal tile of a symmetric product: its panel is operand B's (A == B), rows in their own order
-        uint32_t vo[8];
+      if (ditem) {   // a diagonal tile of a symmetric product: its panels are rows in their own order
+        uint32_t vo[8], voB[8];
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
           const int row = (q * 4 + wave) * 8 + (lane >> 3);
-          vo[q] = (uint32_t)(row * (int)g.ldb + (((lane & 7) ^ swz(row)) * 8)) * 2u;
+          vo[q] = (uint32_t)(row * (int)g.lda + (((lane & 7) ^ swz(row)) * 8)) * 2u;
+          voB[q] = (uint32_t)(row * (int)g.ldb + (((lane & 7) ^ swz(row)) * 8)) * 2u;
         }
-        diag_item<F16, MODE>(g, m0, n, smem, vo, gB, ldsw, lane, wave);
+        diag_item<F16, MODE>(g, m0, n, smem, vo, voB, gA, gB, ldsw, lane, wave);
         __syncthreads();   // the next item's copies land in the memory the staging just used
         continue;
       }
@@ -1666,7 +1712,7 @@ __device__ __forceinline__ void rounds(const FastArgs& p, unsigned char* smem) {
     }
 
     {   // a whole tile, a part of one along k, or a half tile (never on the diagonal of a symmetric product)
-      const bool diag = (NI == 4 || form_scales(FORM)) && g.symmetric && ti == tj;
+      const bool diag = NI == 4 && g.symmetric && ti == tj;
       float* const slot = NI == 4 && n != p.nk ? p.partials + (size_t)slot_id * PART_FLOATS : nullptr;
       const bool draws = NI == 4 && p.sub64 && p.tickets != nullptr && round == p.rounds - 1 && tickets_live;
       whole_tile16<F16, MODE, 2 * NI>(g, diag, n, slot, smem, fa16, voA, voB, gA, gB, ldsw, m0 + wm * (32 * NI), n0 + wn * 128,
@@ -2093,10 +2139,10 @@ static double estimate_half_round(long long half_items, int nk, int grid) {
   return nk * (0.50 + 0.78 * (occ > 0.6 ? occ - 0.6 : 0.0)) + 13.0;
 }
 
-// half items of all matrices: a diagonal tile of A A^T is one, of the product of two matrices two
+// half items of all matrices: a diagonal tile of a symmetric product is one
 static long long half_item_count(const GemmArgs& a) {
   const long long tm = a.Ma / BM, tn = a.Nb / BN, nb = a.batch < 1 ? 1 : a.batch;
-  return (!a.symmetric ? 2 * tm * tn : a.A == a.B ? tm * tm : tm * (tm + 1)) * nb;
+  return (a.symmetric ? tm * tm : 2 * tm * tn) * nb;
 }
 
 // The half-tile schedule (128x256 items, a diagonal tile of a symmetric product as one item) is
