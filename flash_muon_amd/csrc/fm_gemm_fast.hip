@@ -987,6 +987,7 @@ struct FastArgs {
   unsigned long long* tickets;
   unsigned long long epoch;   // this launch's number (48 bits, never 0)
   int half;             // the items are 128x256 half tiles, never cut (the NI == 2 kernels)
+  int tail_tile0;       // >= 0: the halves of the tiles from this one on, two items each (the second of a diagonal tile is none)
 };
 
 // k stages [kb, ke) of base part `part` of `parts`, or of its sub-part `sub` of `subs`
@@ -1674,7 +1675,16 @@ __device__ __forceinline__ void rounds(const FastArgs& p, unsigned char* smem) {
     const int n = ke - kb;
     int bi, ti, tj, half = 0;
     bool ditem = false;   // NI == 2: a whole diagonal tile of a symmetric product
-    if constexpr (NI == 2) half_item_at(p.g, item, bi, ti, tj, half, ditem);
+    if constexpr (NI == 2) {
+      if (p.tail_tile0 >= 0) {
+        tile_at(p.g, p.tail_tile0 + (item >> 1), bi, ti, tj);
+        half = item & 1;
+        ditem = p.g.symmetric && ti == tj;
+        if (ditem && half) continue;
+      } else {
+        half_item_at(p.g, item, bi, ti, tj, half, ditem);
+      }
+    }
     else tile_at(p.g, p.ksplit > 1 ? item / p.ksplit : item, bi, ti, tj);
     const GemmArgs g = batch_view(p.g, bi);
     const int m0 = ti * BM + half * 128, n0 = tj * BN;
@@ -2159,6 +2169,14 @@ static bool half_schedule_chosen(long long half_items, long long tiles, int nk, 
   return estimate_half_round(half_items, nk, grid) < estimate_whole_round(tiles, nk, auto_ksplit(tiles, nk, grid), grid);
 }
 
+// The tiles left over after full rounds, at most half as many as CUs: a round of parts of them along k, which go to memory, and a second
+// kernel that adds them (33 us beside the stages), or a launch of their halves behind the rounds (21: it waits for the slowest XCD).  us, parts / halves:
+// X X^T 6656 x 1024 (95 tiles left) 78.5 / 64.0, 5888 x 2048 96 / 92; five steps on 8 of 3072^2 4446 / 4258, on 32 of 2048^2 5571 / 5405, on 24 of 2048 x 5504 6797 / 6593; but
+// on 8 of 4096 x 11008 (64 left, 64 stages) 13853 / 13988.
+static bool half_tail_pays(int rem, int split, int nk, int grid) {
+  return estimate_half_round(2LL * rem, nk, grid) + 8.0 < 0.95 * ((nk / split) * 1.3 + 33.0);
+}
+
 // Few tiles (at most a sixteenth of the workgroups) can also run as 64x64 sub-tiles over the whole
 // k, 16 workgroups per tile, the way the tiles left after the last full round do: one launch, no
 // fp32 parts, and sixteen times the workgroups of whole tiles.  A sub-tile stage moves four times
@@ -2300,6 +2318,7 @@ int launch_gemm_fast(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) 
   const long long have = (long long)(slot_bytes / (PART_FLOATS * sizeof(float)));
   fast_schedule(a.num_tiles, f.nk, have < kMaxSlots ? have : kMaxSlots, f);
   f.half = 0;
+  f.tail_tile0 = -1;
   int grid = cu_count() < kMaxGrid ? cu_count() : kMaxGrid;
   const long long kg = knob(kKnobGrid);
   if (kg > 0 && kg < grid) grid = (int)kg;
@@ -2345,6 +2364,23 @@ int launch_gemm_fast(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) 
     if (f.epoch != 0)
       f.tickets = reinterpret_cast<unsigned long long*>(static_cast<unsigned char*>(ws) + (ws_bytes / kTicketBytes - 1) * kTicketBytes);
   }
+  // Tiles left over that would be cut along k: as half tiles in a launch behind the full rounds instead, where that is estimated to be
+  // shorter (no fp32 parts through memory and no second kernel to add them).
+  FastArgs tail;
+  const bool halves = !f.half && f.rounds > 0 && f.ksplit == 1 && f.split > 1 && 2 * f.rem <= grid && knob(kKnobHalf) < 0 && knob(kKnobKsplit) < 0 &&
+                      half_tail_pays(f.rem, f.split, f.nk, grid);
+  if (halves) {
+    tail = f;
+    tail.half = 1;
+    tail.tail_tile0 = f.rounds * f.grid;
+    tail.grid = 2 * f.rem;
+    tail.rounds = 1;
+    tail.rem = 0;
+    tail.split = 1;
+    f.rem = 0;
+    f.split = 1;
+    f.reduce_tile0 = a.num_tiles;
+  }
   const int slots = f.tail_slot0 + f.rem * f.split;
   const int reduce_tiles = a.num_tiles - f.reduce_tile0;
   if (!f.half && reduce_tiles > 0 && (slots > have || f.ksplit * f.split > kMaxParts)) return kErrWorkspace;
@@ -2355,6 +2391,7 @@ int launch_gemm_fast(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) 
       break;                                                                                                           \
     }                                                                                                                  \
     hipLaunchKernelGGL((KERNEL<F16, MODE, 4>), dim3(f.grid), dim3(256), 0, stream, f);                                  \
+    if (halves) hipLaunchKernelGGL((KERNEL<F16, MODE, 2>), dim3(tail.grid), dim3(256), 0, stream, tail);                 \
     if (reduce_tiles > 0) hipLaunchKernelGGL((gemm_nt_reduce_kernel<F16, FORM>), dim3(reduce_tiles * 16), dim3(256), 0, stream, f); \
   } while (0)
   if (a.form == kFormPoly) FM_ROUNDS(gemm_nt_form_kernel, true, kFormPoly, kFormPoly);

@@ -63,9 +63,9 @@ def _library_call(Gs, steps, coeffs=NS_COEFFS):
 
 
 # 64x64 sub-tiles alone; 128-tiles, one per CU; the same with A = X X^T cut along k; in pairs; half tiles; whole 256-tiles in one round;
-# rounds with sub-tiles behind them, handed out by ticket, and with their last tiles cut along k; diagonal tiles last
+# rounds with sub-tiles behind them, handed out by ticket, with their last tiles as halves, and cut along k; diagonal tiles last
 @pytest.mark.parametrize("rows,cols,batch", [(512, 1024, 1), (1664, 3328, 1), (640, 10240, 1), (1664, 3328, 4), (3072, 6144, 1), (4096, 8192, 1),
-                                             (4096, 8192, 2), (2816, 5632, 5), (8192, 16384, 1)])
+                                             (4096, 8192, 2), (2816, 5632, 5), (4096, 8192, 8), (8192, 16384, 1)])
 def test_every_schedule_of_the_chain(rows, cols, batch):
     Gs = [_inputs(rows, cols, torch.bfloat16, 7 + i) for i in range(batch)]
     outs = _library_call(Gs, 5)
