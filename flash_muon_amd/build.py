@@ -13,7 +13,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJDIR = os.path.join(HERE, "build")
 LIB_PATH = os.path.join(HERE, "libflashmuon_hip.so")
-SOURCES = ["fm_gemm.hip", "fm_gemm_fast.hip", "fm_gemm_f32.hip", "fm_gemm_ragged.hip", "fm_flow.hip", "fm_elementwise.hip", "fm_api.hip"]
+SOURCES = ["fm_gemm.hip", "fm_gemm_fast.hip", "fm_gemm_f32.hip", "fm_gemm_ragged.hip", "fm_gemm_slim.hip", "fm_flow.hip", "fm_elementwise.hip", "fm_api.hip"]
 # a measurement aid (MFMA-only loop) that only `bench.py --mfma-probe` loads; a library of its own
 PROBE_LIB_PATH = os.path.join(HERE, "libflashmuon_probe.so")
 PROBE_SOURCES = [os.path.join("probe", "fm_probe.hip")]

@@ -188,7 +188,7 @@ constexpr int64_t kSyrkRaggedMinElems = 256 * 256;
 static bool whole_tiles(int M, int K) { return M % 128 == 0 && K % 64 == 0; }
 static bool syrk_ragged_layout(int M, int K, SyrkRagged* p) {
   if (M <= 0 || K <= 0 || (int64_t)M * K < kSyrkRaggedMinElems || K >= (1 << 22)) return false;
-  if (whole_tiles(M, K) && (M % 256 == 0 || any_knob_set() || !syrk_whole_in_place(M, K, cu_count()))) return false;
+  if (whole_tiles(M, K) && (M % 256 == 0 || any_knob_set() || syrk_whole_slim(M, K) || !syrk_whole_in_place(M, K, cu_count()))) return false;
   p->Kp = (K + 63) / 64 * 64;
   p->slots = syrk_ragged_workspace_bytes(M, K);
   p->x = align_up(p->slots, 256);   // (a copy has as many stages, and so the same pieces)

@@ -2132,7 +2132,14 @@ static int mid_ksplit(long long tiles, int nk, int grid) {
   }
   return mid_parts(tiles, nk, grid);
 }
-static double estimate_mid(long long tiles, int nk, int grid, bool with_e) { return mid_us(tiles, nk, grid, mid_ksplit(tiles, nk, grid), with_e); }
+static bool pair_eligible(const GemmArgs& a);
+// the better way on 128x128 tiles or halves of them
+static double estimate_mid(const GemmArgs& a, long long tiles, int nk, int grid) {
+  const double t = mid_us(tiles, nk, grid, mid_ksplit(tiles, nk, grid), a.E != nullptr);
+  if (any_knob_set() || !pair_eligible(a) || !gemm_slim_fits(a, grid)) return t;
+  const double slim = slim_us(tiles, nk, grid, a.E != nullptr);
+  return slim < t ? slim : t;
+}
 
 // Estimates in microseconds, from measured costs of a k stage and of a tile's start and write-out.
 // The clock the power cap allows falls as the chip fills, so a stage costs more the more CUs work.
@@ -2181,8 +2188,8 @@ static bool half_tail_pays(int rem, int split, int nk, int grid) {
 // k, 16 workgroups per tile, the way the tiles left after the last full round do: one launch, no
 // fp32 parts, and sixteen times the workgroups of whole tiles.  A sub-tile stage moves four times
 // the operand bytes per flop, so this pays up to about 64-80 k stages; beyond, the 128x128 tiles cut
-// along k win.  Measured on X X^T: 6.5 us + 0.205 us per stage (1024 x 1024 10, 1024 x 2048 13,
-// 1024 x 4096 20, 1024 x 8192 34 us); five Newton-Schulz steps at 1024^2 200 -> 176 us, 512 x 2048
+// along k win.  Measured on X X^T: 6.2 us + 0.175 us per stage (512 x 2048 11.4, 1024 x 2048 11.8,
+// 768 x 4096 16.4, 1024 x 4096 17.0 us; more per stage beyond 80 of them); five Newton-Schulz steps at 1024^2 200 -> 176 us, 512 x 2048
 // 204 -> 170, 768^2 185 -> 160.
 static bool sub64_schedule_chosen(const GemmArgs& a, long long tiles, int nk, int grid) {
   const long long ns = knob(kKnobNoSub64);       // 1: never; 0: whenever it fits; left alone: by the estimate below
@@ -2190,9 +2197,9 @@ static bool sub64_schedule_chosen(const GemmArgs& a, long long tiles, int nk, in
   if (ns == 0) return true;
   if (knob(kKnobKsplit) >= 0 || knob(kKnobHalf) >= 0 || knob(kKnobFastMinUnits) >= 0) return false;
   const long long tm = a.Ma / BM, tn = a.Nb / BN, nb = a.batch < 1 ? 1 : a.batch;
-  const double t_sub = nk * 0.205 + 6.5 + (a.E ? 2.0 : 0.0);
+  const double t_sub = (nk <= 80 ? nk * 0.175 + 6.2 : nk * 0.205 + 6.5) + (a.E ? 2.0 : 0.0);
   const long long small_tiles = (a.symmetric ? 2 * tm * (2 * tm + 1) / 2 : 4 * tm * tn) * nb;
-  double t_best = estimate_mid(small_tiles, nk, grid, a.E != nullptr);
+  double t_best = estimate_mid(a, small_tiles, nk, grid);
   const int ksplit = auto_ksplit(tiles, nk, grid);
   const double t_large = (nk / ksplit) * 1.45 + 15.0 + (ksplit > 1 ? 25.0 : 0.0);
   if (t_large < t_best) t_best = t_large;
@@ -2223,7 +2230,7 @@ bool gemm_fast_eligible(const GemmArgs& a) {
   const int ksplit = auto_ksplit(tiles, nk, cus);
   const double t_large = (nk / ksplit) * 1.45 + 15.0 + (ksplit > 1 ? 25.0 : 0.0);
   const long long small_tiles = (a.symmetric ? 2 * tm * (2 * tm + 1) / 2 : 4 * tm * tn) * (a.batch < 1 ? 1 : a.batch);
-  const double t_small = estimate_mid(small_tiles, nk, cus, a.E != nullptr);
+  const double t_small = estimate_mid(a, small_tiles, nk, cus);
   const long long half_items = half_item_count(a);
   // (the 128x128 tiles keep the benefit of the doubt against half tiles)
   if (half_schedule_chosen(half_items, tiles, nk, cus) && estimate_half_round(half_items, nk, cus) < 0.9 * t_small) return true;
@@ -2238,11 +2245,22 @@ static bool pair_eligible(const GemmArgs& a) {
   return !a.E || (a.ET && a.ldet % 8 == 0 && a.ldet < (1 << 21) && (reinterpret_cast<uintptr_t>(a.ET) & 15) == 0 && (a.batch < 2 || a.bs_et % 8 == 0));
 }
 
+// Halves of the 128x128 tiles, at most one a CU, rather than whole tiles on half of the CUs or less, and than those cut along k (slim_us).
+static bool slim_chosen(const GemmArgs& a, const void* ws, size_t ws_bytes) {
+  const int cus = cu_count() < kMaxGrid ? cu_count() : kMaxGrid, nk = a.Kc / BKF;
+  if (any_knob_set() || !pair_eligible(a) || !gemm_slim_fits(a, cus)) return false;
+  const long long tm = a.Ma / MID_T, tn = a.Nb / MID_T, tiles = (a.symmetric ? tm * (tm + 1) / 2 : tm * tn) * (a.batch < 1 ? 1 : a.batch);
+  const int parts = mid_parts(tiles, nk, cus);
+  if (parts == 1 || (a.form && a.elem == kElemF16) || !ws || (size_t)tiles * parts * MID_PART_FLOATS * sizeof(float) > ws_bytes) return true;
+  return slim_us(tiles, nk, cus, a.E != nullptr) < mid_us(tiles, nk, cus, parts, a.E != nullptr);
+}
+
 int launch_gemm_mid(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) {
   a.tiles_m = a.Ma / MID_T;
   a.tiles_n = a.Nb / MID_T;
   if (a.batch < 1) a.batch = 1;
   a.num_tiles = (a.symmetric ? a.tiles_m * (a.tiles_m + 1) / 2 : a.tiles_m * a.tiles_n) * a.batch;
+  if (slim_chosen(a, ws, ws_bytes)) return launch_gemm_slim(a, stream);
   MidSplit sp;
   sp.ksplit = mid_ksplit(a.num_tiles, a.Kc / BKF, cu_count() < kMaxGrid ? cu_count() : kMaxGrid);
   sp.partials = static_cast<float*>(ws);

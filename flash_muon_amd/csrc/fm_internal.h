@@ -185,6 +185,9 @@ size_t gemm_fast_workspace_bytes(int Ma, int Nb, int batch);
 int launch_gemm_fast(GemmArgs args, void* ws, size_t ws_bytes, hipStream_t stream);
 bool gemm_mid_eligible(const GemmArgs& a);
 int launch_gemm_mid(GemmArgs args, void* ws, size_t ws_bytes, hipStream_t stream);
+// the same problems as halves of their 128x128 tiles, at most one a CU (fm_gemm_slim.hip); E through ET
+bool gemm_slim_fits(const GemmArgs& args, int cus);
+int launch_gemm_slim(const GemmArgs& args, hipStream_t stream);
 
 // up to kMaxBatch device pointers, passed to a kernel by value
 struct PtrList { void* p[kMaxBatch]; };

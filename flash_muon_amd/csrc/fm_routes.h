@@ -271,6 +271,18 @@ inline double mid_us(long long tiles, int nk, int grid, int parts, bool with_e) 
   return (double)((tiles + grid - 1) / grid) * (nk * stage + (with_e ? 11.0 : 6.0));
 }
 
+// The same as halves of the tiles, at most one a CU (fm_gemm_slim.hip): a stage of 24 KiB, no cut.  us, whole or cut tiles / halves: X X^T 1536 x
+// 1024 11.8 / 9.7, x 4096 27.4 / 22.2, 1792 x 2048 17.6 / 14.1, x 8192 40.5 / 37.9, 768 x 4096 20.5 / 19.4; cut along a long k 512 x 4096 17.9 / 18.8, x 8192
+// 22.9 / 33.9, 1024 x 8192 24.9 / 35.5, 1536 x 8192 33.7 / 38.0, 1792 x 16384 65.3 / 70.3.
+inline double slim_us(long long tiles, int nk, int grid, bool with_e) {
+  const double occ = 2.0 * tiles >= grid ? 1.0 : 2.0 * (double)tiles / grid;
+  return 5.7 + nk * (0.223 + 0.037 * occ) + (with_e ? 2.0 : 0.0);
+}
+
+// X X^T of an odd number of whole 128-tiles on those halves rather than in place or on whole tiles (below).  us, otherwise / halves: 640 x 2048 13.4 / 12.1, 896 x
+// 1024 9.3 / 8.7, 1152 x 2048 14.6 / 12.4, 1664 x 4096 25.5 / 22.7, 1920 x 4096 27.7 / 24.0; but 640 x 4096 15.4 / 18.9, 1152 x 8192 24.0 / 26.9.
+inline bool syrk_whole_slim(int M, int K) { return M <= 1920 && K >= 1024 && K <= (M >= 1664 ? 4096 : 2048); }
+
 // X X^T of an odd number of whole 128-tiles, rows on lines: in place on tiles that share a CU in pairs (fm_gemm_ragged.hip), or on the
 // tiles above.  us, above / in place: more tiles than CUs 2944^2 46.7 / 38.2, 4224^2 96 / 78, 5504 x 2048 81 / 62, 8064 x 1024 114 / 70; 121 to
 // 256 of them 2176^2 20.7 / 21.8, 2688^2 26.3 / 26.9.  Fewer: the deeper ring above starts later (4 us) and takes 0.36 us a stage where
