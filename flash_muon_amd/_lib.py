@@ -98,10 +98,15 @@ def dtype_code(dtype):
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
+def _index(device):
+    """The index of a torch.device, or of what names one; None: the current device."""
+    return (device if isinstance(device, torch.device) else torch.device(device)).index
+
+
 def stream_ptr(device):
     """The hipStream_t of torch's current stream on `device`, as an integer."""
     if _raw_stream is not None:      # the same value without building a Stream object (a few us per call)
-        idx = torch.device(device).index
+        idx = _index(device)
         return _raw_stream(torch.cuda.current_device() if idx is None else idx)
     return torch.cuda.current_stream(device).cuda_stream
 
@@ -120,7 +125,7 @@ _NO_GUARD = _NoGuard()
 def on_device(device):
     """Context that makes `device` the current one for the kernel launches of a call; nothing to
     enter or leave when it is current already."""
-    idx = torch.device(device).index
+    idx = _index(device)
     if idx is None or idx == torch.cuda.current_device():
         return _NO_GUARD
     return torch.cuda.device(idx)
@@ -144,7 +149,7 @@ def gemm_workspace(nbytes, device, stream=None):
     per call."""
     if nbytes == 0:
         return None, 0
-    key = (torch.device(device).index, stream_ptr(device) if stream is None else stream)
+    key = (_index(device), stream_ptr(device) if stream is None else stream)
     ws = _gemm_ws.get(key)
     if ws is None or ws.numel() < nbytes:
         # zeroed once: its last 256 bytes hold the word the library counts sub-tile tickets in, which
