@@ -36,10 +36,8 @@ struct NsLayout {
   bool padded;
   int edge_s, edge_x;    // tiles of the one-launch iteration
   bool flow;             // one launch for all products: x[0], a and p hold kFlowSteps (+ 1) iterates and squares
-  bool groups;           // the steps in groups (ns_groups_chosen); in one launch x[0] and a hold kFlowGroups (+ 1) and kFlowSlots
   size_t counters;
 };
-constexpr int kFlowSteps = 5;   // steps per launch of the one-launch iteration
 // 64x64 tiles for X' as long as every CU gets at most one, and for the symmetric products as long as they are
 // about one round (a longer K makes the 64-tiles of A = X X^T pay a little further): 512^2 104 us on 64x64
 // tiles, 115 with X' on 128x128, 144 all on 128x128; 8 of 384 x 768 152, 111 and 133; 24 of 768^2 520, 423 and 360.
@@ -59,18 +57,14 @@ void ns_flow_edges(int batch, int m, int k, int* es, int* ex) {
 // 2816 x 7168 26).  The long side alone goes to a multiple of 256 where the short one is one already
 // (32 of 2048 x 5504 15.4 ms, of 2048 x 5632 11.9; one matrix 0.72 and 0.59; below 1536 rows a single
 // matrix gains nothing).
-// `how`: launches per product, or in one launch, each with the steps one by one or in groups (for which the long side is at least twice the
-// short one, so that the iterate to come has room for two M x M matrices).
-enum NsHow { kNsLaunches = 0, kNsGroups = 1, kNsFlow = 2, kNsFlowGroups = 3 };
-NsLayout ns_layout(int batch, int rows, int cols, NsHow how) {
+// `flow`: one launch where that is the faster one (ns_flow_chosen).
+NsLayout ns_layout(int batch, int rows, int cols, bool flow) {
   const int m = rows < cols ? rows : cols, k = rows < cols ? cols : rows;
   const size_t B = (size_t)batch;
   NsLayout l = {};
-  l.flow = how == kNsFlow || how == kNsFlowGroups;
-  l.groups = how == kNsGroups || how == kNsFlowGroups;
-  if (l.flow) {
-    if (l.groups) l.edge_s = l.edge_x = 128;
-    else ns_flow_edges(batch, m, k, &l.edge_s, &l.edge_x);
+  if (flow && !any_knob_set() && ns_flow_chosen(batch, m, k)) {
+    l.flow = true;
+    ns_flow_edges(batch, m, k, &l.edge_s, &l.edge_x);
     l.M = (m + l.edge_x - 1) / l.edge_x * l.edge_x;
     l.K = (k + l.edge_x - 1) / l.edge_x * l.edge_x;
     l.padded = l.M != m || l.K != k;
@@ -79,11 +73,11 @@ NsLayout ns_layout(int batch, int rows, int cols, NsHow how) {
     const size_t M = (size_t)l.M, K = (size_t)l.K;
     l.partials = take(B * kSumsqBlocks * sizeof(float));
     l.pdiag_stride = M;
-    l.pdiag = take(B * M * (l.groups ? kFlowGroups : kFlowSteps) * sizeof(float));
-    l.x[0] = take(B * M * K * 2 * ((l.groups ? kFlowGroups : kFlowSteps) + 1));
-    l.a = take(B * M * M * 2 * (l.groups ? kFlowSlots : kFlowSteps));
-    if (!l.groups) l.p = take(B * M * M * 2 * kFlowSteps);
-    l.counters = take((size_t)flow_counter_words(batch, l.groups ? kFlowSlots + kFlowGroups : 3 * kFlowSteps) * sizeof(unsigned));
+    l.pdiag = take(B * M * kFlowSteps * sizeof(float));
+    l.x[0] = take(B * M * K * 2 * (kFlowSteps + 1));
+    l.a = take(B * M * M * 2 * kFlowSteps);
+    l.p = take(B * M * M * 2 * kFlowSteps);
+    l.counters = take((size_t)flow_counter_words(batch, kFlowSteps) * sizeof(unsigned));
     l.gemm = off;
     l.total = off;
     return l;
@@ -93,12 +87,10 @@ NsLayout ns_layout(int batch, int rows, int cols, NsHow how) {
   {
     const int64_t t = (l.M + 255) / 256;
     const bool near_square = k < m + m / 5;
-    const bool both = l.groups ? ns_groups_on_256(batch, m, k)
-                               : l.M >= (batch == 1 && near_square ? 2816 : 2176) || (l.M >= 1152 && (int64_t)batch * t * (t + 1) / 2 >= 120);
+    const bool both = l.M >= (batch == 1 && near_square ? 2816 : 2176) || (l.M >= 1152 && (int64_t)batch * t * (t + 1) / 2 >= 120);
     if (both) l.M = (int)t * 256;
     if (l.M % 256 == 0 && (both || l.M >= 1536 || (batch >= 4 && l.M >= 768))) l.K = (k + 255) / 256 * 256;
   }
-  if (l.groups && l.K < 2 * l.M) l.K = 2 * l.M;
   l.padded = l.M != m || l.K != k;
   const size_t M = (size_t)l.M, K = (size_t)l.K;
   size_t off = 0;
@@ -114,15 +106,6 @@ NsLayout ns_layout(int batch, int rows, int cols, NsHow how) {
   l.gemm = take(g1 > g2 ? g1 : g2);
   l.total = off;
   return l;
-}
-
-// which way the steps of a call take by choice; `grouped`: they may run in groups (enough steps, coefficients that fit)
-NsHow ns_how(int batch, int rows, int cols, bool grouped) {
-  const int m = rows < cols ? rows : cols, k = rows < cols ? cols : rows;
-  const bool one_by_one_in_flow = !any_knob_set() && ns_flow_chosen(batch, m, k);
-  if (any_knob_set() || !grouped || !ns_grouped(m, k)) return one_by_one_in_flow ? kNsFlow : kNsLaunches;
-  const NsWay way = ns_grouped_way(batch, m, k);
-  return way == kWayFlow ? kNsFlow : way == kWayFlowGroups ? kNsFlowGroups : kNsGroups;
 }
 
 // ---- scratch of fm_syrk_bf16_static -------------------------------------------------------------
@@ -429,14 +412,12 @@ int fm_scale_cast_bf16(const void* G, int dtype, int rows, int cols, int64_t ldg
 
 size_t fm_newtonschulz_batched_workspace_bytes(int batch, int rows, int cols) {
   if (batch <= 0 || rows <= 0 || cols <= 0) return 0;
-  // (few steps, or many)
-  const size_t few = ns_layout(batch, rows, cols, ns_how(batch, rows, cols, false)).total, many = ns_layout(batch, rows, cols, ns_how(batch, rows, cols, true)).total;
-  return few > many ? few : many;
+  return ns_layout(batch, rows, cols, true).total;
 }
 
 size_t fm_newtonschulz_batched_min_workspace_bytes(int batch, int rows, int cols) {
   if (batch <= 0 || rows <= 0 || cols <= 0) return 0;
-  const size_t best = ns_layout(batch, rows, cols, ns_how(batch, rows, cols, false)).total, launches = ns_layout(batch, rows, cols, kNsLaunches).total;
+  const size_t best = ns_layout(batch, rows, cols, true).total, launches = ns_layout(batch, rows, cols, false).total;
   return best < launches ? best : launches;
 }
 
@@ -456,6 +437,7 @@ size_t fm_newtonschulz_workspace_bytes(int rows, int cols) {
 // of spectra from M = 512 and K = 2 M on, but one (columns scaled over three decades, 1024 x 2048 6.8e-3 / 7.3e-3).
 // In bf16 the same chain loses (rows with a common part, 256 x 1024: 7.4e-3 / 5.0e-2), and so do all five steps as one
 // (2.0e-2 on gradients) and squarer matrices (columns as above, 2048^2: 5.9e-3 / 7.7e-3), which would gain no time either.
+constexpr float kGramA = 16384.0f, kGramQ = 8192.0f, kGramR = 4096.0f;   // scales of A and Q A, of Q, of Q_2 Q_1
 // A of a group, at scale kGramA (fp16), to the product of the group's n factors, in A (bf16, its diagonal to pdiag).  Q, V and W:
 // room for one more matrix each (stride bs_q, bs_vw between matrices).
 static int launch_gram_chain(int n, bf16_t* A, bf16_t* Q, int64_t mm, bf16_t* V, bf16_t* W, int64_t bs_vw, float* pdiag, int64_t bs_diag,
@@ -511,13 +493,8 @@ static int ns_impl(const void* const* G, int dtype, int batch, int rows, int col
       if (j != i && overlaps(mat_range(out[j], rows, cols, ldout, 2), oi)) return FM_ERR_ALIAS;
     }
   }
-  // Where the scratch does not hold what the chosen way needs: the other ones, least scratch last (launches one by one keep
-  // two iterates, one launch keeps one for every step or group)
-  const bool grouped = steps >= kGroupedSteps && ns_grouped(rows < cols ? rows : cols, rows < cols ? cols : rows) && ns_groups_fit(steps, a, b, c);
-  NsLayout l = ns_layout(batch, rows, cols, ns_how(batch, rows, cols, grouped));
-  if (l.groups && ws_bytes < l.total) l = ns_layout(batch, rows, cols, ns_how(batch, rows, cols, false));
-  if (l.flow && ws_bytes < l.total) l = ns_layout(batch, rows, cols, kNsLaunches);
-  if (!l.flow && grouped && !any_knob_set() && l.K >= 2 * (int64_t)l.M) l.groups = true;   // (room for groups all the same)
+  NsLayout l = ns_layout(batch, rows, cols, true);
+  if (l.flow && ws_bytes < l.total) l = ns_layout(batch, rows, cols, false);   // which keeps two iterates, not one for every step
   if (!ws || ws_bytes < l.total) return FM_ERR_WORKSPACE;
   if (reinterpret_cast<uintptr_t>(ws) % 256 != 0) return FM_ERR_ALIGN;
   {
@@ -550,7 +527,7 @@ static int ns_impl(const void* const* G, int dtype, int batch, int rows, int col
     float* sumsq = reinterpret_cast<float*>(w + l.partials);
     const int parts = sumsq_parts((int64_t)rows * cols);
     unsigned* counters = reinterpret_cast<unsigned*>(w + l.counters);
-    const int n_counters = flow_counter_words(batch, l.groups ? kFlowSlots + kFlowGroups : 3 * (steps < kFlowSteps ? steps : kFlowSteps));
+    const int n_counters = flow_counter_words(batch, steps < kFlowSteps ? steps : kFlowSteps);
     const int64_t mk = (int64_t)l.M * l.K;
     bf16_t* X = reinterpret_cast<bf16_t*>(w + l.x[0]);
     if (squares(sumsq, counters, n_counters)) return FM_ERR_LAUNCH;
@@ -560,41 +537,26 @@ static int ns_impl(const void* const* G, int dtype, int batch, int rows, int col
                                   hs, tall ? l.K : l.M, tall ? l.M : l.K))
       return FM_ERR_LAUNCH;
     FlowProblem f = {};
-    f.X = X; f.x_step = batch * mk;
     f.A = reinterpret_cast<bf16_t*>(w + l.a); f.P = reinterpret_cast<bf16_t*>(w + l.p); f.a_step = (int64_t)batch * l.M * l.M;
     f.pdiag = reinterpret_cast<float*>(w + l.pdiag); f.d_step = (int64_t)batch * l.pdiag_stride; f.d_mat = (int64_t)l.pdiag_stride;
     f.M = l.M; f.K = l.K; f.batch = batch; f.edge_s = l.edge_s; f.edge_x = l.edge_x;
     f.a = a; f.b = b; f.c = c;
     f.counters = counters;
-    for (int s = 0; s < steps;) {
-      const int s0 = s;
-      int iterates;   // of this launch
-      if (l.groups) {
-        f.group[0] = ns_group(steps, s);
-        s += f.group[0];
-        f.groups = 1;
-        if (s < steps && f.group[0] + ns_group(steps, s) <= kFlowSteps) {   // (two groups of three would take more slots)
-          f.group[1] = ns_group(steps, s);
-          s += f.group[1];
-          f.groups = 2;
-        }
-        iterates = f.groups;
-      } else {
-        iterates = f.steps = steps - s < kFlowSteps ? steps - s : kFlowSteps;
-        s += f.steps;
-      }
-      const bool last = s == steps;
+    const int64_t bmk = batch * mk;
+    for (int i = 0; i * kFlowSteps < steps; ++i) {
+      const NsFlowLaunch n = ns_flow_launch(steps, i);
+      f.steps = n.steps;
+      f.X = X + n.from * bmk; f.x_step = n.turn * bmk;
+      const bool last = n.first + n.steps == steps;
       // what is not the last launch leaves its result in the slot behind its own, from where the next one
       // goes the other way
       void* o[kMaxBatch];
-      for (int i = 0; i < batch; ++i) o[i] = last ? out[i] : (void*)(f.X + iterates * f.x_step + i * mk);
+      for (int j = 0; j < batch; ++j) o[j] = last ? out[j] : (void*)(f.X + n.steps * f.x_step + j * mk);
       f.out = o;
       f.ldout = last ? ldout : l.K;
       f.rows = last ? rows : l.M; f.cols = last ? cols : l.K; f.tall = last && tall;
-      if (s0 > 0 && launch_zero_words(counters, n_counters, hs)) return FM_ERR_LAUNCH;
+      if (i > 0 && launch_zero_words(counters, n_counters, hs)) return FM_ERR_LAUNCH;
       if (launch_ns_flow(f, hs)) return FM_ERR_LAUNCH;
-      f.X += iterates * f.x_step;
-      f.x_step = -f.x_step;
     }
     return FM_OK;
   }
@@ -642,9 +604,10 @@ static int ns_impl(const void* const* G, int dtype, int batch, int rows, int col
   // for the copy out of the padded one).
   bool cut_out = padded && rows % 128 == 0 && cols % 128 == 0 && ldout % 8 == 0 && ldout < (1 << 21);
   for (int i = 0; i < batch; ++i) cut_out = cut_out && (reinterpret_cast<uintptr_t>(out[i]) & 15) == 0;
+  const bool grouped = !any_knob_set() && ns_grouped(M, K, steps) && ns_groups_fit(steps, a, b, c);
   int turn = 0;   // which pair of iterates holds X
   for (int s = 0; s < steps;) {
-    const int n = l.groups ? ns_group(steps, s) : 1;
+    const int n = grouped ? ns_group(steps, s) : 1;
     const bool last = s + n == steps;
     turn ^= 1;
     bf16_t* Xn = reinterpret_cast<bf16_t*>(w + l.x[turn]);

@@ -28,10 +28,6 @@
 // the LDS, whose 750 cycles per stage and 128x128 tile are 0.38 us under load, and about 4 us of every tile that
 // the CU's other workgroup does not cover.  24 of 768^2 360 us, in launches 393; 8 of 1024 x 2816 583 and 700;
 // 16 of 512^2 137 and 185.
-//
-// Long matrices iterate in groups of steps (fm_api.hip): their products are A, then on M x M matrices in fp16 Q = a I + b A + c A^2,
-// Q A, the next A = Q (Q A) and so on to the product R of the Q, and X' = R X.  These matrices have a slot of their own each.  18
-// products instead of 15, but two thirds of the work: 8 of 1024 x 2816 571 -> 458 us, 16 of 768 x 3072 683 -> 508, 16 of 1408 x 3784 2412 -> 1707.
 #include "fm_tile64.h"
 
 namespace fm {
@@ -56,53 +52,21 @@ struct FlowArgs {
   PtrList out; int64_t ldout;
   int rows, cols;                     // of the output
   int tall, vec;
-  // in groups: the slots (A is the first), a_step apart, and the steps of each group
-  int groups, group[kFlowGroups];
 };
 
 constexpr int kEnd = -1, kFlush = -2;   // messages that are no item
-struct Item { int prod, m, tile; };   // product 3 step + {0: A, 1: P, 2: X'}, or in groups as below
-
-// Products of a group of n steps: product i < sym_count(n) is symmetric and goes to slot i, the last one is X'.  In the order of their
-// slots: A, Q, Q A, A', Q', Q' A', A'', then of three steps Q' Q, Q'', Q'' (Q' Q), of two Q' Q behind Q'.  Each depends on the one before
-// it, but Q' Q on Q' alone and the last one of three on two: whoever waits for the last tiles of A'' finds Q' Q ready.
-__device__ __forceinline__ int sym_count(int n) { return n == 3 ? 10 : 6; }
-struct Place { int g, i, base, n; };   // group, product of the group, number of its first product and slots before it, steps
-__device__ __forceinline__ Place place_of(const FlowArgs& p, int prod) {
-  const int n0 = sym_count(p.group[0]) + 1;
-  if (prod < n0) return Place{0, prod, 0, p.group[0]};
-  return Place{1, prod - n0, n0 - 1, p.group[1]};
-}
+struct Item { int prod, m, tile; };   // product 3 step + {0: A, 1: P, 2: X'}
 
 // items of queue q in a product of n tiles in all: [n q / 8, n (q + 1) / 8)
 __device__ __forceinline__ int run_begin(int n, int q) { return (int)((unsigned)n * (unsigned)q >> 3); }
 
-template <bool GROUPS>
 __device__ __forceinline__ int queue_total(const FlowArgs& p, int q) {
   const int ns = p.sym_tiles * p.batch, nr = p.rect_tiles * p.batch;
-  if constexpr (GROUPS) {
-    const int syms = sym_count(p.group[0]) + (p.groups > 1 ? sym_count(p.group[1]) : 0);
-    return syms * (run_begin(ns, q + 1) - run_begin(ns, q)) + p.groups * (run_begin(nr, q + 1) - run_begin(nr, q));
-  }
   return p.steps * (2 * (run_begin(ns, q + 1) - run_begin(ns, q)) + run_begin(nr, q + 1) - run_begin(nr, q));
 }
-template <bool GROUPS>
 __device__ __forceinline__ Item item_at(const FlowArgs& p, int q, int t) {
   const int ns = p.sym_tiles * p.batch, nr = p.rect_tiles * p.batch;
   const int s0 = run_begin(ns, q), r0 = run_begin(nr, q), cs = run_begin(ns, q + 1) - s0, cr = run_begin(nr, q + 1) - r0;
-  if constexpr (GROUPS) {
-    const int syms0 = sym_count(p.group[0]);
-    int first = 0, syms = syms0;
-    if (t >= syms0 * cs + cr) {
-      t -= syms0 * cs + cr;
-      first = syms0 + 1;
-      syms = sym_count(p.group[1]);
-    }
-    const bool rect = t >= syms * cs;
-    const int op = rect ? syms : t / cs, i = rect ? r0 + t - syms * cs : s0 + t - op * cs, tiles = rect ? p.rect_tiles : p.sym_tiles;
-    const int m = i / tiles;
-    return Item{first + op, m, i - m * tiles};
-  }
   const int per = 2 * cs + cr, step = t / per;
   t -= step * per;
   Item it;
@@ -121,33 +85,14 @@ __device__ __forceinline__ void count_up(unsigned* p) { __hip_atomic_fetch_add(p
 __device__ __forceinline__ unsigned* counts(const FlowArgs& p, int prod, int m) {
   return p.done + (size_t)((prod * p.batch + m) * p.subs) * kLine;
 }
-// What an item waits for is looked at by a whole wave: lane i reads word i of the product before, in groups of the first product that
-// it depends on, lane 16 + i that of the second, if there is one; `enough` adds them up.
-struct Needs { int first, count; unsigned tiles; };
-__device__ __forceinline__ Needs needs_of(const FlowArgs& p, int prod) {
-  const Place at = place_of(p, prod);
-  if (at.i == 0) return Needs{prod - 1, 1, (unsigned)p.rect_tiles};
-  if (at.n == 3 && at.i == 7) return Needs{prod - 3, 1, (unsigned)p.sym_tiles};
-  if (at.n == 3 && at.i == 8) return Needs{prod - 2, 1, (unsigned)p.sym_tiles};
-  if (at.n == 3 && at.i == 9) return Needs{prod - 2, 2, 2u * p.sym_tiles};
-  return Needs{prod - 1, 1, (unsigned)p.sym_tiles};
-}
-template <bool GROUPS>
+// What an item waits for is looked at by a whole wave: lane i reads word i, `enough` adds them up.
 __device__ __forceinline__ unsigned look_at(const FlowArgs& p, const Item& it, int lane) {
-  if constexpr (GROUPS) {
-    if (it.prod == 0) return 0u;
-    const Needs n = needs_of(p, it.prod);
-    const int sub = lane & (kMaxSubs - 1), of = lane / kMaxSubs;
-    return of < n.count && sub < p.subs ? load_agent(counts(p, n.first + of, it.m) + sub * kLine) : 0u;
-  }
   return it.prod > 0 && lane < p.subs ? load_agent(counts(p, it.prod - 1, it.m) + lane * kLine) : 0u;
 }
-template <bool GROUPS>
 __device__ __forceinline__ bool enough(const FlowArgs& p, const Item& it, unsigned seen) {
   if (it.prod == 0) return true;
 #pragma unroll
-  for (int o = GROUPS ? kMaxSubs : kMaxSubs / 2; o > 0; o >>= 1) seen += __shfl_xor(seen, o, 64);
-  if constexpr (GROUPS) return __builtin_amdgcn_readfirstlane(seen) >= needs_of(p, it.prod).tiles;
+  for (int o = kMaxSubs / 2; o > 0; o >>= 1) seen += __shfl_xor(seen, o, 64);
   return __builtin_amdgcn_readfirstlane(seen) >= (unsigned)(it.prod % 3 == 0 ? p.rect_tiles : p.sym_tiles);   // of the product before
 }
 __device__ __forceinline__ unsigned draw(unsigned* head, int lane) {
@@ -158,14 +103,13 @@ __device__ __forceinline__ unsigned draw(unsigned* head, int lane) {
 
 // an item for a workgroup that waits for one of product `prod`: the head of some queue, if it is of an earlier
 // product and ready
-template <bool GROUPS>
 __device__ bool help(const FlowArgs& p, int prod, Item& it, int lane) {
   for (int q = 0; q < kQueues; ++q) {
     unsigned* const head = p.tickets + q * kLine;
     unsigned t = __builtin_amdgcn_readfirstlane(load_agent(head));
-    if ((int)t >= queue_total<GROUPS>(p, q)) continue;
-    const Item c = item_at<GROUPS>(p, q, (int)t);
-    if (c.prod >= prod || !enough<GROUPS>(p, c, look_at<GROUPS>(p, c, lane))) continue;
+    if ((int)t >= queue_total(p, q)) continue;
+    const Item c = item_at(p, q, (int)t);
+    if (c.prod >= prod || !enough(p, c, look_at(p, c, lane))) continue;
     int got = 0;
     if (lane == 0) got = __hip_atomic_compare_exchange_strong(head, &t, t + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (__builtin_amdgcn_readfirstlane(got)) {
@@ -179,8 +123,8 @@ __device__ bool help(const FlowArgs& p, int prod, Item& it, int lane) {
 // cache policy of stores that other XCDs read (sc1: written through to memory)
 constexpr int kThrough = 16;
 
-// Edges of the tiles, 128 or 64: ES of the symmetric products, EX of X'.  GROUPS: steps in groups, on 128-tiles.
-template <int ES, int EX, bool GROUPS = false>
+// Edges of the tiles, 128 or 64: ES of the symmetric products, EX of X'
+template <int ES, int EX>
 __global__ __launch_bounds__(256, 2) void ns_flow_kernel(FlowArgs p) {
   __shared__ __align__(1024) unsigned char smem[t128::SMEM];   // the ring of either tile size
   const int lane = threadIdx.x & 63;
@@ -210,8 +154,8 @@ __global__ __launch_bounds__(256, 2) void ns_flow_kernel(FlowArgs p) {
         if (!drawn) next = draw(p.tickets + q * kLine, lane);
         const int t = (int)__builtin_amdgcn_readfirstlane(next);
         drawn = false;
-        if (t < queue_total<GROUPS>(p, q)) {
-          mine = item_at<GROUPS>(p, q, t);
+        if (t < queue_total(p, q)) {
+          mine = item_at(p, q, t);
           holding = true;
         } else {
           q = (q + 1) & (kQueues - 1);
@@ -219,15 +163,15 @@ __global__ __launch_bounds__(256, 2) void ns_flow_kernel(FlowArgs p) {
         }
       }
       if (holding) {
-        if (enough<GROUPS>(p, mine, looked ? seen : look_at<GROUPS>(p, mine, lane))) {
+        if (enough(p, mine, looked ? seen : look_at(p, mine, lane))) {
           now = mine;
           holding = false;
         } else if (open) {   // nothing to go on with: first say that the item before is done
           now.prod = kFlush;
         } else {
           for (int n = 1;; ++n) {
-            if (enough<GROUPS>(p, mine, look_at<GROUPS>(p, mine, lane))) { now = mine; holding = false; break; }
-            if ((n & 63) == 0 && help<GROUPS>(p, mine.prod, now, lane)) break;
+            if (enough(p, mine, look_at(p, mine, lane))) { now = mine; holding = false; break; }
+            if ((n & 63) == 0 && help(p, mine.prod, now, lane)) break;
           }
         }
         looked = false;
@@ -258,13 +202,11 @@ __global__ __launch_bounds__(256, 2) void ns_flow_kernel(FlowArgs p) {
       if (prod == kEnd) break;
       continue;
     }
-    const Place at = GROUPS ? place_of(p, prod) : Place{prod / 3, prod % 3, 0, 1};
-    const int step = at.g, op = !GROUPS ? at.i : at.i < sym_count(at.n) ? 0 : 2;
+    const int step = prod / 3, op = prod - 3 * step;
     const int64_t mk = (int64_t)p.M * p.K, mm = (int64_t)p.M * p.M;
     const bf16_t* const X = p.X + step * p.x_step + m * mk;
-    // (in groups A is the group's first slot and P its last, which holds R)
-    bf16_t* const A = p.A + (GROUPS ? at.base : step) * p.a_step + m * mm;
-    bf16_t* const P = GROUPS ? A + (sym_count(at.n) - 1) * p.a_step : p.P + step * p.a_step + m * mm;
+    bf16_t* const A = p.A + step * p.a_step + m * mm;
+    bf16_t* const P = p.P + step * p.a_step + m * mm;
     float* const pd = p.pdiag + step * p.d_step + m * p.d_mat;
     int l = lane;
     asm volatile("" : "+v"(l));   // per-lane addresses derived anew for every item
@@ -272,62 +214,18 @@ __global__ __launch_bounds__(256, 2) void ns_flow_kernel(FlowArgs p) {
     auto look = [&]() {
       if (wave == 0 && drawn) {
         const int t = (int)__builtin_amdgcn_readfirstlane(next);
-        if (t < queue_total<GROUPS>(p, q)) {
-          ahead = item_at<GROUPS>(p, q, t);
-          seen = look_at<GROUPS>(p, ahead, lane);
+        if (t < queue_total(p, q)) {
+          ahead = item_at(p, q, t);
+          seen = look_at(p, ahead, lane);
           looked = true;
         }
       }
     };
-    const bool last = step + 1 == (GROUPS ? p.groups : p.steps);
+    const bool last = step + 1 == p.steps;
     if (op < 2) {
       int ti, tj;
       band_tri_decode(tile, p.ts, ti, tj);
-      if constexpr (GROUPS) {
-        f32x4_t acc[4][4];
-        uint32_t voA[4], voB[4];
-        const t128::Lane L = t128::lane_setup(smem, l, wave);
-        const int64_t r0 = (int64_t)ti * 128, c0 = (int64_t)tj * 128;
-        const int row0 = ti * 128 + (wave >> 1) * 64, col0 = tj * 128 + (wave & 1) * 64;
-        unsigned char* const staging = smem + wave * 16384;
-        t128::Out o;
-        o.C = o.C2 = A + at.i * p.a_step;
-        o.c_rs = o.c2_rs = p.M;
-        o.row_alpha = nullptr;
-        o.diag_out = nullptr;
-        if (at.i == 0) {
-          t128::copy_offsets(voA, voB, p.K, p.K, l, wave);
-          t128::main_loop<false>(acc, p.K / t128::BK, smem, L, voA, voB, X + r0 * p.K, X + c0 * p.K, count);
-          look();
-          o.beta = kGramA;
-          t128::write_block<false, kThrough, false, kFormScaledF16>(o, ti == tj, acc, staging, row0, col0, l);
-        } else {
-          const bool whole = at.i == sym_count(at.n) - 1, poly = !whole && (at.i < 7 ? at.i % 3 == 1 : at.i == 8), r1 = at.n == 3 && at.i == 7;
-          // operands: A; Q and A; Q and Q A; Q' and Q; Q'' and Q' Q
-          const int sa = poly ? (at.i == 8 ? 6 : at.i - 1) : r1 || (whole && at.n == 2) ? 4 : whole ? 8 : at.i % 3 == 2 ? at.i - 1 : at.i - 2;
-          const int sb = poly ? sa : r1 || (whole && at.n == 2) ? 1 : whole ? 7 : at.i % 3 == 2 ? at.i - 2 : at.i - 1;
-          const bf16_t* const Sa = A + sa * p.a_step;
-          const bf16_t* const Sb = A + sb * p.a_step;
-          t128::copy_offsets(voA, voB, p.M, p.M, l, wave);
-          t128::main_loop<true>(acc, p.M / t128::BK, smem, L, voA, voB, Sa + r0 * p.M, Sb + c0 * p.M, count);
-          look();
-          if (poly) {
-            o.ET = Sa;
-            o.ldet = p.M;
-            o.alpha = p.b * (kGramQ / kGramA);
-            o.beta = p.c * (kGramQ / kGramA / kGramA);
-            o.diag_add = p.a * kGramQ;
-            t128::write_block<true, kThrough, false, kFormPoly>(o, ti == tj, acc, staging, row0, col0, l);
-          } else if (whole) {
-            o.beta = at.n == 2 ? 1.0f / (kGramQ * kGramQ) : 1.0f / (kGramQ * kGramR);
-            o.diag_out = pd;
-            t128::write_block<true, kThrough, false, kFormScaledBf16>(o, ti == tj, acc, staging, row0, col0, l);
-          } else {
-            o.beta = r1 ? kGramR / (kGramQ * kGramQ) : 1.0f / kGramQ;
-            t128::write_block<true, kThrough, false, kFormScaledF16>(o, ti == tj, acc, staging, row0, col0, l);
-          }
-        }
-      } else if constexpr (ES == 128) {
+      if constexpr (ES == 128) {
         f32x4_t acc[4][4];
         uint32_t voA[4], voB[4];
         const bf16_t* const S = op == 0 ? X : A;
@@ -400,7 +298,7 @@ __global__ __launch_bounds__(256, 2) void ns_flow_kernel(FlowArgs p) {
         t128::main_loop_t(acc, p.M / t128::KK_BK, smem, L, voX, voP, X + tj * 128, t128::KK_BK * p.K, P + ti * 128,
                           t128::KK_BK * p.M, count);
         look();
-        const t128::OutT o = {Xn, ld, GROUPS ? 0.0f : p.a, rows_v, cols_v, tall, vec};
+        const t128::OutT o = {Xn, ld, p.a, rows_v, cols_v, tall, vec};
         t128::write_block_t<kThrough>(o, pre, acc, smem + wave * 16384, j0, i0, l);
       } else {
         const int r0 = tj * 64, c0 = ti * 64;
@@ -433,7 +331,7 @@ static int flow_subs(int batch) {
   while (s > 1 && s * batch > 64) s >>= 1;
   return s;
 }
-int flow_counter_words(int batch, int products) { return (kQueues + products * batch * flow_subs(batch)) * kLine; }
+int flow_counter_words(int batch, int steps) { return (kQueues + 3 * steps * batch * flow_subs(batch)) * kLine; }
 
 int launch_ns_flow(const FlowProblem& f, hipStream_t stream) {
   FlowArgs p = {};
@@ -455,15 +353,12 @@ int launch_ns_flow(const FlowProblem& f, hipStream_t stream) {
     p.out.p[i] = f.out[i];
     if (reinterpret_cast<uintptr_t>(f.out[i]) & 15) p.vec = 0;
   }
-  p.groups = f.groups;
-  for (int g = 0; g < kFlowGroups; ++g) p.group[g] = f.group[g];
   // as many workgroups as the largest product has items, in whole rounds of the queues
   const int64_t most = (int64_t)(p.rect_tiles > p.sym_tiles ? p.rect_tiles : p.sym_tiles) * f.batch;
   int grid = 2 * cu_count();
   if (grid > most) grid = (int)(most + kQueues - 1) / kQueues * kQueues;
 #define FM_FLOW(ES, EX) hipLaunchKernelGGL((ns_flow_kernel<ES, EX>), dim3((unsigned)grid), dim3(256), 0, stream, p)
-  if (f.groups) hipLaunchKernelGGL((ns_flow_kernel<128, 128, true>), dim3((unsigned)grid), dim3(256), 0, stream, p);
-  else if (f.edge_x == 64) FM_FLOW(64, 64);
+  if (f.edge_x == 64) FM_FLOW(64, 64);
   else if (f.edge_s == 64) FM_FLOW(64, 128);
   else FM_FLOW(128, 128);
 #undef FM_FLOW

@@ -98,8 +98,6 @@ template <bool F16> __device__ __forceinline__ float elem_to_f32(unsigned short 
 constexpr int kFormPoly = 2;         // fp16, with E: v = alpha E + beta acc, and diag_add more on the diagonal
 constexpr int kFormScaledF16 = 3;    // v = beta acc, rounded to fp16; operands bf16 or fp16
 constexpr int kFormScaledBf16 = 4;   // v = beta acc, rounded to bf16, the diagonal to diag_out; operands fp16
-// ... and the scales its matrices are held at: A = X X^T and Q A, Q = a I + b A + c A^2, the product of two Q
-constexpr float kGramA = 16384.0f, kGramQ = 8192.0f, kGramR = 4096.0f;
 
 // Arguments of the one NT contraction every GEMM-shaped kernel here is an instance of:
 //     acc[i][j] = sum_k A[i][k] * B[j][k]            (A: Ma x Kc, B: Nb x Kc, k contiguous)
@@ -219,8 +217,6 @@ int launch_momentum_nesterov(void* g, void* buf, int dtype, int64_t n, float w_b
 int launch_weight_update(void* p, int p_dtype, const bf16_t* u, int64_t n, float decay_mul,
                          float alpha, hipStream_t stream);
 
-constexpr int kFlowGroups = 2, kFlowSlots = 16;   // of one launch: a group of three steps has ten M x M matrices, of two six
-
 // The Newton-Schulz iteration of a batch in one launch (fm_flow.hip).  M and K are whole multiples of the edges; X
 // holds step 0's iterate and room for `steps` of them, A, P and pdiag for as many.
 struct FlowProblem {
@@ -233,11 +229,8 @@ struct FlowProblem {
   unsigned* counters;                 // flow_counter_words of them, zero
   void* const* out; int64_t ldout;    // rows x cols, X' of the last step or (tall) its transpose
   int rows, cols, tall;
-  // Steps in groups of two or three (0: one by one): an iterate and a diagonal per group, and behind A kFlowSlots matrices for
-  // the products of both groups
-  int groups, group[kFlowGroups];
 };
-int flow_counter_words(int batch, int products);
+int flow_counter_words(int batch, int steps);
 int launch_ns_flow(const FlowProblem& f, hipStream_t stream);
 
 int launch_zero_words(unsigned* p, int n, hipStream_t stream);

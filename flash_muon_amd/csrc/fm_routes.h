@@ -2,8 +2,6 @@
 // host compiler can build it by itself and the rules can be checked without a GPU.
 #pragma once
 #include <stdint.h>
-#include <cmath>
-#include <initializer_list>
 
 namespace fm {
 
@@ -88,77 +86,38 @@ inline bool ns_flow_short_enough(int batch, int m, int k) {
   return k <= 12288 && x <= (x + 1023) / 1024 * 820;
 }
 inline bool ns_flow_chosen(int batch, int m, int k) { return ns_flow_pays(batch, m, k) && ns_flow_short_enough(batch, m, k); }
+// The one-launch iteration has room for the iterates of kFlowSteps steps and the one they begin with, in slots 0 .. kFlowSteps.  More steps take
+// further launches, which go back and forth over the slots: step i of a launch reads slot `from` + i `turn` and leaves the next iterate in
+// the slot behind it (the very last step in the caller's output).  Every launch but the last has to take all kFlowSteps steps: one
+// that went back by more slots than the one before it went forward would leave the workspace.
+constexpr int kFlowSteps = 5;
+struct NsFlowLaunch { int first, steps, from, turn; };   // first: of its steps
+inline NsFlowLaunch ns_flow_launch(int steps, int i) {   // launch i of the (steps + kFlowSteps - 1) / kFlowSteps
+  const int first = i * kFlowSteps, left = steps - first;
+  return NsFlowLaunch{first, left < kFlowSteps ? left : kFlowSteps, i & 1 ? kFlowSteps : 0, i & 1 ? -1 : 1};
+}
 
 // ---- Newton-Schulz steps in groups on the Gram matrix (fm_api.hip) ---------------------------------
-// Whether the steps of m x k matrices, m <= k, run in groups: five or more, of a matrix long enough that it saves time and loses
-// no accuracy (fm_api.hip has both sides of both).
-constexpr int kGroupedSteps = 5;
-inline bool ns_grouped(int m, int k) { return m >= 512 && k >= 2 * (int64_t)m; }
-// How matrices that may run in groups iterate, by T = ceil(m / 128), x = the 128-tiles of X', r = k / m: in one launch one by one
-// (F), in groups in one launch (FG) or in launches per product, padded to 128-tiles (L128) or 256-tiles (L256).  us, measured over 900 sizes; the choice
-// below is 2 % off the fastest of the four on the mean.
-//   F: little work, where 15 products make a shorter chain than 18.  512 x 1024 115 (FG 181, L128 159), 4 of 640 x 2560 225 (251, 259), 768 x 3072 172 (234, 196), 5 of 768 x
-//   1952 262 (278, 284), 1024 x 4096 213 (280, 232), 2 of 1024 x 2752 280 (301, 295), 1408 x 2816 230 (307, 316); but 8 of 512 x 4096 331 (273, 290), 2 of 768 x 3072 245 (253,
-//   222), 768 x 6144 273 (291, 222), 2 of 1024 x 4096 333 (331, 315), 1152 x 4608 332 (329, 273), 1536 x 3072 356 (386, 336).
-enum NsWay { kWayFlow = 0, kWayFlowGroups = 1, kWayGroups128 = 2, kWayGroups256 = 3 };
-inline bool ns_groups_lose(int batch, int T, double r, int64_t x) {
-  if (T > 11 || x > (T <= 6 ? 512 : T == 7 ? 480 : T <= 9 ? 360 : 250)) return false;
-  return r <= (T == 6 && batch == 2 ? 3.5 : T == 7 && x > 400 ? 3.0 : T <= 8 ? 4.1 : T == 9 ? 3.0 : 2.2) || x <= (T <= 5 ? 256 : T == 6 ? 200 : 0);
-}
-//   FG: several matrices of up to 15 tile rows, while the launches' 256-tiles do not fill whole rounds of the CUs (t (t + 1) / 2 of them per matrix and product).  8 of
-//   512 x 4096 273 / 290 in launches, 8 of 768 x 3072 343 / 411, 32 of 768 x 3072 876 / 1101, 8 of 1024 x 2752 475 / 603, 32 of 1024 x 8192 2779 / 3165, 16 of 1408 x
-//   3784 1707 / 2055, 16 of 1664 x 3328 2267 / 2505; but 4 of 1024 x 2752 358 / 333, 4 of 1152 x 4608 500 / 465, 12 of 1536 x 6144 2046 / 1860 (252 tiles), 16 of 1280 x
-//   10240 2689 / 2520, 8 of 1792 x 7168 2139 / 1846; few of a very long k, which launches cut along it (5 of 1024 x 62008 3427 / 2938).
-inline bool ns_groups_flow(int batch, int T, double r, int64_t x) {
-  if (batch < 3 || T > 15 || (batch < 8 && r > 40.0)) return false;
-  const int t = (T + 1) / 2, n = batch * t * (t + 1) / 2, rounds = (n + 255) / 256;
-  const double full = n / (256.0 * rounds);   // of the 256-tiles' rounds
-  switch (T) {
-    case 4: case 5: return batch >= 5;
-    case 6: return batch >= 4;
-    case 7: return true;
-    case 8: return batch >= 7 || (batch >= 5 && x >= 1100);
-    case 9: return batch >= 5;
-    case 10: return batch >= 5 && (batch < 16 || r <= 3.0);
-    case 11: return batch >= 4;
-    case 12: return batch == 4 || batch == 6 || (batch == 8 && r <= 3.0) || (n > 256 && full < 0.83 && r <= 5.0);
-    case 13: return r <= 5.0 || batch <= 6;
-    case 14: return batch == 3 || (batch == 4 && r <= 3.5) || (n > 256 && full < 0.7);
-    default: return batch <= 4 || (n > 256 && full < 0.77 && r <= 4.1);
-  }
-}
-//   L256 rather than L128, for odd T: 640 x 1720 194 / 219, 1152 x 4608 273 / 298, 16 of 1664 x 13312 5248 / 5927, 8 of 2113 x 8448 .97, 4 of 2432 x 9728 .84; but 3 of 640 x
-//   1720 1.12, 1408 x 5632 380 / 348, 4 of 1408 x 2816 1.22, 2 of 1920 x 5160 821 / 635, one of 2176 x 7728 1.05, of 2432 x 9728 1.10.
-inline bool ns_groups_on_256(int batch, int m, int k) {
-  const int T = (m + 127) / 128;
-  if (T % 2 == 0 || (T >= 9 && k >= 24 * (int64_t)m)) return true;   // (1664 x 47184, two of them 2290 / 2752)
-  return batch == 1 ? T <= 9 || T >= 23 : T >= 17 || (T >= 13 && batch >= 5);
-}
-inline NsWay ns_grouped_way(int batch, int m, int k) {
-  const int T = (m + 127) / 128;
-  const int64_t x = (int64_t)batch * T * (((int64_t)k + 127) / 128);
-  const double r = (double)k / m;
-  if (ns_groups_lose(batch, T, r, x)) return kWayFlow;
-  if (ns_groups_flow(batch, T, r, x)) return kWayFlowGroups;
-  return ns_groups_on_256(batch, m, k) ? kWayGroups256 : kWayGroups128;
-}
-// steps of the group that begins with step s: three, and two where one step would be left at the end
-inline int ns_group(int steps, int s) { return steps - s == 2 || steps - s == 4 ? 2 : 3; }
+// Whether the steps of M x K matrices, as they lie in the workspace, run in groups: five or more, of a matrix long enough that it
+// saves time and loses no accuracy (fm_api.hip has both sides of both).
+inline bool ns_grouped(int M, int K, int steps) { return steps >= 5 && M >= 512 && K >= 2 * (int64_t)M; }
+// steps of the group that begins with step s: three, then two at a time
+inline int ns_group(int steps, int s) { return s == 0 ? 3 : steps - s >= 2 ? 2 : 1; }
 // Whether the coefficients keep the M x M matrices inside fp16's range at the scales they are held at (2^14 A and Q A, 2^13 Q, 2^12 Q_2 Q_1),
 // with half of it to spare for A.  The singular values of X lie in [0, top]: top starts at 1 (the Frobenius norm) and becomes
 // the largest value of sigma q(sigma^2), a hundredth on top for the roundings.  (3.4445, -4.775, 2.0315): top <= 1.22, q <= 3.45.
-inline bool ns_groups_fit(int steps, float fa, float fb, float fc) {
-  const double a = fa, b = fb, c = fc;
+inline bool ns_groups_fit(int steps, float a, float b, float c) {
   double top = 1.01;
   for (int s = 0; s < steps; ++s) {
-    const double end = top * top;   // q over [0, end] and sqrt(l) q(l) take their extremes there or where their derivatives vanish
-    auto q = [&](double l) { const double v = a + b * l + c * l * l; return v < 0 ? -v : v; };
-    const double turn = -b / (2.0 * c), root = std::sqrt(9.0 * b * b - 20.0 * a * c);   // (no number where there is none)
-    if (!(q(0.0) <= 3.7 && q(end) <= 3.7) || (turn > 0.0 && turn < end && !(q(turn) <= 3.7))) return false;
-    double next = top * q(end);
-    for (const double l : {(-3.0 * b + root) / (10.0 * c), (-3.0 * b - root) / (10.0 * c), -a / (3.0 * b)})
-      if (l > 0.0 && l < end && std::sqrt(l) * q(l) > next) next = std::sqrt(l) * q(l);
-    if (!(end <= 2.0 && top * next <= 2.0)) return false;
+    double next = 0.0;
+    for (int i = 0; i <= 256; ++i) {
+      const double x = top * i / 256.0;
+      double q = a + b * x * x + c * x * x * x * x;
+      q = q < 0 ? -q : q;
+      if (!(q <= 3.7)) return false;
+      if (x * q > next) next = x * q;
+    }
+    if (top * top > 2.0 || top * next > 2.0) return false;
     top = 1.01 * next;
   }
   return true;

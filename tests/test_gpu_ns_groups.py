@@ -96,8 +96,8 @@ def test_in_one_launch(rows, cols, batch, dtype):
     assert all(torch.equal(again[i], got[0]) for i in range(batch))   # whatever workgroup draws what and when
 
 
-@pytest.mark.parametrize("steps", [4, 5, 6, 7, 8, 11])
-@pytest.mark.parametrize("batch", [1, 8])   # in launches per product, in one launch per two groups
+@pytest.mark.parametrize("steps", [4, 5, 6, 7, 8, 10, 11, 16])
+@pytest.mark.parametrize("batch", [1, 8])   # both in one launch per five steps
 def test_step_counts(steps, batch):
     G = _inputs(1300, 2700, torch.bfloat16, 3)
     got = fast_newtonschulz(G.expand(batch, *G.shape).contiguous() if batch > 1 else G, steps).view(batch, *G.shape)

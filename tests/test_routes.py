@@ -18,8 +18,9 @@ int syrk_copy_pays(int M, int K, int half) { return fm::syrk_copy_pays(M, K, hal
 int scale_cast_d_on_tiles(long long r, long long c) { return fm::scale_cast_d_on_tiles(r, c); }
 int scale_cast_t_on_128(long long tiles) { return fm::scale_cast_t_on_128(tiles); }
 int ns_flow_chosen(int batch, int m, int k) { return fm::ns_flow_chosen(batch, m, k); }
-int ns_grouped(int m, int k) { return fm::ns_grouped(m, k); }
-int ns_grouped_way(int batch, int m, int k) { return fm::ns_grouped_way(batch, m, k); }
+void ns_flow_launch(int steps, int i, int* out) { const fm::NsFlowLaunch n = fm::ns_flow_launch(steps, i); out[0] = n.first; out[1] = n.steps; out[2] = n.from; out[3] = n.turn; }
+int ns_flow_slots() { return fm::kFlowSteps + 1; }
+int ns_grouped(int M, int K, int steps) { return fm::ns_grouped(M, K, steps); }
 int ns_group(int steps, int s) { return fm::ns_group(steps, s); }
 int ns_groups_fit(int steps, float a, float b, float c) { return fm::ns_groups_fit(steps, a, b, c); }
 }
@@ -148,15 +149,31 @@ def test_a_knob_leads_every_product_to_the_schedules_it_speaks_of(lib, knobs, na
     assert lib.fm_syrk_workspace_bytes(1152, 4096) == lib.fm_gemm_workspace_bytes(1152, 1152)
 
 
-@pytest.mark.parametrize("steps,groups", [(5, [3, 2]), (6, [3, 3]), (7, [3, 2, 2]), (8, [3, 3, 2]), (13, [3, 3, 3, 2, 2])])
+@pytest.mark.parametrize("steps", range(1, 65))
+def test_the_one_launch_iteration_stays_in_its_slots(routes, steps):
+    """Every iterate that a launch reads or leaves behind lies in the workspace, each launch begins where the one before it
+    left off, and what it leaves there is not one that it still reads."""
+    done, at, i, out = 0, 0, 0, (ctypes.c_int * 4)()
+    while done < steps:
+        routes.ns_flow_launch(steps, i, out)
+        first, n, slot, turn = out
+        assert first == done and slot == at and n >= 1 and abs(turn) == 1
+        done, at, i = done + n, at + n * turn, i + 1
+        written = [slot + turn * s for s in range(1, n + (done < steps))]   # the last step of all writes the caller's output
+        assert all(0 <= s < routes.ns_flow_slots() for s in [slot] + written)
+        assert len(set([slot] + written)) == 1 + len(written)
+    assert done == steps
+
+
+@pytest.mark.parametrize("steps,groups", [(5, [3, 2]), (6, [3, 2, 1]), (7, [3, 2, 2]), (8, [3, 2, 2, 1]), (13, [3, 2, 2, 2, 2, 2])])
 def test_groups_of_steps_add_up(routes, steps, groups):
     s, got = 0, []
     while s < steps:
         got.append(routes.ns_group(steps, s))
         s += got[-1]
     assert got == groups
-    assert not routes.ns_grouped(511, 16384) and not routes.ns_grouped(1024, 2047)
-    assert routes.ns_grouped(512, 1024) and routes.ns_grouped(1 << 29, 1 << 30) and not routes.ns_grouped((1 << 30) + 1, 2 ** 31 - 1)
+    assert not routes.ns_grouped(4096, 16384, 4) and not routes.ns_grouped(511, 16384, 5) and not routes.ns_grouped(1024, 2047, 5)
+    assert routes.ns_grouped(512, 1024, 5) and routes.ns_grouped(1 << 20, 1 << 30, 5)
 
 
 # (coefficients, whether A, Q A, Q and Q Q stay inside fp16 at their scales for every number of steps)
@@ -177,18 +194,3 @@ def test_coefficients_whose_matrices_fit_fp16(routes, coeffs, fit):
             assert max(t * t for t in x) * 2 ** 14 < 65504 and max(abs(t * s) for t, s in zip(x, y)) * 2 ** 14 < 65504
             assert max(abs(s) for s in q) * 2 ** 13 < 65504 and max(abs(s) for s in q) ** 2 * 2 ** 12 < 65504
             x = y
-
-
-# (batch, m, k, us one by one in one launch, in groups in one launch, in groups in launches per product on 128- and on 256-tiles), measured
-GROUP_TIMES = [(1, 512, 1024, 115, 181, 159, 163), (4, 640, 2560, 225, 251, 259, 274), (1, 1024, 4096, 213, 280, 232, 232), (1, 1408, 2816, 230, 307, 316, 340),
-               (8, 512, 4096, 331, 273, 290, 293), (2, 768, 3072, 245, 253, 222, 224), (1, 768, 6144, 273, 291, 222, 221), (8, 1024, 2752, 590, 475, 603, 603),
-               (16, 768, 3072, 683, 508, 679, 673), (32, 1024, 8192, 5066, 2779, 3165, 3178), (16, 1408, 3784, 2412, 1707, 2055, 2366),
-               (4, 1024, 2752, 428, 358, 333, 333), (12, 1536, 6144, 3210, 2046, 1866, 1860), (16, 1280, 10240, 5007, 2689, 2520, 2523),
-               (1, 640, 5120, 207, 258, 225, 214), (1, 1152, 4608, 332, 329, 298, 273), (16, 1664, 13312, 10303, 5433, 5927, 5248), (1, 1408, 5632, 430, 409, 348, 380),
-               (4, 1408, 2816, 572, 508, 526, 644), (2, 1920, 5160, 856, 695, 635, 821), (5, 1024, 62008, 7626, 3427, 2938, 2927)]
-
-
-@pytest.mark.parametrize("batch,m,k,flow,flow_groups,groups128,groups256", GROUP_TIMES)
-def test_long_matrices_iterate_the_way_that_measured_fastest(routes, batch, m, k, flow, flow_groups, groups128, groups256):
-    times = (flow, flow_groups, groups128, groups256)
-    assert times[routes.ns_grouped_way(batch, m, k)] <= 1.02 * min(times)
