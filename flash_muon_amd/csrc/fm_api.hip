@@ -425,55 +425,6 @@ size_t fm_newtonschulz_workspace_bytes(int rows, int cols) {
   return fm_newtonschulz_batched_workspace_bytes(1, rows, cols);
 }
 
-// ---- several Newton-Schulz steps on the Gram matrix ----------------------------------------------
-// A step multiplies X by Q = a I + b A + c A^2 with A = X X^T, and the next step's A is Q A Q: n steps are one
-// product X' = R X with R = Q_n ... Q_1, and what leads to R are products of M x M matrices that commute, symmetric all
-// of them, so that half of their tiles are computed.  Five steps of an M x K matrix take, in units of 2 M^3 flops and with
-// r = K / M, 7.5 r + 2.5 one by one and 3 r + 7 as three and two: 4096 x 16384 32.5 and 19, 4096 x 11008 22.7 and 15.
-//   M x M matrices are held in fp16, scaled by powers of two that fill its range (ns_groups_fit
-// bounds their norms), R of a whole group in bf16 with its diagonal in fp32, as P is: 11 bits instead of 8 where the steps one
-// by one round A and P, and two roundings of the iterate instead of five.  The error of five steps against 64 bits, one by
-// one / as three and two: gradients of 2048 x 5504 6.4e-3 / 3.6e-3, of 768 x 3072 8.1e-3 / 4.4e-3, and lower too for 21 other kinds
-// of spectra from M = 512 and K = 2 M on, but one (columns scaled over three decades, 1024 x 2048 6.8e-3 / 7.3e-3).
-// In bf16 the same chain loses (rows with a common part, 256 x 1024: 7.4e-3 / 5.0e-2), and so do all five steps as one
-// (2.0e-2 on gradients) and squarer matrices (columns as above, 2048^2: 5.9e-3 / 7.7e-3), which would gain no time either.
-constexpr float kGramA = 16384.0f, kGramQ = 8192.0f, kGramR = 4096.0f;   // scales of A and Q A, of Q, of Q_2 Q_1
-// A of a group, at scale kGramA (fp16), to the product of the group's n factors, in A (bf16, its diagonal to pdiag).  Q, V and W:
-// room for one more matrix each (stride bs_q, bs_vw between matrices).
-static int launch_gram_chain(int n, bf16_t* A, bf16_t* Q, int64_t mm, bf16_t* V, bf16_t* W, int64_t bs_vw, float* pdiag, int64_t bs_diag,
-                             int M, int batch, float a, float b, float c, void* gws, size_t gws_bytes, hipStream_t hs) {
-  struct Mat { bf16_t* p; int64_t bs; };
-  const Mat mA = {A, mm}, mQ = {Q, mm}, mV = {V, bs_vw}, mW = {W, bs_vw};
-  auto product = [&](Mat x, Mat y, Mat out, int form, float scale) -> int {   // symmetric, of two that commute
-    GemmArgs g = {};
-    g.A = x.p; g.bs_a = x.bs; g.B = y.p; g.bs_b = y.bs; g.lda = g.ldb = M;
-    g.C = g.C2 = out.p; g.bs_c = g.bs_c2 = out.bs; g.c_rs = g.c2_rs = M; g.c_cs = g.c2_cs = 1;
-    g.Ma = g.Nb = g.Kc = M; g.symmetric = 1; g.batch = batch; g.elem = kElemF16;
-    g.form = form; g.beta = scale;
-    if (form == kFormPoly) {   // scale (a I + b A + c A A)
-      g.E = g.ET = x.p; g.lde = g.ldet = M; g.bs_e = g.bs_et = x.bs;
-      g.alpha = scale * b / kGramA; g.beta = scale * c / (kGramA * kGramA); g.diag_add = scale * a;
-    }
-    if (form == kFormScaledBf16) { g.diag_out = pdiag; g.bs_do = bs_diag; }
-    return launch_gemm_nt(g, gws, gws_bytes, hs);
-  };
-  Mat R = mV;        // the product of the factors so far
-  float r = kGramQ;  // its scale
-  int rc = product(mA, mA, R, kFormPoly, kGramQ);
-  for (int i = 1; i < n && rc == 0; ++i) {
-    const Mat q = i == 1 ? mV : mQ;   // the factor before, which A moves on by
-    rc = product(q, mA, mW, kFormScaledF16, 1.0f / kGramQ);
-    if (rc == 0) rc = product(q, mW, mA, kFormScaledF16, 1.0f / kGramQ);
-    if (rc == 0 && i > 1) {           // (behind the use of W)
-      rc = product(mQ, R, mW, kFormScaledF16, kGramR / (kGramQ * r));
-      R = mW;
-      r = kGramR;
-    }
-    if (rc == 0) rc = product(mA, mA, mQ, kFormPoly, kGramQ);
-  }
-  return rc ? rc : product(mQ, R, mA, kFormScaledBf16, 1.0f / (kGramQ * r));
-}
-
 // the momentum update that comes before: of g and buf, one of which is G
 struct NsMomentum { void* const* g; void* const* buf; float w_buf, w_nes; int nesterov; };
 
@@ -604,44 +555,31 @@ static int ns_impl(const void* const* G, int dtype, int batch, int rows, int col
   // for the copy out of the padded one).
   bool cut_out = padded && rows % 128 == 0 && cols % 128 == 0 && ldout % 8 == 0 && ldout < (1 << 21);
   for (int i = 0; i < batch; ++i) cut_out = cut_out && (reinterpret_cast<uintptr_t>(out[i]) & 15) == 0;
-  const bool grouped = !any_knob_set() && ns_grouped(M, K, steps) && ns_groups_fit(steps, a, b, c);
-  int turn = 0;   // which pair of iterates holds X
-  for (int s = 0; s < steps;) {
-    const int n = grouped ? ns_group(steps, s) : 1;
-    const bool last = s + n == steps;
-    turn ^= 1;
-    bf16_t* Xn = reinterpret_cast<bf16_t*>(w + l.x[turn]);
-    bf16_t* XTn = reinterpret_cast<bf16_t*>(w + l.xt[turn]);
-    const bf16_t* factor = P;   // what X' = (a + pdiag) X + factor X multiplies X with
+  for (int s = 0; s < steps; ++s) {
+    const bool last = s + 1 == steps;
+    bf16_t* Xn = reinterpret_cast<bf16_t*>(w + l.x[(s + 1) & 1]);
+    bf16_t* XTn = reinterpret_cast<bf16_t*>(w + l.xt[(s + 1) & 1]);
     GemmArgs g = {};
     // A = X X^T
     g.A = g.B = X; g.lda = g.ldb = K; g.bs_a = g.bs_b = mk;
     g.C = g.C2 = A; g.c_rs = g.c2_rs = M; g.c_cs = g.c2_cs = 1; g.bs_c = g.bs_c2 = mm;
     g.Ma = g.Nb = M; g.Kc = K; g.beta = 1.0f; g.symmetric = 1; g.batch = batch;
-    if (n > 1) { g.form = kFormScaledF16; g.beta = kGramA; }
     if (launch_gemm_nt(g, gws, gws_bytes, hs)) return FM_ERR_LAUNCH;
-    if (n == 1) {
-      // P = b A + c A A, diagonal in fp32
-      g = GemmArgs{};
-      g.A = g.B = g.E = g.ET = A; g.lda = g.ldb = g.lde = g.ldet = M;
-      g.bs_a = g.bs_b = g.bs_e = g.bs_et = mm;
-      g.C = g.C2 = P; g.c_rs = g.c2_rs = M; g.c_cs = g.c2_cs = 1; g.bs_c = g.bs_c2 = mm;
-      g.Ma = g.Nb = g.Kc = M; g.alpha = b; g.beta = c; g.symmetric = 1; g.batch = batch;
-      g.diag_out = pdiag; g.bs_do = (int64_t)l.pdiag_stride;
-      if (launch_gemm_nt(g, gws, gws_bytes, hs)) return FM_ERR_LAUNCH;
-    } else {
-      // (the iterate that is written next is free until then: two more M x M matrices, since K >= 2 M)
-      if (launch_gram_chain(n, A, P, mm, Xn, Xn + mm, mk, pdiag, (int64_t)l.pdiag_stride, M, batch, a, b, c, gws, gws_bytes, hs))
-        return FM_ERR_LAUNCH;
-      factor = A;
-    }
+    // P = b A + c A A, diagonal in fp32
+    g = GemmArgs{};
+    g.A = g.B = g.E = g.ET = A; g.lda = g.ldb = g.lde = g.ldet = M;
+    g.bs_a = g.bs_b = g.bs_e = g.bs_et = mm;
+    g.C = g.C2 = P; g.c_rs = g.c2_rs = M; g.c_cs = g.c2_cs = 1; g.bs_c = g.bs_c2 = mm;
+    g.Ma = g.Nb = g.Kc = M; g.alpha = b; g.beta = c; g.symmetric = 1; g.batch = batch;
+    g.diag_out = pdiag; g.bs_do = (int64_t)l.pdiag_stride;
+    if (launch_gemm_nt(g, gws, gws_bytes, hs)) return FM_ERR_LAUNCH;
     // X' = (a + diag) X + P X, and its transpose; the last step writes the caller's orientation only
     g = GemmArgs{};
-    g.A = factor; g.lda = M; g.bs_a = mm;
+    g.A = P; g.lda = M; g.bs_a = mm;
     g.B = XT; g.ldb = M; g.bs_b = mk;
     g.E = X; g.lde = K; g.bs_e = mk;
     g.ET = XT; g.ldet = M; g.bs_et = mk;
-    g.Ma = M; g.Nb = K; g.Kc = M; g.alpha = n > 1 ? 0.0f : a; g.beta = 1.0f; g.symmetric = 0; g.batch = batch;
+    g.Ma = M; g.Nb = K; g.Kc = M; g.alpha = a; g.beta = 1.0f; g.symmetric = 0; g.batch = batch;
     g.row_alpha = pdiag; g.bs_ra = (int64_t)l.pdiag_stride;
     g.c_cs = g.c2_cs = 1;
     if (!last) {
@@ -660,7 +598,6 @@ static int ns_impl(const void* const* G, int dtype, int batch, int rows, int col
     if (last && cut_out) { g.rows_v = tall ? cols : rows; g.cols_v = tall ? rows : cols; }
     if (launch_gemm_nt(g, gws, gws_bytes, hs)) return FM_ERR_LAUNCH;
     X = Xn; XT = XTn;
-    s += n;
   }
   if (padded && !cut_out) {
     bf16_t* o[kMaxBatch];

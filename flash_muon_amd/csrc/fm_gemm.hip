@@ -232,8 +232,7 @@ int launch_gemm_nt(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) {
     const int rc = launch_gemm_fast(a, ws, ws_bytes, stream);
     if (rc != kErrWorkspace) return rc;
   }
-  if (gemm_mid_eligible(a) && (knob(kKnobNoMid) <= 0 || a.form)) return launch_gemm_mid(a, ws, ws_bytes, stream);
-  if (a.form) return (int)hipErrorInvalidValue;   // (the general path has none of the forms)
+  if (gemm_mid_eligible(a) && knob(kKnobNoMid) <= 0) return launch_gemm_mid(a, ws, ws_bytes, stream);
   return launch_gemm_general(a, stream);
 }
 

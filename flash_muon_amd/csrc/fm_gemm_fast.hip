@@ -194,20 +194,12 @@ __device__ __forceinline__ void stage16(f32x4_t (&acc)[NA][8], Frag16<NA>& f0, F
 // fragments, read once more rather than picked from the six at the cost of vector instructions
 // among the MFMAs).  Both operands are the one 256-row panel, which goes round the three A slots
 // (8 copies per wave and stage, issued two stages ahead); the B slots are idle.
-// MIXED: of the product of two matrices, which has a row panel and a column panel.  The row panel goes round
-// the A slots as above, the column panel round the B slots, its copies for the stage two ahead behind the
-// barrier of a stage (0.9 of a stage to land); a triangle wave reads 4 + 4 fragments.  4096^2, one matrix: 256
-// items in one round take 71 us, 136 whole tiles on as many CUs 96.
 struct DFrag { bf16x8_t f[8]; };   // triangle waves: rows 32q of their square; the others: 2 row, 4 column fragments and the ninth tile's two
 struct DFragAddr { uint32_t lo[8][4], hi[8][4]; };   // A slots 0 and 1 / A slot 2
 
-// whether fragment q of a MIXED item comes from the column panel
-__host__ __device__ constexpr bool d_col(bool tri, int q) { return tri ? q >= 4 : (q >= 2 && q != 6); }
-
-template <int ASLOT, int BSLOT, bool COL>
+template <int ASLOT>
 __device__ __forceinline__ bf16x8_t read_d(const unsigned char* smem, const DFragAddr& fa, int q, int ks) {
-  if constexpr (COL) return *reinterpret_cast<const bf16x8_t*>(smem + fa.lo[q][ks] + BSLOT * OPER_BYTES);
-  else if constexpr (ASLOT == 2) return *reinterpret_cast<const bf16x8_t*>(smem + fa.hi[q][ks]);
+  if constexpr (ASLOT == 2) return *reinterpret_cast<const bf16x8_t*>(smem + fa.hi[q][ks]);
   else return *reinterpret_cast<const bf16x8_t*>(smem + fa.lo[q][ks] + ASLOT * OPER_BYTES);
 }
 
@@ -218,30 +210,23 @@ __host__ __device__ constexpr int tri_c(int i, int j) { return i < 3 ? j : (j < 
 __host__ __device__ constexpr int tri_i(int q) { return q < 2 ? q : q < 5 ? 2 : 3; }
 __host__ __device__ constexpr int tri_j(int q) { return q < 2 ? q : q < 5 ? q - 2 : q - 5; }
 
-// the 9 MFMAs of one substep, with the fragment reads of `ks_next` of slots RSLOT, BSLOT riding on the
-// first ones and copies Q0 .. Q1-1 of the panel two stages ahead on the later ones, or (COPYB) all 8 of the
-// column panel.
-template <bool F16, bool TRI, bool MIXED, int RSLOT, int BSLOT, int Q0, int Q1, int CSLOT, bool COPYB, bool FIRST>
+// the 9 MFMAs of one substep, with the fragment reads of `ks_next` of slot RSLOT riding on the
+// first ones and copies Q0 .. Q1-1 of the panel two stages ahead on the later ones.
+template <bool F16, bool TRI, int RSLOT, int Q0, int Q1, int CSLOT, bool FIRST>
 __device__ __forceinline__ void dsubstep(f32x16_t (&acc)[3][4], const DFrag& cur, DFrag& nxt, const unsigned char* smem,
                                          const DFragAddr& fa, int ks_next, const uint32_t (&vo)[8], const bf16_t* gP,
                                          uint32_t ldsw) {
-  constexpr int NM = 9, NRD = TRI && !MIXED ? 4 : 8;
+  constexpr int NM = 9, NRD = TRI ? 4 : 8;
   constexpr int C0 = 5, CSTEP = 1;   // copies after MFMA 5, 6, 7
 #pragma unroll
   for (int q = 0; q < NM; ++q) {
-    if (q < NRD) {
-      if (MIXED && d_col(TRI, q)) nxt.f[q] = read_d<RSLOT, BSLOT, true>(smem, fa, q, ks_next);
-      else nxt.f[q] = read_d<RSLOT, BSLOT, false>(smem, fa, q, ks_next);
-    }
-    if constexpr (COPYB) {
-      if (q > 0) dma16o(vo[q > 0 ? q - 1 : 0], gP, ldsw, b_slot_off(CSLOT) + (q - 1) * 4096);
-    } else if (q >= C0 && (q - C0) % CSTEP == 0 && Q0 + (q - C0) / CSTEP < Q1) {
+    if (q < NRD) nxt.f[q] = read_d<RSLOT>(smem, fa, q, ks_next);
+    if (q >= C0 && (q - C0) % CSTEP == 0 && Q0 + (q - C0) / CSTEP < Q1)
       dma16o(vo[Q0 + (q - C0) / CSTEP], gP, ldsw, a_slot_off(CSLOT) + (Q0 + (q - C0) / CSTEP) * 4096);
-    }
     const f32x16_t zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     if constexpr (TRI) {
       f32x16_t& c = acc[tri_r(tri_i(q), tri_j(q))][tri_c(tri_i(q), tri_j(q))];
-      c = mfma_32x32x16<F16>(cur.f[tri_i(q)], cur.f[tri_j(q) + (MIXED ? 4 : 0)], FIRST ? zero : c);
+      c = mfma_32x32x16<F16>(cur.f[tri_i(q)], cur.f[tri_j(q)], FIRST ? zero : c);
     } else if (q < 8) {
       f32x16_t& c = acc[q >> 2][q & 3];
       c = mfma_32x32x16<F16>(cur.f[q >> 2], cur.f[2 + (q & 3)], FIRST ? zero : c);
@@ -252,29 +237,19 @@ __device__ __forceinline__ void dsubstep(f32x16_t (&acc)[3][4], const DFrag& cur
   }
 }
 
-// one k stage of the panel in A slot ASLOT (and of the column panel in B slot BSLOT)
-template <bool F16, bool TRI, bool MIXED, int ASLOT, int BSLOT, bool FIRST>
+// one k stage of the panel in A slot ASLOT
+template <bool F16, bool TRI, int ASLOT, bool FIRST>
 __device__ __forceinline__ void dstage(f32x16_t (&acc)[3][4], DFrag& f0, DFrag& f1, const unsigned char* smem,
-                                       const DFragAddr& fa, const uint32_t (&vo)[8], const uint32_t (&voB)[8], const bf16_t* nP,
-                                       const bf16_t* nB, uint32_t ldsw) {
+                                       const DFragAddr& fa, const uint32_t (&vo)[8], const bf16_t* nP, uint32_t ldsw) {
   constexpr int AFREE = (ASLOT + 2) % 3, ANEXT = (ASLOT + 1) % 3;
-  dsubstep<F16, TRI, MIXED, ASLOT, BSLOT, 0, 3, AFREE, false, FIRST>(acc, f0, f1, smem, fa, 1, vo, nP, ldsw);
-  dsubstep<F16, TRI, MIXED, ASLOT, BSLOT, 3, 6, AFREE, false, false>(acc, f1, f0, smem, fa, 2, vo, nP, ldsw);
-  dsubstep<F16, TRI, MIXED, ASLOT, BSLOT, 6, 8, AFREE, false, false>(acc, f0, f1, smem, fa, 3, vo, nP, ldsw);
+  dsubstep<F16, TRI, ASLOT, 0, 3, AFREE, FIRST>(acc, f0, f1, smem, fa, 1, vo, nP, ldsw);
+  dsubstep<F16, TRI, ASLOT, 3, 6, AFREE, false>(acc, f1, f0, smem, fa, 2, vo, nP, ldsw);
+  dsubstep<F16, TRI, ASLOT, 6, 8, AFREE, false>(acc, f0, f1, smem, fa, 3, vo, nP, ldsw);
   // everybody's copies of the next stage have landed (all but the 8 newest, of the stage after),
-  // and nobody reads the slots that the next copies go to
+  // and nobody reads the slot that the next stage's copies go to
   asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  if constexpr (MIXED) dsubstep<F16, TRI, MIXED, ANEXT, BSLOT ^ 1, 0, 0, BSLOT, true, false>(acc, f1, f0, smem, fa, 0, voB, nB, ldsw);
-  else dsubstep<F16, TRI, MIXED, ANEXT, 0, 0, 0, AFREE, false, false>(acc, f1, f0, smem, fa, 0, vo, nP, ldsw);
+  dsubstep<F16, TRI, ANEXT, 0, 0, AFREE, false>(acc, f1, f0, smem, fa, 0, vo, nP, ldsw);
 }
-
-// ---- the forms of GemmArgs ----------------------------------------------------------------------
-// FORM below is GemmArgs::form where a kernel is built for one of them, and 0 for the products that have none: what
-// the elements of the output are, and whether the product is scaled on the way.
-__host__ __device__ constexpr bool out_f16(bool f16, int form) { return form == kFormScaledF16 || (f16 && form != kFormScaledBf16); }
-__host__ __device__ constexpr bool form_scales(int form) { return form == kFormScaledF16 || form == kFormScaledBf16; }
-// of a kernel with the write-out MODE (below), which is the form where there is one
-__host__ __device__ constexpr int mode_form(bool f16, int mode) { return form_scales(mode) || (f16 && mode == kFormPoly) ? mode : 0; }
 
 // ---- the part of a tile after the main loop -----------------------------------------------------
 // Each wave finishes its 128x128 block a quarter (32 rows x 128 columns, one row of MFMA tiles) at
@@ -415,7 +390,7 @@ __device__ __forceinline__ void direct_e_batch(const GemmArgs& g, float* F, cons
   }
 }
 
-template <bool F16, bool HAS_E, bool DIAG, int FORM = 0>
+template <bool F16, bool HAS_E, bool DIAG>
 __device__ __forceinline__ void epilogue_quarter_t(const GemmArgs& g, float* F, const unsigned char* Eb,
                                                    const float* RA, int ra_off, int row_base, int col_base,
                                                    int lane, int it_begin, int it_end, int passes) {
@@ -445,14 +420,7 @@ __device__ __forceinline__ void epilogue_quarter_t(const GemmArgs& g, float* F, 
 #pragma unroll
         for (int k = 0; k < 8; ++k) v[k] = __builtin_fmaf(al, elem_to_f32<F16>(e.s[k]), beta * v[k]);
       }
-      if constexpr (form_scales(FORM)) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] *= beta;
-      }
-      if constexpr (DIAG && FORM == kFormPoly) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] += row - col == k ? g.diag_add : 0.0f;
-      } else if (DIAG) {                                // selects only: no branch per element
+      if (DIAG) {                                       // selects only: no branch per element
         const int kd = row - col;                       // the diagonal element of this row, if 0..7
         float dv = 0.0f;
 #pragma unroll
@@ -464,7 +432,7 @@ __device__ __forceinline__ void epilogue_quarter_t(const GemmArgs& g, float* F, 
         if (dout && (unsigned)kd < 8u) g.diag_out[row] = dv;
       }
 #pragma unroll
-      for (int k = 0; k < 8; ++k) o.s[k] = f32_to_elem<out_f16(F16, FORM)>(v[k]);
+      for (int k = 0; k < 8; ++k) o.s[k] = f32_to_elem<F16>(v[k]);
       if (g.C) *reinterpret_cast<uint4*>(C + (int64_t)row * g.c_rs + col) = o.v;
     }
   }
@@ -480,26 +448,26 @@ __device__ __forceinline__ void epilogue_quarter_t(const GemmArgs& g, float* F, 
       const float a[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       union { uint4 v; unsigned short s[8]; } o;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) o.s[k] = f32_to_elem<out_f16(F16, FORM)>(form_scales(FORM) ? beta * a[k] : a[k]);
+      for (int k = 0; k < 8; ++k) o.s[k] = f32_to_elem<F16>(a[k]);
       *reinterpret_cast<uint4*>(C2 + (int64_t)col * g.c2_rs + row) = o.v;
     }
   }
 }
 
-template <bool F16, int FORM = 0>
+template <bool F16>
 __device__ __forceinline__ void epilogue_quarter(const GemmArgs& g, bool diag, float* F, const unsigned char* Eb,
                                                  const float* RA, int ra_off, int row_base, int col_base,
                                                  int lane, int it_begin, int it_end, int passes) {
   if (g.E && !block_written(g, row_base, col_base)) return;   // (only products with E leave blocks out)
-  if constexpr (!F16 || FORM == kFormPoly) {   // other fp16 problems carry no operand E
+  if constexpr (!F16) {   // fp16 problems carry no operand E
     if (g.E) {
-      if (diag) epilogue_quarter_t<F16, true, true, FORM>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
-      else epilogue_quarter_t<F16, true, false, FORM>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
+      if (diag) epilogue_quarter_t<false, true, true>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
+      else epilogue_quarter_t<false, true, false>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
       return;
     }
   }
-  if (diag) epilogue_quarter_t<F16, false, true, FORM>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
-  else epilogue_quarter_t<F16, false, false, FORM>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
+  if (diag) epilogue_quarter_t<F16, false, true>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
+  else epilogue_quarter_t<F16, false, false>(g, F, Eb, RA, ra_off, row_base, col_base, lane, it_begin, it_end, passes);
 }
 
 // ---- write-out of a whole tile from the accumulators --------------------------------------------
@@ -557,7 +525,7 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
 }
 
 // MODE: 0 without the operand E, 1 with it and beta == 1 (the product is added as it is), 2 with it
-// and any beta; kFormPoly in fp16 and the scaled forms.  A kernel holds one instance only: of identical element reads in several branches
+// and any beta.  A kernel holds one instance only: of identical element reads in several branches
 // the optimizer makes one read of all 256 accumulators ahead of the branch, and they do not fit
 // into the vector registers.
 // The wave's block is 32 NI rows x 128 columns at (row0, col0).  `diag`: the block has no mirror
@@ -586,13 +554,11 @@ __device__ __forceinline__ void epilogue_regs(const GemmArgs& g, bool diag, int 
   // what follows is derived from `lane` anew for every tile: kept in registers across the main
   // loop instead, the per-lane offsets of the write-out would crowd out the loop's own
   asm volatile("" : "+v"(lane));
-  constexpr bool has_e = MODE == 1 || MODE == 2;
-  constexpr int FORM = mode_form(F16, MODE);
-  constexpr bool OF16 = out_f16(F16, FORM);
+  constexpr bool has_e = !F16 && MODE != 0;
   const int lc = lane & 31, lh = lane >> 5, par = lane & 1;
   const bool direct = g.C != nullptr;
   const bool mirror = g.C2 != nullptr && !diag;
-  const bool dout = (KIND == 1 || (KIND == 0 && diag)) && (FORM == kFormPoly || g.diag_out != nullptr);
+  const bool dout = (KIND == 1 || (KIND == 0 && diag)) && g.diag_out != nullptr;
   const float alpha = g.alpha, beta = g.beta;
   const uint32_t sel = par ? 0x03020706u : 0x05040100u;   // odd lanes keep the high halves, even lanes the low ones
   float* const RA = reinterpret_cast<float*>(T + QT_BYTES);
@@ -676,14 +642,7 @@ __device__ __forceinline__ void epilogue_regs(const GemmArgs& g, bool diag, int 
           v[r] = __builtin_fmaf(al[r >> 2][r & 3], ef, v[r]);
         }
       }
-      if constexpr (form_scales(FORM)) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] *= beta;
-      }
-      if constexpr (DOUT && FORM == kFormPoly) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] += lc == 8 * (r >> 2) + 4 * lh + (r & 3) ? g.diag_add : 0.0f;
-      } else if constexpr (DOUT) {
+      if constexpr (DOUT) {
         float dv = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -697,7 +656,7 @@ __device__ __forceinline__ void epilogue_regs(const GemmArgs& g, bool diag, int 
 #pragma unroll
       for (int qq = 0; qq < 4; ++qq)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) P[qq][h] = pack2<OF16>(v[4 * qq + 2 * h], v[4 * qq + 2 * h + 1]);
+        for (int h = 0; h < 2; ++h) P[qq][h] = pack2<F16>(v[4 * qq + 2 * h], v[4 * qq + 2 * h + 1]);
       if (direct) {   // stage the column of the quarter for the direct output
 #pragma unroll
         for (int qq = 0; qq < 4; ++qq)
@@ -793,14 +752,12 @@ __device__ __forceinline__ void epilogue_regs16(const GemmArgs& g, bool diag, in
   constexpr int NQ = NA / 2;   // quarters: groups of 32 rows
   // derived from `lane` anew for every tile (see epilogue_regs)
   asm volatile("" : "+v"(lane));
-  constexpr bool has_e = MODE == 1 || MODE == 2;
-  constexpr int FORM = mode_form(F16, MODE);
-  constexpr bool OF16 = out_f16(F16, FORM);
+  constexpr bool has_e = !F16 && MODE != 0;
   const int n = lane & 15, grp = lane >> 4;
   const bool written = !has_e || block_written(g, row0, col0);   // (only products with E leave blocks out)
   const bool direct = g.C != nullptr && written;
   const bool mirror = g.C2 != nullptr && !diag && written;
-  const bool dout = diag && (FORM == kFormPoly || g.diag_out != nullptr);
+  const bool dout = diag && g.diag_out != nullptr;
   const float alpha = g.alpha, beta = g.beta;
   float* const RA = reinterpret_cast<float*>(T + QT_BYTES);
   // direct staging: this lane writes rows 8 grp + 4 a + r, the 4 bytes of columns 32 J + 2 n .. + 1, at
@@ -874,22 +831,7 @@ __device__ __forceinline__ void epilogue_regs16(const GemmArgs& g, bool diag, in
               }
           }
         }
-        if constexpr (form_scales(FORM)) {
-#pragma unroll
-          for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-              for (int r = 0; r < 4; ++r) v[a][b][r] *= beta;
-        }
-        if constexpr (DOUT && FORM == kFormPoly) {
-#pragma unroll
-          for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-              for (int r = 0; r < 4; ++r) v[a][b][r] += 2 * n + b == 8 * grp + 4 * a + r ? g.diag_add : 0.0f;
-        } else if constexpr (DOUT) {
+        if constexpr (DOUT) {
           // row 8 grp + 4 a + r meets column 2 n + b: the lanes with n / 4 == grp hold two elements of the
           // diagonal, rows 2 n and 2 n + 1 of the sub-block; they are split off in fp32 and stored as zero
           float dv[2] = {0.0f, 0.0f};
@@ -913,7 +855,7 @@ __device__ __forceinline__ void epilogue_regs16(const GemmArgs& g, bool diag, in
           for (int a = 0; a < 2; ++a)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-              *reinterpret_cast<uint32_t*>(tw + (4 * a + r) * QD_PITCH + 64 * (J ^ grp)) = pack2<OF16>(v[a][0][r], v[a][1][r]);
+              *reinterpret_cast<uint32_t*>(tw + (4 * a + r) * QD_PITCH + 64 * (J ^ grp)) = pack2<F16>(v[a][0][r], v[a][1][r]);
         }
         if (mirror) {
 #pragma unroll
@@ -921,7 +863,7 @@ __device__ __forceinline__ void epilogue_regs16(const GemmArgs& g, bool diag, in
 #pragma unroll
             for (int a = 0; a < 2; ++a)
               *reinterpret_cast<uint2*>(mw + (32 * J + b) * QM_PITCH + 64 * (I & 1) + 8 * a) =
-                  uint2{pack2<OF16>(v[a][b][0], v[a][b][1]), pack2<OF16>(v[a][b][2], v[a][b][3])};
+                  uint2{pack2<F16>(v[a][b][0], v[a][b][1]), pack2<F16>(v[a][b][2], v[a][b][3])};
         }
       };
       if (dout && J == I + dshift) block(std::true_type{});
@@ -1111,61 +1053,40 @@ __device__ __forceinline__ void half_item_at(const GemmArgs& g, int e, int& b, i
 
 // The k loop of a diagonal item for one kind of wave; the copies of the first two stages are in
 // flight and stage 0 has landed everywhere.
-template <bool F16, bool TRI, bool MIXED>
+template <bool F16, bool TRI>
 __device__ __forceinline__ void diag_item_loop(f32x16_t (&acc)[3][4], const unsigned char* smem, const DFragAddr& dfa,
-                                               const uint32_t (&vo)[8], const uint32_t (&voB)[8], const bf16_t* gP, const bf16_t* gB, int n,
-                                               uint32_t ldsw) {
+                                               const uint32_t (&vo)[8], const bf16_t* gP, int n, uint32_t ldsw) {
   const int last = n - 1;
   DFrag f0, f1;
 #pragma unroll
-  for (int q = 0; q < (TRI && !MIXED ? 4 : 8); ++q) {
-    if (MIXED && d_col(TRI, q)) f0.f[q] = read_d<0, 0, true>(smem, dfa, q, 0);
-    else f0.f[q] = read_d<0, 0, false>(smem, dfa, q, 0);
-  }
+  for (int q = 0; q < (TRI ? 4 : 8); ++q) f0.f[q] = read_d<0>(smem, dfa, q, 0);
   // stages past the end are the last stage again (into slots nobody reads), so that the number of
   // copies in flight is the same at every wait
-#define FM_DSTAGE(AS, BS, S, FIRST)                                                                          \
-  {                                                                                                          \
-    const int kn = (S) + 2 < last ? (S) + 2 : last;                                                          \
-    dstage<F16, TRI, MIXED, AS, BS, FIRST>(acc, f0, f1, smem, dfa, vo, voB, gP + kn * BKF, gB + kn * BKF, ldsw); \
+#define FM_DSTAGE(AS, S, FIRST)                                                                \
+  {                                                                                            \
+    const int kn = (S) + 2 < last ? (S) + 2 : last;                                            \
+    dstage<F16, TRI, AS, FIRST>(acc, f0, f1, smem, dfa, vo, gP + kn * BKF, ldsw);              \
   }
-  FM_DSTAGE(0, 0, 0, true)
+  FM_DSTAGE(0, 0, true)
   int s = 1;
-  if constexpr (MIXED) {   // the pair of slots comes round every 6 stages
-    for (; s < n; s += 6) {
-      FM_DSTAGE(1, 1, s, false)
-      if (s + 1 >= n) break;
-      FM_DSTAGE(2, 0, s + 1, false)
-      if (s + 2 >= n) break;
-      FM_DSTAGE(0, 1, s + 2, false)
-      if (s + 3 >= n) break;
-      FM_DSTAGE(1, 0, s + 3, false)
-      if (s + 4 >= n) break;
-      FM_DSTAGE(2, 1, s + 4, false)
-      if (s + 5 >= n) break;
-      FM_DSTAGE(0, 0, s + 5, false)
-    }
-  } else {
-    for (; s + 3 <= n; s += 3) {
-      FM_DSTAGE(1, 0, s, false)
-      FM_DSTAGE(2, 0, s + 1, false)
-      FM_DSTAGE(0, 0, s + 2, false)
-    }
-    if (s < n) {
-      FM_DSTAGE(1, 0, s, false)
-      if (s + 1 < n) FM_DSTAGE(2, 0, s + 1, false)
-    }
+  for (; s + 3 <= n; s += 3) {
+    FM_DSTAGE(1, s, false)
+    FM_DSTAGE(2, s + 1, false)
+    FM_DSTAGE(0, s + 2, false)
+  }
+  if (s < n) {
+    FM_DSTAGE(1, s, false)
+    if (s + 1 < n) FM_DSTAGE(2, s + 1, false)
   }
 #undef FM_DSTAGE
   wait_vmcnt<0>();
   __syncthreads();   // no copy in flight and no wave still reading: LDS is free again
 }
 
-// A diagonal tile (at m0 on the diagonal) of a symmetric product, over n k stages from gP (and gB) on.
+// A diagonal tile (at m0 on the diagonal) of a symmetric product, over n k stages from gP on.
 template <bool F16, int MODE>
 __device__ __forceinline__ void diag_item(const GemmArgs& g, int m0, int n, unsigned char* smem, const uint32_t (&vo)[8],
-                                          const uint32_t (&voB)[8], const bf16_t* gP, const bf16_t* gB, uint32_t ldsw, int lane, int wave) {
-  constexpr bool MIXED = F16 && form_scales(mode_form(F16, MODE));
+                                          const bf16_t* gP, uint32_t ldsw, int lane, int wave) {
   const bool tri = wave < 2;
   DFragAddr dfa;
   int dlane = lane;   // derived anew for every such item instead of being kept across the others
@@ -1177,40 +1098,31 @@ __device__ __forceinline__ void diag_item(const GemmArgs& g, int m0, int n, unsi
                        : (q < 2 ? 64 * (wave - 2) + 32 * q : q < 6 ? 128 + 32 * (q - 2) : 128 * (wave - 2) + 32 * (7 - q));
     const int r = r0 + (dlane & 31);
     const uint32_t o = (uint32_t)(r * ROWB + (((dlane >> 5) ^ swz(r)) << 4));
-    const uint32_t slot0 = MIXED && d_col(tri, q) ? b_slot_off(0) : 0;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
-      dfa.lo[q][ks] = (o ^ (ks << 5)) + slot0;
+      dfa.lo[q][ks] = o ^ (ks << 5);
       dfa.hi[q][ks] = (o ^ (ks << 5)) + a_slot_off(2);
     }
   }
   const int k1 = n - 1 < 1 ? n - 1 : 1;
 #pragma unroll
   for (int q = 0; q < 8; ++q) dma16o(vo[q], gP, ldsw, a_slot_off(0) + q * 4096);
-  if constexpr (MIXED) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) dma16o(voB[q], gB, ldsw, b_slot_off(0) + q * 4096);
-  }
 #pragma unroll
   for (int q = 0; q < 8; ++q) dma16o(vo[q], gP + k1 * BKF, ldsw, a_slot_off(1) + q * 4096);
-  if constexpr (MIXED) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) dma16o(voB[q], gB + k1 * BKF, ldsw, b_slot_off(1) + q * 4096);
-  }
-  wait_vmcnt<MIXED ? 16 : 8>();
+  wait_vmcnt<8>();
   __syncthreads();
   unsigned char* const wave_lds = smem + wave * EPI_WAVE_BYTES;
   // (each kind of wave has accumulators of its own, pinned to their registers before the write-out)
   if (tri) {
     f32x16_t acc[3][4];
-    diag_item_loop<F16, true, MIXED>(acc, smem, dfa, vo, voB, gP, gB, n, ldsw);
+    diag_item_loop<F16, true>(acc, smem, dfa, vo, gP, n, ldsw);
 #pragma unroll
     for (int q = 0; q < 9; ++q) asm volatile("" : "+a"(acc[tri_r(tri_i(q), tri_j(q))][tri_c(tri_i(q), tri_j(q))]));
     const int sq = m0 + 128 * wave;
     epilogue_regs<F16, MODE, 2, 1>(g, false, 0, acc, wave_lds, sq, sq, lane);
   } else {
     f32x16_t acc[3][4];
-    diag_item_loop<F16, false, MIXED>(acc, smem, dfa, vo, voB, gP, gB, n, ldsw);
+    diag_item_loop<F16, false>(acc, smem, dfa, vo, gP, n, ldsw);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1260,7 +1172,7 @@ constexpr int SUB_STAGE = 2 * SUB_OPER;
 constexpr int SUB_DEPTH = 8;
 constexpr int SUB_F_PITCH = 36;               // floats per staged column: 32 rows + 4 of padding
 
-template <bool F16, int FORM = 0>
+template <bool F16>
 __device__ __forceinline__ void sub64_tile(const GemmArgs& g, int ti, int tj, int si, int sj, int nk,
                                            unsigned char* smem, int lane, int wave) {
   const bool tdiag = g.symmetric && ti == tj;
@@ -1368,7 +1280,7 @@ __device__ __forceinline__ void sub64_tile(const GemmArgs& g, int ti, int tj, in
   // a block of a diagonal sub-tile holds its own mirror image (or is one of a pair of blocks that
   // hold each other's, bit for bit): such a sub-tile is written once, by the direct pass
   const bool bdiag = tdiag && si == sj;
-  const bool use_e = FORM == kFormPoly || (!F16 && FORM == 0 && g.E != nullptr);
+  const bool use_e = !F16 && g.E != nullptr;
   const bool written = !use_e || block_written(g, m0, n0);   // (only products with E leave blocks out)
   const bool mirror = !bdiag && g.C2 != nullptr && written;
   {
@@ -1386,14 +1298,7 @@ __device__ __forceinline__ void sub64_tile(const GemmArgs& g, int ti, int tj, in
 #pragma unroll
       for (int k = 0; k < 16; ++k) v[k] = __builtin_fmaf(al, elem_to_f32<F16>(e.h[k]), g.beta * v[k]);
     }
-    if constexpr (form_scales(FORM)) {
-#pragma unroll
-      for (int k = 0; k < 16; ++k) v[k] *= g.beta;
-    }
-    if constexpr (FORM == kFormPoly) {
-#pragma unroll
-      for (int k = 0; k < 16; ++k) v[k] += bdiag && wm == wn && r - c0 == k ? g.diag_add : 0.0f;
-    } else if (bdiag && wm == wn && g.diag_out != nullptr) {   // this block lies on the diagonal of the product
+    if (bdiag && wm == wn && g.diag_out != nullptr) {   // this block lies on the diagonal of the product
       const int kd = r - c0;                            // the diagonal element of this row, if 0..15
       float dv = 0.0f;
 #pragma unroll
@@ -1407,8 +1312,8 @@ __device__ __forceinline__ void sub64_tile(const GemmArgs& g, int ti, int tj, in
     union { uint4 q[2]; unsigned short h[16]; } o;
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
-      o.h[k] = f32_to_elem<out_f16(F16, FORM)>(v[k]);
-      if (mirror) F[(c0 + k) * SUB_F_PITCH + r] = elem_to_f32<out_f16(F16, FORM)>(o.h[k]);
+      o.h[k] = f32_to_elem<F16>(v[k]);
+      if (mirror) F[(c0 + k) * SUB_F_PITCH + r] = elem_to_f32<F16>(o.h[k]);
     }
     if (g.C && written) {
       uint4* dst = reinterpret_cast<uint4*>(reinterpret_cast<unsigned short*>(g.C) + (int64_t)row * g.c_rs + col);
@@ -1420,7 +1325,7 @@ __device__ __forceinline__ void sub64_tile(const GemmArgs& g, int ti, int tj, in
     const int c = lane >> 1, r0 = (lane & 1) * 16;
     union { uint4 q[2]; unsigned short h[16]; } o;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) o.h[k] = f32_to_elem<out_f16(F16, FORM)>(F[c * SUB_F_PITCH + r0 + k]);
+    for (int k = 0; k < 16; ++k) o.h[k] = f32_to_elem<F16>(F[c * SUB_F_PITCH + r0 + k]);
     uint4* dst = reinterpret_cast<uint4*>(reinterpret_cast<unsigned short*>(g.C2) + (int64_t)(col0 + c) * g.c2_rs + row0 + r0);
     dst[0] = o.q[0];
     dst[1] = o.q[1];
@@ -1480,7 +1385,7 @@ __device__ __forceinline__ void whole_tile16(const GemmArgs& g, bool diag, int n
       stage16<F16, NA, AS, BS, FIRST>(acc, f0, f1, smem, fa, voA, voB, gA + kn * BKF, gB + kn * BKF, ldsw);  \
     }
 #define FM_STAGE(AS, BS, S) FM_STAGE_T(AS, BS, S, false)
-    if constexpr (MODE != 1 && MODE != 2) {
+    if constexpr (MODE == 0) {
       // the first stage stands apart: its first MFMAs start the sums from zero
       FM_STAGE_T(0, 0, 0, true)
       int s = 1;
@@ -1575,12 +1480,13 @@ __device__ __forceinline__ void whole_tile16(const GemmArgs& g, bool diag, int n
   }
 }
 
-// MODE: how whole tiles are written out (see epilogue_regs); chosen by the host from E and beta.
-// smem: the operand ring during the main loop (five slots of 32 KiB: A0 A1 B0 B1 A2), the staging of
-// the four waves' write-out afterwards
+// MODE: how whole tiles are written out (see epilogue_regs); chosen by the host from E and beta
 template <bool F16, int MODE, int NI>
-__device__ __forceinline__ void rounds(const FastArgs& p, unsigned char* smem) {
-  constexpr int FORM = mode_form(F16, MODE);
+__global__ __launch_bounds__(256) void gemm_nt_rounds_kernel(FastArgs p) {
+  // the operand ring during the main loop (five slots of 32 KiB: A0 A1 B0 B1 A2), the staging of
+  // the four waves' write-out afterwards
+  __shared__ __align__(1024) unsigned char smem[SMEM_BYTES];
+
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
@@ -1631,7 +1537,7 @@ __device__ __forceinline__ void rounds(const FastArgs& p, unsigned char* smem) {
         int sbi, sti, stj;
         tile_at(p.g, p.rounds * p.grid + (w >> 4), sbi, sti, stj);
         const GemmArgs sg = batch_view(p.g, sbi);
-        sub64_tile<F16, FORM>(sg, sti, stj, (w >> 2) & 3, w & 3, p.nk, smem, lane, wave);
+        sub64_tile<F16>(sg, sti, stj, (w >> 2) & 3, w & 3, p.nk, smem, lane, wave);
         break;
       }
       // The workgroups do not leave the last full round together: the XCDs of one chip differ by
@@ -1661,7 +1567,7 @@ __device__ __forceinline__ void rounds(const FastArgs& p, unsigned char* smem) {
         int sbi, sti, stj;
         tile_at(p.g, p.rounds * p.grid + tile, sbi, sti, stj);
         const GemmArgs sg = batch_view(p.g, sbi);
-        sub64_tile<F16, FORM>(sg, sti, stj, si, sj, p.nk, smem, lane, wave);
+        sub64_tile<F16>(sg, sti, stj, si, sj, p.nk, smem, lane, wave);
         if (t == kNoTickets) break;
       }
       break;
@@ -1693,15 +1599,14 @@ __device__ __forceinline__ void rounds(const FastArgs& p, unsigned char* smem) {
     const bf16_t* gB = g.B + (int64_t)n0 * g.ldb + (int64_t)kb * BKF;
 
     if constexpr (NI == 2) {
-      if (ditem) {   // a diagonal tile of a symmetric product: its panels are rows in their own order
-        uint32_t vo[8], voB[8];
+      if (ditem) {   // a diagonal tile of a symmetric product: its panel is operand B's (A == B), rows in their own order
+        uint32_t vo[8];
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
           const int row = (q * 4 + wave) * 8 + (lane >> 3);
-          vo[q] = (uint32_t)(row * (int)g.lda + (((lane & 7) ^ swz(row)) * 8)) * 2u;
-          voB[q] = (uint32_t)(row * (int)g.ldb + (((lane & 7) ^ swz(row)) * 8)) * 2u;
+          vo[q] = (uint32_t)(row * (int)g.ldb + (((lane & 7) ^ swz(row)) * 8)) * 2u;
         }
-        diag_item<F16, MODE>(g, m0, n, smem, vo, voB, gA, gB, ldsw, lane, wave);
+        diag_item<F16, MODE>(g, m0, n, smem, vo, gB, ldsw, lane, wave);
         __syncthreads();   // the next item's copies land in the memory the staging just used
         continue;
       }
@@ -1733,23 +1638,11 @@ __device__ __forceinline__ void rounds(const FastArgs& p, unsigned char* smem) {
   }
 }
 
-template <bool F16, int MODE, int NI>
-__global__ __launch_bounds__(256) void gemm_nt_rounds_kernel(FastArgs p) {
-  __shared__ __align__(1024) unsigned char smem[SMEM_BYTES];
-  rounds<F16, MODE, NI>(p, smem);
-}
-// the same for the forms of GemmArgs
-template <bool F16, int FORM, int NI>
-__global__ __launch_bounds__(256) void gemm_nt_form_kernel(FastArgs p) {
-  __shared__ __align__(1024) unsigned char smem[SMEM_BYTES];
-  rounds<F16, FORM, NI>(p, smem);
-}
-
 // Second kernel, for the tiles that were not computed whole: one workgroup per (tile, 128x128
 // block, quarter).  Its four waves add the tile's parts in k order, so the bits do not depend on
 // which workgroup finished when, into one staging buffer, and then share the iterations of the
 // same epilogue the main kernel runs.
-template <bool F16, int FORM>
+template <bool F16>
 __global__ __launch_bounds__(256) void gemm_nt_reduce_kernel(FastArgs p) {
   __shared__ __align__(1024) unsigned char smem[EPI_WAVE_BYTES];
   __shared__ int s_slot[kMaxParts];
@@ -1788,9 +1681,9 @@ __global__ __launch_bounds__(256) void gemm_nt_reduce_kernel(FastArgs p) {
   __syncthreads();
   const bool diag = g.symmetric && ti == tj;
   // direct pass, then (after everybody has put its rounded values back) the transposed pass
-  epilogue_quarter<F16, FORM>(g, diag, L.F, L.E[0], L.RA, 32 * q, row0 + 32 * q, col0, lane, wave * 2, wave * 2 + 2, 1);
+  epilogue_quarter<F16>(g, diag, L.F, L.E[0], L.RA, 32 * q, row0 + 32 * q, col0, lane, wave * 2, wave * 2 + 2, 1);
   __syncthreads();
-  epilogue_quarter<F16, FORM>(g, diag, L.F, L.E[0], L.RA, 32 * q, row0 + 32 * q, col0, lane, wave * 2, wave * 2 + 2, 2);
+  epilogue_quarter<F16>(g, diag, L.F, L.E[0], L.RA, 32 * q, row0 + 32 * q, col0, lane, wave * 2, wave * 2 + 2, 2);
 }
 
 // ---- 128x128 tiles, one per workgroup, for problems too small for the rounds above --------------
@@ -1817,7 +1710,7 @@ struct MidSplit {
 };
 constexpr int MID_PART_FLOATS = MID_T * MID_T;   // one fp32 partial tile: 64 KiB
 
-template <bool F16, int FORM>
+template <bool F16>
 __global__ __launch_bounds__(256) void gemm_nt_mid_kernel(GemmArgs gb, MidSplit sp) {
   __shared__ __align__(1024) unsigned char smem[MID_SMEM];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1841,7 +1734,7 @@ __global__ __launch_bounds__(256) void gemm_nt_mid_kernel(GemmArgs gb, MidSplit 
   const int row0 = m0 + wave * 32, col0 = n0;
 
   // the epilogue operand and the per-row additions first: they are long there when needed
-  const bool use_e = (!F16 || FORM == kFormPoly) && g.E != nullptr && sp.ksplit == 1;
+  const bool use_e = !F16 && g.E != nullptr && sp.ksplit == 1;
   unsigned char* const e_buf = smem + MID_RING + wave * QE_BYTES;
   float ra = 0.0f;
   if (use_e) {
@@ -1965,14 +1858,14 @@ __global__ __launch_bounds__(256) void gemm_nt_mid_kernel(GemmArgs gb, MidSplit 
     return;
   }
   const bool diag = g.symmetric && ti == tj;
-  epilogue_quarter<F16, FORM>(g, diag, F, e_buf, RA, 0, row0, col0, lane, 0, 8, 3);
+  epilogue_quarter<F16>(g, diag, F, e_buf, RA, 0, row0, col0, lane, 0, 8, 3);
 }
 
 // The same tiles by workgroups that share a CU in pairs (fm_tile128.h), for more whole tiles than CUs: one workgroup's
 // start, first stages and write-out lie under the other's multiplications, where the kernel above leaves them bare
 // between its tiles.  X' of 1664 x 6400 (650 tiles of 26 stages) 60 -> 46 us, fast_newtonschulz(5) of it 596 -> 527, of 1408 x 5632
 // 436 -> 377, 2 of 1600^2 393 -> 345.  Bound by the copies into the LDS (fm_gemm_ragged.hip): 0.43 us a stage, tile and CU.
-template <bool F16, int FORM>
+template <bool F16>
 __global__ __launch_bounds__(256, 2) void gemm_nt_pair_kernel(GemmArgs gb) {
   __shared__ __align__(1024) unsigned char smem[t128::SMEM];
   const int lane = threadIdx.x & 63;
@@ -2000,14 +1893,13 @@ __global__ __launch_bounds__(256, 2) void gemm_nt_pair_kernel(GemmArgs gb) {
   o.alpha = g.alpha; o.beta = g.beta;
   o.row_alpha = g.row_alpha;
   o.diag_out = g.diag_out;
-  if constexpr (FORM == kFormPoly) o.diag_add = g.diag_add;
-  t128::write_block<F16, 0, false, FORM>(o, g.symmetric && ti == tj, acc, smem + wave * 16384, ti * MID_T + (wave >> 1) * 64, tj * MID_T + (wave & 1) * 64, lane);
+  t128::write_block<F16, 0>(o, g.symmetric && ti == tj, acc, smem + wave * 16384, ti * MID_T + (wave >> 1) * 64, tj * MID_T + (wave & 1) * 64, lane);
 }
 
 // Second kernel of the cut 128x128 tiles: one workgroup per (tile, quarter).  Its four waves add
 // the quarter's parts in k order, so the bits do not depend on which workgroup finished when, and
 // share the iterations of its epilogue.
-template <bool F16, int FORM>
+template <bool F16>
 __global__ __launch_bounds__(256) void gemm_nt_mid_reduce_kernel(GemmArgs gb, MidSplit sp) {
   __shared__ __align__(1024) unsigned char smem[EPI_WAVE_BYTES];
   __shared__ int s_slot[kMaxParts];
@@ -2030,9 +1922,9 @@ __global__ __launch_bounds__(256) void gemm_nt_mid_reduce_kernel(GemmArgs gb, Mi
   __syncthreads();
   const bool diag = g.symmetric && ti == tj;
   // direct pass, then (after everybody has put its rounded values back) the transposed pass
-  epilogue_quarter<F16, FORM>(g, diag, L.F, L.E[0], L.RA, 0, row0, col0, lane, wave * 2, wave * 2 + 2, 1);
+  epilogue_quarter<F16>(g, diag, L.F, L.E[0], L.RA, 0, row0, col0, lane, wave * 2, wave * 2 + 2, 1);
   __syncthreads();
-  epilogue_quarter<F16, FORM>(g, diag, L.F, L.E[0], L.RA, 0, row0, col0, lane, wave * 2, wave * 2 + 2, 2);
+  epilogue_quarter<F16>(g, diag, L.F, L.E[0], L.RA, 0, row0, col0, lane, wave * 2, wave * 2 + 2, 2);
 }
 
 }  // namespace
@@ -2102,7 +1994,7 @@ static void fast_schedule(int num_tiles, int nk, long long max_slots, FastArgs& 
 // what both tile shapes ask of a problem: whole tiles of edge `tile`, whole k stages, 16-byte
 // accesses everywhere
 static bool tiled_dma_eligible(const GemmArgs& a, int tile) {
-  if (a.elem == kElemF16 && a.E && a.form == 0) return false;
+  if (a.elem == kElemF16 && a.E) return false;
   if (a.Kc < BKF || a.Kc % BKF != 0) return false;
   if (a.lda % 8 != 0 || a.ldb % 8 != 0) return false;
   if ((reinterpret_cast<uintptr_t>(a.A) & 15) || (reinterpret_cast<uintptr_t>(a.B) & 15)) return false;
@@ -2156,12 +2048,6 @@ static double estimate_half_round(long long half_items, int nk, int grid) {
   return nk * (0.50 + 0.78 * (occ > 0.6 ? occ - 0.6 : 0.0)) + 13.0;
 }
 
-// half items of all matrices: a diagonal tile of a symmetric product is one
-static long long half_item_count(const GemmArgs& a) {
-  const long long tm = a.Ma / BM, tn = a.Nb / BN, nb = a.batch < 1 ? 1 : a.batch;
-  return (a.symmetric ? tm * tm : 2 * tm * tn) * nb;
-}
-
 // The half-tile schedule (128x256 items, a diagonal tile of a symmetric product as one item) is
 // taken when all its items fit into one round and that round is estimated to be shorter than the
 // round of whole tiles: those would leave about half of the CUs idle, and half items are never
@@ -2203,7 +2089,7 @@ static bool sub64_schedule_chosen(const GemmArgs& a, long long tiles, int nk, in
   const int ksplit = auto_ksplit(tiles, nk, grid);
   const double t_large = (nk / ksplit) * 1.45 + 15.0 + (ksplit > 1 ? 25.0 : 0.0);
   if (t_large < t_best) t_best = t_large;
-  const long long half_items = half_item_count(a);
+  const long long half_items = (a.symmetric ? tm * tm : 2 * tm * tn) * nb;
   if (half_schedule_chosen(half_items, tiles, nk, grid)) {
     const double t_half = estimate_half_round(half_items, nk, grid);
     if (t_half < t_best) t_best = t_half;
@@ -2231,7 +2117,7 @@ bool gemm_fast_eligible(const GemmArgs& a) {
   const double t_large = (nk / ksplit) * 1.45 + 15.0 + (ksplit > 1 ? 25.0 : 0.0);
   const long long small_tiles = (a.symmetric ? 2 * tm * (2 * tm + 1) / 2 : 4 * tm * tn) * (a.batch < 1 ? 1 : a.batch);
   const double t_small = estimate_mid(a, small_tiles, nk, cus);
-  const long long half_items = half_item_count(a);
+  const long long half_items = (a.symmetric ? tm * tm : 2 * tm * tn) * (a.batch < 1 ? 1 : a.batch);
   // (the 128x128 tiles keep the benefit of the doubt against half tiles)
   if (half_schedule_chosen(half_items, tiles, nk, cus) && estimate_half_round(half_items, nk, cus) < 0.9 * t_small) return true;
   return t_large < t_small;
@@ -2251,7 +2137,7 @@ static bool slim_chosen(const GemmArgs& a, const void* ws, size_t ws_bytes) {
   if (any_knob_set() || !pair_eligible(a) || !gemm_slim_fits(a, cus)) return false;
   const long long tm = a.Ma / MID_T, tn = a.Nb / MID_T, tiles = (a.symmetric ? tm * (tm + 1) / 2 : tm * tn) * (a.batch < 1 ? 1 : a.batch);
   const int parts = mid_parts(tiles, nk, cus);
-  if (parts == 1 || (a.form && a.elem == kElemF16) || !ws || (size_t)tiles * parts * MID_PART_FLOATS * sizeof(float) > ws_bytes) return true;
+  if (parts == 1 || !ws || (size_t)tiles * parts * MID_PART_FLOATS * sizeof(float) > ws_bytes) return true;
   return slim_us(tiles, nk, cus, a.E != nullptr) < mid_us(tiles, nk, cus, parts, a.E != nullptr);
 }
 
@@ -2266,28 +2152,18 @@ int launch_gemm_mid(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) {
   sp.partials = static_cast<float*>(ws);
   // without room for the parts the tiles stay whole
   if (sp.ksplit > 1 && (!ws || (size_t)a.num_tiles * sp.ksplit * MID_PART_FLOATS * sizeof(float) > ws_bytes)) sp.ksplit = 1;
-  // (the products of two M x M matrices are never cut: where they have few tiles their k is short)
-  if (a.form && a.elem == kElemF16) sp.ksplit = 1;
   const unsigned grid = (unsigned)(a.num_tiles * sp.ksplit);
-  const bool pairs = sp.ksplit == 1 && a.num_tiles > cu_count() && pair_eligible(a);
-#define FM_MID(F16, FORM)                                                                                                          \
-  do {                                                                                                                             \
-    if (pairs) {                                                                                                                   \
-      hipLaunchKernelGGL((gemm_nt_pair_kernel<F16, FORM>), dim3(grid), dim3(256), 0, stream, a);                                    \
-      break;                                                                                                                       \
-    }                                                                                                                              \
-    hipLaunchKernelGGL((gemm_nt_mid_kernel<F16, FORM>), dim3(grid), dim3(256), 0, stream, a, sp);                                   \
-    if constexpr (!F16 || FORM == 0) {                                                                                              \
-      if (sp.ksplit > 1) hipLaunchKernelGGL((gemm_nt_mid_reduce_kernel<F16, FORM>), dim3(a.num_tiles * 4), dim3(256), 0, stream, a, sp); \
-    }                                                                                                                              \
-  } while (0)
-  if (a.form == kFormPoly) FM_MID(true, kFormPoly);
-  else if (a.form == kFormScaledBf16) FM_MID(true, kFormScaledBf16);
-  else if (a.form == kFormScaledF16 && a.elem == kElemF16) FM_MID(true, kFormScaledF16);
-  else if (a.form == kFormScaledF16) FM_MID(false, kFormScaledF16);
-  else if (a.elem == kElemF16) FM_MID(true, 0);
-  else FM_MID(false, 0);
-#undef FM_MID
+  if (sp.ksplit == 1 && a.num_tiles > cu_count() && pair_eligible(a)) {
+    if (a.elem == kElemF16) hipLaunchKernelGGL(gemm_nt_pair_kernel<true>, dim3(grid), dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL(gemm_nt_pair_kernel<false>, dim3(grid), dim3(256), 0, stream, a);
+    return (int)hipGetLastError();
+  }
+  if (a.elem == kElemF16) hipLaunchKernelGGL(gemm_nt_mid_kernel<true>, dim3(grid), dim3(256), 0, stream, a, sp);
+  else hipLaunchKernelGGL(gemm_nt_mid_kernel<false>, dim3(grid), dim3(256), 0, stream, a, sp);
+  if (sp.ksplit > 1) {
+    if (a.elem == kElemF16) hipLaunchKernelGGL(gemm_nt_mid_reduce_kernel<true>, dim3(a.num_tiles * 4), dim3(256), 0, stream, a, sp);
+    else hipLaunchKernelGGL(gemm_nt_mid_reduce_kernel<false>, dim3(a.num_tiles * 4), dim3(256), 0, stream, a, sp);
+  }
   return (int)hipGetLastError();
 }
 
@@ -2340,7 +2216,7 @@ int launch_gemm_fast(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) 
   int grid = cu_count() < kMaxGrid ? cu_count() : kMaxGrid;
   const long long kg = knob(kKnobGrid);
   if (kg > 0 && kg < grid) grid = (int)kg;
-  const long long half_items = half_item_count(a);
+  const long long half_items = a.symmetric ? (long long)a.tiles_m * a.tiles_m * a.batch : 2LL * a.num_tiles;   // a diagonal tile is one item
   if (sub64_schedule_chosen(a, a.num_tiles, f.nk, grid)) {   // every tile as 16 sub-tiles of 64x64, one workgroup each
     f.grid = a.num_tiles * 16;
     f.ksplit = 1;
@@ -2402,24 +2278,20 @@ int launch_gemm_fast(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) 
   const int slots = f.tail_slot0 + f.rem * f.split;
   const int reduce_tiles = a.num_tiles - f.reduce_tile0;
   if (!f.half && reduce_tiles > 0 && (slots > have || f.ksplit * f.split > kMaxParts)) return kErrWorkspace;
-#define FM_ROUNDS(KERNEL, F16, MODE, FORM)                                                                             \
-  do {                                                                                                                 \
-    if (f.half) {                                                                                                      \
-      hipLaunchKernelGGL((KERNEL<F16, MODE, 2>), dim3(f.grid), dim3(256), 0, stream, f);                                \
-      break;                                                                                                           \
-    }                                                                                                                  \
-    hipLaunchKernelGGL((KERNEL<F16, MODE, 4>), dim3(f.grid), dim3(256), 0, stream, f);                                  \
-    if (halves) hipLaunchKernelGGL((KERNEL<F16, MODE, 2>), dim3(tail.grid), dim3(256), 0, stream, tail);                 \
-    if (reduce_tiles > 0) hipLaunchKernelGGL((gemm_nt_reduce_kernel<F16, FORM>), dim3(reduce_tiles * 16), dim3(256), 0, stream, f); \
+#define FM_ROUNDS(F16, MODE)                                                                                              \
+  do {                                                                                                                    \
+    if (f.half) {                                                                                                         \
+      hipLaunchKernelGGL((gemm_nt_rounds_kernel<F16, MODE, 2>), dim3(f.grid), dim3(256), 0, stream, f);                    \
+      break;                                                                                                              \
+    }                                                                                                                     \
+    hipLaunchKernelGGL((gemm_nt_rounds_kernel<F16, MODE, 4>), dim3(f.grid), dim3(256), 0, stream, f);                      \
+    if (halves) hipLaunchKernelGGL((gemm_nt_rounds_kernel<F16, MODE, 2>), dim3(tail.grid), dim3(256), 0, stream, tail);     \
+    if (reduce_tiles > 0) hipLaunchKernelGGL(gemm_nt_reduce_kernel<F16>, dim3(reduce_tiles * 16), dim3(256), 0, stream, f); \
   } while (0)
-  if (a.form == kFormPoly) FM_ROUNDS(gemm_nt_form_kernel, true, kFormPoly, kFormPoly);
-  else if (a.form == kFormScaledBf16) FM_ROUNDS(gemm_nt_form_kernel, true, kFormScaledBf16, kFormScaledBf16);
-  else if (a.form == kFormScaledF16 && a.elem == kElemF16) FM_ROUNDS(gemm_nt_form_kernel, true, kFormScaledF16, kFormScaledF16);
-  else if (a.form == kFormScaledF16) FM_ROUNDS(gemm_nt_form_kernel, false, kFormScaledF16, kFormScaledF16);
-  else if (a.elem == kElemF16) FM_ROUNDS(gemm_nt_rounds_kernel, true, 0, 0);
-  else if (!a.E) FM_ROUNDS(gemm_nt_rounds_kernel, false, 0, 0);
-  else if (a.beta == 1.0f) FM_ROUNDS(gemm_nt_rounds_kernel, false, 1, 0);
-  else FM_ROUNDS(gemm_nt_rounds_kernel, false, 2, 0);
+  if (a.elem == kElemF16) FM_ROUNDS(true, 0);
+  else if (!a.E) FM_ROUNDS(false, 0);
+  else if (a.beta == 1.0f) FM_ROUNDS(false, 1);
+  else FM_ROUNDS(false, 2);
 #undef FM_ROUNDS
   return (int)hipGetLastError();
 }

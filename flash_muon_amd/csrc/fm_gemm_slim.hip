@@ -182,12 +182,11 @@ __device__ __forceinline__ void load_e(Pre& pre, const GemmArgs& g, int row0, in
 // through wave-private LDS and out 16 bytes per lane.  `diag`: in a diagonal tile of a symmetric product.  KIND 1 and 2: the upper and lower
 // half of a 64x64 square on the diagonal, of which the wave holds columns 0 .. 31 above, whose other columns are written as the
 // mirror image of columns 0 .. 31 below.
-template <bool F16, int FORM, int KIND = 0>
+template <bool F16, int KIND = 0>
 __device__ __forceinline__ void write_block(const GemmArgs& g, bool use_e, const Pre& pre, const f32x4_t (&a0)[4], const f32x4_t (&a1)[4],
                                             bool direct, bool mirror, bool diag, int row0, int col0, unsigned char* T, int lane) {
-  constexpr bool SCALES = FORM == kFormScaledF16 || FORM == kFormScaledBf16, OF16 = FORM == kFormScaledF16 || (F16 && FORM != kFormScaledBf16);
   const int n = lane & 15, grp = lane >> 4;
-  const bool dout = diag && (FORM == kFormPoly || g.diag_out != nullptr);
+  const bool dout = diag && g.diag_out != nullptr;
   unsigned char* const T2 = T + 32 * 128;
 #pragma unroll
   for (int J = 0; J < (KIND == 1 ? 1 : 2); ++J) {
@@ -205,46 +204,33 @@ __device__ __forceinline__ void write_block(const GemmArgs& g, bool use_e, const
           v[b][k] = __builtin_fmaf(pre.al[k], elem_to_f32<F16>((unsigned short)((k & 1) ? (e[k >> 1] >> 16) : (e[k >> 1] & 0xffffu))), g.beta * v[b][k]);
       }
     }
-    if constexpr (SCALES) {
+    if (dout && row0 - col0 == 32 * J) {   // this 32x32 sub-block lies on the diagonal: the lanes with n / 4 == grp hold rows 2 n and 2 n + 1 of it
+      float dv[2] = {0.0f, 0.0f};
 #pragma unroll
       for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[b][k] *= g.beta;
-    }
-    if (dout && row0 - col0 == 32 * J) {   // this 32x32 sub-block lies on the diagonal
-      if constexpr (FORM == kFormPoly) {
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int k = 0; k < 8; ++k) v[b][k] += 2 * n + b == 8 * grp + k ? g.diag_add : 0.0f;
-      } else {   // the lanes with n / 4 == grp hold rows 2 n and 2 n + 1 of it
-        float dv[2] = {0.0f, 0.0f};
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            const bool on = 2 * n + b == 8 * grp + k;
-            dv[b] = on ? v[b][k] : dv[b];
-            v[b][k] = on ? 0.0f : v[b][k];
-          }
-        if ((n >> 2) == grp) {
-          g.diag_out[row0 + 2 * n] = dv[0];
-          g.diag_out[row0 + 2 * n + 1] = dv[1];
+        for (int k = 0; k < 8; ++k) {
+          const bool on = 2 * n + b == 8 * grp + k;
+          dv[b] = on ? v[b][k] : dv[b];
+          v[b][k] = on ? 0.0f : v[b][k];
         }
+      if ((n >> 2) == grp) {
+        g.diag_out[row0 + 2 * n] = dv[0];
+        g.diag_out[row0 + 2 * n + 1] = dv[1];
       }
     }
     if (direct) {   // row R of the block in LDS row R ^ (R / 16 % 2), its 64-byte halves swapped where R / 8 is odd
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const int R = 8 * grp + k;
-        *reinterpret_cast<uint32_t*>(T + ((R ^ (grp >> 1)) * 128) + ((J ^ (grp & 1)) * 64) + 4 * n) = pack2<OF16>(v[0][k], v[1][k]);
+        *reinterpret_cast<uint32_t*>(T + ((R ^ (grp >> 1)) * 128) + ((J ^ (grp & 1)) * 64) + 4 * n) = pack2<F16>(v[0][k], v[1][k]);
       }
     }
     if (mirror && (KIND != 2 || J == 0)) {
 #pragma unroll
       for (int b = 0; b < 2; ++b)
         *reinterpret_cast<uint4*>(T2 + (32 * J + 2 * n + b) * MIRROR_PITCH + 16 * grp) =
-            uint4{pack2<OF16>(v[b][0], v[b][1]), pack2<OF16>(v[b][2], v[b][3]), pack2<OF16>(v[b][4], v[b][5]), pack2<OF16>(v[b][6], v[b][7])};
+            uint4{pack2<F16>(v[b][0], v[b][1]), pack2<F16>(v[b][2], v[b][3]), pack2<F16>(v[b][4], v[b][5]), pack2<F16>(v[b][6], v[b][7])};
     }
   }
   if (direct) {
@@ -271,10 +257,9 @@ __device__ __forceinline__ void write_block(const GemmArgs& g, bool use_e, const
   }
 }
 
-template <bool F16, int FORM>
+template <bool F16>
 __global__ __launch_bounds__(256) void gemm_nt_slim_kernel(GemmArgs gb, int diag_items) {
   __shared__ __align__(1024) unsigned char smem[DEPTH * STAGE];
-  constexpr bool SCALES = FORM == kFormScaledF16 || FORM == kFormScaledBf16;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 1, wn = wave & 1;
   // workgroups are dealt round-robin to the 8 XCDs: give each XCD a contiguous run of tiles
@@ -287,7 +272,7 @@ __global__ __launch_bounds__(256) void gemm_nt_slim_kernel(GemmArgs gb, int diag
   item_at(gb, diag_items, w, bi, ti, tj, h);
   const GemmArgs g = batch_view(gb, bi);
   const int m0 = ti * 128 + h * TM, n0 = tj * TN;
-  const bool use_e = FORM == kFormPoly || (!F16 && !SCALES && g.E != nullptr);
+  const bool use_e = !F16 && g.E != nullptr;   // (fp16 problems carry no operand E)
   if (use_e && !block_written(g, ti * 128, n0)) return;
 
   Lane L;
@@ -313,49 +298,47 @@ __global__ __launch_bounds__(256) void gemm_nt_slim_kernel(GemmArgs gb, int diag
   const bf16_t* const gB = g.B + (int64_t)n0 * g.ldb;
   const int nk = g.Kc / BK, last = nk - 1;
 
-  if constexpr (!SCALES || !F16) {   // (the products of two matrices have no such items)
-    if (diag_items && ti == tj) {
-      DLane D;
-      D.ldsw = L.ldsw;
+  if (diag_items && ti == tj) {
+    DLane D;
+    D.ldsw = L.ldsw;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) D.vo[q] = L.voB[q];
-      const int dr = wave < 2 ? 64 * wave : 32 * wave, dc = wave < 2 ? 64 * wave : 0;   // (waves 2 and 3: rows 64 and 96)
+    for (int q = 0; q < 4; ++q) D.vo[q] = L.voB[q];
+    const int dr = wave < 2 ? 64 * wave : 32 * wave, dc = wave < 2 ? 64 * wave : 0;   // (waves 2 and 3: rows 64 and 96)
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
+    for (int kk = 0; kk < 2; ++kk) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int rb = dc + 16 * i + (lane & 15);
-          D.fb[kk][i] = (uint32_t)(A_BYTES + rb * ROW + (((4 * kk + (lane >> 4)) ^ swz(rb)) << 4));
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = gather_row((dr & ~31) + 16 * i + (lane & 15)) & (TN - 1);   // (fragments 2 and 3 of waves 2 and 3 are not read)
-          D.fa[kk][i] = (uint32_t)(A_BYTES + r * ROW + (((4 * kk + (lane >> 4)) ^ swz(r)) << 4));
-        }
+      for (int i = 0; i < 2; ++i) {
+        const int rb = dc + 16 * i + (lane & 15);
+        D.fb[kk][i] = (uint32_t)(A_BYTES + rb * ROW + (((4 * kk + (lane >> 4)) ^ swz(rb)) << 4));
       }
 #pragma unroll
-      for (int s = 0; s < DEPTH; ++s) {
-        const int k = s < last ? s : last;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) copy16(D.vo[q], gB + k * BK, D.ldsw, s * STAGE + A_BYTES + q * 4096);
+      for (int i = 0; i < 4; ++i) {
+        const int r = gather_row((dr & ~31) + 16 * i + (lane & 15)) & (TN - 1);   // (fragments 2 and 3 of waves 2 and 3 are not read)
+        D.fa[kk][i] = (uint32_t)(A_BYTES + r * ROW + (((4 * kk + (lane >> 4)) ^ swz(r)) << 4));
       }
-      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"((DEPTH - 1) * 4) : "memory");
-      f32x4_t acc[4][4];
-      if (wave < 2) diag_loop<F16, 4>(acc, nk, smem, D, gB);
-      else diag_loop<F16, 2>(acc, nk, smem, D, gB);
-      unsigned char* const T = smem + wave * STAGING;
-      Pre pre;
-      if (wave < 2) {
-        if (use_e) load_e(pre, g, n0 + dr, n0 + dc, lane);
-        write_block<F16, FORM, 1>(g, use_e, pre, acc[0], acc[1], true, false, true, n0 + dr, n0 + dc, T, lane);
-        if (use_e) load_e(pre, g, n0 + dr + 32, n0 + dc, lane);
-        write_block<F16, FORM, 2>(g, use_e, pre, acc[2], acc[3], true, true, true, n0 + dr + 32, n0 + dc, T, lane);
-      } else {
-        if (use_e) load_e(pre, g, n0 + dr, n0 + dc, lane);
-        write_block<F16, FORM>(g, use_e, pre, acc[0], acc[1], true, true, false, n0 + dr, n0 + dc, T, lane);
-      }
-      return;
     }
+#pragma unroll
+    for (int s = 0; s < DEPTH; ++s) {
+      const int k = s < last ? s : last;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) copy16(D.vo[q], gB + k * BK, D.ldsw, s * STAGE + A_BYTES + q * 4096);
+    }
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"((DEPTH - 1) * 4) : "memory");
+    f32x4_t acc[4][4];
+    if (wave < 2) diag_loop<F16, 4>(acc, nk, smem, D, gB);
+    else diag_loop<F16, 2>(acc, nk, smem, D, gB);
+    unsigned char* const T = smem + wave * STAGING;
+    Pre pre;
+    if (wave < 2) {
+      if (use_e) load_e(pre, g, n0 + dr, n0 + dc, lane);
+      write_block<F16, 1>(g, use_e, pre, acc[0], acc[1], true, false, true, n0 + dr, n0 + dc, T, lane);
+      if (use_e) load_e(pre, g, n0 + dr + 32, n0 + dc, lane);
+      write_block<F16, 2>(g, use_e, pre, acc[2], acc[3], true, true, true, n0 + dr + 32, n0 + dc, T, lane);
+    } else {
+      if (use_e) load_e(pre, g, n0 + dr, n0 + dc, lane);
+      write_block<F16>(g, use_e, pre, acc[0], acc[1], true, true, false, n0 + dr, n0 + dc, T, lane);
+    }
+    return;
   }
 
   const int row0 = m0 + wm * 32, col0 = n0 + wn * 64;
@@ -399,29 +382,22 @@ __global__ __launch_bounds__(256) void gemm_nt_slim_kernel(GemmArgs gb, int diag
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
   const bool tdiag = g.symmetric && ti == tj;   // both halves of such a tile hold their own mirror images
-  write_block<F16, FORM>(g, use_e, pre, acc[0], acc[1], g.C != nullptr, g.C2 != nullptr && !tdiag, tdiag, row0, col0, smem + wave * STAGING, lane);
+  write_block<F16>(g, use_e, pre, acc[0], acc[1], g.C != nullptr, g.C2 != nullptr && !tdiag, tdiag, row0, col0, smem + wave * STAGING, lane);
 }
 
 }  // namespace
 
 bool gemm_slim_fits(const GemmArgs& a, int cus) {
   const long long tm = a.Ma / 128, tn = a.Nb / 128, nb = a.batch < 1 ? 1 : a.batch;
-  if (a.symmetric && a.A == a.B && tm * tm * nb <= cus) return true;
-  return (a.symmetric ? tm * (tm + 1) : 2 * tm * tn) * nb <= cus;
+  return (a.symmetric ? tm * tm : 2 * tm * tn) * nb <= cus;
 }
 
 int launch_gemm_slim(const GemmArgs& a, hipStream_t stream) {   // tiles_m, tiles_n and num_tiles are those of 128x128 tiles
   // diagonal tiles as one item where they may be and their halves would be too many
   const int diag_items = 2 * a.num_tiles > cu_count();
   const dim3 grid((unsigned)(diag_items ? a.tiles_m * a.tiles_m * a.batch : 2 * a.num_tiles)), block(256);
-#define FM_SLIM(F16, FORM) hipLaunchKernelGGL((gemm_nt_slim_kernel<F16, FORM>), grid, block, 0, stream, a, diag_items)
-  if (a.form == kFormPoly) FM_SLIM(true, kFormPoly);
-  else if (a.form == kFormScaledBf16) FM_SLIM(true, kFormScaledBf16);
-  else if (a.form == kFormScaledF16 && a.elem == kElemF16) FM_SLIM(true, kFormScaledF16);
-  else if (a.form == kFormScaledF16) FM_SLIM(false, kFormScaledF16);
-  else if (a.elem == kElemF16) FM_SLIM(true, 0);
-  else FM_SLIM(false, 0);
-#undef FM_SLIM
+  if (a.elem == kElemF16) hipLaunchKernelGGL(gemm_nt_slim_kernel<true>, grid, block, 0, stream, a, diag_items);
+  else hipLaunchKernelGGL(gemm_nt_slim_kernel<false>, grid, block, 0, stream, a, diag_items);
   return (int)hipGetLastError();
 }
 

@@ -93,12 +93,6 @@ template <bool F16> __device__ __forceinline__ float elem_to_f32(unsigned short 
   else return __builtin_bit_cast(float, (uint32_t)h << 16);
 }
 
-// Forms of the contraction below for the chain of M x M products that several Newton-Schulz steps are folded into
-// (fm_api.hip).  They run on whole, aligned 128-tiles only.
-constexpr int kFormPoly = 2;         // fp16, with E: v = alpha E + beta acc, and diag_add more on the diagonal
-constexpr int kFormScaledF16 = 3;    // v = beta acc, rounded to fp16; operands bf16 or fp16
-constexpr int kFormScaledBf16 = 4;   // v = beta acc, rounded to bf16, the diagonal to diag_out; operands fp16
-
 // Arguments of the one NT contraction every GEMM-shaped kernel here is an instance of:
 //     acc[i][j] = sum_k A[i][k] * B[j][k]            (A: Ma x Kc, B: Nb x Kc, k contiguous)
 //     v         = E ? (alpha + row_alpha[i]) * E[i][j] + beta * acc : acc   (row_alpha optional)
@@ -106,8 +100,7 @@ constexpr int kFormScaledBf16 = 4;   // v = beta acc, rounded to bf16, the diago
 //     C [i*c_rs  + j*c_cs ] = round(v)               (if C  != nullptr)
 //     C2[j*c2_rs + i*c2_cs] = round(v)               (if C2 != nullptr; the mirrored copy)
 // A, B, E, C and C2 hold bf16; without E they may hold fp16 instead (`elem`; pointers stay typed bf16_t).
-// With `symmetric` set, only tiles on or above the diagonal are computed and C2 == C; A == B but for the scaled forms,
-// whose operands may be two matrices that commute.
+// With `symmetric` set, A == B, only tiles on or above the diagonal are computed and C2 == C.
 struct GemmArgs {
   const bf16_t* A;  int64_t lda;
   const bf16_t* B;  int64_t ldb;
@@ -134,9 +127,6 @@ struct GemmArgs {
   int diag_last;          // 256x256 schedule, one symmetric matrix: its last `diag_last` diagonal tiles end the tile order
   // with E: the rows and columns of C (columns and rows of C2) that are written, whole multiples of 128; 0: all of them
   int rows_v, cols_v;
-  // 0, or one of the forms above; diag_add: of kFormPoly
-  int form;
-  float diag_add;
 };
 
 // whether the block of C at (row, col), of at most 128x128 and on a multiple of its size, is written

@@ -97,32 +97,6 @@ inline NsFlowLaunch ns_flow_launch(int steps, int i) {   // launch i of the (ste
   return NsFlowLaunch{first, left < kFlowSteps ? left : kFlowSteps, i & 1 ? kFlowSteps : 0, i & 1 ? -1 : 1};
 }
 
-// ---- Newton-Schulz steps in groups on the Gram matrix (fm_api.hip) ---------------------------------
-// Whether the steps of M x K matrices, as they lie in the workspace, run in groups: five or more, of a matrix long enough that it
-// saves time and loses no accuracy (fm_api.hip has both sides of both).
-inline bool ns_grouped(int M, int K, int steps) { return steps >= 5 && M >= 512 && K >= 2 * (int64_t)M; }
-// steps of the group that begins with step s: three, then two at a time
-inline int ns_group(int steps, int s) { return s == 0 ? 3 : steps - s >= 2 ? 2 : 1; }
-// Whether the coefficients keep the M x M matrices inside fp16's range at the scales they are held at (2^14 A and Q A, 2^13 Q, 2^12 Q_2 Q_1),
-// with half of it to spare for A.  The singular values of X lie in [0, top]: top starts at 1 (the Frobenius norm) and becomes
-// the largest value of sigma q(sigma^2), a hundredth on top for the roundings.  (3.4445, -4.775, 2.0315): top <= 1.22, q <= 3.45.
-inline bool ns_groups_fit(int steps, float a, float b, float c) {
-  double top = 1.01;
-  for (int s = 0; s < steps; ++s) {
-    double next = 0.0;
-    for (int i = 0; i <= 256; ++i) {
-      const double x = top * i / 256.0;
-      double q = a + b * x * x + c * x * x * x * x;
-      q = q < 0 ? -q : q;
-      if (!(q <= 3.7)) return false;
-      if (x * q > next) next = x * q;
-    }
-    if (top * top > 2.0 || top * next > 2.0) return false;
-    top = 1.01 * next;
-  }
-  return true;
-}
-
 // ---- X X^T in 16 bits of sides that the 256-tiles do not fit -------------------------------------
 // The in-place kernel's schedule (fm_gemm_ragged.hip): 128x128 tiles in full rounds of 512 workgroups; of those left over `whole` in one
 // piece and `cut` in `parts` pieces along k each.

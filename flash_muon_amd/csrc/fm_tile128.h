@@ -305,7 +305,6 @@ struct Out {
   const float* row_alpha;
   float* diag_out;                // fp32 diagonal split off (blocks on the diagonal of a symmetric product)
   int limit;                      // EDGE: rows and columns of the output that exist
-  float diag_add;                 // kFormPoly: added to the diagonal
 };
 
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -340,15 +339,14 @@ __device__ __forceinline__ void store_edge(bf16_t* C, int64_t ld, int r, int c, 
 }
 
 // AUX: cache policy of the stores (0, or 16: written through to memory, for readers on other XCDs).  EDGE: blocks may
-// beyond the output, whose rows may start at any element.  FORM: of GemmArgs.
-template <bool F16, int AUX, bool EDGE = false, int FORM = 0>
+// reach beyond the output, whose rows may start at any element.
+template <bool F16, int AUX, bool EDGE = false>
 __device__ __forceinline__ void write_block(const Out& o, bool diag, const f32x4_t (&acc)[4][4], unsigned char* T, int row0,
                                             int col0, int lane) {
   asm volatile("" : "+v"(lane));   // offsets derived anew for every tile, not kept across the main loop
   const int n = lane & 15, g = lane >> 4;
-  constexpr bool SCALES = FORM == kFormScaledF16 || FORM == kFormScaledBf16, OF16 = FORM == kFormScaledF16 || (F16 && FORM != kFormScaledBf16);
-  const bool use_e = FORM == kFormPoly || (!F16 && !SCALES && o.ET != nullptr), direct = o.C != nullptr, mirror = o.C2 != nullptr && !diag;
-  const bool dout = diag && row0 == col0 && (FORM == kFormPoly || o.diag_out != nullptr);
+  const bool use_e = !F16 && o.ET != nullptr, direct = o.C != nullptr, mirror = o.C2 != nullptr && !diag;
+  const bool dout = diag && row0 == col0 && o.diag_out != nullptr;
   unsigned char* const T2 = T + 8192;
   uint4 ev[2][2][2];
   float al[2][8];
@@ -390,20 +388,7 @@ __device__ __forceinline__ void write_block(const Out& o, bool diag, const f32x4
           }
         }
       }
-      if constexpr (SCALES) {
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int k = 0; k < 8; ++k) v[b][k] *= o.beta;
-      }
-      if constexpr (FORM == kFormPoly) {
-        if (dout && I == J) {
-#pragma unroll
-          for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int k = 0; k < 8; ++k) v[b][k] += 2 * n + b == 8 * g + k ? o.diag_add : 0.0f;
-        }
-      } else if (dout && I == J) {   // the lanes with n / 4 == g hold rows 2 n and 2 n + 1 of the sub-block's diagonal
+      if (dout && I == J) {   // the lanes with n / 4 == g hold rows 2 n and 2 n + 1 of the sub-block's diagonal
         float dv[2] = {0.0f, 0.0f};
 #pragma unroll
         for (int b = 0; b < 2; ++b)
@@ -430,7 +415,7 @@ __device__ __forceinline__ void write_block(const Out& o, bool diag, const f32x4
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
           const int R = 32 * I + 8 * g + k;
-          *reinterpret_cast<uint32_t*>(T + ((R ^ (g >> 1)) * 128) + ((J ^ (g & 1)) * 64) + 4 * n) = pack2<OF16>(v[0][k], v[1][k]);
+          *reinterpret_cast<uint32_t*>(T + ((R ^ (g >> 1)) * 128) + ((J ^ (g & 1)) * 64) + 4 * n) = pack2<F16>(v[0][k], v[1][k]);
         }
       }
       if (mirror) {
@@ -439,7 +424,7 @@ __device__ __forceinline__ void write_block(const Out& o, bool diag, const f32x4
         for (int b = 0; b < 2; ++b) {
           const int c = 32 * J + 2 * n + b;
           *reinterpret_cast<uint4*>(T2 + ((c ^ (n >> 3)) * 128) + (((4 * I + g) ^ (n & 7)) << 4)) =
-              uint4{pack2<OF16>(v[b][0], v[b][1]), pack2<OF16>(v[b][2], v[b][3]), pack2<OF16>(v[b][4], v[b][5]), pack2<OF16>(v[b][6], v[b][7])};
+              uint4{pack2<F16>(v[b][0], v[b][1]), pack2<F16>(v[b][2], v[b][3]), pack2<F16>(v[b][4], v[b][5]), pack2<F16>(v[b][6], v[b][7])};
         }
       }
     }

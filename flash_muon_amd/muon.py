@@ -1,7 +1,7 @@
 """fast_newtonschulz and the single-GPU Muon optimizer on libflashmuon_hip.so.
 
 Signatures, defaults, state keys and error behaviour follow flash_muon/muon.py:6-110.  The
-Newton-Schulz loop (muon.py:25-29) runs as three fused products per step, or in groups of steps, inside
+Newton-Schulz loop (muon.py:25-29) runs as three fused kernels per step inside
 fm_newtonschulz_bf16; the momentum and weight updates (muon.py:99-100, 87-89) are one kernel
 each.  The all-gather of muon.py:108 has no counterpart: only world_size == 1 is implemented,
 and no process group is needed.

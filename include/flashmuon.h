@@ -217,12 +217,10 @@ FM_API int fm_scale_cast_bf16(const void* G, int dtype, int rows, int cols, int6
  * The whole quintic Newton-Schulz orthogonalisation of one matrix: G is rows x cols of `dtype`
  * (row stride ldg), out is rows x cols bf16 (row stride ldout).  Runs the sum of squares, the scaled
  * cast and `steps` x (fm_syrk_bf16, fm_syrk_poly_bf16, fm_gemm_axpby_bf16) on
- * `stream`, iterating on the wide orientation (M = min(rows, cols)).  From five steps, M = 512 and K = 2 M on the
- * steps run in groups of three and two, each of which works on the Gram matrix X X^T, held in scaled fp16, and multiplies X once (with
- * coefficients that keep fp16's range): less work, and closer to the exact result.  Matrices of up to 512 to 1920 rows
+ * `stream`, iterating on the wide orientation (M = min(rows, cols)).  Matrices of up to 512 to 1920 rows
  * (by size, shape and number; not with a long K) run all products of up to five steps as one launch, whose workgroups wait
  * for each other inside it but need not be resident together; their workspace holds every step's
- * iterate and squares (6 M K + 10 M^2 bf16 per matrix, in groups 3 M K + 16 M^2, against 4 M K + 2 M^2 otherwise), and with less they run
+ * iterate and squares (6 M K + 10 M^2 bf16 per matrix, against 4 M K + 2 M^2 otherwise), and with less they run
  * a launch per product (fm_newtonschulz_batched_min_workspace_bytes).
  * steps == 0 returns the normalised input.  out must not overlap G.  A matrix whose sides are not whole multiples of 128
  * (of 256 where whole 256x256 tiles are estimated to pay for the padding) is iterated on zero-padded to whole tiles inside the workspace (zero rows and columns stay zero

@@ -20,9 +20,6 @@ int scale_cast_t_on_128(long long tiles) { return fm::scale_cast_t_on_128(tiles)
 int ns_flow_chosen(int batch, int m, int k) { return fm::ns_flow_chosen(batch, m, k); }
 void ns_flow_launch(int steps, int i, int* out) { const fm::NsFlowLaunch n = fm::ns_flow_launch(steps, i); out[0] = n.first; out[1] = n.steps; out[2] = n.from; out[3] = n.turn; }
 int ns_flow_slots() { return fm::kFlowSteps + 1; }
-int ns_grouped(int M, int K, int steps) { return fm::ns_grouped(M, K, steps); }
-int ns_group(int steps, int s) { return fm::ns_group(steps, s); }
-int ns_groups_fit(int steps, float a, float b, float c) { return fm::ns_groups_fit(steps, a, b, c); }
 }
 """
 
@@ -163,34 +160,3 @@ def test_the_one_launch_iteration_stays_in_its_slots(routes, steps):
         assert all(0 <= s < routes.ns_flow_slots() for s in [slot] + written)
         assert len(set([slot] + written)) == 1 + len(written)
     assert done == steps
-
-
-@pytest.mark.parametrize("steps,groups", [(5, [3, 2]), (6, [3, 2, 1]), (7, [3, 2, 2]), (8, [3, 2, 2, 1]), (13, [3, 2, 2, 2, 2, 2])])
-def test_groups_of_steps_add_up(routes, steps, groups):
-    s, got = 0, []
-    while s < steps:
-        got.append(routes.ns_group(steps, s))
-        s += got[-1]
-    assert got == groups
-    assert not routes.ns_grouped(4096, 16384, 4) and not routes.ns_grouped(511, 16384, 5) and not routes.ns_grouped(1024, 2047, 5)
-    assert routes.ns_grouped(512, 1024, 5) and routes.ns_grouped(1 << 20, 1 << 30, 5)
-
-
-# (coefficients, whether A, Q A, Q and Q Q stay inside fp16 at their scales for every number of steps)
-@pytest.mark.parametrize("coeffs,fit", [((3.4445, -4.775, 2.0315), 1), ((1.5, -0.5, 0.0), 1), ((1.875, -1.25, 0.375), 1), ((2.0, -1.5, 0.5), 1),
-                                        ((4.0, -6.0, 3.0), 0), ((2.0, 0.0, 0.0), 0), ((3.0, 0.0, -9.0), 0), ((float("nan"), 0.0, 0.0), 0),
-                                        ((1.0, 0.0, float("inf")), 0), ((0.0, 0.0, 0.0), 1)])
-def test_coefficients_whose_matrices_fit_fp16(routes, coeffs, fit):
-    f = ctypes.c_float
-    routes.ns_groups_fit.argtypes = [ctypes.c_int, f, f, f]
-    for steps in (5, 8, 30):
-        assert routes.ns_groups_fit(steps, *coeffs) == fit
-    if fit:   # the bounds, from the scalars that the singular values go through
-        a, b, c = coeffs
-        x = [i / 4000 for i in range(4001)]
-        for _ in range(8):
-            q = [a + b * t * t + c * t ** 4 for t in x]
-            y = [t * s for t, s in zip(x, q)]
-            assert max(t * t for t in x) * 2 ** 14 < 65504 and max(abs(t * s) for t, s in zip(x, y)) * 2 ** 14 < 65504
-            assert max(abs(s) for s in q) * 2 ** 13 < 65504 and max(abs(s) for s in q) ** 2 * 2 ** 12 < 65504
-            x = y
