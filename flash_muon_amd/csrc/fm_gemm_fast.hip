@@ -2027,10 +2027,10 @@ static int mid_ksplit(long long tiles, int nk, int grid) {
 static bool pair_eligible(const GemmArgs& a);
 // the better way on 128x128 tiles or halves of them
 static double estimate_mid(const GemmArgs& a, long long tiles, int nk, int grid) {
-  const double t = mid_us(tiles, nk, grid, mid_ksplit(tiles, nk, grid), a.E != nullptr);
-  if (any_knob_set() || !pair_eligible(a) || !gemm_slim_fits(a, grid)) return t;
-  const double slim = slim_us(tiles, nk, grid, a.E != nullptr);
-  return slim < t ? slim : t;
+  const int parts = mid_ksplit(tiles, nk, grid);
+  if (!any_knob_set() && pair_eligible(a) && gemm_slim_fits(a, grid) && slim_pays(tiles, nk, grid, parts, a.E != nullptr))
+    return slim_us(tiles, nk, grid, a.E != nullptr);
+  return mid_us(tiles, nk, grid, parts, a.E != nullptr);
 }
 
 // Estimates in microseconds, from measured costs of a k stage and of a tile's start and write-out.
@@ -2131,14 +2131,14 @@ static bool pair_eligible(const GemmArgs& a) {
   return !a.E || (a.ET && a.ldet % 8 == 0 && a.ldet < (1 << 21) && (reinterpret_cast<uintptr_t>(a.ET) & 15) == 0 && (a.batch < 2 || a.bs_et % 8 == 0));
 }
 
-// Halves of the 128x128 tiles, at most one a CU, rather than whole tiles on half of the CUs or less, and than those cut along k (slim_us).
+// Halves of the 128x128 tiles, at most one a CU, rather than whole tiles on half of the CUs or less, and than those cut along k.
 static bool slim_chosen(const GemmArgs& a, const void* ws, size_t ws_bytes) {
   const int cus = cu_count() < kMaxGrid ? cu_count() : kMaxGrid, nk = a.Kc / BKF;
   if (any_knob_set() || !pair_eligible(a) || !gemm_slim_fits(a, cus)) return false;
   const long long tm = a.Ma / MID_T, tn = a.Nb / MID_T, tiles = (a.symmetric ? tm * (tm + 1) / 2 : tm * tn) * (a.batch < 1 ? 1 : a.batch);
   const int parts = mid_parts(tiles, nk, cus);
-  if (parts == 1 || !ws || (size_t)tiles * parts * MID_PART_FLOATS * sizeof(float) > ws_bytes) return true;
-  return slim_us(tiles, nk, cus, a.E != nullptr) < mid_us(tiles, nk, cus, parts, a.E != nullptr);
+  if (!ws || (size_t)tiles * parts * MID_PART_FLOATS * sizeof(float) > ws_bytes) return true;   // (no room for parts)
+  return slim_pays(tiles, nk, cus, parts, a.E != nullptr);
 }
 
 int launch_gemm_mid(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) {

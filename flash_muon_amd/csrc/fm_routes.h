@@ -204,15 +204,23 @@ inline double mid_us(long long tiles, int nk, int grid, int parts, bool with_e) 
   return (double)((tiles + grid - 1) / grid) * (nk * stage + (with_e ? 11.0 : 6.0));
 }
 
-// The same as halves of the tiles, at most one a CU (fm_gemm_slim.hip): a stage of 24 KiB, no cut.  us, whole or cut tiles / halves: X X^T 1536 x
-// 1024 11.8 / 9.7, x 4096 27.4 / 22.2, 1792 x 2048 17.6 / 14.1, x 8192 40.5 / 37.9, 768 x 4096 20.5 / 19.4; cut along a long k 512 x 4096 17.9 / 18.8, x 8192
-// 22.9 / 33.9, 1024 x 8192 24.9 / 35.5, 1536 x 8192 33.7 / 38.0, 1792 x 16384 65.3 / 70.3.
+// The same as halves of the tiles, at most one a CU (fm_gemm_slim.hip): a stage of 24 KiB, no cut.  us, whole tiles / halves: X X^T 1536 x
+// 1024 11.1 / 8.8, x 4096 27.8 / 22.1, 1792 x 2048 17.4 / 14.1, x 6144 39.7 / 33.0, 2048^2 17.8 / 15.1, x
+// 8192 50.8 / 43.2.  (Beyond 72 stages all of these kernels take 3 to 4 us more than their stages before, and a
+// stage of 2048 rows beyond 336 of them 0.30 to 0.32: x 20480 100, x 22528 122, x 24576 123, x 32768 164, where 256-tiles cut along k, whose estimate is
+// as high, take 105 and 130 for the last two.)
 inline double slim_us(long long tiles, int nk, int grid, bool with_e) {
   const double occ = 2.0 * tiles >= grid ? 1.0 : 2.0 * (double)tiles / grid;
-  return 5.7 + nk * (0.223 + 0.037 * occ) + (with_e ? 2.0 : 0.0);
+  return 5.7 + nk * (0.223 + 0.037 * occ) * (nk > 336 ? 1.25 : 1.0) + (nk > 72 ? 3.0 : 0.0) + (with_e ? 2.0 : 0.0);
+}
+// Halves rather than whole tiles always, and than tiles cut into `parts` along a long k where they are estimated to be 5 % faster: they
+// hardly ever are.  us, cut / halves: 1536 x 5120 27.5 / 29.8, x 6144 30.0 / 32.2, x 8192 33.7 / 38.0, 1664 x 7680 37.7 / 40.5, 1792 x 8128 42.1 / 43.8, x
+// 16384 65.3 / 70.3, 512 x 8192 22.9 / 33.9, 1024 x 8192 24.9 / 35.5; near ties 1664 x 8192 38.5 / 39.6, 1792 x 8192 41.1 / 39.1.
+inline bool slim_pays(long long tiles, int nk, int grid, int parts, bool with_e) {
+  return parts == 1 || slim_us(tiles, nk, grid, with_e) < 0.95 * mid_us(tiles, nk, grid, parts, with_e);
 }
 
-// X X^T of an odd number of whole 128-tiles on those halves rather than in place or on whole tiles (below).  us, otherwise / halves: 640 x 2048 13.4 / 12.1, 896 x
+// X X^T of an odd number of whole 128-tiles on halves of them rather than in place or on whole tiles (below).  us, otherwise / halves: 640 x 2048 13.4 / 12.1, 896 x
 // 1024 9.3 / 8.7, 1152 x 2048 14.6 / 12.4, 1664 x 4096 25.5 / 22.7, 1920 x 4096 27.7 / 24.0; but 640 x 4096 15.4 / 18.9, 1152 x 8192 24.0 / 26.9.
 inline bool syrk_whole_slim(int M, int K) { return M <= 1920 && K >= 1024 && K <= (M >= 1664 ? 4096 : 2048); }
 

@@ -18,6 +18,7 @@ int syrk_copy_pays(int M, int K, int half) { return fm::syrk_copy_pays(M, K, hal
 int scale_cast_d_on_tiles(long long r, long long c) { return fm::scale_cast_d_on_tiles(r, c); }
 int scale_cast_t_on_128(long long tiles) { return fm::scale_cast_t_on_128(tiles); }
 int ns_flow_chosen(int batch, int m, int k) { return fm::ns_flow_chosen(batch, m, k); }
+int slim_pays(int tiles, int nk) { return fm::slim_pays(tiles, nk, 256, fm::mid_parts(tiles, nk, 256), false); }
 void ns_flow_launch(int steps, int i, int* out) { const fm::NsFlowLaunch n = fm::ns_flow_launch(steps, i); out[0] = n.first; out[1] = n.steps; out[2] = n.from; out[3] = n.turn; }
 int ns_flow_slots() { return fm::kFlowSteps + 1; }
 }
@@ -122,6 +123,18 @@ WHOLE_TIMES = [(128, 2048, 14.7, 12.0), (128, 65536, 34.5, 28.6), (384, 32768, 2
 @pytest.mark.parametrize("M,K,apart,in_place", WHOLE_TIMES)
 def test_odd_numbers_of_whole_tiles_are_multiplied_in_place_where_it_measured_faster(routes, M, K, apart, in_place):
     assert bool(routes.syrk_whole_in_place(M, K)) == (in_place < apart)
+
+
+# (M, K, us on whole 128-tiles or tiles cut along k, us on their halves): even numbers of tiles
+SLIM_TIMES = [(1536, 1024, 11.1, 8.8), (1536, 4096, 27.8, 22.1), (1792, 2048, 17.4, 14.1), (1792, 4608, 30.7, 24.8), (1792, 6144, 39.7, 33.0),
+              (512, 8192, 22.9, 33.9), (1024, 8192, 24.9, 35.5), (1536, 5120, 27.5, 29.8), (1536, 6144, 30.0, 32.2), (1536, 8192, 33.7, 38.0), (1664, 7680, 37.7, 40.5),
+              (1792, 8128, 42.1, 43.8), (1920, 9216, 47.1, 48.1), (1792, 16384, 65.3, 70.3)]
+
+
+@pytest.mark.parametrize("M,K,whole,halves", SLIM_TIMES)
+def test_halves_of_tiles_are_taken_where_they_measured_faster(routes, M, K, whole, halves):
+    T = M // 128
+    assert bool(routes.slim_pays(T * (T + 1) // 2, K // 64)) == (halves < whole)
 
 
 # (M, K, us in place, us behind a copy of X): rows that 16-byte copies can take and that lie on no lines
