@@ -2062,14 +2062,6 @@ static bool half_schedule_chosen(long long half_items, long long tiles, int nk, 
   return estimate_half_round(half_items, nk, grid) < estimate_whole_round(tiles, nk, auto_ksplit(tiles, nk, grid), grid);
 }
 
-// The tiles left over after full rounds, at most half as many as CUs: a round of parts of them along k, which go to memory, and a second
-// kernel that adds them (33 us beside the stages), or a launch of their halves behind the rounds (21: it waits for the slowest XCD).  us, parts / halves:
-// X X^T 6656 x 1024 (95 tiles left) 78.5 / 64.0, 5888 x 2048 96 / 92; five steps on 8 of 3072^2 4446 / 4258, on 32 of 2048^2 5571 / 5405, on 24 of 2048 x 5504 6797 / 6593; but
-// on 8 of 4096 x 11008 (64 left, 64 stages) 13853 / 13988.
-static bool half_tail_pays(int rem, int split, int nk, int grid) {
-  return estimate_half_round(2LL * rem, nk, grid) + 8.0 < 0.95 * ((nk / split) * 1.3 + 33.0);
-}
-
 // Few tiles (at most a sixteenth of the workgroups) can also run as 64x64 sub-tiles over the whole
 // k, 16 workgroups per tile, the way the tiles left after the last full round do: one launch, no
 // fp32 parts, and sixteen times the workgroups of whole tiles.  A sub-tile stage moves four times
@@ -2258,8 +2250,7 @@ int launch_gemm_fast(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) 
     if (f.epoch != 0)
       f.tickets = reinterpret_cast<unsigned long long*>(static_cast<unsigned char*>(ws) + (ws_bytes / kTicketBytes - 1) * kTicketBytes);
   }
-  // Tiles left over that would be cut along k: as half tiles in a launch behind the full rounds instead, where that is estimated to be
-  // shorter (no fp32 parts through memory and no second kernel to add them).
+  // Tiles left over that would be cut along k: as half tiles in a launch behind the full rounds instead (half_tail_pays)
   FastArgs tail;
   const bool halves = !f.half && f.rounds > 0 && f.ksplit == 1 && f.split > 1 && 2 * f.rem <= grid && knob(kKnobHalf) < 0 && knob(kKnobKsplit) < 0 &&
                       half_tail_pays(f.rem, f.split, f.nk, grid);

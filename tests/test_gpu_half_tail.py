@@ -1,4 +1,4 @@
-"""Tiles left over after full rounds of 256-tiles that run as halves in a launch of their own: exact on integers against int64, and
+"""Tiles left over after full rounds of 256-tiles that run as halves in a launch of their own: exact on integers, and
 the bits of the other schedules but for the order of their sums."""
 import pytest
 import torch
@@ -15,19 +15,27 @@ def _ints(rows, cols, dtype, seed):
     return torch.randint(-2, 3, (rows, cols), generator=gen, device=DEV).to(dtype)
 
 
-# 20, 44, 95 and 122 tiles left of a symmetric product, diagonal ones among them; 1, 5 and 33 stages of 64
-@pytest.mark.parametrize("M", [5888, 6144, 6656, 6912])
-@pytest.mark.parametrize("K,dtype", [(64, torch.bfloat16), (320, torch.float16), (2112, torch.bfloat16)])
+# 20, 44, 69, 95 and 122 tiles left of a symmetric product, diagonal ones among them; 2, 5, 16 and 33 stages of 64
+HALVES = [(M, K, dtype) for M in (5888, 6144, 6400, 6656, 6912)
+          for K, dtype in [(128, torch.bfloat16), (320, torch.float16), (1024, torch.bfloat16), (2112, torch.bfloat16)] if (M, K) != (5888, 2112)]
+# one stage, which cannot be cut along k; and what is cut
+OTHERS = [(M, 64, torch.bfloat16) for M in (5888, 6144, 6656, 6912)] + [(5888, 2112, torch.bfloat16)]
+
+
+@pytest.mark.parametrize("M,K,dtype", HALVES + OTHERS)
 def test_symmetric_products_exact(M, K, dtype):
     X = _ints(M, K, dtype, M + K)
     Y = matmul_transpose(X)
     assert torch.equal(Y, Y.T)
-    want = X.float() @ X.float().T          # integers below 2^24: exact in any order
+    want = X.float() @ X.float().T          # integers below 2^24: exact in fp32, in any order
     assert torch.equal(Y, want.to(dtype))
 
 
-# 17 and 104 tiles left of a product with an operand E and a transposed output
-@pytest.mark.parametrize("M,K", [(3328, 5376), (2304, 10240)])
+# 20 and 104 tiles left of a product with an operand E and a transposed output, as halves; 17, cut along k
+AXPBY_HALVES = [(512, 35328), (2304, 10240)]
+
+
+@pytest.mark.parametrize("M,K", AXPBY_HALVES + [(3328, 5376)])
 def test_axpby_exact(lib, M, K):
     P, X = _ints(M, M, torch.bfloat16, 1), _ints(M, K, torch.bfloat16, 2)
     Xo, XoT = gemm_axpby(lib, P, X, 3.0)

@@ -5,6 +5,8 @@ import subprocess
 
 import pytest
 
+import test_gpu_half_tail as half_tail
+
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "flash_muon_amd", "csrc")
 INT32_MAX = 2 ** 31 - 1
 
@@ -18,6 +20,7 @@ int syrk_copy_pays(int M, int K, int half) { return fm::syrk_copy_pays(M, K, hal
 int scale_cast_d_on_tiles(long long r, long long c) { return fm::scale_cast_d_on_tiles(r, c); }
 int scale_cast_t_on_128(long long tiles) { return fm::scale_cast_t_on_128(tiles); }
 int ns_flow_chosen(int batch, int m, int k) { return fm::ns_flow_chosen(batch, m, k); }
+int half_tail_pays(int rem, int split, int nk) { return fm::half_tail_pays(rem, split, nk, 256); }
 int slim_pays(int tiles, int nk) { return fm::slim_pays(tiles, nk, 256, fm::mid_parts(tiles, nk, 256), false); }
 void ns_flow_launch(int steps, int i, int* out) { const fm::NsFlowLaunch n = fm::ns_flow_launch(steps, i); out[0] = n.first; out[1] = n.steps; out[2] = n.from; out[3] = n.turn; }
 int ns_flow_slots() { return fm::kFlowSteps + 1; }
@@ -123,6 +126,32 @@ WHOLE_TIMES = [(128, 2048, 14.7, 12.0), (128, 65536, 34.5, 28.6), (384, 32768, 2
 @pytest.mark.parametrize("M,K,apart,in_place", WHOLE_TIMES)
 def test_odd_numbers_of_whole_tiles_are_multiplied_in_place_where_it_measured_faster(routes, M, K, apart, in_place):
     assert bool(routes.syrk_whole_in_place(M, K)) == (in_place < apart)
+
+
+# (M, K, us with the 256-tiles left over cut along k, us with their halves in a launch of their own)
+TAIL_TIMES = [(5888, 256, 40.9, 33.0), (5888, 1024, 63.3, 54.7), (6144, 256, 45.2, 34.1), (6144, 2048, 91.5, 86.4), (6400, 1024, 69.5, 57.2), (6400, 4096, 155.8, 148.5),
+              (6400, 6144, 198.0, 207.0), (6400, 7168, 238.6, 241.6), (6656, 1024, 73.2, 58.0), (6656, 4096, 168.0, 151.4), (6656, 8192, 292.5, 276.0),
+              (6912, 256, 54.6, 35.3), (6912, 4096, 173.6, 156.5)]
+
+
+def _takes_halves(routes, tiles, nk):
+    rem = tiles % 256
+    return tiles >= 256 and 16 < rem <= 128 and nk > 1 and bool(routes.half_tail_pays(rem, min(256 // rem, nk, 16), nk))
+
+
+@pytest.mark.parametrize("M,K,cut,halves", TAIL_TIMES)
+def test_left_over_tiles_run_as_halves_where_it_measured_faster(routes, M, K, cut, halves):
+    T = M // 256
+    assert _takes_halves(routes, T * (T + 1) // 2, K // 64) == (halves < cut)
+
+
+def test_what_the_gpu_tests_of_halves_run_on(routes):
+    for M, K, _ in half_tail.HALVES:
+        assert _takes_halves(routes, (M // 256) * (M // 256 + 1) // 2, K // 64), (M, K)
+    for M, K, _ in half_tail.OTHERS:
+        assert not _takes_halves(routes, (M // 256) * (M // 256 + 1) // 2, K // 64), (M, K)
+    for M, K in half_tail.AXPBY_HALVES:
+        assert _takes_halves(routes, (M // 256) * (K // 256), M // 64), (M, K)
 
 
 # (M, K, us on whole 128-tiles or tiles cut along k, us on their halves): even numbers of tiles
