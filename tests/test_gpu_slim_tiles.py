@@ -1,10 +1,12 @@
 """Halves of 128x128 tiles, at most one a CU: exact on integers for every write-out it has, diagonal tiles as two items and as one, 1 to 40
-stages (around the six of its ring), batches, and an operand E."""
+stages (around the six of its ring), and an operand E; batches of all three products of a Newton-Schulz step."""
 import pytest
 import torch
 
 from flash_muon_amd import matmul_transpose
+from flash_muon_amd.muon import NS_EPS
 from gpu_util import gemm_axpby, syrk_poly
+from test_gpu_ns_long import _library_call, _one_by_one
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -59,3 +61,20 @@ def test_axpby_exact(lib, M, K, x, xt):
     want = ((3.0 + ra)[:, None] * X.float() + P.float() @ X.float()).bfloat16()
     assert not x or torch.equal(Xo, want)
     assert not xt or torch.equal(XoT, want.T)
+
+
+# A and P of 4 matrices of 8 tile rows and 2 of 11: 256 and 242 items, a diagonal tile as one; of 3 of 7: 168, as two; X' of 2 of 5 x 12: 240
+@pytest.mark.parametrize("batch,M,K", [(4, 1024, 2816), (2, 1408, 2816), (3, 896, 1792), (2, 640, 1536)])
+@pytest.mark.parametrize("tall", [False, True])
+def test_batches(batch, M, K, tall):
+    """One step, in launches per product, of matrices that differ: each against the same roundings in fp32, whose sums have another order (that turns
+    less than one rounding in a hundred, by a unit of 2^-8 at most: 8e-4 on the root mean square); and of equal ones, whose bits are equal."""
+    Gs = [torch.randn(M, K, generator=torch.Generator(device=DEV).manual_seed(i), device=DEV).bfloat16() for i in range(batch)]
+    put = (lambda G: G.T.contiguous()) if tall else (lambda G: G)
+    for G, out in zip(Gs, _library_call([put(G) for G in Gs], 1)):
+        X = G.float()
+        want = _one_by_one(X / (X.norm() + NS_EPS), 1, (3.4445, -4.7750, 2.0315))
+        got = (out.T if tall else out).float()
+        assert float((got - want).norm() / want.norm()) < 8e-4
+    outs = _library_call([put(Gs[-1])] * batch, 1)
+    assert all(torch.equal(outs[0], o) for o in outs) and torch.equal(outs[0], _library_call([put(G) for G in Gs], 1)[-1])
