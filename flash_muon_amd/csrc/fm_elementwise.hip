@@ -512,14 +512,9 @@ int launch_momentum_nesterov_batched(void* const* g, void* const* buf, int batch
 // just rounded, in the partition and order of sumsq_partial_kernel: the same bits), which spares a pass over them.
 // Bound by the memory; the two kernels, this one: 12 fp32 tensors of 3072 x 768 75 + 20 us, 81 (5.6 TB/s); 24 of 768^2 38 + 12, 43; 32 bf16
 // ones of 2048^2 168 + 80, 186.
-//   keep: what is orthogonalised is stored through the caches, for the scaled cast behind this kernel, where both tensors as they are written
-// fit into the 256 MB memory-side cache (kKeptBytes of each).  Muon.step, us, never / so: 12 layers of 768 in fp32 (113 MB of 3072 x 768) 1973 / 1941, 6 of
-// 1536 in bf16 (113 MB) 4445 / 4395, 3 of 1280 in fp32 1725 / 1708; but 8 of 1024 in fp32 (134 MB) 2308 / 2331.  Larger batches in
-// pieces of that size, momentum and cast by turns, lose more by the launches than they gain: 12 of 2048 in bf16 15850 / 15936.
-constexpr int64_t kKeptBytes = 120ll << 20;
 template <int DT>
 __global__ __launch_bounds__(256) void momentum_sumsq_kernel(PtrList gl, PtrList bl, int64_t nv, float w_buf, float w_nes, int nesterov,
-                                                             int keep, float* partials, unsigned* zero, int n_zero) {
+                                                             float* partials, unsigned* zero, int n_zero) {
   typedef typename Elem<DT>::raw raw;
   constexpr int V = 16 / sizeof(raw);
   __shared__ float red[4];
@@ -533,12 +528,8 @@ __global__ __launch_bounds__(256) void momentum_sumsq_kernel(PtrList gl, PtrList
   auto update = [&](int64_t i, Unit& ug, Unit& ub) {
 #pragma unroll
     for (int e = 0; e < V; ++e) momentum_one<DT>(ug.e[e], ub.e[e], w_buf, w_nes, nesterov);
-    if (keep && !nesterov) b4[i] = ub.v;
-    else st_stream(b4 + i, ub.v);
-    if (nesterov) {
-      if (keep) g4[i] = ug.v;
-      else st_stream(g4 + i, ug.v);
-    }
+    st_stream(b4 + i, ub.v);
+    if (nesterov) st_stream(g4 + i, ug.v);
     add_squares<DT>(s4, nesterov ? ug.e : ub.e);
   };
   int64_t i = i0 + threadIdx.x;
@@ -568,10 +559,9 @@ bool launch_momentum_sumsq_batched(void* const* g, void* const* buf, int batch, 
     gl.p[i] = g[i]; bl.p[i] = buf[i];
     if ((reinterpret_cast<uintptr_t>(g[i]) & 15) || (reinterpret_cast<uintptr_t>(buf[i]) & 15)) return false;
   }
-  const int keep = (int64_t)batch * n * (16 / V) <= kKeptBytes;
   dim3 grid((unsigned)sumsq_parts(n), (unsigned)batch), block(256);
 #define FM_MOMENTUM_SUMSQ(DT) hipLaunchKernelGGL(momentum_sumsq_kernel<DT>, grid, block, 0, stream, gl, bl, n / V, w_buf, w_nes, nesterov, \
-                                                 keep, partials, zero, n_zero)
+                                                 partials, zero, n_zero)
   if (dtype == 0) FM_MOMENTUM_SUMSQ(0);
   else if (dtype == 1) FM_MOMENTUM_SUMSQ(1);
   else FM_MOMENTUM_SUMSQ(2);

@@ -2117,8 +2117,7 @@ bool gemm_fast_eligible(const GemmArgs& a) {
 
 bool gemm_mid_eligible(const GemmArgs& a) { return tiled_dma_eligible(a, MID_T); }
 
-// (with up to one tile per CU the deeper ring of gemm_nt_mid_kernel is as fast or faster: 2048^2 19.2 us, 20.2 in pairs)
-// what gemm_nt_pair_kernel asks for besides: E through its transpose
+// what gemm_nt_pair_kernel and fm_gemm_slim.hip ask for besides: E through its transpose
 static bool pair_eligible(const GemmArgs& a) {
   return !a.E || (a.ET && a.ldet % 8 == 0 && a.ldet < (1 << 21) && (reinterpret_cast<uintptr_t>(a.ET) & 15) == 0 && (a.batch < 2 || a.bs_et % 8 == 0));
 }
@@ -2145,6 +2144,7 @@ int launch_gemm_mid(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) {
   // without room for the parts the tiles stay whole
   if (sp.ksplit > 1 && (!ws || (size_t)a.num_tiles * sp.ksplit * MID_PART_FLOATS * sizeof(float) > ws_bytes)) sp.ksplit = 1;
   const unsigned grid = (unsigned)(a.num_tiles * sp.ksplit);
+  // (with up to one tile per CU the deeper ring of gemm_nt_mid_kernel is as fast or faster: 2048^2 19.2 us, 20.2 in pairs)
   if (sp.ksplit == 1 && a.num_tiles > cu_count() && pair_eligible(a)) {
     if (a.elem == kElemF16) hipLaunchKernelGGL(gemm_nt_pair_kernel<true>, dim3(grid), dim3(256), 0, stream, a);
     else hipLaunchKernelGGL(gemm_nt_pair_kernel<false>, dim3(grid), dim3(256), 0, stream, a);

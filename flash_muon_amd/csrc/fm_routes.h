@@ -246,8 +246,8 @@ inline bool syrk_whole_in_place(int M, int K, int cus) {
 // or a launch of their halves behind the rounds.  What the halves gain, fitted to X X^T of 23 to 27 tile rows (us): 7 and 0.105 a tile for the
 // parts' way through memory and the second kernel, and a stage of a part (1.3 / split) against one of a half (0.3 to 0.7, by the CUs they fill).
 //   20 left (5888 rows) K 1024 63.3 / 54.7; 44 (6144) K 1024 65.4 / 56.3, 2048 91.5 / 86.4; 69 (6400) K 1024 69.5 / 57.2, 4096 155.8 / 148.5, but 6144 198 / 207, 7168
-// 239 / 242; 95 (6656) K 1024 73.2 / 58.0, 4096 168 / 151, 8192 292 / 275; 122 (6912) K 256 54.6 / 35.3, 4096 173.5 / 156.5; 32 of 2048^2, five Newton-Schulz steps
-// (128 left) 5900 / 5580.
+// 239 / 242; 95 (6656) K 1024 73.2 / 58.0, 4096 168 / 151, 8192 292 / 275; 122 (6912) K 256 54.6 / 35.3, 4096 173.5 / 156.5; five Newton-Schulz steps on 32 of 2048^2
+// (128 left) 5600 / 5450, on 8 of 3072^2 (112) 4440 / 4270.
 inline bool half_tail_pays(int rem, int split, int nk, int grid) {
   const double fill = 0.3 + 0.6 * 2.0 * rem / grid, half = fill < 0.7 ? fill : 0.7;
   return 7.0 + 0.105 * rem + nk * (1.3 / split - half) > 2.0;

@@ -38,7 +38,7 @@ def _fused(lib, gs, bufs, outs, nesterov, ws, steps=5):
 @pytest.mark.parametrize("batch,rows,cols,dtype,offset", [
     (3, 64, 100, torch.float32, 0), (2, 33, 77, torch.bfloat16, 0), (2, 96, 128, torch.float32, 1), (5, 300, 200, torch.float16, 0),
     (2, 1600, 700, torch.bfloat16, 0), (1, 1544, 1600, torch.float32, 0), (1, 2304, 2048, torch.bfloat16, 0), (2, 200, 12000, torch.float32, 0),
-    (30, 1024, 1024, torch.float32, 0), (31, 1024, 1024, torch.float32, 0)])   # 120 MiB, which the caches keep for the cast, and more
+    (30, 1024, 1024, torch.float32, 0), (31, 1024, 1024, torch.float32, 0)])   # 120 MiB and more
 @pytest.mark.parametrize("nesterov", [1, 0])
 def test_same_bits_as_the_two_calls(lib, batch, rows, cols, dtype, offset, nesterov):
     gs = _tensors(batch, rows, cols, dtype, 1e-2, 1, offset)
