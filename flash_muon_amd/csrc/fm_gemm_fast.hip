@@ -928,8 +928,9 @@ struct FastArgs {
   // Sub-tiles handed out in the order the workgroups arrive (below), or nullptr: sub-tile w to workgroup w.
   unsigned long long* tickets;
   unsigned long long epoch;   // this launch's number (48 bits, never 0)
-  int half;             // the items are 128x256 half tiles, never cut (the NI == 2 kernels)
-  int tail_tile0;       // >= 0: the halves of the tiles from this one on, two items each (the second of a diagonal tile is none)
+  // 1: the items are 128x256 half tiles, never cut (the NI == 2 kernels); 2 + t: those of the tiles from t on, two items each (the
+  // second of a diagonal tile is none)
+  int half;
 };
 
 // k stages [kb, ke) of base part `part` of `parts`, or of its sub-part `sub` of `subs`
@@ -1582,8 +1583,8 @@ __global__ __launch_bounds__(256) void gemm_nt_rounds_kernel(FastArgs p) {
     int bi, ti, tj, half = 0;
     bool ditem = false;   // NI == 2: a whole diagonal tile of a symmetric product
     if constexpr (NI == 2) {
-      if (p.tail_tile0 >= 0) {
-        tile_at(p.g, p.tail_tile0 + (item >> 1), bi, ti, tj);
+      if (p.half > 1) {
+        tile_at(p.g, p.half - 2 + (item >> 1), bi, ti, tj);
         half = item & 1;
         ditem = p.g.symmetric && ti == tj;
         if (ditem && half) continue;
@@ -2204,7 +2205,6 @@ int launch_gemm_fast(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) 
   const long long have = (long long)(slot_bytes / (PART_FLOATS * sizeof(float)));
   fast_schedule(a.num_tiles, f.nk, have < kMaxSlots ? have : kMaxSlots, f);
   f.half = 0;
-  f.tail_tile0 = -1;
   int grid = cu_count() < kMaxGrid ? cu_count() : kMaxGrid;
   const long long kg = knob(kKnobGrid);
   if (kg > 0 && kg < grid) grid = (int)kg;
@@ -2256,8 +2256,7 @@ int launch_gemm_fast(GemmArgs a, void* ws, size_t ws_bytes, hipStream_t stream) 
                       half_tail_pays(f.rem, f.split, f.nk, grid);
   if (halves) {
     tail = f;
-    tail.half = 1;
-    tail.tail_tile0 = f.rounds * f.grid;
+    tail.half = 2 + f.rounds * f.grid;
     tail.grid = 2 * f.rem;
     tail.rounds = 1;
     tail.rem = 0;
