@@ -236,3 +236,18 @@ def test_five_blocks_of_a_scaled_tile_fit_a_cu(elementwise):
         if m and "scale_cast_tile128_kernel" in kernel:
             sizes[kernel] = int(m.group(1))
     assert len(sizes) == 12 and all(5 * n <= 160 * 1024 for n in sizes.values()), sizes
+
+
+def test_the_momentum_kernel_streams_its_momenta_and_keeps_what_is_cast_next(elementwise):
+    """Two stores of different kinds in branches of one `if` become one of the plain kind: the unit's three pairs of stores are told apart in
+    the code as built (with nesterov the momentum streamed and G plain, without it the momentum streamed)."""
+    kernel, stores = None, {}
+    for line in elementwise:
+        m = re.match(r"^(_Z\w+):", line)
+        if m:
+            kernel = m.group(1) if "momentum_sumsq_kernel" in m.group(1) else None
+        if kernel and line.strip().startswith("global_store_dwordx4"):
+            stores.setdefault(kernel, []).append(" nt" in line)
+    assert len(stores) == 3
+    for name, nt in stores.items():
+        assert nt.count(False) == 3 and nt.count(True) >= 3, (name, nt)
