@@ -268,7 +268,7 @@ def _extras(Xd, steps, warmup, torch):
         diff = (params[i].detach().float() - q.detach().float())
         rel = float(diff.norm() / moved.norm())
         ex["muon_step_llama7b_%s_vs_one_per_launch_rel_fro" % name] = rel
-        assert rel < 0.1, "Muon.step at 32 per launch and at 1 per launch moved a %s parameter differently: %g" % (name, rel)
+        assert rel < 6e-3, "Muon.step at 32 per launch and at 1 per launch moved a %s parameter differently: %g" % (name, rel)
         assert torch.equal(q.grad, params[i].grad), "momentum / Nesterov state differs"
         if i == last_sq:   # the orthogonalised update itself, as the last step left it in the group's buffer
             ub = [g["update_buffer"][0] for g in opt.param_groups if g["params"][-1] is params[i]]

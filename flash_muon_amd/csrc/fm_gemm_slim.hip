@@ -4,8 +4,8 @@
 // Bound by the rate at which a CU copies into its LDS (some 90 KB/us, whatever the others do): 24 KiB per 64-wide k stage, 0.27 us,
 // where a 128x128 tile takes 0.36 for its 32; the waves' 32x64 blocks read 48 KiB of fragments a stage beside that, and their 16
 // MFMAs a stage are a quarter of the time.  So the ring is as deep as the LDS allows, six stages with five on their way.
-// us, 128x128 tiles / this: X X^T 1536 x 2048 17.4 / 14.1, 1792 x 4096 28.4 / 23.3, 2048^2 17.8 / 15.6, 2048 x 4096 28.2 / 24.8; five Newton-Schulz steps
-// on 6400 x 1600 422 / 383, 1536^2 257 / 230, 1408 x 5632 346 / 302, 2 of 1024 x 4096 314 / 262.
+// us, 128x128 tiles / this: X X^T 1536 x 2048 17.1 / 13.7, 1792 x 4096 27.9 / 22.5, 2048^2 17.8 / 15.1, 2048 x 4096 28.4 / 24.3; five Newton-Schulz steps
+// on 6400 x 1600 518 / 506, 1536^2 254 / 231, 2048^2 317 / 290, 2 of 1024 x 4096 335 / 297, 4 of 768 x 3072 327 / 295.
 #include "fm_routes.h"
 #include "fm_tile128.h"
 
